@@ -4,6 +4,7 @@
 // calls from different threads never touch common mutable state -- but for the cache of device
 // allocations below, which is behind a mutex.
 #include "../../include/galvatron_dp_hip.h"
+#include "gdp_bounds.h"
 #include "gdp_kernels.h"
 #include "gdp_host.h"
 
@@ -15,6 +16,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <condition_variable>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <string>
@@ -674,7 +676,8 @@ int gdp_validate_f0(const gdp_problem *p, int i, bool *f0_live)
     return gdp_fail(what == 2 ? GDP_E_BADARG : GDP_E_NONFINITE, buf);
 }
 
-int gdp_validate(const gdp_problem *p, int i)
+// *magnitude: sum over the layers of the largest finite magnitudes of the cost arrays.
+static int validate_costs(const gdp_problem *p, int i, double *magnitude)
 {
     char buf[160];
     auto bad = [&](int code, const char *why) {
@@ -736,7 +739,14 @@ int gdp_validate(const gdp_problem *p, int i)
         if (p->other_mem[k] < 0) return bad(GDP_E_BADARG, "negative other_mem entry (start row above the table)");
     }
     if (!(bound < COST_BOUND)) return bad(GDP_E_NONFINITE, "cost magnitudes could overflow binary64");
+    *magnitude = bound;
     return GDP_OK;
+}
+
+int gdp_validate(const gdp_problem *p, int i)
+{
+    double magnitude = 0;
+    return validate_costs(p, i, &magnitude);
 }
 
 namespace {
@@ -2439,12 +2449,361 @@ void gdp_cache_trim(void)
     lane_trim();
 }
 
+// ---- smaller instances in place of whole ones ------------------------------------------------------
+// Strategies that no best path can use are taken out of an instance before its DP runs (why that changes no result:
+// gdp_bounds.hip).  What stays is an instance of its own for the launch schemes above: fewer strategies (padded to
+// a multiple of 4 with ones that cost +inf), the budget lowered by the memory that every choice needs and capped
+// where it stops to bind.
+struct Reduced {
+    gdp_problem q = {};
+    gdp_result r = {};
+    std::vector<int32_t> mem, res, remaining;
+    std::vector<double> intra, inter, total;
+    std::vector<int64_t> other_mem, spare;   // per key: budget beyond the cap
+    std::vector<int32_t> kept;               // [L][S of q] strategy of the whole instance, -1: padding
+};
+
+// Dense relaxations of a batch from which on the bounds are worth their launches (GALVATRON_DP_REDUCE=1 takes them for
+// every instance that has the form, =0 for none).  They take 0.08 (L = 32, S = 44) to 0.2 ms (L = 80, S = 64) and a round
+// trip; per call, whole / reduced: L = 28, S = 40, V = 29493 (1.3e9) 0.30 / 0.32 ms; L = 32, S = 44, V = 65536 (4e9)
+// 0.67 / 0.43 ms, but 0.67 / 0.74 ms where the caller's array of initial costs comes from memory and not from a
+// cache: looking through it is hidden behind the device's work, and less of that is left; L = 80, S = 64,
+// V = 131072 (4.3e10) 3.06 / 0.96 ms; L = 48, S = 88, V = 262144 (9.7e10) 10.8 / 4.5 ms; 256 instances of S = 44 49 / 7.8 ms.
+static constexpr double REDUCE_MIN_WORK = 6e9;
+static constexpr size_t REDUCE_MAX_BYTES = (size_t)4 << 30;   // of device memory for the tables of the passes
+
+static bool reducible(const gdp_problem *q, double magnitude)
+{
+    constexpr uint32_t whole = GDP_EXPORT_F | GDP_EXPORT_MARK | GDP_COMPUTE_ALL | GDP_KEEP_MARKS | GDP_LAUNCH_FUSED | GDP_LAUNCH_PER_LAYER;
+    if ((q->flags & whole) || q->L < 2 || q->L > GDP_BOUND_MAX_L || q->S < 2 || q->S > GDP_BOUND_MAX_S ||
+        q->n_key < 1 || q->n_key > GDP_BOUND_MAX_KEY || q->L * q->S > GDP_BOUND_MAX_LS || !(magnitude < 1e100))
+        return false;
+    // a memory cost of 0 reads the layer's own row: the recurrence is not a path through the layers then
+    for (size_t k = 0; k < (size_t)q->L * q->S; ++k)
+        if (q->mem[k] == 0) return false;
+    return true;
+}
+
+// The multipliers of an instance: 0 and a geometric series around (range of times) / (range of memory costs).
+static void multipliers(const gdp_problem *q, int n_lam, double *lam)
+{
+    double t0 = INFINITY, t1 = -INFINITY, m0 = INFINITY, m1 = 0;
+    for (size_t k = 0; k < (size_t)q->L * q->S; ++k) {
+        if (q->mem[k] >= q->V || !(q->intra[k] < INFINITY)) continue;
+        t0 = std::min(t0, q->intra[k]);
+        t1 = std::max(t1, q->intra[k]);
+        m0 = std::min(m0, (double)q->mem[k]);
+        m1 = std::max(m1, (double)q->mem[k]);
+    }
+    const double range = t1 > t0 ? t1 - t0 : 1.0, base = range / std::max(1.0, m1 - m0);
+    lam[0] = 0.0;
+    for (int i = 1; i < n_lam; ++i) lam[i] = base * std::exp2(-6.0 + 12.0 * (i - 1) / (n_lam - 2));
+}
+
+// The smaller instance of q, given what stays ([L][S]); false where it would not be a good deal smaller.
+static bool build_reduced(const gdp_problem *q, const HostInst &h, const uint8_t *keep, const int64_t *budget, Reduced &d)
+{
+    const int L = q->L, S = q->S;
+    int most = 0;
+    int64_t base = 0, span = 0;   // memory that every path needs beyond 1 per layer, and what a path can need on top
+    std::vector<int32_t> low((size_t)L);
+    std::vector<int> count((size_t)L);
+    for (int l = 0; l < L; ++l) {
+        int n = 0, lo = INT32_MAX, hi = 0;
+        for (int s = 0; s < S; ++s) {
+            if (!keep[(size_t)l * S + s]) continue;
+            const int32_t m = q->mem[(size_t)l * S + s];
+            if (m >= q->V) return false;   // (cannot be: its bound is +inf)
+            ++n;
+            lo = std::min(lo, m);
+            hi = std::max(hi, m);
+        }
+        if (n == 0) return false;
+        most = std::max(most, n);
+        count[(size_t)l] = n;
+        low[(size_t)l] = lo;
+        base += lo - 1;
+        span += hi - lo + 1;
+    }
+    const int R = (most + 3) / 4 * 4;
+    int64_t top = 0;
+    for (int k = 0; k < q->n_key; ++k)
+        if (budget[k] >= 0) top = std::max(top, std::min(budget[k] - base, span));
+    if (top < 1) return false;
+    const int64_t V = top + 1;
+    if ((double)R * R * (double)V > 0.5 * (double)S * S * (double)q->V) return false;
+    d.q.L = L;
+    d.q.S = R;
+    d.q.V = (int32_t)V;
+    d.q.n_inter = L;
+    d.q.n_key = q->n_key;
+    d.q.other_time = q->other_time;
+    d.q.flags = q->flags;
+    d.kept.assign((size_t)L * R, -1);
+    d.mem.resize((size_t)L * R);
+    d.intra.assign((size_t)L * R, INFINITY);
+    d.inter.assign((size_t)L * R * R, 0.0);
+    for (int l = 0; l < L; ++l) {
+        int32_t *kept = d.kept.data() + (size_t)l * R;
+        int n = 0;
+        for (int s = 0; s < S; ++s)
+            if (keep[(size_t)l * S + s]) kept[n++] = s;
+        const double *M = h.matrix_at(q, h.matrix(q, l));
+        double *to = d.inter.data() + (size_t)l * R * R;
+        for (int j = 0; j < R; ++j) {
+            const int s = kept[std::min(j, n - 1)];
+            d.mem[(size_t)l * R + j] = q->mem[(size_t)l * S + s] - low[(size_t)l] + 1;
+            if (j >= n) continue;
+            d.intra[(size_t)l * R + j] = q->intra[(size_t)l * S + s];
+            if (l == 0) {   // the zeros before the first layer are reached from every strategy: its cheapest transition
+                double c = INFINITY;
+                for (int sp = 0; sp < S; ++sp) c = std::min(c, 0.0 + M[(size_t)sp * S + s]);
+                for (int i = 0; i < R; ++i) to[(size_t)i * R + j] = c;
+            } else {
+                const int32_t *from = d.kept.data() + (size_t)(l - 1) * R;
+                for (int i = 0; i < count[(size_t)l - 1]; ++i) to[(size_t)i * R + j] = M[(size_t)from[i] * S + s];
+            }
+        }
+    }
+    d.other_mem.resize((size_t)q->n_key);
+    d.spare.assign((size_t)q->n_key, 0);
+    for (int k = 0; k < q->n_key; ++k) {
+        const int64_t left = budget[k] < 0 ? -1 : budget[k] - base;
+        const int64_t v0 = std::min(left, top);
+        d.spare[(size_t)k] = left - v0;
+        d.other_mem[(size_t)k] = v0 < 0 ? V : V - 1 - v0;   // V: infeasible, as before
+    }
+    d.total.assign((size_t)q->n_key, 0.0);
+    d.remaining.assign((size_t)q->n_key, 0);
+    d.res.assign((size_t)q->n_key * L, -1);
+    d.q.mem = d.mem.data();
+    d.q.intra = d.intra.data();
+    d.q.inter = d.inter.data();
+    d.q.other_mem = d.other_mem.data();
+    d.r.total = d.total.data();
+    d.r.remaining = d.remaining.data();
+    d.r.res = d.res.data();
+    return true;
+}
+
+// Bounds of the instances of a batch that have the form, all in one set of launches, and the smaller instances that
+// follow (out[i] stays empty where instance i is solved whole).  Initial costs are taken to be zeros.
+static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vector<double> &magnitude,
+                        std::vector<std::unique_ptr<Reduced>> &out)
+{
+    const char *env = getenv("GALVATRON_DP_REDUCE"), *skip = getenv("GALVATRON_DP_SKIP");
+    const bool forced = env && *env && atoi(env) != 0;
+    if ((env && *env && !forced) || (skip && *skip && atoi(skip) == 0)) return GDP_OK;
+    double total = 0;
+    for (int i = 0; i < n; ++i) total += (double)p[i]->L * p[i]->V * (double)p[i]->S * p[i]->S;
+    if (!forced && total < REDUCE_MIN_WORK) return GDP_OK;
+
+    struct Entry {
+        int orig, table_of;   // table_of: the entry whose matrices this one reads
+        HostInst h;
+        std::vector<int64_t> budget;
+        size_t off_mem, off_intra, off_inter, off_index, off_lam, off_budget, off_inter_t, off_P, off_Q, off_time, off_pmem, off_path, off_ub, off_keep;
+    };
+    std::vector<Entry> es;
+    std::vector<int2> pairs;
+    size_t at = 0;
+    auto place = [&](size_t bytes) { const size_t o = at; at = align_up(at + bytes, 256); return o; };
+    for (int i = 0; i < n; ++i) {
+        if (!reducible(p[i], magnitude[(size_t)i])) continue;
+        const gdp_problem *q = p[i];
+        Entry e;
+        e.orig = i;
+        e.table_of = (int)es.size();
+        int64_t least = 0;
+        for (int l = 0; l < q->L; ++l) least += *std::min_element(q->mem + (size_t)l * q->S, q->mem + (size_t)(l + 1) * q->S);
+        bool any = false;
+        for (int k = 0; k < q->n_key; ++k) {
+            const int64_t b = (int64_t)q->V - 1 - q->other_mem[k];
+            e.budget.push_back(b >= least ? b : -1);
+            any = any || b >= least;
+        }
+        if (!any) continue;
+        e.h.S = q->S;
+        e.h.n_inter = q->inter_index ? q->n_inter : q->L;
+        if (!q->inter_index) share_equal_matrices(q, e.h);
+        for (size_t j = es.size(); q->inter_index && j-- > 0;) {   // the stages of one fit, the tasks of one sweep
+            const gdp_problem *o = p[es[j].orig];
+            if (o->inter_index && o->inter == q->inter && o->S == q->S && o->n_inter == q->n_inter) {
+                e.table_of = es[j].table_of;
+                break;
+            }
+            if (es.size() - j >= 8) break;
+        }
+        es.push_back(std::move(e));
+    }
+    if (es.empty()) return GDP_OK;
+    const int m = (int)es.size(), n_lam = m <= 4 ? GDP_BOUND_MAX_LAM : GDP_BOUND_MAX_LAM / 2;
+    int max_LS = 0, max_S = 0, max_K = 0, elements = 1;
+    // what is uploaded, what is copied back, what stays on the device
+    const size_t off_inst = place(sizeof(GdpBoundInst) * (size_t)m);
+    for (int j = 0; j < m; ++j) {
+        Entry &e = es[(size_t)j];
+        const gdp_problem *q = p[e.orig];
+        const size_t LS = (size_t)q->L * q->S;
+        e.off_mem = place(4 * LS);
+        e.off_intra = place(8 * LS);
+        e.off_index = place(4 * (size_t)q->L);
+        e.off_lam = place(8 * (size_t)n_lam);
+        e.off_budget = place(8 * (size_t)q->n_key);
+        if (e.table_of == j) {
+            e.off_inter = place(8 * (size_t)e.h.n_inter * q->S * q->S);
+            for (int t = 0; t < e.h.n_inter; ++t) pairs.push_back(make_int2(j, t));
+        }
+        max_LS = std::max(max_LS, (int)LS);
+        max_S = std::max(max_S, q->S);
+        max_K = std::max(max_K, q->n_key);
+        elements = std::max(elements, gdp_bound_elements(q->S));
+    }
+    const size_t off_pairs = place(sizeof(int2) * pairs.size());
+    const size_t up_bytes = at;
+    for (Entry &e : es) {
+        const gdp_problem *q = p[e.orig];
+        e.off_ub = place(8 * (size_t)q->n_key);
+        e.off_keep = place((size_t)q->L * q->S);
+    }
+    const size_t back_bytes = at - up_bytes;
+    for (int j = 0; j < m; ++j) {
+        Entry &e = es[(size_t)j];
+        const gdp_problem *q = p[e.orig];
+        const size_t LS = (size_t)q->L * q->S;
+        if (e.table_of == j) e.off_inter_t = place(8 * (size_t)e.h.n_inter * q->S * q->S);
+        e.off_P = place(8 * LS * (size_t)n_lam);
+        e.off_Q = place(8 * LS * (size_t)n_lam);
+        e.off_time = place(8 * (size_t)n_lam);
+        e.off_pmem = place(8 * (size_t)n_lam);
+        e.off_path = place((size_t)q->L * (size_t)n_lam);
+    }
+    if (at > REDUCE_MAX_BYTES || m > 65535) return GDP_OK;
+
+    int device = 0;
+    GDP_HIP(hipGetDevice(&device));
+    Lane lane;
+    char *dev = nullptr;
+    size_t dev_bytes = 0;
+    GDP_HIP(lane_take(device, back_bytes, up_bytes, &lane));
+    hipError_t err = arena_take(device, at, &dev, &dev_bytes);
+    if (err != hipSuccess) {
+        (void)hipGetLastError();
+        lane_give(lane);
+        return GDP_OK;   // a device this full solves the instances whole, in the parts that fit
+    }
+    std::vector<char> pageable;
+    char *up = lane.up;
+    try {
+        if (lane.up_bytes < up_bytes) {
+            pageable.resize(up_bytes);
+            up = pageable.data();
+        }
+    } catch (const std::bad_alloc &) {
+        arena_give(device, dev, dev_bytes);
+        lane_give(lane);
+        throw;
+    }
+    for (int j = 0; j < m; ++j) {
+        Entry &e = es[(size_t)j];
+        const Entry &te = es[(size_t)e.table_of];
+        const gdp_problem *q = p[e.orig];
+        const size_t LS = (size_t)q->L * q->S, SS = (size_t)q->S * q->S;
+        memcpy(up + e.off_mem, q->mem, 4 * LS);
+        memcpy(up + e.off_intra, q->intra, 8 * LS);
+        for (int l = 0; l < q->L; ++l) reinterpret_cast<int32_t *>(up + e.off_index)[l] = e.h.matrix(q, l);
+        multipliers(q, n_lam, reinterpret_cast<double *>(up + e.off_lam));
+        memcpy(up + e.off_budget, e.budget.data(), 8 * e.budget.size());
+        if (e.table_of == j)
+            for (int t = 0; t < e.h.n_inter; ++t) memcpy(up + e.off_inter + 8 * SS * (size_t)t, e.h.matrix_at(q, t), 8 * SS);
+        GdpBoundInst b;
+        b.mem = reinterpret_cast<const int32_t *>(dev + e.off_mem);
+        b.intra = reinterpret_cast<const double *>(dev + e.off_intra);
+        b.inter = reinterpret_cast<const double *>(dev + te.off_inter);
+        b.inter_t = reinterpret_cast<const double *>(dev + te.off_inter_t);
+        b.index = reinterpret_cast<const int32_t *>(dev + e.off_index);
+        b.lam = reinterpret_cast<const double *>(dev + e.off_lam);
+        b.budget = reinterpret_cast<const int64_t *>(dev + e.off_budget);
+        b.P = reinterpret_cast<double *>(dev + e.off_P);
+        b.Q = reinterpret_cast<double *>(dev + e.off_Q);
+        b.path_time = reinterpret_cast<double *>(dev + e.off_time);
+        b.path_mem = reinterpret_cast<int64_t *>(dev + e.off_pmem);
+        b.path = reinterpret_cast<uint8_t *>(dev + e.off_path);
+        b.ub = reinterpret_cast<double *>(dev + e.off_ub);
+        b.keep = reinterpret_cast<uint8_t *>(dev + e.off_keep);
+        b.magnitude = magnitude[(size_t)e.orig];
+        b.L = q->L;
+        b.V = q->V;
+        b.S = q->S;
+        b.K = q->n_key;
+        memcpy(up + off_inst + sizeof b * (size_t)j, &b, sizeof b);
+    }
+    memcpy(up + off_pairs, pairs.data(), sizeof(int2) * pairs.size());
+    bool stats = false;
+    {
+        std::lock_guard<std::mutex> lk(g_stats_mu);
+        stats = g_stats_on;
+    }
+    err = hipMemcpyAsync(dev, up, up_bytes, hipMemcpyHostToDevice, lane.stream);
+    if (err == hipSuccess && stats) err = hipEventRecord(lane.ev_begin, lane.stream);
+    if (err == hipSuccess)
+        err = gdp_launch_bounds(reinterpret_cast<const GdpBoundInst *>(dev + off_inst), m, n_lam, max_LS, max_S, max_K, elements,
+                                reinterpret_cast<const int2 *>(dev + off_pairs), (int)pairs.size(), lane.stream);
+    if (err == hipSuccess && stats) err = hipEventRecord(lane.ev_end, lane.stream);
+    if (err == hipSuccess) err = hipMemcpyAsync(lane.back, dev + up_bytes, back_bytes, hipMemcpyDeviceToHost, lane.stream);
+    const hipError_t es2 = hipStreamSynchronize(lane.stream);
+    if (err == hipSuccess) err = es2;
+    float ms = 0;
+    if (err == hipSuccess && stats) err = hipEventElapsedTime(&ms, lane.ev_begin, lane.ev_end);
+    if (stats) {
+        std::lock_guard<std::mutex> lk(g_stats_mu);
+        g_stats.device_ms += ms;
+    }
+    arena_give(device, dev, dev_bytes);
+    int rc = err == hipSuccess ? GDP_OK : fail_hip(err, "bounds");
+    try {
+        for (int j = 0; j < m && rc == GDP_OK; ++j) {
+            const Entry &e = es[(size_t)j];
+            const gdp_problem *q = p[e.orig];
+            const double *ub = reinterpret_cast<const double *>(lane.back + (e.off_ub - up_bytes));
+            bool bounded = true;   // a key whose budget no path was found for keeps everything
+            for (int k = 0; k < q->n_key; ++k) bounded = bounded && (e.budget[(size_t)k] < 0 || ub[k] < INFINITY);
+            if (!bounded) continue;
+            std::unique_ptr<Reduced> d(new Reduced());
+            if (build_reduced(q, e.h, reinterpret_cast<const uint8_t *>(lane.back + (e.off_keep - up_bytes)), e.budget.data(), *d))
+                out[(size_t)e.orig] = std::move(d);
+        }
+    } catch (const std::bad_alloc &) {
+        lane_give(lane);
+        throw;
+    }
+    lane_give(lane);
+    return rc;
+}
+
+// The results of a smaller instance in the terms of the whole one.
+static int expand_result(const gdp_problem *q, const Reduced &d, gdp_result *out)
+{
+    if (!out) return fail(GDP_E_BADARG, "null result");
+    if (!out->total || !out->remaining || !out->res) return fail(GDP_E_BADARG, "null result array");
+    for (int k = 0; k < q->n_key; ++k) {
+        out->total[k] = d.total[(size_t)k];
+        out->remaining[k] = d.remaining[(size_t)k];
+        if (d.remaining[(size_t)k] == -1) continue;
+        out->remaining[k] += (int32_t)d.spare[(size_t)k];
+        for (int l = 0; l < q->L; ++l)
+            out->res[(size_t)k * q->L + l] = d.kept[(size_t)l * d.q.S + d.res[(size_t)k * q->L + l]];
+    }
+    return GDP_OK;
+}
+
 // The parts of gdp_solve_batch.  f0_live: per problem, whether its initial costs are to be uploaded.
 // scan_f0_late: the initial costs have not been looked at yet -- the batch is one part, and they are looked
 // through while the device works on it; *f0_found says afterwards whether any hold more than zeros (or are
-// refused: then the return code says so), in which case nothing has been written to the results.
+// refused: then the return code says so), in which case nothing has been written to the results.  whole: the
+// caller's problems, where p holds smaller ones in place of some of them.
 static int solve_parts(int32_t n, const gdp_problem *const *p, gdp_result *const *r, size_t budget, std::vector<char> &f0_live,
-                       bool scan_f0_late, bool *f0_found)
+                       bool scan_f0_late, const gdp_problem *const *whole, bool *f0_found)
 {
     int begin = 0, prev_begin = 0;
     gdp_plan *prev = nullptr;
@@ -2508,7 +2867,7 @@ static int solve_parts(int32_t n, const gdp_problem *const *p, gdp_result *const
     }
     int rs = GDP_OK;
     if (scan_f0_late) {
-        rs = validate_f0_all(n, p, f0_live);
+        rs = validate_f0_all(n, whole, f0_live);
         for (char c : f0_live) *f0_found = *f0_found || c != 0;
     }
     int rc = finish(prev);
@@ -2524,33 +2883,61 @@ int gdp_solve_batch(int32_t n, const gdp_problem *const *p, gdp_result *const *r
     if (!r) return fail(GDP_E_BADARG, "null results");
     if (n < 1 || !p) return fail(GDP_E_BADARG, "need at least one problem");
     bool any_f0 = false;
-    for (int i = 0; i < n; ++i) {  // all of them first: nothing is written when one is rejected
-        const int rc = gdp_validate(p[i], i);
-        if (rc != GDP_OK) return rc;
-        any_f0 = any_f0 || p[i]->f0 != nullptr;
-    }
-    // A batch whose cost buffers would take more than GALVATRON_DP_ARENA_MB (default 8192) of device
-    // memory is solved in consecutive parts that reuse one allocation: the time to obtain device
-    // memory grows with its size, the time to solve a part does not grow faster than its share.
-    const size_t budget = std::max<size_t>(env_mb("GALVATRON_DP_ARENA_MB", 8192), (size_t)1 << 20);
     try {
+        std::vector<double> magnitude((size_t)n, 0.0);
+        for (int i = 0; i < n; ++i) {  // all of them first: nothing is written when one is rejected
+            const int rc = validate_costs(p[i], i, &magnitude[(size_t)i]);
+            if (rc != GDP_OK) return rc;
+            any_f0 = any_f0 || p[i]->f0 != nullptr;
+        }
+        // A batch whose cost buffers would take more than GALVATRON_DP_ARENA_MB (default 8192) of device
+        // memory is solved in consecutive parts that reuse one allocation: the time to obtain device
+        // memory grows with its size, the time to solve a part does not grow faster than its share.
+        const size_t budget = std::max<size_t>(env_mb("GALVATRON_DP_ARENA_MB", 8192), (size_t)1 << 20);
         std::vector<char> f0_live((size_t)n, 0);
+        std::vector<std::unique_ptr<Reduced>> small((size_t)n);
+        int rc = reduce_batch(n, p, magnitude, small);
+        if (rc != GDP_OK) return rc;
+        std::vector<const gdp_problem *> q(p, p + n);
+        std::vector<gdp_result *> qr(r, r + n);
+        for (int i = 0; i < n; ++i)
+            if (small[(size_t)i]) {
+                q[(size_t)i] = &small[(size_t)i]->q;
+                qr[(size_t)i] = &small[(size_t)i]->r;
+            }
         // Initial costs (gdp_problem.f0) are zeros in every call the reference's own code makes, and looking
         // through V x S doubles takes as long as solving a small instance.  A batch of one part is therefore
         // started as if they were zeros and the arrays are looked through while the device works; should one
-        // of them hold anything else, that solve is dropped and the batch solved again with them.
+        // of them hold anything else, that solve is dropped and the batch solved again with them, whole.
         size_t bytes = 0;
-        for (int i = 0; i < n && bytes <= budget; ++i) bytes += footprint(p[i]);
+        for (int i = 0; i < n && bytes <= budget; ++i) bytes += footprint(q[(size_t)i]);
         const bool late = any_f0 && n <= 65535 && bytes <= budget;
         if (any_f0 && !late) {
-            const int rc = validate_f0_all(n, p, f0_live);
+            rc = validate_f0_all(n, p, f0_live);
             if (rc != GDP_OK) return rc;
+            for (int i = 0; i < n; ++i)
+                if (f0_live[(size_t)i]) {
+                    small[(size_t)i].reset();
+                    q[(size_t)i] = p[i];
+                    qr[(size_t)i] = r[i];
+                }
         }
         bool f0_found = false;
-        int rc = solve_parts(n, p, r, budget, f0_live, late, &f0_found);
+        rc = solve_parts(n, q.data(), qr.data(), budget, f0_live, late, p, &f0_found);
         if (rc == GDP_OK && f0_found) {
             f0_found = false;
-            rc = solve_parts(n, p, r, budget, f0_live, false, &f0_found);
+            return solve_parts(n, p, r, budget, f0_live, false, p, &f0_found);
+        }
+        double left_out = 0;
+        for (int i = 0; i < n && rc == GDP_OK; ++i)
+            if (small[(size_t)i]) {
+                rc = expand_result(p[i], *small[(size_t)i], r[i]);
+                const gdp_problem &d = small[(size_t)i]->q;
+                left_out += (double)p[i]->L * (double)p[i]->V * p[i]->S * p[i]->S - (double)d.L * (double)d.V * d.S * d.S;
+            }
+        if (rc == GDP_OK && left_out > 0) {   // statistics count the relaxations of the whole instances
+            std::lock_guard<std::mutex> lk(g_stats_mu);
+            if (g_stats_on) g_stats.relaxations += left_out;
         }
         return rc;
     } catch (const std::bad_alloc &) {

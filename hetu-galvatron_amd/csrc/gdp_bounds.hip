@@ -1,0 +1,301 @@
+// Lower bounds per (layer, strategy), so that the DP runs over the strategies that can matter only.
+//
+// For a multiplier lam >= 0 per bin of memory the budget can be priced instead of counted: with costs
+// intra + lam * mem the cheapest path through the layers is a plain min-plus product of L vectors and matrices,
+// S*S operations per layer instead of V*S*S.  P[l][s] is the cheapest way from the first layer to (l, s), both ends
+// included, Q[l][s] the cheapest way on from there; every path that uses (l, s) and fits the budget B takes at least
+//     P[l][s] + Q[l][s] - lam * B
+// of time.  Any path that fits gives an upper bound U on the optimum.  Where the lower bound exceeds U (by more than
+// the rounding of both) no optimal path of that budget uses (l, s), and no path that ties with one does: the DP
+// without (l, s) has the same value in every cell of an optimal path -- a cheaper way into such a cell through
+// (l, s) would be a path below U -- and values elsewhere can only be larger, so that no candidate ties that did not
+// tie before.  The optimum, its strategies (ties to the lowest index: the order of what stays is kept) and what is
+// left of the budget are those of the whole instance, bit for bit.
+//
+// The bounds are loose by what the last layers before the budget waste, a fraction of one layer, while most
+// strategies lose more than that against the best ones: of 64 strategies 2 to 5 per layer stay (random costs), of 40
+// of a layer that is repeated 28 times some 13.
+#include "gdp_bounds.h"
+
+#include <math.h>
+
+namespace {
+
+__device__ __forceinline__ double lagrangian(int32_t mem, double intra, double lam, int V)
+{
+    return mem < V && intra < INFINITY ? intra + lam * (double)mem : (double)INFINITY;
+}
+
+// inter_t: grid (pairs, 16-row bands of the largest matrix), 256 threads; LDS turns the band around so that both
+// sides are read and written along rows.
+__global__ __launch_bounds__(256) void gdp_bound_transpose_kernel(const GdpBoundInst *inst, const int2 *pairs)
+{
+    __shared__ double tile[16][GDP_BOUND_MAX_S + 1];
+    const int2 w = pairs[blockIdx.x];
+    const GdpBoundInst &I = inst[w.x];
+    const int S = I.S, r0 = (int)blockIdx.y * 16;
+    if (r0 >= S) return;
+    const int rows = S - r0 < 16 ? S - r0 : 16;
+    const double *src = I.inter + (size_t)w.y * S * S;
+    double *dst = const_cast<double *>(I.inter_t) + (size_t)w.y * S * S;
+    for (int e = threadIdx.x; e < rows * S; e += 256) tile[e / S][e % S] = src[(size_t)r0 * S + e];
+    __syncthreads();
+    for (int e = threadIdx.x; e < rows * S; e += 256) {
+        const int c = e / rows, r = e % rows;
+        dst[(size_t)c * S + r0 + r] = tile[r][c];
+    }
+}
+
+// One pass over the layers of one instance under one multiplier: forwards (P, the path and its cost) or backwards
+// (Q).  grid (2 * multipliers, instances): the serial chain of L steps is what takes the time, so everything that
+// does not depend on it runs side by side -- multipliers and directions in workgroups of their own, a step's S*S
+// candidates on up to 1024 threads (thread = target strategy + S * part, its sources part, part + G, ...: loads run
+// along the rows), and the matrix of the next step is on its way to registers while this one is reduced.
+template <int E>
+__global__ __launch_bounds__(GDP_BOUND_THREADS) void gdp_bound_pass_kernel(const GdpBoundInst *inst)
+{
+    extern __shared__ uint8_t arg_of[];   // [L][S], forwards only
+    __shared__ double X[GDP_BOUND_MAX_S], part_v[GDP_BOUND_THREADS];
+    __shared__ uint8_t part_i[GDP_BOUND_THREADS];
+    __shared__ int32_t mat[GDP_BOUND_MAX_L];
+    __shared__ uint8_t path[GDP_BOUND_MAX_L];
+    const GdpBoundInst &I = inst[blockIdx.y];
+    const int L = I.L, S = I.S, V = I.V, t = (int)threadIdx.x, li = (int)blockIdx.x >> 1;
+    const bool back = blockIdx.x & 1u;
+    const double lam = I.lam[li];
+    const int G = min(GDP_BOUND_THREADS / S, GDP_BOUND_PARTS), s = t % S, g = t / S;
+    const bool active = g < G;
+    const size_t SS = (size_t)S * S;
+    for (int l = t; l < L; l += GDP_BOUND_THREADS) mat[l] = I.index[l];
+    if (t < S) X[t] = 0.0;
+    __syncthreads();
+    const double *tables = back ? I.inter_t : I.inter;
+    double *out = (back ? I.Q : I.P) + (size_t)li * L * S;
+
+    double m_now[E], m_next[E], c_now = 0.0, c_next = 0.0;
+    auto fetch = [&](int l, double (&m)[E], double &c) {
+        const double *M = tables + (size_t)mat[l] * SS;
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+            const int sp = g + k * G;
+            m[k] = active && sp < S ? M[(size_t)sp * S + s] : (double)INFINITY;
+        }
+        if (t < S) c = lagrangian(I.mem[(size_t)l * S + t], I.intra[(size_t)l * S + t], lam, V);
+    };
+    const int first = back ? L - 1 : 0, step = back ? -1 : 1;
+    fetch(first, m_now, c_now);
+    for (int i = 0, l = first; i < L; ++i, l += step) {
+        if (i + 1 < L) fetch(l + step, m_next, c_next);
+        if (back) {
+            // X is Q[l]; what lies before layer l sees the cost of (l, s) on top of it
+            if (t < S) {
+                out[(size_t)l * S + t] = X[t];
+                X[t] += c_now;
+            }
+            if (l == 0) break;
+            __syncthreads();
+        }
+        double best = INFINITY;
+        int arg = 0;
+        if (active) {
+#pragma unroll
+            for (int k = 0; k < E; ++k) {
+                const int sp = g + k * G;
+                if (sp < S) {
+                    const double v = X[sp] + m_now[k];
+                    if (v < best) { best = v; arg = sp; }
+                }
+            }
+            part_v[t] = best;
+            part_i[t] = (uint8_t)arg;
+        }
+        __syncthreads();
+        if (t < S) {   // thread t is part 0 of target t
+            for (int p = 1; p < G; ++p)
+                if (part_v[p * S + t] < best) { best = part_v[p * S + t]; arg = part_i[p * S + t]; }
+            if (back) {
+                X[t] = best;
+            } else {
+                X[t] = best + c_now;
+                out[(size_t)l * S + t] = X[t];
+                arg_of[l * S + t] = (uint8_t)arg;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < E; ++k) m_now[k] = m_next[k];
+        c_now = c_next;
+    }
+    if (back) return;
+    if (t == 0) {
+        int b = 0;
+        for (int k = 1; k < S; ++k)
+            if (X[k] < X[b]) b = k;
+        for (int l = L - 1; l >= 0; --l) {
+            path[l] = (uint8_t)b;
+            b = arg_of[l * S + b];
+        }
+    }
+    __syncthreads();
+    // what the path costs: one layer per thread (L <= 512), summed in LDS
+    double time = 0.0, memory = 0.0;
+    if (t < L) {
+        const int b = path[t], a = arg_of[t * S + b];
+        I.path[(size_t)li * L + t] = (uint8_t)b;
+        const int32_t m = I.mem[(size_t)t * S + b];
+        time = tables[(size_t)mat[t] * SS + (size_t)a * S + b] + (m < V ? I.intra[(size_t)t * S + b] : (double)INFINITY);
+        memory = (double)m;   // whole numbers below 2^41: exact
+    }
+    part_v[t] = time;
+    __syncthreads();
+    for (int w = GDP_BOUND_THREADS / 2; w > 0; w >>= 1) {
+        if (t < w) part_v[t] += part_v[t + w];
+        __syncthreads();
+    }
+    if (t == 0) I.path_time[li] = part_v[0];
+    __syncthreads();
+    part_v[t] = memory;
+    __syncthreads();
+    for (int w = GDP_BOUND_THREADS / 2; w > 0; w >>= 1) {
+        if (t < w) part_v[t] += part_v[t + w];
+        __syncthreads();
+    }
+    if (t == 0) I.path_mem[li] = (int64_t)part_v[0];
+}
+
+// Upper bound of one key: the best of the multipliers' paths that fit, and of the paths that follow one of the
+// last paths that do not fit up to some layer and the first one that does from there on (or the other way round) --
+// where all layers are alike every layer changes its strategy at the same multiplier, and only such a
+// splice comes near the budget.  grid (keys, instances), 256 threads; a candidate per thread from running sums.
+__global__ __launch_bounds__(256) void gdp_bound_upper_kernel(const GdpBoundInst *inst, int n_lam)
+{
+    __shared__ double pt[GDP_BOUND_LOW + 1][GDP_BOUND_MAX_L + 1], pm[GDP_BOUND_LOW + 1][GDP_BOUND_MAX_L + 1];
+    __shared__ uint8_t st[GDP_BOUND_LOW + 1][GDP_BOUND_MAX_L];
+    __shared__ double red[256];
+    __shared__ int which[GDP_BOUND_LOW + 1];
+    const GdpBoundInst &I = inst[blockIdx.y];
+    const int key = (int)blockIdx.x, t = (int)threadIdx.x, L = I.L, S = I.S;
+    if (key >= I.K) return;
+    const int64_t B = I.budget[key];
+    const size_t SS = (size_t)S * S;
+    double best = INFINITY;
+    if (t < n_lam && I.path_mem[t] <= B && I.path_time[t] < INFINITY) best = I.path_time[t];
+    if (t == 0) {
+        int fit = -1, low = 0;
+        for (int q = 0; q <= GDP_BOUND_LOW; ++q) which[q] = -1;
+        for (int i = 0; i < n_lam && fit < 0; ++i)
+            if (I.path_mem[i] <= B && I.path_time[i] < INFINITY) fit = i;
+        which[0] = fit;
+        for (int i = fit - 1; i >= 0 && low < GDP_BOUND_LOW; --i)
+            if (I.path_time[i] < INFINITY) which[1 + low++] = i;
+    }
+    __syncthreads();
+    if (which[0] >= 0 && which[1] >= 0) {   // the same in every thread
+        for (int e = t; e < (GDP_BOUND_LOW + 1) * L; e += 256) {
+            const int q = e / L, l = e % L;
+            if (which[q] < 0) continue;
+            const uint8_t *p = I.path + (size_t)which[q] * L;
+            const int b = p[l];
+            st[q][l] = (uint8_t)b;
+            // the first layer comes from whatever strategy is cheapest: P under lam[0] = 0 is that plus its own cost
+            const double x = l == 0 ? I.P[b]
+                                    : I.inter[(size_t)I.index[l] * SS + (size_t)p[l - 1] * S + b] + I.intra[(size_t)l * S + b];
+            pt[q][l + 1] = x;
+            pm[q][l + 1] = (double)I.mem[(size_t)l * S + b];
+        }
+        __syncthreads();
+        if (t <= GDP_BOUND_LOW && which[t] >= 0) {
+            pt[t][0] = pm[t][0] = 0.0;
+            for (int l = 1; l <= L; ++l) {
+                pt[t][l] += pt[t][l - 1];
+                pm[t][l] += pm[t][l - 1];
+            }
+        }
+        __syncthreads();
+        for (int e = t; e < 2 * GDP_BOUND_LOW * (L - 1); e += 256) {
+            const int c = 1 + e % (L - 1), d = e / (L - 1), q = 1 + (d >> 1);
+            if (which[q] < 0) continue;
+            const int a = d & 1 ? 0 : q, b = d & 1 ? q : 0;   // a up to layer c, then b
+            if (pm[a][c] + (pm[b][L] - pm[b][c]) > (double)B) continue;
+            const double *M = I.inter + (size_t)I.index[c] * SS;
+            const double turn = M[(size_t)st[a][c - 1] * S + st[b][c]], was = M[(size_t)st[b][c - 1] * S + st[b][c]];
+            const double x = pt[a][c] + (pt[b][L] - pt[b][c]) + (turn - was);
+            if (x < best) best = x;
+        }
+    }
+    red[t] = best;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if (t < w && red[t + w] < red[t]) red[t] = red[t + w];
+        __syncthreads();
+    }
+    if (t == 0) I.ub[key] = red[0];
+}
+
+// What stays: (l, s) is out when for every key some multiplier's bound lies above that key's upper bound.  The
+// margin covers the rounding of the bound, of the upper bound and of the DP's own sums: each is a sum of at most
+// 4 L + 4 terms whose magnitudes add up to no more than `magnitude` + lam * (L + 1) * V.
+// grid (64-element groups of the largest table, instances), one wave per workgroup.
+__global__ __launch_bounds__(64) void gdp_bound_keep_kernel(const GdpBoundInst *inst, int n_lam)
+{
+    const GdpBoundInst &I = inst[blockIdx.y];
+    const int e = (int)(blockIdx.x * 64 + threadIdx.x), LS = I.L * I.S;
+    if (e >= LS) return;
+    unsigned alive = 0;
+    double ub[GDP_BOUND_MAX_KEY], budget[GDP_BOUND_MAX_KEY];
+#pragma unroll
+    for (int k = 0; k < GDP_BOUND_MAX_KEY; ++k) {
+        ub[k] = INFINITY;
+        budget[k] = 0.0;
+        if (k < I.K && I.budget[k] >= 0) {
+            alive |= 1u << k;
+            ub[k] = I.ub[k];
+            budget[k] = (double)I.budget[k];
+        }
+    }
+    const double ulp = 16.0 * (double)(I.L + 4) * 0x1p-53;
+#pragma unroll 4
+    for (int i = 0; i < n_lam; ++i) {
+        const double lam = I.lam[i];
+        const double r = I.P[(size_t)i * LS + e] + I.Q[(size_t)i * LS + e];
+        const double margin = ulp * (I.magnitude + lam * (double)(I.L + 1) * (double)I.V);
+#pragma unroll
+        for (int k = 0; k < GDP_BOUND_MAX_KEY; ++k)
+            if (r - lam * budget[k] > ub[k] + margin) alive &= ~(1u << k);
+    }
+    I.keep[e] = alive != 0;
+}
+
+}  // namespace
+
+int gdp_bound_elements(int S)
+{
+    const int G = GDP_BOUND_THREADS / S < GDP_BOUND_PARTS ? GDP_BOUND_THREADS / S : GDP_BOUND_PARTS;
+    for (int e = 1; e < 16; e *= 2)
+        if (e * G >= S) return e;
+    return 16;   // S <= 128: G >= 8
+}
+
+hipError_t gdp_launch_bounds(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K,
+                             int elements, const int2 *pairs, int n_pairs, hipStream_t stream)
+{
+    gdp_bound_transpose_kernel<<<dim3((unsigned)n_pairs, (unsigned)((max_S + 15) / 16)), 256, 0, stream>>>(inst, pairs);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const dim3 grid(2u * (unsigned)n_lam, (unsigned)n);
+    const size_t lds = (size_t)max_LS;
+    switch (elements) {
+    case 1: gdp_bound_pass_kernel<1><<<grid, GDP_BOUND_THREADS, lds, stream>>>(inst); break;
+    case 2: gdp_bound_pass_kernel<2><<<grid, GDP_BOUND_THREADS, lds, stream>>>(inst); break;
+    case 4: gdp_bound_pass_kernel<4><<<grid, GDP_BOUND_THREADS, lds, stream>>>(inst); break;
+    case 8: gdp_bound_pass_kernel<8><<<grid, GDP_BOUND_THREADS, lds, stream>>>(inst); break;
+    default: gdp_bound_pass_kernel<16><<<grid, GDP_BOUND_THREADS, lds, stream>>>(inst); break;
+    }
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    gdp_bound_upper_kernel<<<dim3((unsigned)max_K, (unsigned)n), 256, 0, stream>>>(inst, n_lam);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    gdp_bound_keep_kernel<<<dim3((unsigned)((max_LS + 63) / 64), (unsigned)n), 64, 0, stream>>>(inst, n_lam);
+    return hipGetLastError();
+}

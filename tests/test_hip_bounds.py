@@ -1,0 +1,105 @@
+"""Instances whose strategies are thinned out by bounds before the DP: results against the C oracle, which sees the
+whole instance.  The bounds take part in every instance of the form here (``GALVATRON_DP_REDUCE=1``; by default
+only from a certain amount of work on)."""
+import numpy as np
+import pytest
+
+import helpers as H
+from galvatron_dp import _lib, workloads as W
+from oracle import dp_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# L, S, V: two layers and the most; strategies around the parts of a pass (32, 33, 64, 65), elements per thread 1 to
+# 16 (89 and 128 need 16) and the largest; budgets from a few bins on
+SHAPES = [(2, 2, 40), (2, 128, 300), (3, 5, 64), (5, 31, 400), (4, 32, 333), (6, 33, 500), (4, 44, 1000), (3, 64, 700),
+          (7, 65, 512), (5, 88, 900), (4, 89, 600), (12, 9, 3000), (40, 6, 4001), (24, 22, 2500), (512, 3, 2600)]
+
+
+def _instance(rng, L, S, V, kind):
+    per = max(2, V // L)
+    same = kind in ("same", "ties_same")
+    n = 1 if same else L
+    mem = rng.integers(max(1, per // 4), 3 * per + 1, size=(n, S)).astype(np.int32)
+    if kind.startswith("ties"):
+        intra, inter = rng.integers(1, 5, size=(n, S)).astype(float), rng.integers(0, 3, size=(n, S, S)).astype(float)
+        mem = (mem // 4 + 1).astype(np.int32)
+    else:
+        intra, inter = rng.lognormal(2.5, 0.5, size=(n, S)), rng.uniform(0, 5, size=(n, S, S))
+    if kind == "negative":
+        intra, inter = intra - 20.0, inter - 2.5
+    if kind == "holes":
+        intra[rng.uniform(size=intra.shape) < 0.2] = np.inf
+        inter[rng.uniform(size=inter.shape) < 0.2] = np.inf
+        mem[rng.uniform(size=mem.shape) < 0.2] = V + 3
+        intra[:, 0], mem[:, 0] = 10.0, max(1, per // 2)
+        inter[:, 0, 0] = 0.0
+    if kind == "loose":
+        mem = np.minimum(mem, max(1, per // 2)).astype(np.int32)
+    if n == 1:
+        mem, intra, inter = np.repeat(mem, L, 0), np.repeat(intra, L, 0), np.repeat(inter, L, 0)
+    # a key with the whole budget, tighter ones, one without a solution, one below the table
+    om = {1: 0, 2: V // 10, 4: V // 4, 8: V - 2, 16: V + 5}
+    ot = {k: float(k) / 3 for k in om}
+    return mem, intra, inter, om, ot
+
+
+def _problem(x, V):
+    mem, intra, inter, om, ot = x
+    keys = sorted(om)
+    return _lib.Problem(mem, intra, inter, V, [om[k] for k in keys], [ot[k] for k in keys])
+
+
+def _check(x, V, prob, tag):
+    mem, intra, inter, om, ot = x
+    keys = sorted(om)
+    got = ({k: prob.total[i] for i, k in enumerate(keys)}, {k: [int(v) for v in prob.res[i]] for i, k in enumerate(keys)},
+           {k: int(prob.remaining[i]) for i, k in enumerate(keys)})
+    wt, wr, wm = O.solve(mem, intra, inter, V, om, ot)[:3]
+    H.assert_same_results(got, (wt, wr, wm), tag)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_reduced_instances_against_oracle(shape, monkeypatch):
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    L, S, V = shape
+    for n, kind in enumerate(["each", "same", "ties", "ties_same", "negative", "holes", "loose"]):
+        x = _instance(np.random.Generator(np.random.PCG64([5, L, S, n])), L, S, V, kind)
+        prob = _problem(x, V)
+        _lib.solve_batch([prob])
+        _check(x, V, prob, f"{shape} {kind}")
+
+
+def test_batch_of_different_shapes_and_shared_tables(monkeypatch):
+    """One set of launches over instances of different sizes, some of them without the form (a memory cost of 0), some
+    of them with the same matrices."""
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    rng = np.random.Generator(np.random.PCG64(99))
+    xs, probs = [], []
+    for n, (L, S, V) in enumerate(SHAPES[:12]):
+        x = _instance(rng, L, S, V, ["each", "ties", "same"][n % 3])
+        if n == 5:
+            x[0][1, 1] = 0
+        xs.append((x, V))
+        probs.append(_problem(x, V))
+    tables = rng.uniform(0, 4, size=(2, 20, 20))
+    for L in (4, 7, 9):
+        mem, intra, _, om, ot = _instance(rng, L, 20, 800, "each")
+        index = (np.arange(L) % 2).astype(np.int32)
+        x = (mem, intra, tables[index], om, ot)
+        keys = sorted(om)
+        xs.append((x, 800))
+        probs.append(_lib.Problem(mem, intra, tables, 800, [om[k] for k in keys], [ot[k] for k in keys], inter_index=index))
+    _lib.solve_batch(probs)
+    for n, ((x, V), prob) in enumerate(zip(xs, probs)):
+        _check(x, V, prob, f"instance {n}")
+
+
+def test_initial_costs_that_are_not_zeros(monkeypatch):
+    """The bounds take the initial costs to be zeros; a caller's array with others is solved whole."""
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    rng = np.random.Generator(np.random.PCG64(3))
+    inst = W.with_initial_costs(W.random_instance(rng, 6, 12, 700, mem_hi=200), rng)
+    got = H.hip_solve(inst)
+    want = O.solve(inst.mem, inst.intra, inst.inter, inst.V, inst.other_mem, inst.other_time, f0=inst.f0)[:3]
+    H.assert_same_results(got, want)
