@@ -20,6 +20,8 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <unordered_map>
 #include <vector>
 
@@ -656,6 +658,82 @@ static int scan_f0(const gdp_problem *p, bool *live, double *maxabs)
     *maxabs = m;
     return 0;
 }
+
+namespace {
+
+// Looks through the initial costs of a batch for anything but zeros, on threads beside the one that prepares and
+// waits for the device: one thread reads 20 GB/s from memory, so the 184 MB of a call with S = 88, V = 262144 took 4.5 ms
+// of its own once the device needed less, and the 23 MB of S = 44, V = 65536 0.6 ms.  The arrays are cut into
+// pieces that the threads draw from a counter; the caller helps with what is left when it needs the answer, so a
+// thread that could not be had only costs time.  One thread per 4 MB, at most 7 and what the machine has, from 16 MB
+// on: starting one takes some 30 us, and the 9 MB of S = 40, V = 29493 are looked through behind the device's work
+// (0.30 ms per call without threads, 0.37 with two).  Per call, one thread / with helpers: S = 88, V = 262144
+// 4.5 / 1.1 ms, S = 44, V = 65536 0.74 / 0.41 ms.
+class InitialScan {
+public:
+    void start(int32_t n, const gdp_problem *const *p)
+    {
+        size_t bytes = 0;
+        for (int i = 0; i < n; ++i) {
+            if (!p[i]->f0) continue;
+            const size_t words = (size_t)p[i]->V * (size_t)p[i]->S;
+            for (size_t k = 0; k < words; k += PIECE) pieces_.push_back({p[i]->f0 + k, std::min(PIECE, words - k)});
+            bytes += 8 * words;
+        }
+        const size_t cores = std::max(1u, std::thread::hardware_concurrency());
+        const size_t want = bytes < HELPED_FROM ? 0 : std::min({bytes >> 22, cores - 1, (size_t)7});
+        helpers_.reserve(want);
+        try {
+            for (size_t k = 0; k < want; ++k) helpers_.emplace_back([this] { work(); });
+        } catch (const std::system_error &) {   // no thread to be had: the caller does what is left
+        }
+    }
+    // true: some array holds more than zeros
+    bool finish()
+    {
+        work();
+        join();
+        return found_.load(std::memory_order_relaxed);
+    }
+    ~InitialScan()
+    {
+        next_.store(pieces_.size(), std::memory_order_relaxed);
+        join();
+    }
+
+private:
+    static constexpr size_t HELPED_FROM = (size_t)16 << 20;
+    static constexpr size_t PIECE = (size_t)1 << 16;   // doubles: half a megabyte
+    struct Piece {
+        const double *at;
+        size_t n;
+    };
+    void work()
+    {
+        while (!found_.load(std::memory_order_relaxed)) {
+            const size_t k = next_.fetch_add(1, std::memory_order_relaxed);
+            if (k >= pieces_.size()) return;
+            uint64_t any = 0;
+            for (size_t j = 0; j < pieces_[k].n; ++j) {
+                uint64_t w;
+                memcpy(&w, pieces_[k].at + j, sizeof w);
+                any |= w;
+            }
+            if (any) found_.store(true, std::memory_order_relaxed);
+        }
+    }
+    void join()
+    {
+        for (std::thread &t : helpers_) t.join();
+        helpers_.clear();
+    }
+    std::vector<Piece> pieces_;
+    std::vector<std::thread> helpers_;
+    std::atomic<size_t> next_{0};
+    std::atomic<bool> found_{false};
+};
+
+}  // namespace
 
 // The magnitudes of the cost arrays may add up to COST_BOUND and those of the initial costs reach it, so that
 // no partial sum can overflow.
@@ -2465,11 +2543,10 @@ struct Reduced {
 
 // Dense relaxations of a batch from which on the bounds are worth their launches (GALVATRON_DP_REDUCE=1 takes them for
 // every instance that has the form, =0 for none).  They take 0.08 (L = 32, S = 44) to 0.2 ms (L = 80, S = 64) and a round
-// trip; per call, whole / reduced: L = 28, S = 40, V = 29493 (1.3e9) 0.30 / 0.32 ms; L = 32, S = 44, V = 65536 (4e9)
-// 0.67 / 0.43 ms, but 0.67 / 0.74 ms where the caller's array of initial costs comes from memory and not from a
-// cache: looking through it is hidden behind the device's work, and less of that is left; L = 80, S = 64,
-// V = 131072 (4.3e10) 3.06 / 0.96 ms; L = 48, S = 88, V = 262144 (9.7e10) 10.8 / 4.5 ms; 256 instances of S = 44 49 / 7.8 ms.
-static constexpr double REDUCE_MIN_WORK = 6e9;
+// trip; per call, whole / reduced: L = 24, S = 22, V = 16384 (1.9e8) 0.16 / 0.27 ms; L = 28, S = 40, V = 29493 (1.3e9)
+// 0.30 / 0.32; L = 32, S = 44, V = 65536 (4e9) 0.67 / 0.41; L = 80, S = 64, V = 131072 (4.3e10) 3.06 / 0.97; L = 48,
+// S = 88, V = 262144 (9.7e10) 10.8 / 1.1; 256 instances of S = 44 49 / 7.8 ms.
+static constexpr double REDUCE_MIN_WORK = 3e9;
 static constexpr size_t REDUCE_MAX_BYTES = (size_t)4 << 30;   // of device memory for the tables of the passes
 
 static bool reducible(const gdp_problem *q, double magnitude)
@@ -2798,12 +2875,11 @@ static int expand_result(const gdp_problem *q, const Reduced &d, gdp_result *out
 }
 
 // The parts of gdp_solve_batch.  f0_live: per problem, whether its initial costs are to be uploaded.
-// scan_f0_late: the initial costs have not been looked at yet -- the batch is one part, and they are looked
-// through while the device works on it; *f0_found says afterwards whether any hold more than zeros (or are
-// refused: then the return code says so), in which case nothing has been written to the results.  whole: the
-// caller's problems, where p holds smaller ones in place of some of them.
+// scan: the initial costs have not been looked through yet -- the batch is one part, and they are while the device
+// works on it; *f0_found says afterwards whether any hold more than zeros, in which case nothing has been written
+// to the results.
 static int solve_parts(int32_t n, const gdp_problem *const *p, gdp_result *const *r, size_t budget, std::vector<char> &f0_live,
-                       bool scan_f0_late, const gdp_problem *const *whole, bool *f0_found)
+                       InitialScan *scan, bool *f0_found)
 {
     int begin = 0, prev_begin = 0;
     gdp_plan *prev = nullptr;
@@ -2865,13 +2941,8 @@ static int solve_parts(int32_t n, const gdp_problem *const *p, gdp_result *const
         prev_begin = begin;
         begin = end;
     }
-    int rs = GDP_OK;
-    if (scan_f0_late) {
-        rs = validate_f0_all(n, whole, f0_live);
-        for (char c : f0_live) *f0_found = *f0_found || c != 0;
-    }
+    if (scan) *f0_found = scan->finish();
     int rc = finish(prev);
-    if (rs != GDP_OK) rc = rs;
     if (rc == GDP_OK && !*f0_found) rc = fetch(prev, r + prev_begin);
     destroy(prev);
     return rc;
@@ -2895,6 +2966,8 @@ int gdp_solve_batch(int32_t n, const gdp_problem *const *p, gdp_result *const *r
         // memory grows with its size, the time to solve a part does not grow faster than its share.
         const size_t budget = std::max<size_t>(env_mb("GALVATRON_DP_ARENA_MB", 8192), (size_t)1 << 20);
         std::vector<char> f0_live((size_t)n, 0);
+        InitialScan scan;
+        if (any_f0) scan.start(n, p);
         std::vector<std::unique_ptr<Reduced>> small((size_t)n);
         int rc = reduce_batch(n, p, magnitude, small);
         if (rc != GDP_OK) return rc;
@@ -2912,21 +2985,12 @@ int gdp_solve_batch(int32_t n, const gdp_problem *const *p, gdp_result *const *r
         size_t bytes = 0;
         for (int i = 0; i < n && bytes <= budget; ++i) bytes += footprint(q[(size_t)i]);
         const bool late = any_f0 && n <= 65535 && bytes <= budget;
-        if (any_f0 && !late) {
-            rc = validate_f0_all(n, p, f0_live);
-            if (rc != GDP_OK) return rc;
-            for (int i = 0; i < n; ++i)
-                if (f0_live[(size_t)i]) {
-                    small[(size_t)i].reset();
-                    q[(size_t)i] = p[i];
-                    qr[(size_t)i] = r[i];
-                }
-        }
-        bool f0_found = false;
-        rc = solve_parts(n, q.data(), qr.data(), budget, f0_live, late, p, &f0_found);
+        bool f0_found = any_f0 && !late && scan.finish();
+        if (!f0_found) rc = solve_parts(n, q.data(), qr.data(), budget, f0_live, late ? &scan : nullptr, &f0_found);
         if (rc == GDP_OK && f0_found) {
+            rc = validate_f0_all(n, p, f0_live);
             f0_found = false;
-            return solve_parts(n, p, r, budget, f0_live, false, p, &f0_found);
+            return rc == GDP_OK ? solve_parts(n, p, r, budget, f0_live, nullptr, &f0_found) : rc;
         }
         double left_out = 0;
         for (int i = 0; i < n && rc == GDP_OK; ++i)
