@@ -2542,7 +2542,7 @@ struct Reduced {
 };
 
 // Dense relaxations of a batch from which on the bounds are worth their launches (GALVATRON_DP_REDUCE=1 takes them for
-// every instance that has the form, =0 for none).  They take 0.08 (L = 32, S = 44) to 0.2 ms (L = 80, S = 64) and a round
+// every instance that has the form, =0 for none).  They take 0.1 (L = 32, S = 44) to 0.2 ms (L = 80, S = 64) and a round
 // trip; per call, whole / reduced: L = 24, S = 22, V = 16384 (1.9e8) 0.16 / 0.27 ms; L = 28, S = 40, V = 29493 (1.3e9)
 // 0.30 / 0.32; L = 32, S = 44, V = 65536 (4e9) 0.67 / 0.41; L = 80, S = 64, V = 131072 (4.3e10) 3.06 / 0.97; L = 48,
 // S = 88, V = 262144 (9.7e10) 10.8 / 1.1; 256 instances of S = 44 49 / 7.8 ms.
@@ -2715,7 +2715,7 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
     }
     if (es.empty()) return GDP_OK;
     const int m = (int)es.size(), n_lam = m <= 4 ? GDP_BOUND_MAX_LAM : GDP_BOUND_MAX_LAM / 2;
-    int max_LS = 0, max_S = 0, max_K = 0, elements = 1;
+    int max_LS = 0, max_S = 0, max_K = 0, elements = 1, narrow = 1;
     // what is uploaded, what is copied back, what stays on the device
     const size_t off_inst = place(sizeof(GdpBoundInst) * (size_t)m);
     for (int j = 0; j < m; ++j) {
@@ -2734,8 +2734,14 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
         max_LS = std::max(max_LS, (int)LS);
         max_S = std::max(max_S, q->S);
         max_K = std::max(max_K, q->n_key);
-        elements = std::max(elements, gdp_bound_elements(q->S));
+        const int half = gdp_bound_elements(q->S, GDP_BOUND_THREADS / 2);
+        elements = std::max(elements, gdp_bound_elements(q->S, GDP_BOUND_THREADS));
+        narrow = narrow && half ? std::max(narrow, half) : 0;
     }
+    // With more passes than the device holds at a time what counts is not the chain of a pass but how many run
+    // side by side: half as many threads and few enough registers for
+    // four passes per compute unit (256 instances of S = 44, L = 32: 1.67 -> 0.65 ms).
+    const int threads = narrow && (int64_t)m * n_lam * 2 > 1024 ? GDP_BOUND_THREADS / 2 : GDP_BOUND_THREADS;
     const size_t off_pairs = place(sizeof(int2) * pairs.size());
     const size_t up_bytes = at;
     for (Entry &e : es) {
@@ -2824,7 +2830,8 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
     err = hipMemcpyAsync(dev, up, up_bytes, hipMemcpyHostToDevice, lane.stream);
     if (err == hipSuccess && stats) err = hipEventRecord(lane.ev_begin, lane.stream);
     if (err == hipSuccess)
-        err = gdp_launch_bounds(reinterpret_cast<const GdpBoundInst *>(dev + off_inst), m, n_lam, max_LS, max_S, max_K, elements,
+        err = gdp_launch_bounds(reinterpret_cast<const GdpBoundInst *>(dev + off_inst), m, n_lam, max_LS, max_S, max_K,
+                                threads == GDP_BOUND_THREADS ? elements : narrow, threads,
                                 reinterpret_cast<const int2 *>(dev + off_pairs), (int)pairs.size(), lane.stream);
     if (err == hipSuccess && stats) err = hipEventRecord(lane.ev_end, lane.stream);
     if (err == hipSuccess) err = hipMemcpyAsync(lane.back, dev + up_bytes, back_bytes, hipMemcpyDeviceToHost, lane.stream);

@@ -10,7 +10,7 @@ constexpr int GDP_BOUND_MAX_L = 512;      // layers (running sums of four paths 
 constexpr int GDP_BOUND_MAX_LS = 40960;   // layers x strategies: the argmin table of a pass lives in LDS
 constexpr int GDP_BOUND_MAX_LAM = 64;     // multipliers
 constexpr int GDP_BOUND_MAX_KEY = 8;
-constexpr int GDP_BOUND_THREADS = 1024;
+constexpr int GDP_BOUND_THREADS = 1024;    // at most, per pass; at least GDP_BOUND_MAX_L
 constexpr int GDP_BOUND_PARTS = 32;       // at most this many threads share a target strategy
 constexpr int GDP_BOUND_LOW = 3;          // paths above the budget that are spliced with the one below it
 
@@ -32,10 +32,11 @@ struct GdpBoundInst {
     int32_t L, V, S, K;
 };
 
-// Elements of a transition matrix per thread that instances of S strategies need (1, 2, 4, 8 or 16).
-__attribute__((visibility("hidden"))) int gdp_bound_elements(int S);
+// Elements of a transition matrix per thread that instances of S strategies need with that many threads per pass (1, 2,
+// 4, 8 or 16; 0: more than that many threads take).
+__attribute__((visibility("hidden"))) int gdp_bound_elements(int S, int threads);
 // Transposes the matrices, runs the passes of all multipliers, finds the upper bounds and marks what stays.
 // pairs: {instance, matrix} of every matrix that is to be transposed.
 __attribute__((visibility("hidden")))
 hipError_t gdp_launch_bounds(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K,
-                             int elements, const int2 *pairs, int n_pairs, hipStream_t stream);
+                             int elements, int threads, const int2 *pairs, int n_pairs, hipStream_t stream);

@@ -50,9 +50,11 @@ __global__ __launch_bounds__(256) void gdp_bound_transpose_kernel(const GdpBound
 // (Q).  grid (2 * multipliers, instances): the serial chain of L steps is what takes the time, so everything that
 // does not depend on it runs side by side -- multipliers and directions in workgroups of their own, a step's S*S
 // candidates on up to 1024 threads (thread = target strategy + S * part, its sources part, part + G, ...: loads run
-// along the rows), and the matrix of the next step is on its way to registers while this one is reduced.
-template <int E>
-__global__ __launch_bounds__(GDP_BOUND_THREADS) void gdp_bound_pass_kernel(const GdpBoundInst *inst)
+// along the rows), and the matrices of the next two steps are on their way to registers meanwhile.  A step is then two
+// barriers and the reduction over the parts: L = 80, S = 64 207 -> 132 us, L = 48, S = 88 147 -> 102 us and L = 32,
+// S = 44 79 -> 50 us against loads one step ahead behind comparisons.
+template <int E, int NT>
+__global__ __launch_bounds__(NT, NT == GDP_BOUND_THREADS ? 4 : 8) void gdp_bound_pass_kernel(const GdpBoundInst *inst)
 {
     extern __shared__ uint8_t arg_of[];   // [L][S], forwards only
     __shared__ double X[GDP_BOUND_MAX_S], part_v[GDP_BOUND_THREADS];
@@ -63,69 +65,88 @@ __global__ __launch_bounds__(GDP_BOUND_THREADS) void gdp_bound_pass_kernel(const
     const int L = I.L, S = I.S, V = I.V, t = (int)threadIdx.x, li = (int)blockIdx.x >> 1;
     const bool back = blockIdx.x & 1u;
     const double lam = I.lam[li];
-    const int G = min(GDP_BOUND_THREADS / S, GDP_BOUND_PARTS), s = t % S, g = t / S;
-    const bool active = g < G;
+    const int G = min(NT / S, GDP_BOUND_PARTS), s = t % S, g = min(t / S, G - 1), c_at = min(t, S - 1);
     const size_t SS = (size_t)S * S;
-    for (int l = t; l < L; l += GDP_BOUND_THREADS) mat[l] = I.index[l];
+    for (int l = t; l < L; l += NT) mat[l] = I.index[l];
     if (t < S) X[t] = 0.0;
     __syncthreads();
-    const double *tables = back ? I.inter_t : I.inter;
-    double *out = (back ? I.Q : I.P) + (size_t)li * L * S;
+    // Global memory, said so: the compiler takes a pointer that comes from memory for one that may point anywhere.
+    typedef const __attribute__((address_space(1))) double *gdouble;
+    typedef const __attribute__((address_space(1))) int32_t *gint;
+    typedef __attribute__((address_space(1))) double *gout;
+    const gdouble tables = (gdouble)(uintptr_t)(back ? I.inter_t : I.inter), intra = (gdouble)(uintptr_t)I.intra;
+    const gint mem = (gint)(uintptr_t)I.mem;
+    const gout out = (gout)(uintptr_t)((back ? I.Q : I.P) + (size_t)li * L * S);
 
-    double m_now[E], m_next[E], c_now = 0.0, c_next = 0.0;
-    auto fetch = [&](int l, double (&m)[E], double &c) {
-        const double *M = tables + (size_t)mat[l] * SS;
+    // What a step needs from memory: its part of the matrix and the layer's costs of strategy t.  Sources beyond the last
+    // are the last once more, so that nothing here depends on a comparison and the loads of a step leave together.
+    struct Inputs {
+        double m[E], intra;
+        int32_t mem;
+    };
+    auto from = [&](int k) { return min(g + k * G, S - 1); };
+    constexpr int AHEAD = E <= 8 ? 2 : 1;   // steps: two sets of 16 elements do not fit the registers of 1024 threads
+    auto fetch = [&](int l, Inputs &in) {
+        const gdouble M = tables + (size_t)__builtin_amdgcn_readfirstlane(mat[l]) * SS;
 #pragma unroll
-        for (int k = 0; k < E; ++k) {
-            const int sp = g + k * G;
-            m[k] = active && sp < S ? M[(size_t)sp * S + s] : (double)INFINITY;
-        }
-        if (t < S) c = lagrangian(I.mem[(size_t)l * S + t], I.intra[(size_t)l * S + t], lam, V);
+        for (int k = 0; k < E; ++k) in.m[k] = M[from(k) * S + s];
+        in.mem = mem[l * S + c_at];
+        in.intra = intra[l * S + c_at];
     };
     const int first = back ? L - 1 : 0, step = back ? -1 : 1;
-    fetch(first, m_now, c_now);
-    for (int i = 0, l = first; i < L; ++i, l += step) {
-        if (i + 1 < L) fetch(l + step, m_next, c_next);
+    // Step i; its registers are filled again for step i + AHEAD as soon as they have been read.
+    auto pass = [&](int i, Inputs &in) {
+        const int l = first + i * step;
+        const double c = lagrangian(in.mem, in.intra, lam, V);
         if (back) {
             // X is Q[l]; what lies before layer l sees the cost of (l, s) on top of it
             if (t < S) {
                 out[(size_t)l * S + t] = X[t];
-                X[t] += c_now;
+                X[t] += c;
             }
-            if (l == 0) break;
+            if (l == 0) return;
             __syncthreads();
         }
         double best = INFINITY;
         int arg = 0;
-        if (active) {
 #pragma unroll
-            for (int k = 0; k < E; ++k) {
-                const int sp = g + k * G;
-                if (sp < S) {
-                    const double v = X[sp] + m_now[k];
-                    if (v < best) { best = v; arg = sp; }
-                }
-            }
+        for (int k = 0; k < E; ++k) {
+            const double v = X[from(k)] + in.m[k];
+            arg = v < best ? from(k) : arg;
+            best = v < best ? v : best;
+        }
+        if (i + AHEAD < L) fetch(l + AHEAD * step, in);
+        if (t < G * S) {
             part_v[t] = best;
             part_i[t] = (uint8_t)arg;
         }
         __syncthreads();
         if (t < S) {   // thread t is part 0 of target t
-            for (int p = 1; p < G; ++p)
-                if (part_v[p * S + t] < best) { best = part_v[p * S + t]; arg = part_i[p * S + t]; }
+#pragma unroll 8
+            for (int p = 1; p < G; ++p) {   // no branch: the reads of all parts are in flight together
+                const double v = part_v[p * S + t];
+                const int a = part_i[p * S + t];
+                arg = v < best ? a : arg;
+                best = v < best ? v : best;
+            }
             if (back) {
                 X[t] = best;
             } else {
-                X[t] = best + c_now;
+                X[t] = best + c;
                 out[(size_t)l * S + t] = X[t];
                 arg_of[l * S + t] = (uint8_t)arg;
             }
         }
         __syncthreads();
+    };
+    Inputs in[AHEAD];
 #pragma unroll
-        for (int k = 0; k < E; ++k) m_now[k] = m_next[k];
-        c_now = c_next;
-    }
+    for (int a = 0; a < AHEAD; ++a)
+        if (a < L) fetch(first + a * step, in[a]);
+    for (int i = 0; i < L; i += AHEAD)
+#pragma unroll
+        for (int a = 0; a < AHEAD; ++a)
+            if (i + a < L) pass(i + a, in[a]);
     if (back) return;
     if (t == 0) {
         int b = 0;
@@ -142,13 +163,13 @@ __global__ __launch_bounds__(GDP_BOUND_THREADS) void gdp_bound_pass_kernel(const
     if (t < L) {
         const int b = path[t], a = arg_of[t * S + b];
         I.path[(size_t)li * L + t] = (uint8_t)b;
-        const int32_t m = I.mem[(size_t)t * S + b];
-        time = tables[(size_t)mat[t] * SS + (size_t)a * S + b] + (m < V ? I.intra[(size_t)t * S + b] : (double)INFINITY);
+        const int32_t m = mem[t * S + b];
+        time = tables[(size_t)mat[t] * SS + (size_t)a * S + b] + (m < V ? intra[t * S + b] : (double)INFINITY);
         memory = (double)m;   // whole numbers below 2^41: exact
     }
     part_v[t] = time;
     __syncthreads();
-    for (int w = GDP_BOUND_THREADS / 2; w > 0; w >>= 1) {
+    for (int w = NT / 2; w > 0; w >>= 1) {
         if (t < w) part_v[t] += part_v[t + w];
         __syncthreads();
     }
@@ -156,7 +177,7 @@ __global__ __launch_bounds__(GDP_BOUND_THREADS) void gdp_bound_pass_kernel(const
     __syncthreads();
     part_v[t] = memory;
     __syncthreads();
-    for (int w = GDP_BOUND_THREADS / 2; w > 0; w >>= 1) {
+    for (int w = NT / 2; w > 0; w >>= 1) {
         if (t < w) part_v[t] += part_v[t + w];
         __syncthreads();
     }
@@ -253,12 +274,15 @@ __global__ __launch_bounds__(64) void gdp_bound_keep_kernel(const GdpBoundInst *
             budget[k] = (double)I.budget[k];
         }
     }
+    typedef const __attribute__((address_space(1))) double *gdouble;
+    const gdouble P = (gdouble)(uintptr_t)I.P, Q = (gdouble)(uintptr_t)I.Q, lams = (gdouble)(uintptr_t)I.lam;
+    const double reach = (double)(I.L + 1) * (double)I.V, magnitude = I.magnitude;
     const double ulp = 16.0 * (double)(I.L + 4) * 0x1p-53;
-#pragma unroll 4
+#pragma unroll 8
     for (int i = 0; i < n_lam; ++i) {
-        const double lam = I.lam[i];
-        const double r = I.P[(size_t)i * LS + e] + I.Q[(size_t)i * LS + e];
-        const double margin = ulp * (I.magnitude + lam * (double)(I.L + 1) * (double)I.V);
+        const double lam = lams[i];
+        const double r = P[(size_t)i * LS + e] + Q[(size_t)i * LS + e];
+        const double margin = ulp * (magnitude + lam * reach);
 #pragma unroll
         for (int k = 0; k < GDP_BOUND_MAX_KEY; ++k)
             if (r - lam * budget[k] > ub[k] + margin) alive &= ~(1u << k);
@@ -268,28 +292,39 @@ __global__ __launch_bounds__(64) void gdp_bound_keep_kernel(const GdpBoundInst *
 
 }  // namespace
 
-int gdp_bound_elements(int S)
+int gdp_bound_elements(int S, int threads)
 {
-    const int G = GDP_BOUND_THREADS / S < GDP_BOUND_PARTS ? GDP_BOUND_THREADS / S : GDP_BOUND_PARTS;
-    for (int e = 1; e < 16; e *= 2)
+    const int G = threads / S < GDP_BOUND_PARTS ? threads / S : GDP_BOUND_PARTS;
+    const int most = threads == GDP_BOUND_THREADS ? 16 : 4;   // S <= 128: with 1024 threads G >= 8, so 16 are enough
+    for (int e = 1; e <= most; e *= 2)
         if (e * G >= S) return e;
-    return 16;   // S <= 128: G >= 8
+    return 0;
 }
 
 hipError_t gdp_launch_bounds(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K,
-                             int elements, const int2 *pairs, int n_pairs, hipStream_t stream)
+                             int elements, int threads, const int2 *pairs, int n_pairs, hipStream_t stream)
 {
     gdp_bound_transpose_kernel<<<dim3((unsigned)n_pairs, (unsigned)((max_S + 15) / 16)), 256, 0, stream>>>(inst, pairs);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const dim3 grid(2u * (unsigned)n_lam, (unsigned)n);
     const size_t lds = (size_t)max_LS;
-    switch (elements) {
-    case 1: gdp_bound_pass_kernel<1><<<grid, GDP_BOUND_THREADS, lds, stream>>>(inst); break;
-    case 2: gdp_bound_pass_kernel<2><<<grid, GDP_BOUND_THREADS, lds, stream>>>(inst); break;
-    case 4: gdp_bound_pass_kernel<4><<<grid, GDP_BOUND_THREADS, lds, stream>>>(inst); break;
-    case 8: gdp_bound_pass_kernel<8><<<grid, GDP_BOUND_THREADS, lds, stream>>>(inst); break;
-    default: gdp_bound_pass_kernel<16><<<grid, GDP_BOUND_THREADS, lds, stream>>>(inst); break;
+    auto launch = [&](auto kernel) { kernel<<<grid, threads, lds, stream>>>(inst); };
+    constexpr int WIDE = GDP_BOUND_THREADS, HALF = GDP_BOUND_THREADS / 2;
+    if (threads == WIDE) {
+        switch (elements) {
+        case 1: launch(gdp_bound_pass_kernel<1, WIDE>); break;
+        case 2: launch(gdp_bound_pass_kernel<2, WIDE>); break;
+        case 4: launch(gdp_bound_pass_kernel<4, WIDE>); break;
+        case 8: launch(gdp_bound_pass_kernel<8, WIDE>); break;
+        default: launch(gdp_bound_pass_kernel<16, WIDE>); break;
+        }
+    } else {
+        switch (elements) {
+        case 1: launch(gdp_bound_pass_kernel<1, HALF>); break;
+        case 2: launch(gdp_bound_pass_kernel<2, HALF>); break;
+        default: launch(gdp_bound_pass_kernel<4, HALF>); break;
+        }
     }
     e = hipGetLastError();
     if (e != hipSuccess) return e;
