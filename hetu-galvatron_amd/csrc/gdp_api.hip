@@ -2565,8 +2565,10 @@ struct Reduced {
 // every instance that has the form, =0 for none).  They take 0.1 (L = 32, S = 44) to 0.2 ms (L = 80, S = 64) and a round
 // trip; per call, whole / reduced: L = 24, S = 22, V = 16384 (1.9e8) 0.16 / 0.27 ms; L = 28, S = 40, V = 29493 (1.3e9)
 // 0.30 / 0.32; L = 32, S = 44, V = 65536 (4e9) 0.67 / 0.41; L = 80, S = 64, V = 131072 (4.3e10) 3.06 / 0.97; L = 48,
-// S = 88, V = 262144 (9.7e10) 10.8 / 1.1; 256 instances of S = 44 49 / 7.8 ms.
-static constexpr double REDUCE_MIN_WORK = 3e9;
+// S = 88, V = 262144 (9.7e10) 10.8 / 1.1; 256 instances of S = 44 49 / 7.8 ms.  Instances of different S run in launches
+// of their own, one after the other, and what is left of them mostly in one: a batch of four S (the 15 stages of a
+// fit, L = 30, S = 37, 19, 10 and 5, V = 23593, 1.3e9) gains from a quarter of the work on, 0.93 / 0.62 ms.
+static constexpr double REDUCE_MIN_WORK = 2e9;
 static constexpr size_t REDUCE_MAX_BYTES = (size_t)4 << 30;   // of device memory for the tables of the passes
 
 static bool reducible(const gdp_problem *q, double magnitude)
@@ -2692,8 +2694,14 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
     const bool forced = env && *env && atoi(env) != 0;
     if ((env && *env && !forced) || (skip && *skip && atoi(skip) == 0)) return GDP_OK;
     double total = 0;
-    for (int i = 0; i < n; ++i) total += (double)p[i]->L * p[i]->V * (double)p[i]->S * p[i]->S;
-    if (!forced && total < REDUCE_MIN_WORK) return GDP_OK;
+    std::vector<char> seen(GDP_MAX_S + 1, 0);
+    int groups = 0;
+    for (int i = 0; i < n; ++i) {
+        total += (double)p[i]->L * p[i]->V * (double)p[i]->S * p[i]->S;
+        groups += !seen[(size_t)p[i]->S];
+        seen[(size_t)p[i]->S] = 1;
+    }
+    if (!forced && total * std::min(groups, 4) < REDUCE_MIN_WORK) return GDP_OK;
 
     struct Entry {
         int orig, table_of;   // table_of: the entry whose matrices this one reads
