@@ -21,6 +21,9 @@
 
 namespace {
 
+static_assert(GDP_BOUND_MAX_S <= 128, "the cheapest end of a path: two strategies per lane");
+static_assert(GDP_BOUND_MAX_LAM <= 64 && GDP_BOUND_LOW + 1 == 4, "the upper bounds: a multiplier per lane, a path per wave");
+
 __device__ __forceinline__ double lagrangian(int32_t mem, double intra, double lam, int V)
 {
     return mem < V && intra < INFINITY ? intra + lam * (double)mem : (double)INFINITY;
@@ -148,14 +151,27 @@ __global__ __launch_bounds__(NT, NT == GDP_BOUND_THREADS ? 4 : 8) void gdp_bound
         for (int a = 0; a < AHEAD; ++a)
             if (i + a < L) pass(i + a, in[a]);
     if (back) return;
-    if (t == 0) {
-        int b = 0;
-        for (int k = 1; k < S; ++k)
-            if (X[k] < X[b]) b = k;
-        for (int l = L - 1; l >= 0; --l) {
-            path[l] = (uint8_t)b;
-            b = arg_of[l * S + b];
+    if (t < 64) {   // the cheapest end: two strategies per lane at most, then across the wave
+        int b = t < S ? t : 0;
+        double least = X[b];
+        if (t + 64 < S && X[t + 64] < least) {
+            b = t + 64;
+            least = X[b];
         }
+#pragma unroll
+        for (int w = 32; w > 0; w >>= 1) {
+            const double v = __shfl_xor(least, w);
+            const int a = __shfl_xor(b, w);
+            if (v < least || (v == least && a < b)) {
+                least = v;
+                b = a;
+            }
+        }
+        if (t == 0)
+            for (int l = L - 1; l >= 0; --l) {
+                path[l] = (uint8_t)b;
+                b = arg_of[l * S + b];
+            }
     }
     __syncthreads();
     // what the path costs: one layer per thread (L <= 512), summed in LDS
@@ -187,7 +203,9 @@ __global__ __launch_bounds__(NT, NT == GDP_BOUND_THREADS ? 4 : 8) void gdp_bound
 // Upper bound of one key: the best of the multipliers' paths that fit, and of the paths that follow one of the
 // last paths that do not fit up to some layer and the first one that does from there on (or the other way round) --
 // where all layers are alike every layer changes its strategy at the same multiplier, and only such a
-// splice comes near the budget.  grid (keys, instances), 256 threads; a candidate per thread from running sums.
+// splice comes near the budget.  grid (keys, instances), 256 threads; a candidate per thread from running sums.  Choosing
+// the paths and summing them up are a wave's work instead of one thread's walk through memory (L = 80, S = 64 11.5 ->
+// 7.0 us, 256 instances of S = 44 8.4 -> 6.9 us).
 __global__ __launch_bounds__(256) void gdp_bound_upper_kernel(const GdpBoundInst *inst, int n_lam)
 {
     __shared__ double pt[GDP_BOUND_LOW + 1][GDP_BOUND_MAX_L + 1], pm[GDP_BOUND_LOW + 1][GDP_BOUND_MAX_L + 1];
@@ -200,15 +218,17 @@ __global__ __launch_bounds__(256) void gdp_bound_upper_kernel(const GdpBoundInst
     const int64_t B = I.budget[key];
     const size_t SS = (size_t)S * S;
     double best = INFINITY;
-    if (t < n_lam && I.path_mem[t] <= B && I.path_time[t] < INFINITY) best = I.path_time[t];
-    if (t == 0) {
-        int fit = -1, low = 0;
-        for (int q = 0; q <= GDP_BOUND_LOW; ++q) which[q] = -1;
-        for (int i = 0; i < n_lam && fit < 0; ++i)
-            if (I.path_mem[i] <= B && I.path_time[i] < INFINITY) fit = i;
-        which[0] = fit;
-        for (int i = fit - 1; i >= 0 && low < GDP_BOUND_LOW; --i)
-            if (I.path_time[i] < INFINITY) which[1 + low++] = i;
+    if (t < 64) {   // a multiplier per lane: which paths fit, and which there are, are two ballots
+        const double time = t < n_lam ? I.path_time[t] : (double)INFINITY;
+        const bool fits = time < INFINITY && I.path_mem[t] <= B;
+        if (fits) best = time;
+        const unsigned long long fit = __ballot(fits), any = __ballot(time < INFINITY);
+        if (t <= GDP_BOUND_LOW) {
+            const int first = fit ? __ffsll(fit) - 1 : -1;
+            unsigned long long below = first > 0 ? any & ((1ull << first) - 1) : 0;
+            for (int q = 1; q < t && below; ++q) below ^= 1ull << (63 - __clzll(below));
+            which[t] = t == 0 ? first : below ? 63 - __clzll(below) : -1;
+        }
     }
     __syncthreads();
     if (which[0] >= 0 && which[1] >= 0) {   // the same in every thread
@@ -225,11 +245,30 @@ __global__ __launch_bounds__(256) void gdp_bound_upper_kernel(const GdpBoundInst
             pm[q][l + 1] = (double)I.mem[(size_t)l * S + b];
         }
         __syncthreads();
-        if (t <= GDP_BOUND_LOW && which[t] >= 0) {
-            pt[t][0] = pm[t][0] = 0.0;
-            for (int l = 1; l <= L; ++l) {
-                pt[t][l] += pt[t][l - 1];
-                pm[t][l] += pm[t][l - 1];
+        // running sums: a path per wave, 64 layers at a time (their rounding, in whatever order, is within the margin)
+        const int q = t >> 6, lane = t & 63;
+        if (which[q] >= 0) {
+            double time = 0.0, memory = 0.0;   // of the layers before the 64
+            if (lane == 0) pt[q][0] = pm[q][0] = 0.0;
+            for (int l0 = 1; l0 <= L; l0 += 64) {
+                const int l = l0 + lane;
+                double x = l <= L ? pt[q][l] : 0.0, y = l <= L ? pm[q][l] : 0.0;
+#pragma unroll
+                for (int w = 1; w < 64; w <<= 1) {
+                    const double u = __shfl_up(x, w), v = __shfl_up(y, w);
+                    if (lane >= w) {
+                        x += u;
+                        y += v;
+                    }
+                }
+                x += time;
+                y += memory;
+                if (l <= L) {
+                    pt[q][l] = x;
+                    pm[q][l] = y;
+                }
+                time = __shfl(x, 63);
+                memory = __shfl(y, 63);
             }
         }
         __syncthreads();
@@ -256,19 +295,25 @@ __global__ __launch_bounds__(256) void gdp_bound_upper_kernel(const GdpBoundInst
 // What stays: (l, s) is out when for every key some multiplier's bound lies above that key's upper bound.  The
 // margin covers the rounding of the bound, of the upper bound and of the DP's own sums: each is a sum of at most
 // 4 L + 4 terms whose magnitudes add up to no more than `magnitude` + lam * (L + 1) * V.
-// grid (64-element groups of the largest table, instances), one wave per workgroup.
-__global__ __launch_bounds__(64) void gdp_bound_keep_kernel(const GdpBoundInst *inst, int n_lam)
+// grid (64-element groups of the largest table, instances), PARTS waves with 8 multipliers at a time each.  What takes
+// the time is the round trips of the loads: with 8 waves all 64 multipliers of an element are asked for at once (L = 80,
+// S = 64 26.8 -> 6.3 us, L = 48, S = 88 25.0 -> 5.7 us).  A batch that fills the device with one wave per 64 elements
+// hides them by itself and would only start more waves (256 instances of S = 44 23.6 us with 1 wave, 40 with 8).
+template <int PARTS>
+__global__ __launch_bounds__(64 * PARTS) void gdp_bound_keep_kernel(const GdpBoundInst *inst, int n_lam)
 {
+    __shared__ unsigned left[PARTS][64];
     const GdpBoundInst &I = inst[blockIdx.y];
-    const int e = (int)(blockIdx.x * 64 + threadIdx.x), LS = I.L * I.S;
-    if (e >= LS) return;
+    const int LS = I.L * I.S, K = I.K, lane = (int)threadIdx.x & 63, part = (int)threadIdx.x >> 6;
+    if ((int)blockIdx.x * 64 >= LS) return;   // the whole workgroup
+    const int e = (int)blockIdx.x * 64 + lane, at = min(e, LS - 1);
     unsigned alive = 0;
     double ub[GDP_BOUND_MAX_KEY], budget[GDP_BOUND_MAX_KEY];
 #pragma unroll
     for (int k = 0; k < GDP_BOUND_MAX_KEY; ++k) {
         ub[k] = INFINITY;
         budget[k] = 0.0;
-        if (k < I.K && I.budget[k] >= 0) {
+        if (k < K && I.budget[k] >= 0) {
             alive |= 1u << k;
             ub[k] = I.ub[k];
             budget[k] = (double)I.budget[k];
@@ -278,15 +323,29 @@ __global__ __launch_bounds__(64) void gdp_bound_keep_kernel(const GdpBoundInst *
     const gdouble P = (gdouble)(uintptr_t)I.P, Q = (gdouble)(uintptr_t)I.Q, lams = (gdouble)(uintptr_t)I.lam;
     const double reach = (double)(I.L + 1) * (double)I.V, magnitude = I.magnitude;
     const double ulp = 16.0 * (double)(I.L + 4) * 0x1p-53;
-#pragma unroll 8
-    for (int i = 0; i < n_lam; ++i) {
-        const double lam = lams[i];
-        const double r = P[(size_t)i * LS + e] + Q[(size_t)i * LS + e];
-        const double margin = ulp * (magnitude + lam * reach);
+    for (int i0 = 8 * part; i0 < n_lam; i0 += 8 * PARTS) {
+        double p[8], q[8];
 #pragma unroll
-        for (int k = 0; k < GDP_BOUND_MAX_KEY; ++k)
-            if (r - lam * budget[k] > ub[k] + margin) alive &= ~(1u << k);
+        for (int i = 0; i < 8; ++i) {   // beyond the last: the last once more
+            const size_t row = (size_t)min(i0 + i, n_lam - 1) * LS + at;
+            p[i] = P[row];
+            q[i] = Q[row];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const double lam = lams[min(i0 + i, n_lam - 1)];
+            const double r = p[i] + q[i];
+            const double margin = ulp * (magnitude + lam * reach);
+#pragma unroll
+            for (int k = 0; k < GDP_BOUND_MAX_KEY; ++k)
+                if (k < K && r - lam * budget[k] > ub[k] + margin) alive &= ~(1u << k);
+        }
     }
+    left[part][lane] = alive;
+    __syncthreads();
+    if (part != 0 || e >= LS) return;
+#pragma unroll
+    for (int w = 1; w < PARTS; ++w) alive &= left[w][lane];
     I.keep[e] = alive != 0;
 }
 
@@ -331,6 +390,10 @@ hipError_t gdp_launch_bounds(const GdpBoundInst *inst, int n, int n_lam, int max
     gdp_bound_upper_kernel<<<dim3((unsigned)max_K, (unsigned)n), 256, 0, stream>>>(inst, n_lam);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    gdp_bound_keep_kernel<<<dim3((unsigned)((max_LS + 63) / 64), (unsigned)n), 64, 0, stream>>>(inst, n_lam);
+    const dim3 elements64((unsigned)((max_LS + 63) / 64), (unsigned)n);
+    if ((int64_t)elements64.x * n <= 1024)   // 8 waves of each are on the device at a time
+        gdp_bound_keep_kernel<8><<<elements64, 512, 0, stream>>>(inst, n_lam);
+    else
+        gdp_bound_keep_kernel<1><<<elements64, 64, 0, stream>>>(inst, n_lam);
     return hipGetLastError();
 }

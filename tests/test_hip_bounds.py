@@ -103,3 +103,34 @@ def test_initial_costs_that_are_not_zeros(monkeypatch):
     got = H.hip_solve(inst)
     want = O.solve(inst.mem, inst.intra, inst.inter, inst.V, inst.other_mem, inst.other_time, f0=inst.f0)[:3]
     H.assert_same_results(got, want)
+
+
+@pytest.mark.parametrize("strategies", [(22,), (23, 32), (33, 44, 9), (45, 8)])
+def test_batches_with_narrow_passes(strategies, monkeypatch):
+    """From 17 instances on a pass has 512 threads where 4 elements per thread are enough (up to 44 strategies)."""
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    rng = np.random.Generator(np.random.PCG64([7, *strategies]))
+    V, xs = 400, []
+    for n in range(18):
+        L, S = (2, 5, 9)[n % 3], strategies[n % len(strategies)]
+        xs.append(_instance(rng, L, S, V, ["each", "same", "ties", "negative", "holes", "loose"][n % 6]))
+    probs = [_problem(x, V) for x in xs]
+    _lib.solve_batch(probs)
+    for n, (x, prob) in enumerate(zip(xs, probs)):
+        _check(x, V, prob, f"{strategies} instance {n}")
+
+
+@pytest.mark.parametrize("many", [63, 64, 80])
+def test_instances_of_very_different_budgets(many, monkeypatch):
+    """From 64 instances of one S on those within a factor of 4 of the budget form a group of their own."""
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "0")
+    rng = np.random.Generator(np.random.PCG64(many))
+    xs, probs = [], []
+    for n in range(many):
+        V = (40, 41, 160, 161, 640, 2560, 33, 50)[n % 8] if n else 2560
+        x = _instance(rng, 3 + n % 4, 9, V, ["each", "ties"][n % 2])
+        xs.append((x, V))
+        probs.append(_problem(x, V))
+    _lib.solve_batch(probs)
+    for n, ((x, V), prob) in enumerate(zip(xs, probs)):
+        _check(x, V, prob, f"instance {n}")
