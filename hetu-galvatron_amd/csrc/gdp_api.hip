@@ -663,32 +663,38 @@ static int scan_f0(const gdp_problem *p, bool *live, double *maxabs)
 namespace {
 
 // Looks through the initial costs of a batch for anything but zeros, on threads beside the one that prepares and
-// waits for the device: one thread reads 20 GB/s from memory, so the 184 MB of a call with S = 88, V = 262144 took 4.5 ms
-// of its own once the device needed less, and the 23 MB of S = 44, V = 65536 0.6 ms.  The arrays are cut into
-// pieces that the threads draw from a counter; the caller helps with what is left when it needs the answer, so a
-// thread that could not be had only costs time.  One thread per 4 MB, at most 7 and what the machine has, from 16 MB
-// on: starting one takes some 30 us, and the 9 MB of S = 40, V = 29493 are looked through behind the device's work
-// (0.30 ms per call without threads, 0.37 with two).  Per call, one thread / with helpers: S = 88, V = 262144
-// 4.5 / 1.1 ms, S = 44, V = 65536 0.74 / 0.41 ms.
+// waits for the device: one thread reads 35 GB/s from memory, so the 184 MB of a call with S = 88, V = 262144 took 4.5 ms
+// of its own once the device needed less.  The arrays are cut into pieces that the threads draw from a counter; the
+// caller helps with what is left when it needs the answer, so a thread that could not be had only costs time.  One
+// thread per 4 MB, at most 7 and what the machine has, from 64 MB on.  An array that fits the caller's last-level cache
+// stays with the caller: lines that other cores have read are slow to write again, and a caller who fills the next
+// array into the same memory pays more than the scan gains (S = 44, V = 65536, 23 MB: the call 1.04 -> 0.48 ms, filling
+// the next array 0.98 -> 1.90 ms).  At 184 MB: the call 4.5 -> 1.1 ms, filling as before (9.6 and 9.8 ms).
 class InitialScan {
 public:
-    void start(int32_t n, const gdp_problem *const *p)
+    void start(int32_t n, const gdp_problem *const *p, double relaxations)
     {
-        size_t bytes = 0;
         for (int i = 0; i < n; ++i) {
             if (!p[i]->f0) continue;
             const size_t words = (size_t)p[i]->V * (size_t)p[i]->S;
             for (size_t k = 0; k < words; k += PIECE) pieces_.push_back({p[i]->f0 + k, std::min(PIECE, words - k)});
-            bytes += 8 * words;
+            bytes_ += 8 * words;
         }
+        if (bytes_ < HELPED_FROM || !device_bound(relaxations, bytes_)) return;
         const size_t cores = std::max(1u, std::thread::hardware_concurrency());
-        const size_t want = bytes < HELPED_FROM ? 0 : std::min({bytes >> 22, cores - 1, (size_t)7});
+        const size_t want = std::min({bytes_ >> 22, cores - 1, (size_t)7});
         helpers_.reserve(want);
         try {
             for (size_t k = 0; k < want; ++k) helpers_.emplace_back([this] { work(); });
         } catch (const std::system_error &) {   // no thread to be had: the caller does what is left
         }
     }
+    // A caller that looks through `bytes` (35 GB/s) for longer than the whole instances' relaxations keep the device
+    // (10^13 a second) waits for itself: bounds would come on top, and what helpers save is lost when the array is
+    // filled again (75 MB: the call 1.60 -> 1.00 ms, filling the next array 3.7 -> 5.3 ms).
+    static bool device_bound(double relaxations, size_t bytes) { return relaxations / 1e13 >= 1.5 * (double)bytes / 35e9; }
+    // bytes that the calling thread has to look through by itself
+    size_t alone() const { return helpers_.empty() ? bytes_ : 0; }
     // true: some array holds more than zeros
     bool finish()
     {
@@ -703,7 +709,7 @@ public:
     }
 
 private:
-    static constexpr size_t HELPED_FROM = (size_t)16 << 20;
+    static constexpr size_t HELPED_FROM = (size_t)64 << 20;
     static constexpr size_t PIECE = (size_t)1 << 16;   // doubles: half a megabyte
     struct Piece {
         const double *at;
@@ -728,6 +734,7 @@ private:
         for (std::thread &t : helpers_) t.join();
         helpers_.clear();
     }
+    size_t bytes_ = 0;
     std::vector<Piece> pieces_;
     std::vector<std::thread> helpers_;
     std::atomic<size_t> next_{0};
@@ -1116,12 +1123,14 @@ void PlanBuilder::describe_instances()
     constexpr int MANY = 64, WASTE = 3;
     std::unordered_map<int, std::pair<int64_t, std::pair<int64_t, int64_t>>> by_S;   // instances, sum and maximum of V
     for (const HostInst &h : inst) {
+        if (n < MANY) break;
         auto &e = by_S[h.S];
         e.first++;
         e.second.first += h.V;
         e.second.second = std::max<int64_t>(e.second.second, h.V);
     }
     for (HostInst &h : inst) {
+        if (n < MANY) break;
         const auto &e = by_S[h.S];
         if (e.first < MANY || e.first * e.second.second < WASTE * e.second.first) continue;
         for (int64_t v = h.V; 4 * v <= e.second.second; v *= 4) h.size_class++;
@@ -2564,7 +2573,8 @@ struct Reduced {
 // Dense relaxations of a batch from which on the bounds are worth their launches (GALVATRON_DP_REDUCE=1 takes them for
 // every instance that has the form, =0 for none).  They take 0.1 (L = 32, S = 44) to 0.2 ms (L = 80, S = 64) and a round
 // trip; per call, whole / reduced: L = 24, S = 22, V = 16384 (1.9e8) 0.16 / 0.27 ms; L = 28, S = 40, V = 29493 (1.3e9)
-// 0.30 / 0.32; L = 32, S = 44, V = 65536 (4e9) 0.67 / 0.41; L = 80, S = 64, V = 131072 (4.3e10) 3.06 / 0.97; L = 48,
+// 0.30 / 0.32; L = 32, S = 44, V = 65536 (4e9, no initial costs)
+// 0.67 / 0.29; L = 80, S = 64, V = 131072 (4.3e10) 3.06 / 0.97; L = 48,
 // S = 88, V = 262144 (9.7e10) 10.8 / 1.1; 256 instances of S = 44 49 / 7.8 ms.  Instances of different S run in launches
 // of their own, one after the other, and what is left of them mostly in one: a batch of four S (the 15 stages of a
 // fit, L = 30, S = 37, 19, 10 and 5, V = 23593, 1.3e9) gains from a quarter of the work on, 0.93 / 0.62 ms.
@@ -2685,19 +2695,28 @@ static bool build_reduced(const gdp_problem *q, const HostInst &h, const uint8_t
     return true;
 }
 
+static double dense_work(int32_t n, const gdp_problem *const *p)
+{
+    double work = 0;
+    for (int i = 0; i < n; ++i) work += (double)p[i]->L * p[i]->V * (double)p[i]->S * p[i]->S;
+    return work;
+}
+
 // Bounds of the instances of a batch that have the form, all in one set of launches, and the smaller instances that
-// follow (out[i] stays empty where instance i is solved whole).  Initial costs are taken to be zeros.
-static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vector<double> &magnitude,
+// follow (out[i] stays empty where instance i is solved whole).  Initial costs are taken to be zeros; scanned: bytes of
+// them that the calling thread looks through while the device works.
+static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vector<double> &magnitude, size_t scanned,
                         std::vector<std::unique_ptr<Reduced>> &out)
 {
     const char *env = getenv("GALVATRON_DP_REDUCE"), *skip = getenv("GALVATRON_DP_SKIP");
     const bool forced = env && *env && atoi(env) != 0;
     if ((env && *env && !forced) || (skip && *skip && atoi(skip) == 0)) return GDP_OK;
-    double total = 0;
+    const double total = dense_work(n, p);
+    if (!forced && total * std::min(n, 4) < REDUCE_MIN_WORK) return GDP_OK;
+    if (!forced && !InitialScan::device_bound(total, scanned)) return GDP_OK;
     std::vector<char> seen(GDP_MAX_S + 1, 0);
     int groups = 0;
     for (int i = 0; i < n; ++i) {
-        total += (double)p[i]->L * p[i]->V * (double)p[i]->S * p[i]->S;
         groups += !seen[(size_t)p[i]->S];
         seen[(size_t)p[i]->S] = 1;
     }
@@ -3002,9 +3021,9 @@ int gdp_solve_batch(int32_t n, const gdp_problem *const *p, gdp_result *const *r
         const size_t budget = std::max<size_t>(env_mb("GALVATRON_DP_ARENA_MB", 8192), (size_t)1 << 20);
         std::vector<char> f0_live((size_t)n, 0);
         InitialScan scan;
-        if (any_f0) scan.start(n, p);
+        if (any_f0) scan.start(n, p, dense_work(n, p));
         std::vector<std::unique_ptr<Reduced>> small((size_t)n);
-        int rc = reduce_batch(n, p, magnitude, small);
+        int rc = reduce_batch(n, p, magnitude, scan.alone(), small);
         if (rc != GDP_OK) return rc;
         std::vector<const gdp_problem *> q(p, p + n);
         std::vector<gdp_result *> qr(r, r + n);

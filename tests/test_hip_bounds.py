@@ -134,3 +134,27 @@ def test_instances_of_very_different_budgets(many, monkeypatch):
     _lib.solve_batch(probs)
     for n, ((x, V), prob) in enumerate(zip(xs, probs)):
         _check(x, V, prob, f"instance {n}")
+
+
+@pytest.mark.parametrize("shape", [(36, 96, 87000), (36, 96, 88000), (8, 96, 88000)])
+@pytest.mark.parametrize("at", [None, 0, -1])
+def test_large_initial_costs(shape, at):
+    """Initial costs around 64 MB, from where on several threads look through them where the device takes longer (not
+    with 8 layers): a call with zeros gives what one without gives, and one with a single other value at either end
+    what a plan gives, which uploads them as they are."""
+    L, S, V = shape
+    x = _instance(np.random.Generator(np.random.PCG64([L, V])), L, S, V, "each")
+    mem, intra, inter, om, ot = x
+    f0 = np.zeros((V, S))
+    if at is not None:
+        f0.reshape(-1)[at] = -3.0
+    keys = sorted(om)
+    def problem(f):
+        return _lib.Problem(mem, intra, inter, V, [om[k] for k in keys], [ot[k] for k in keys], f0=f)
+    got, want = problem(f0), problem(None if at is None else f0)
+    _lib.solve_batch([got])
+    plan = _lib.Plan([want])
+    plan.run()
+    plan.fetch()
+    assert got.total.tobytes() == want.total.tobytes()
+    assert np.array_equal(got.remaining, want.remaining) and np.array_equal(got.res, want.res)
