@@ -2118,7 +2118,7 @@ int audit_groups(const gdp_plan *pl, const gdp_problem *const *p)
             if (seg.lds_bytes > 65536u) return bad("dynamic LDS of a fused launch", seg.lds_bytes, 0, 0);
         }
         if (pl->flow_ready) {
-            // flow launch: grid = (workgroups of the widest band, layers, instances); a task's row offsets are
+            // flow launch: grid = (workgroups of the widest band, instances, layers); a task's row offsets are
             // ro[part * nsrc + u], u < nsrc (inside the SU entries checked below), its cost rows and gate cells
             // the elements a per-layer task reads
             if (g.flow_blocks < 0 || g.max_L > 65535 || g.count > 65535) return bad("grid of a flow launch", g.flow_blocks, g.max_L, g.count);

@@ -106,6 +106,22 @@ def test_flow_launch_batch_of_small_instances(golden, monkeypatch):
                 _check_against_golden(prob, golden[n], f"{n} run {rep}")
 
 
+def test_flow_launch_takes_the_instances_of_a_batch_side_by_side():
+    """The chains of 32 small instances hide each other: 1.3 times one instance's time as measured, 7 times where
+    they run one after the other.  The bound lies in between."""
+    if any(k in os.environ for k in _PRESETS):
+        pytest.skip("the environment presets the layout")
+    rng = np.random.Generator(np.random.PCG64(40))
+
+    def device_ms(n):
+        with _lib.Plan([_problem(W.random_instance(rng, 40, 16, 1000, mem_hi=60)) for _ in range(n)]) as plan:
+            ts = [plan.run(1) for _ in range(9)]
+            assert all(t.flow == 1 for t in ts)
+            return sorted(t.total_ms for t in ts)[4]
+    one, many = device_ms(1), device_ms(32)
+    assert many < 3 * one, (one, many)
+
+
 def test_flow_switched_off_and_on_again(golden):
     """A plan laid out for the flow launch runs per layer when told to, and flows again afterwards (the
     cells are reset first); a plan laid out for something else refuses the option."""
