@@ -386,7 +386,6 @@ struct HostInst {
     // byte offsets inside the device allocation
     size_t off_H, off_M, off_inter, off_intra, off_index, off_roff, off_mem;
     bool has_zero = false;  // some memory cost is 0 (see gdp_launch_zero_pass)
-    int size_class = 0;     // instances of one group have the same (PlanBuilder::describe_instances)
     size_t off_zcols = 0;
     // a dense [L,S,S] transition array whose equal matrices are kept once (share_equal_matrices):
     std::vector<int32_t> mat_of;   // layer -> kept matrix
@@ -434,7 +433,7 @@ void share_equal_matrices(const gdp_problem *q, HostInst &h)
     h.n_inter = (int)h.mat_src.size();
 }
 
-struct Group {  // instances with the same S (and size class), sorted by L descending
+struct Group {  // instances with the same S, sorted by L descending
     int first, count, SP, S, max_L, max_ntile, variant, ntb, nbt;   // ntb: wave tasks per tile (with the parts of split tasks)
     int split = 1;            // fused launches: waves that share the source strategies of a task (1, or 2: see relax_task)
     int xcd_group = 1;        // consecutive block tasks handed to one XCD (whole tiles)
@@ -1115,30 +1114,12 @@ void PlanBuilder::describe_instances()
                 for (int s2 = 0; s2 < q->S; ++s2) h.f0t[(size_t)s2 * q->V + v] = q->f0[(size_t)v * q->S + s2];
         }
     }
-    // The grids of a group are those of its widest instance, and a workgroup without work still has to be started:
-    // 256 thinned-out instances with budgets from 50 to 35000 bins are 1.5 million workgroups in the kernel that
-    // prepares the buffers and another million in the flow launch, most of them empty (1.1 and 3.1 ms).  Where
-    // many instances of one S differ that much, those within a factor of 4 form a group (0.2 and 1.7 ms); a launch
-    // per group costs a chain of layers of its own, so few or similar instances stay together.
-    constexpr int MANY = 64, WASTE = 3;
-    std::unordered_map<int, std::pair<int64_t, std::pair<int64_t, int64_t>>> by_S;   // instances, sum and maximum of V
-    for (const HostInst &h : inst) {
-        if (n < MANY) break;
-        auto &e = by_S[h.S];
-        e.first++;
-        e.second.first += h.V;
-        e.second.second = std::max<int64_t>(e.second.second, h.V);
-    }
-    for (HostInst &h : inst) {
-        if (n < MANY) break;
-        const auto &e = by_S[h.S];
-        if (e.first < MANY || e.first * e.second.second < WASTE * e.second.first) continue;
-        for (int64_t v = h.V; 4 * v <= e.second.second; v *= 4) h.size_class++;
-    }
-    // group by S and size, then by L descending (stable, so equal shapes keep the caller's order)
+    // group by S, then by L descending (stable, so equal shapes keep the caller's order).  Instances of one S and very
+    // different budgets stay in one group: in groups of their own (within a factor of 4 of V) batches of two sizes ran
+    // up to 1.5 times as fast, but every group is a chain of layers more, and batches of all sizes were as much
+    // slower (plans of 64, V = 640 to 40000: S = 9 0.43 -> 0.74 ms, S = 24 1.04 -> 1.19; 256 of S = 24 2.61 -> 3.00).
     std::stable_sort(inst.begin(), inst.end(), [](const HostInst &a, const HostInst &b) {
         if (a.S != b.S) return a.S < b.S;
-        if (a.size_class != b.size_class) return a.size_class < b.size_class;
         return a.L > b.L;
     });
 }
@@ -1151,7 +1132,7 @@ int PlanBuilder::form_groups()
         Group g;
         g.first = i; g.S = inst[(size_t)i].S;
         int j = i;
-        while (j < n && inst[(size_t)j].S == g.S && inst[(size_t)j].size_class == inst[(size_t)i].size_class) ++j;
+        while (j < n && inst[(size_t)j].S == g.S) ++j;
         g.count = j - i;
         // Register tile.  Width: pick_ts.  Height: the tallest whose first layer still gives every
         // resident wave at least two tasks, so that the stores of one task drain under the arithmetic

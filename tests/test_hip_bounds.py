@@ -122,7 +122,7 @@ def test_batches_with_narrow_passes(strategies, monkeypatch):
 
 @pytest.mark.parametrize("many", [63, 64, 80])
 def test_instances_of_very_different_budgets(many, monkeypatch):
-    """From 64 instances of one S on those within a factor of 4 of the budget form a group of their own."""
+    """Many instances of one S whose budgets differ by a factor of 80: one group, and with it one launch."""
     monkeypatch.setenv("GALVATRON_DP_REDUCE", "0")
     rng = np.random.Generator(np.random.PCG64(many))
     xs, probs = [], []
@@ -134,6 +134,9 @@ def test_instances_of_very_different_budgets(many, monkeypatch):
     _lib.solve_batch(probs)
     for n, ((x, V), prob) in enumerate(zip(xs, probs)):
         _check(x, V, prob, f"instance {n}")
+    with _lib.Plan(probs) as plan:
+        t = plan.run(1)
+        assert t.relax_launches == (1 if t.fused or t.flow else max(prob.L for prob in probs))
 
 
 @pytest.mark.parametrize("shape", [(36, 96, 87000), (36, 96, 88000), (8, 96, 88000)])
