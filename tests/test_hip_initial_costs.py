@@ -113,3 +113,38 @@ def test_rejected_initial_costs_raise_before_any_device_work():
             shim.dynamic_programming_core(inst.L, inst.V, inst.S, inst.mem, None, f, inst.inter, inst.intra,
                                           inst.other_mem, inst.other_time, res)
         assert all((r == -1).all() for r in res.values())
+
+
+@pytest.mark.parametrize("reduce", ["0", "1"])
+def test_costs_of_ones_own_are_seen_before_anything_is_solved(reduce, monkeypatch):
+    """An array full of costs is noticed at a glance: the call neither takes bounds (which assume zeros) nor solves
+    the instance as if there were none first."""
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", reduce)
+    inst = _case(670, L=6, S=22, V=3000)
+    prob = _problem(inst)
+    _lib.batch_stats_begin()
+    _lib.solve_batch([prob])
+    s = _lib.batch_stats_end()
+    assert s.parts == 1 and s.instances == 1 and s.relaxations == prob.relaxations
+    want = O.solve(inst.mem, inst.intra, inst.inter, inst.V, inst.other_mem, inst.other_time, f0=inst.f0)
+    H.assert_same_results(_results(prob, inst), want)
+
+
+@pytest.mark.parametrize("reduce", ["0", "1"])
+@pytest.mark.parametrize("value", [-7.5, np.nan, -np.inf, -0.0])
+def test_one_value_among_zeros(value, reduce, monkeypatch):
+    """... and one that is not is found while the device works on the speculative solve: the same results, the same
+    refusals, and nothing written by a refused call."""
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", reduce)
+    inst = _case(671, L=6, S=22, V=3000)
+    inst.f0 = np.zeros_like(inst.f0)
+    inst.f0[1234, 5] = value
+    prob = _problem(inst)
+    if value == -7.5:
+        _lib.solve_batch([prob])
+        want = O.solve(inst.mem, inst.intra, inst.inter, inst.V, inst.other_mem, inst.other_time, f0=inst.f0)
+        H.assert_same_results(_results(prob, inst), want)
+    else:
+        with pytest.raises(ValueError, match="f0"):
+            _lib.solve_batch([prob])
+        assert np.isinf(prob.total).all() and (prob.remaining == -1).all() and (prob.res == -1).all()
