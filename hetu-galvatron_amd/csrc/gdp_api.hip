@@ -2576,7 +2576,7 @@ struct Reduced {
 // of their own, one after the other, and what is left of them mostly in one: a batch of four S (the 15 stages of a
 // fit, L = 30, S = 37, 19, 10 and 5, V = 23593, 1.3e9) gains from a quarter of the work on, 0.93 / 0.62 ms.
 static constexpr double REDUCE_MIN_WORK = 2e9;
-static constexpr size_t REDUCE_MAX_BYTES = (size_t)4 << 30;   // of device memory for the tables of the passes
+static constexpr size_t REDUCE_MAX_BYTES = (size_t)4 << 30;   // of device memory for the bounds of a slice (GALVATRON_DP_ARENA_MB if less)
 
 static bool reducible(const gdp_problem *q, double magnitude)
 {
@@ -2699,71 +2699,47 @@ static double dense_work(int32_t n, const gdp_problem *const *p)
     return work;
 }
 
-// Bounds of the instances of a batch that have the form, all in one set of launches, and the smaller instances that
-// follow (out[i] stays empty where instance i is solved whole).  Initial costs are taken to be zeros; scanned: bytes of
-// them that the calling thread looks through while the device works.
-static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vector<double> &magnitude, size_t scanned,
+// An instance whose bounds are taken, and where its arrays lie in the allocation of its slice.
+struct BoundEntry {
+    int orig, table_of;   // table_of: the entry of the slice whose matrices this one reads
+    HostInst h;
+    std::vector<int64_t> budget;
+    size_t off_mem, off_intra, off_inter, off_index, off_lam, off_budget, off_inter_t, off_P, off_Q, off_time, off_pmem, off_path, off_ub, off_keep;
+};
+
+// Device memory that the bounds of an instance take at most, with matrices of its own.
+static size_t bound_bytes(const gdp_problem *q, const HostInst &h, int n_lam)
+{
+    const size_t L = (size_t)q->L, LS = L * q->S, T = (size_t)h.n_inter, K = (size_t)q->n_key, NL = (size_t)n_lam;
+    constexpr size_t ARRAYS = 16;   // aligned to 256 bytes each
+    return sizeof(GdpBoundInst) + T * sizeof(int2) + 13 * LS + 4 * L + 16 * K + 16 * T * (size_t)q->S * q->S +
+           NL * (24 + 16 * LS + L) + 256 * ARRAYS;
+}
+
+// Bounds of the instances of one slice in one set of launches, and the smaller instances that follow (out[i] stays
+// empty where instance i is solved whole).
+static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &magnitude, BoundEntry *es, int m, int n_lam,
                         std::vector<std::unique_ptr<Reduced>> &out)
 {
-    const char *env = getenv("GALVATRON_DP_REDUCE"), *skip = getenv("GALVATRON_DP_SKIP");
-    const bool forced = env && *env && atoi(env) != 0;
-    if ((env && *env && !forced) || (skip && *skip && atoi(skip) == 0)) return GDP_OK;
-    const double total = dense_work(n, p);
-    if (!forced && total * std::min(n, 4) < REDUCE_MIN_WORK) return GDP_OK;
-    if (!forced && !InitialScan::device_bound(total, scanned)) return GDP_OK;
-    std::vector<char> seen(GDP_MAX_S + 1, 0);
-    int groups = 0;
-    for (int i = 0; i < n; ++i) {
-        groups += !seen[(size_t)p[i]->S];
-        seen[(size_t)p[i]->S] = 1;
-    }
-    if (!forced && total * std::min(groups, 4) < REDUCE_MIN_WORK) return GDP_OK;
-
-    struct Entry {
-        int orig, table_of;   // table_of: the entry whose matrices this one reads
-        HostInst h;
-        std::vector<int64_t> budget;
-        size_t off_mem, off_intra, off_inter, off_index, off_lam, off_budget, off_inter_t, off_P, off_Q, off_time, off_pmem, off_path, off_ub, off_keep;
-    };
-    std::vector<Entry> es;
     std::vector<int2> pairs;
     size_t at = 0;
     auto place = [&](size_t bytes) { const size_t o = at; at = align_up(at + bytes, 256); return o; };
-    for (int i = 0; i < n; ++i) {
-        if (!reducible(p[i], magnitude[(size_t)i])) continue;
-        const gdp_problem *q = p[i];
-        Entry e;
-        e.orig = i;
-        e.table_of = (int)es.size();
-        int64_t least = 0;
-        for (int l = 0; l < q->L; ++l) least += *std::min_element(q->mem + (size_t)l * q->S, q->mem + (size_t)(l + 1) * q->S);
-        bool any = false;
-        for (int k = 0; k < q->n_key; ++k) {
-            const int64_t b = (int64_t)q->V - 1 - q->other_mem[k];
-            e.budget.push_back(b >= least ? b : -1);
-            any = any || b >= least;
-        }
-        if (!any) continue;
-        e.h.S = q->S;
-        e.h.n_inter = q->inter_index ? q->n_inter : q->L;
-        if (!q->inter_index) share_equal_matrices(q, e.h);
-        for (size_t j = es.size(); q->inter_index && j-- > 0;) {   // the stages of one fit, the tasks of one sweep
+    for (int i = 0; i < m; ++i) {   // the stages of one fit and the tasks of one sweep share their matrices
+        const gdp_problem *q = p[es[i].orig];
+        es[i].table_of = i;
+        for (int j = i; q->inter_index && j-- > std::max(0, i - 8);) {
             const gdp_problem *o = p[es[j].orig];
             if (o->inter_index && o->inter == q->inter && o->S == q->S && o->n_inter == q->n_inter) {
-                e.table_of = es[j].table_of;
+                es[i].table_of = es[j].table_of;
                 break;
             }
-            if (es.size() - j >= 8) break;
         }
-        es.push_back(std::move(e));
     }
-    if (es.empty()) return GDP_OK;
-    const int m = (int)es.size(), n_lam = m <= 4 ? GDP_BOUND_MAX_LAM : GDP_BOUND_MAX_LAM / 2;
     int max_LS = 0, max_S = 0, max_K = 0, elements = 1, narrow = 1;
     // what is uploaded, what is copied back, what stays on the device
     const size_t off_inst = place(sizeof(GdpBoundInst) * (size_t)m);
     for (int j = 0; j < m; ++j) {
-        Entry &e = es[(size_t)j];
+        BoundEntry &e = es[j];
         const gdp_problem *q = p[e.orig];
         const size_t LS = (size_t)q->L * q->S;
         e.off_mem = place(4 * LS);
@@ -2788,14 +2764,15 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
     const int threads = narrow && (int64_t)m * n_lam * 2 > 1024 ? GDP_BOUND_THREADS / 2 : GDP_BOUND_THREADS;
     const size_t off_pairs = place(sizeof(int2) * pairs.size());
     const size_t up_bytes = at;
-    for (Entry &e : es) {
+    for (int j = 0; j < m; ++j) {
+        BoundEntry &e = es[j];
         const gdp_problem *q = p[e.orig];
         e.off_ub = place(8 * (size_t)q->n_key);
         e.off_keep = place((size_t)q->L * q->S);
     }
     const size_t back_bytes = at - up_bytes;
     for (int j = 0; j < m; ++j) {
-        Entry &e = es[(size_t)j];
+        BoundEntry &e = es[j];
         const gdp_problem *q = p[e.orig];
         const size_t LS = (size_t)q->L * q->S;
         if (e.table_of == j) e.off_inter_t = place(8 * (size_t)e.h.n_inter * q->S * q->S);
@@ -2805,7 +2782,6 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
         e.off_pmem = place(8 * (size_t)n_lam);
         e.off_path = place((size_t)q->L * (size_t)n_lam);
     }
-    if (at > REDUCE_MAX_BYTES || m > 65535) return GDP_OK;
 
     int device = 0;
     GDP_HIP(hipGetDevice(&device));
@@ -2832,8 +2808,8 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
         throw;
     }
     for (int j = 0; j < m; ++j) {
-        Entry &e = es[(size_t)j];
-        const Entry &te = es[(size_t)e.table_of];
+        BoundEntry &e = es[j];
+        const BoundEntry &te = es[e.table_of];
         const gdp_problem *q = p[e.orig];
         const size_t LS = (size_t)q->L * q->S, SS = (size_t)q->S * q->S;
         memcpy(up + e.off_mem, q->mem, 4 * LS);
@@ -2891,7 +2867,7 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
     int rc = err == hipSuccess ? GDP_OK : fail_hip(err, "bounds");
     try {
         for (int j = 0; j < m && rc == GDP_OK; ++j) {
-            const Entry &e = es[(size_t)j];
+            const BoundEntry &e = es[j];
             const gdp_problem *q = p[e.orig];
             const double *ub = reinterpret_cast<const double *>(lane.back + (e.off_ub - up_bytes));
             bool bounded = true;   // a key whose budget no path was found for keeps everything
@@ -2906,6 +2882,62 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
         throw;
     }
     lane_give(lane);
+    return rc;
+}
+
+// Bounds of the instances of a batch that have the form, in consecutive slices of at most `limit` bytes of device
+// memory each; instances that need more by themselves are solved whole.  Initial costs are taken to be zeros; scanned:
+// bytes of them that the calling thread looks through while the device works.
+static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vector<double> &magnitude, size_t scanned,
+                        size_t limit, std::vector<std::unique_ptr<Reduced>> &out)
+{
+    const char *env = getenv("GALVATRON_DP_REDUCE"), *skip = getenv("GALVATRON_DP_SKIP");
+    const bool forced = env && *env && atoi(env) != 0;
+    if ((env && *env && !forced) || (skip && *skip && atoi(skip) == 0)) return GDP_OK;
+    const double total = dense_work(n, p);
+    if (!forced && total * std::min(n, 4) < REDUCE_MIN_WORK) return GDP_OK;
+    if (!forced && !InitialScan::device_bound(total, scanned)) return GDP_OK;
+    std::vector<char> seen(GDP_MAX_S + 1, 0);
+    int groups = 0;
+    for (int i = 0; i < n; ++i) {
+        groups += !seen[(size_t)p[i]->S];
+        seen[(size_t)p[i]->S] = 1;
+    }
+    if (!forced && total * std::min(groups, 4) < REDUCE_MIN_WORK) return GDP_OK;
+
+    std::vector<BoundEntry> es;
+    for (int i = 0; i < n; ++i) {
+        if (!reducible(p[i], magnitude[(size_t)i])) continue;
+        const gdp_problem *q = p[i];
+        BoundEntry e;
+        e.orig = i;
+        int64_t least = 0;
+        for (int l = 0; l < q->L; ++l) least += *std::min_element(q->mem + (size_t)l * q->S, q->mem + (size_t)(l + 1) * q->S);
+        bool any = false;
+        for (int k = 0; k < q->n_key; ++k) {
+            const int64_t b = (int64_t)q->V - 1 - q->other_mem[k];
+            e.budget.push_back(b >= least ? b : -1);
+            any = any || b >= least;
+        }
+        if (!any) continue;
+        e.h.S = q->S;
+        e.h.n_inter = q->inter_index ? q->n_inter : q->L;
+        if (!q->inter_index) share_equal_matrices(q, e.h);
+        es.push_back(std::move(e));
+    }
+    const int n_lam = es.size() <= 4 ? GDP_BOUND_MAX_LAM : GDP_BOUND_MAX_LAM / 2;
+    int rc = GDP_OK;
+    for (size_t begin = 0; begin < es.size() && rc == GDP_OK;) {
+        size_t end = begin, bytes = 0;
+        while (end < es.size() && end - begin < 65535) {
+            const size_t b = bound_bytes(p[es[end].orig], es[end].h, n_lam);
+            if (bytes + b > limit) break;
+            bytes += b;
+            ++end;
+        }
+        if (end > begin) rc = reduce_slice(p, magnitude, es.data() + begin, (int)(end - begin), n_lam, out);
+        begin = std::max(end, begin + 1);
+    }
     return rc;
 }
 
@@ -3030,7 +3062,7 @@ int gdp_solve_batch(int32_t n, const gdp_problem *const *p, gdp_result *const *r
             return rv == GDP_OK ? solve_parts(n, p, r, budget, f0_live, nullptr, nullptr, nullptr) : rv;
         }
         std::vector<std::unique_ptr<Reduced>> small((size_t)n);
-        int rc = reduce_batch(n, p, magnitude, scan.alone(), small);
+        int rc = reduce_batch(n, p, magnitude, scan.alone(), std::min(budget, REDUCE_MAX_BYTES), small);
         if (rc != GDP_OK) return rc;
         std::vector<const gdp_problem *> q(p, p + n);
         std::vector<gdp_result *> qr(r, r + n);

@@ -95,6 +95,36 @@ def test_batch_of_different_shapes_and_shared_tables(monkeypatch):
         _check(x, V, prob, f"instance {n}")
 
 
+def _work(probs):
+    """Relaxations carried out of all a batch stands for."""
+    _lib.batch_stats_begin()
+    _lib.solve_batch(probs)
+    s = _lib.batch_stats_end()
+    assert s.instances == len(probs) and s.relaxations == sum(prob.relaxations for prob in probs)
+    return s.executed / s.relaxations
+
+
+@pytest.mark.parametrize("limit_mb", [32, 1])
+def test_bounds_stay_within_the_largest_allocation(limit_mb, monkeypatch):
+    """40 instances whose bounds take 1.1 MB of device memory each: within GALVATRON_DP_ARENA_MB = 32 they are taken in
+    two slices; with 1 MB, less than an instance needs, all instances are solved whole.  (The first limit is one the
+    device sets as well.)"""
+    rng = np.random.Generator(np.random.PCG64(32))
+    L, S, V = 24, 40, 2500
+    xs = [_instance(rng, L, S, V, "each") for _ in range(40)]
+    probs = [_problem(x, V) for x in xs]
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "0")
+    whole = _work(probs)
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    monkeypatch.setenv("GALVATRON_DP_ARENA_MB", str(limit_mb))
+    if limit_mb == 32:
+        monkeypatch.setenv("GALVATRON_DP_DEVICE_LIMIT_MB", str(limit_mb))
+    done = _work(probs)
+    assert done < 0.3 * whole if limit_mb == 32 else done > 0.7 * whole   # (the tiles of a part are those of its size)
+    for n, (x, prob) in enumerate(zip(xs[::13], probs[::13])):
+        _check(x, V, prob, f"instance {13 * n}")
+
+
 def test_initial_costs_that_are_not_zeros(monkeypatch):
     """The bounds take the initial costs to be zeros; a caller's array with others is solved whole."""
     monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
