@@ -2567,27 +2567,95 @@ struct Reduced {
     std::vector<int32_t> kept;               // [L][S of q] strategy of the whole instance, -1: padding
 };
 
-// Dense relaxations of a batch from which on the bounds are worth their launches (GALVATRON_DP_REDUCE=1 takes them for
-// every instance that has the form, =0 for none).  They take 0.1 (L = 32, S = 44) to 0.2 ms (L = 80, S = 64) and a round
-// trip; per call, whole / reduced: L = 24, S = 22, V = 16384 (1.9e8) 0.16 / 0.27 ms; L = 28, S = 40, V = 29493 (1.3e9)
-// 0.30 / 0.32; L = 32, S = 44, V = 65536 (4e9, no initial costs)
-// 0.67 / 0.29; L = 80, S = 64, V = 131072 (4.3e10) 3.06 / 0.97; L = 48,
-// S = 88, V = 262144 (9.7e10) 10.8 / 1.1; 256 instances of S = 44 49 / 7.8 ms.  Instances of different S run in launches
-// of their own, one after the other, and what is left of them mostly in one: a batch of four S (the 15 stages of a
-// fit, L = 30, S = 37, 19, 10 and 5, V = 23593, 1.3e9) gains from a quarter of the work on, 0.93 / 0.62 ms.
-static constexpr double REDUCE_MIN_WORK = 2e9;
 static constexpr size_t REDUCE_MAX_BYTES = (size_t)4 << 30;   // of device memory for the bounds of a slice (GALVATRON_DP_ARENA_MB if less)
+
+static bool has_bounds_form(const gdp_problem *q)
+{
+    constexpr uint32_t whole = GDP_EXPORT_F | GDP_EXPORT_MARK | GDP_COMPUTE_ALL | GDP_KEEP_MARKS | GDP_LAUNCH_FUSED | GDP_LAUNCH_PER_LAYER;
+    return !(q->flags & whole) && q->L >= 2 && q->L <= GDP_BOUND_MAX_L && q->S >= 2 && q->S <= GDP_BOUND_MAX_S &&
+           q->n_key >= 1 && q->n_key <= GDP_BOUND_MAX_KEY && q->L * q->S <= GDP_BOUND_MAX_LS;
+}
 
 static bool reducible(const gdp_problem *q, double magnitude)
 {
-    constexpr uint32_t whole = GDP_EXPORT_F | GDP_EXPORT_MARK | GDP_COMPUTE_ALL | GDP_KEEP_MARKS | GDP_LAUNCH_FUSED | GDP_LAUNCH_PER_LAYER;
-    if ((q->flags & whole) || q->L < 2 || q->L > GDP_BOUND_MAX_L || q->S < 2 || q->S > GDP_BOUND_MAX_S ||
-        q->n_key < 1 || q->n_key > GDP_BOUND_MAX_KEY || q->L * q->S > GDP_BOUND_MAX_LS || !(magnitude < 1e100))
-        return false;
+    if (!has_bounds_form(q) || !(magnitude < 1e100)) return false;
     // a memory cost of 0 reads the layer's own row: the recurrence is not a path through the layers then
     for (size_t k = 0; k < (size_t)q->L * q->S; ++k)
         if (q->mem[k] == 0) return false;
     return true;
+}
+
+static int bound_multipliers(size_t instances) { return instances <= 4 ? GDP_BOUND_MAX_LAM : GDP_BOUND_MAX_LAM / 2; }
+
+// Share of the strategies of a layer that are cheaper in time than every one that needs no more memory: most others
+// go.  From one layer each of at most 8 instances (batches of 2 to 1000, share of the relaxations left: random costs
+// 0.15 on average and 0.06; costs where memory is traded for time 0.44 and 0.40).
+static double undominated(int32_t n, const gdp_problem *const *p)
+{
+    constexpr int32_t LOOKED_AT = 8;
+    std::vector<std::pair<int32_t, double>> layer;
+    double share = 0;
+    const int32_t m = std::min(n, LOOKED_AT);
+    for (int32_t k = 0; k < m; ++k) {
+        const gdp_problem *q = p[(int64_t)n * k / m];
+        const size_t row = (size_t)(q->L / 2) * q->S;
+        layer.clear();
+        for (int s = 0; s < q->S; ++s) layer.emplace_back(q->mem[row + s], q->intra[row + s]);
+        std::sort(layer.begin(), layer.end());
+        double least = INFINITY;
+        int stay = 0;
+        for (const auto &s : layer) {
+            stay += s.first < q->V && s.second < least;
+            least = s.first < q->V ? std::min(least, s.second) : least;
+        }
+        share += (double)stay / q->S;
+    }
+    return share / m;
+}
+
+// Whether the bounds of a batch are worth their time (GALVATRON_DP_REDUCE=1 takes them for every instance that has the
+// form, =0 for none).  What they can save is the dense recurrence, 10^13 relaxations a second; where the instances
+// have several S it runs in launches of their own, one after the other, which cost as much again up to 0.1 ms each, and
+// what is left of them mostly runs in one.  They cost
+// * a round trip, 0.1 ms, and two chains of max L steps -- the passes, then the DP on what is left --, whatever V is:
+//   5 us a step, 25 us where a thread of a pass has 16 elements (S > 88: 16 us a step of the passes instead of 1.65);
+// * from 1024 passes (2 per multiplier and instance) on the device's time for all steps instead, 1.5 and 13 us;
+// * in batches the host's: layout, matrices of what stays and their upload, 3 ns per transition cost times the share of
+//   strategies that stay at least (undominated); the arrays of a single instance stay in its caches.
+// How much is left is not known before: random costs leave a tenth, 128 equal layers four fifths.  So the line lies
+// where the calls on it gain on average.  Of 4500 calls tried on either side of it 1500 gain, to 0.55 on average, and 250 lose
+// more than 8 % -- those that are not thinned out, mostly a fifth, up to a half, single ones more.  Some of them, ms whole / with bounds, random costs; costs that follow a layout, all layers alike:
+//   L = 24, S = 64   1.0e9 0.25 / 0.26; 0.24 / 0.30    2.0e9 0.38 / 0.29; 0.35 / 0.34    1.0e10 0.92 / 0.33; 0.83 / 0.63
+//   L = 64, S = 64   2.0e9 0.62 / 0.56; 0.57 / 0.67    4.0e9 0.81 / 0.58; 0.80 / 0.93    1.0e10 1.37 / 0.57; 1.43 / 1.00
+//   L = 256, S = 32  4.0e9 1.66 / 1.50; 1.59 / 2.03    1.0e10 2.64 / 1.53; 2.56 / 2.99
+//   L = 32, S = 128  4.0e9 0.90 / 0.95; 0.78 / 1.26    1.0e10 1.51 / 0.96; 1.56 / 1.81
+//   32 x L = 14, S = 40  V = 8000 0.75 / 0.62; 0.76 / 1.08    V = 30000 2.11 / 0.82; 2.23 / 1.73
+//   64 x L = 28, S = 64  V = 8000 5.0 / 2.7; 5.3 / 8.0        16 x L = 28, S = 40, V = 30000 2.02 / 1.19; 2.05 / 2.07
+//   15 stages of a fit, L = 8 to 1, S = 60 to 8, V = 16583 (6.5e8) -; 0.44 / 0.37
+static bool bounds_pay(int32_t n, const gdp_problem *const *p)
+{
+    constexpr double RATE = 1e13, FLOOR = 0.2e-3, STEP = 5e-6, STEP_16 = 25e-6, BUSY = 1.5e-6, BUSY_16 = 13e-6, ENTRY = 3e-9, GROUP = 0.1e-3;
+    double work = 0, layers = 0, entries = 0;
+    int max_L = 0, max_S = 0, groups = 0;
+    uint64_t seen[GDP_MAX_S / 64 + 1] = {};
+    for (int i = 0; i < n; ++i) {
+        const gdp_problem *q = p[i];
+        uint64_t &word = seen[q->S / 64], bit = 1ull << (q->S % 64);
+        groups += !(word & bit);
+        word |= bit;
+        if (!has_bounds_form(q)) continue;
+        const double SS = (double)q->S * q->S;
+        work += (double)q->L * q->V * SS;
+        layers += q->L;
+        entries += q->L * SS;
+        max_L = std::max(max_L, q->L);
+        max_S = std::max(max_S, q->S);
+    }
+    const double dense = work / RATE, save = dense + (std::min(groups, 4) - 1) * std::min(dense, GROUP);
+    if (save < FLOOR) return false;
+    const bool wide = gdp_bound_elements(max_S, GDP_BOUND_THREADS) == 16;
+    const double passes = layers * 2 * bound_multipliers((size_t)n) / 1024;
+    return save >= std::max(max_L * (wide ? STEP_16 : STEP), passes * (wide ? BUSY_16 : BUSY)) + (n > 1 ? entries * ENTRY * undominated(n, p) : 0.0);
 }
 
 // The multipliers of an instance: 0 and a geometric series around (range of times) / (range of memory costs).
@@ -2894,16 +2962,7 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
     const char *env = getenv("GALVATRON_DP_REDUCE"), *skip = getenv("GALVATRON_DP_SKIP");
     const bool forced = env && *env && atoi(env) != 0;
     if ((env && *env && !forced) || (skip && *skip && atoi(skip) == 0)) return GDP_OK;
-    const double total = dense_work(n, p);
-    if (!forced && total * std::min(n, 4) < REDUCE_MIN_WORK) return GDP_OK;
-    if (!forced && !InitialScan::device_bound(total, scanned)) return GDP_OK;
-    std::vector<char> seen(GDP_MAX_S + 1, 0);
-    int groups = 0;
-    for (int i = 0; i < n; ++i) {
-        groups += !seen[(size_t)p[i]->S];
-        seen[(size_t)p[i]->S] = 1;
-    }
-    if (!forced && total * std::min(groups, 4) < REDUCE_MIN_WORK) return GDP_OK;
+    if (!forced && (!bounds_pay(n, p) || !InitialScan::device_bound(dense_work(n, p), scanned))) return GDP_OK;
 
     std::vector<BoundEntry> es;
     for (int i = 0; i < n; ++i) {
@@ -2925,7 +2984,7 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
         if (!q->inter_index) share_equal_matrices(q, e.h);
         es.push_back(std::move(e));
     }
-    const int n_lam = es.size() <= 4 ? GDP_BOUND_MAX_LAM : GDP_BOUND_MAX_LAM / 2;
+    const int n_lam = bound_multipliers(es.size());
     int rc = GDP_OK;
     for (size_t begin = 0; begin < es.size() && rc == GDP_OK;) {
         size_t end = begin, bytes = 0;

@@ -26,6 +26,8 @@ def _instance(rng, L, S, V, kind):
         mem = (mem // 4 + 1).astype(np.int32)
     else:
         intra, inter = rng.lognormal(2.5, 0.5, size=(n, S)), rng.uniform(0, 5, size=(n, S, S))
+    if kind == "trade":                    # what saves memory costs time: few strategies are dominated by another
+        intra = 40.0 * per / mem * rng.uniform(0.98, 1.02, size=mem.shape)
     if kind == "negative":
         intra, inter = intra - 20.0, inter - 2.5
     if kind == "holes":
@@ -102,6 +104,28 @@ def _work(probs):
     s = _lib.batch_stats_end()
     assert s.instances == len(probs) and s.relaxations == sum(prob.relaxations for prob in probs)
     return s.executed / s.relaxations
+
+
+# instances, L, S, V: on the far side of each term of the rule -- too little work, chains of too many steps, steps of
+# 16 elements, too many transition costs that stay in a batch -- and on the near one
+@pytest.mark.parametrize("shape,kind,bounds", [
+    ((1, 24, 40, 30000), "each", False), ((1, 16, 64, 40000), "each", True), ((1, 256, 16, 33000), "each", False),
+    ((1, 40, 64, 30000), "each", True), ((1, 24, 96, 12000), "each", False), ((1, 4, 96, 80000), "each", True),
+    ((64, 14, 40, 4000), "trade", False), ((64, 14, 40, 4000), "each", True), ((8, 14, 24, 45000), "each", True)])
+def test_bounds_are_taken_where_they_pay(shape, kind, bounds, monkeypatch):
+    n, L, S, V = shape
+    rng = np.random.Generator(np.random.PCG64(list(shape)))
+    xs = [_instance(rng, L, S, V, kind) for _ in range(n)]
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "0")
+    whole = [_problem(x, V) for x in xs]
+    all_of_it = _work(whole)
+    monkeypatch.delenv("GALVATRON_DP_REDUCE")
+    probs = [_problem(x, V) for x in xs]
+    done = _work(probs)
+    assert done < 0.5 * all_of_it if bounds else done == all_of_it
+    for a, b in zip(probs, whole):
+        assert a.total.tobytes() == b.total.tobytes()
+        assert np.array_equal(a.remaining, b.remaining) and np.array_equal(a.res, b.res)
 
 
 @pytest.mark.parametrize("limit_mb", [32, 1])
