@@ -218,6 +218,8 @@ void lane_release(Lane &ln)  // the lane's device is current
 // Page-locked memory of at least `bytes` behind *ptr (grown in steps of `grain`, contents not kept).
 hipError_t pinned_reserve(char **ptr, size_t *have, size_t bytes, size_t grain)
 {
+    // test aid: requests above GALVATRON_DP_PINNED_LIMIT_MB are answered like a host that has no page-locked memory left
+    if (getenv("GALVATRON_DP_PINNED_LIMIT_MB") && bytes > env_mb("GALVATRON_DP_PINNED_LIMIT_MB", 0)) return hipErrorOutOfMemory;
     if (*have >= bytes) return hipSuccess;
     if (*ptr) (void)hipHostFree(*ptr);
     *ptr = nullptr;
@@ -2784,6 +2786,24 @@ static size_t bound_bytes(const gdp_problem *q, const HostInst &h, int n_lam)
            NL * (24 + 16 * LS + L) + 256 * ARRAYS;
 }
 
+// What the bounds of a slice work with; given back on every way out, the stream idle.
+struct BoundLease {
+    int device = 0;
+    Lane lane;
+    char *dev = nullptr;
+    size_t dev_bytes = 0;
+    void give_device_memory()
+    {
+        if (dev) arena_give(device, dev, dev_bytes);
+        dev = nullptr;
+    }
+    ~BoundLease()
+    {
+        give_device_memory();
+        lane_give(lane);
+    }
+};
+
 // Bounds of the instances of one slice in one set of launches, and the smaller instances that follow (out[i] stays
 // empty where instance i is solved whole).
 static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &magnitude, BoundEntry *es, int m, int n_lam,
@@ -2851,29 +2871,22 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
         e.off_path = place((size_t)q->L * (size_t)n_lam);
     }
 
-    int device = 0;
-    GDP_HIP(hipGetDevice(&device));
-    Lane lane;
-    char *dev = nullptr;
-    size_t dev_bytes = 0;
-    GDP_HIP(lane_take(device, back_bytes, up_bytes, &lane));
-    hipError_t err = arena_take(device, at, &dev, &dev_bytes);
-    if (err != hipSuccess) {
+    // A device or a host that is out of memory solves the instances whole, in the parts that fit; what else may be
+    // wrong with the device is found, and reported, there.
+    BoundLease lease;
+    if (hipGetDevice(&lease.device) != hipSuccess || lane_take(lease.device, back_bytes, up_bytes, &lease.lane) != hipSuccess ||
+        arena_take(lease.device, at, &lease.dev, &lease.dev_bytes) != hipSuccess) {
         (void)hipGetLastError();
-        lane_give(lane);
-        return GDP_OK;   // a device this full solves the instances whole, in the parts that fit
+        lease.dev = nullptr;
+        return GDP_OK;
     }
+    const Lane &lane = lease.lane;
+    char *const dev = lease.dev;
     std::vector<char> pageable;
     char *up = lane.up;
-    try {
-        if (lane.up_bytes < up_bytes) {
-            pageable.resize(up_bytes);
-            up = pageable.data();
-        }
-    } catch (const std::bad_alloc &) {
-        arena_give(device, dev, dev_bytes);
-        lane_give(lane);
-        throw;
+    if (lane.up_bytes < up_bytes) {
+        pageable.resize(up_bytes);
+        up = pageable.data();
     }
     for (int j = 0; j < m; ++j) {
         BoundEntry &e = es[j];
@@ -2915,7 +2928,7 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
         std::lock_guard<std::mutex> lk(g_stats_mu);
         stats = g_stats_on;
     }
-    err = hipMemcpyAsync(dev, up, up_bytes, hipMemcpyHostToDevice, lane.stream);
+    hipError_t err = hipMemcpyAsync(dev, up, up_bytes, hipMemcpyHostToDevice, lane.stream);
     if (err == hipSuccess && stats) err = hipEventRecord(lane.ev_begin, lane.stream);
     if (err == hipSuccess)
         err = gdp_launch_bounds(reinterpret_cast<const GdpBoundInst *>(dev + off_inst), m, n_lam, max_LS, max_S, max_K,
@@ -2931,26 +2944,20 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
         std::lock_guard<std::mutex> lk(g_stats_mu);
         g_stats.device_ms += ms;
     }
-    arena_give(device, dev, dev_bytes);
-    int rc = err == hipSuccess ? GDP_OK : fail_hip(err, "bounds");
-    try {
-        for (int j = 0; j < m && rc == GDP_OK; ++j) {
-            const BoundEntry &e = es[j];
-            const gdp_problem *q = p[e.orig];
-            const double *ub = reinterpret_cast<const double *>(lane.back + (e.off_ub - up_bytes));
-            bool bounded = true;   // a key whose budget no path was found for keeps everything
-            for (int k = 0; k < q->n_key; ++k) bounded = bounded && (e.budget[(size_t)k] < 0 || ub[k] < INFINITY);
-            if (!bounded) continue;
-            std::unique_ptr<Reduced> d(new Reduced());
-            if (build_reduced(q, e.h, reinterpret_cast<const uint8_t *>(lane.back + (e.off_keep - up_bytes)), e.budget.data(), *d))
-                out[(size_t)e.orig] = std::move(d);
-        }
-    } catch (const std::bad_alloc &) {
-        lane_give(lane);
-        throw;
+    lease.give_device_memory();
+    if (err != hipSuccess) return fail_hip(err, "bounds");
+    for (int j = 0; j < m; ++j) {
+        const BoundEntry &e = es[j];
+        const gdp_problem *q = p[e.orig];
+        const double *ub = reinterpret_cast<const double *>(lane.back + (e.off_ub - up_bytes));
+        bool bounded = true;   // a key whose budget no path was found for keeps everything
+        for (int k = 0; k < q->n_key; ++k) bounded = bounded && (e.budget[(size_t)k] < 0 || ub[k] < INFINITY);
+        if (!bounded) continue;
+        std::unique_ptr<Reduced> d(new Reduced());
+        if (build_reduced(q, e.h, reinterpret_cast<const uint8_t *>(lane.back + (e.off_keep - up_bytes)), e.budget.data(), *d))
+            out[(size_t)e.orig] = std::move(d);
     }
-    lane_give(lane);
-    return rc;
+    return GDP_OK;
 }
 
 // Bounds of the instances of a batch that have the form, in consecutive slices of at most `limit` bytes of device
@@ -3121,7 +3128,11 @@ int gdp_solve_batch(int32_t n, const gdp_problem *const *p, gdp_result *const *r
             return rv == GDP_OK ? solve_parts(n, p, r, budget, f0_live, nullptr, nullptr, nullptr) : rv;
         }
         std::vector<std::unique_ptr<Reduced>> small((size_t)n);
-        int rc = reduce_batch(n, p, magnitude, scan.alone(), std::min(budget, REDUCE_MAX_BYTES), small);
+        int rc = GDP_OK;
+        try {
+            rc = reduce_batch(n, p, magnitude, scan.alone(), std::min(budget, REDUCE_MAX_BYTES), small);
+        } catch (const std::bad_alloc &) {   // instances without bounds by then are solved whole, which takes less
+        }
         if (rc != GDP_OK) return rc;
         std::vector<const gdp_problem *> q(p, p + n);
         std::vector<gdp_result *> qr(r, r + n);

@@ -149,6 +149,25 @@ def test_bounds_stay_within_the_largest_allocation(limit_mb, monkeypatch):
         _check(x, V, prob, f"instance {13 * n}")
 
 
+def test_no_page_locked_memory_for_the_bounds(monkeypatch):
+    """260 instances whose marks of what stays are 1.7 MB, and whose results are less than the 1 MB that can be had:
+    solved whole, in two parts.  (The inputs of a part, 18 MB and more, are laid out in ordinary memory anyway.)"""
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    monkeypatch.setenv("GALVATRON_DP_PINNED_LIMIT_MB", "1")
+    rng = np.random.Generator(np.random.PCG64(260))
+    L, S, V, n = 60, 100, 200, 260
+    tables = rng.uniform(0, 5, size=(1, S, S))
+    index = np.zeros(L, np.int32)
+    mem, intra, _, om, ot = _instance(rng, L, S, V, "same")
+    keys = sorted(om)
+    probs = []
+    for i in range(n):
+        probs.append(_lib.Problem(mem, np.roll(intra, i, axis=1), tables, V, [om[k] for k in keys], [ot[k] for k in keys], inter_index=index))
+    _lib.solve_batch(probs)
+    for i in (0, 17, n - 1):
+        _check((mem, probs[i].intra, np.repeat(tables, L, 0), om, ot), V, probs[i], f"instance {i}")
+
+
 def test_initial_costs_that_are_not_zeros(monkeypatch):
     """The bounds take the initial costs to be zeros; a caller's array with others is solved whole."""
     monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
