@@ -666,11 +666,14 @@ namespace {
 // Looks through the initial costs of a batch for anything but zeros, on threads beside the one that prepares and
 // waits for the device: one thread reads 35 GB/s from memory, so the 184 MB of a call with S = 88, V = 262144 took 4.5 ms
 // of its own once the device needed less.  The arrays are cut into pieces that the threads draw from a counter; the
-// caller helps with what is left when it needs the answer, so a thread that could not be had only costs time.  One
-// thread per 4 MB, at most 7 and what the machine has, from 64 MB on.  An array that fits the caller's last-level cache
-// stays with the caller: lines that other cores have read are slow to write again, and a caller who fills the next
-// array into the same memory pays more than the scan gains (S = 44, V = 65536, 23 MB: the call 1.04 -> 0.48 ms, filling
-// the next array 0.98 -> 1.90 ms).  At 184 MB: the call 4.5 -> 1.1 ms, filling as before (9.6 and 9.8 ms).
+// caller helps with what is left when it needs the answer, so a thread that could not be had only costs time.  7 threads
+// (GALVATRON_DP_SCAN_THREADS: so many, 0 for none) where the machine has them, from 64 MB on.  Lines that other cores
+// have read are slow to write again, and a caller who fills the next array into the same memory waits for that.  An
+// array that fits the caller's last-level cache stays with the caller, since more is lost there than the scan gains (S = 44,
+// V = 65536, 23 MB: the call 1.04 -> 0.48 ms, filling the next array 0.98 -> 1.90 ms).  Larger ones lose less than the
+// call gains, in ms without bounds and helpers -> with both: the call; filling the same array; np.full of a new one
+//   67 MB  2.6 -> 1.2;  1.6 -> 3.2;  2.9 -> 4.0      102 MB  6.1 -> 1.3;  2.5 -> 5.1;  4.8 -> 6.4
+//   185 MB 9.6 -> 1.5;  4.6 -> 9.0;  8.6 -> 11.4
 class InitialScan {
 public:
     void start(int32_t n, const gdp_problem *const *p, double relaxations)
@@ -684,7 +687,8 @@ public:
         }
         if (found() || bytes_ < HELPED_FROM || !device_bound(relaxations, bytes_)) return;
         const size_t cores = std::max(1u, std::thread::hardware_concurrency());
-        const size_t want = std::min({bytes_ >> 22, cores - 1, (size_t)7});
+        const char *env = getenv("GALVATRON_DP_SCAN_THREADS");
+        const size_t want = std::min(cores - 1, env && *env ? (size_t)std::max(0, std::min(atoi(env), 64)) : HELPERS);
         helpers_.reserve(want);
         try {
             for (size_t k = 0; k < want; ++k) helpers_.emplace_back([this] { work(); });
@@ -713,7 +717,7 @@ public:
     }
 
 private:
-    static constexpr size_t HELPED_FROM = (size_t)64 << 20;
+    static constexpr size_t HELPED_FROM = (size_t)64 << 20, HELPERS = 7;
     static constexpr size_t PIECE = (size_t)1 << 16;   // doubles: half a megabyte
     struct Piece {
         const double *at;

@@ -137,7 +137,11 @@ int gdp_solve(const gdp_problem *p, gdp_result *r);
  * bsz x chunk sweep: the DPAlg.fit calls issued from dynamic_programming.py:446-488 and
  * search_engine.py:477-498) with one launch grid per layer index.  A batch whose cost buffers would
  * exceed GALVATRON_DP_ARENA_MB (default 8192) of device memory is solved in consecutive parts that
- * reuse one allocation. */
+ * reuse one allocation.
+ * Where it pays, strategies that no best path can use are taken out of an instance by lower bounds before it is
+ * solved (GALVATRON_DP_REDUCE=0: never); the results are those of the whole instance, bit for bit.
+ * f0 arrays of 64 MB or more in all may be read by up to 7 threads that the call starts and joins before it
+ * returns, on every path (GALVATRON_DP_SCAN_THREADS=n: at most n, 0: only the calling thread reads them). */
 int gdp_solve_batch(int32_t n, const gdp_problem *const *p, gdp_result *const *r);
 
 /* gdp_solve for callers that cannot allocate.  No counterpart in the reference: it exists for callers that
@@ -231,9 +235,11 @@ void gdp_debug_shared_device(int32_t seems_shared);
  * part to its last one: relaxation launches and backtrack), so the host's share of a sweep's wall time is
  * what is left of the wall clock. */
 typedef struct gdp_batch_stats {
-    double relaxations;   /* sum over the solved instances of L*V*S*S                      */
-    double executed;      /* of those, carried out (see gdp_timing.executed)               */
-    double device_ms;     /* sum over the parts of first kernel -> last kernel              */
+    double relaxations;   /* sum over the solved instances of L*V*S*S, as the caller gave them; what initial costs
+                             that were found late made the call solve again counts again    */
+    double executed;      /* of those, carried out (see gdp_timing.executed); where strategies were taken out by
+                             bounds, those of the smaller instance that was solved          */
+    double device_ms;     /* sum over the parts of first kernel -> last kernel, and of the bounds' kernels */
     int64_t instances;
     int64_t parts;        /* plans (a batch above GALVATRON_DP_ARENA_MB is solved in parts) */
     int64_t flow_parts, fused_parts, per_layer_parts; /* by launch scheme of the run        */

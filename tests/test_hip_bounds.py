@@ -234,3 +234,23 @@ def test_large_initial_costs(shape, at):
     plan.fetch()
     assert got.total.tobytes() == want.total.tobytes()
     assert np.array_equal(got.remaining, want.remaining) and np.array_equal(got.res, want.res)
+
+
+@pytest.mark.parametrize("threads", ["0", "1", "64"])
+def test_as_many_helper_threads_as_told(threads, monkeypatch):
+    """GALVATRON_DP_SCAN_THREADS: none, one and more than the machine may have look through the array as the caller's
+    thread does, a single value included."""
+    L, S, V = 36, 96, 88000
+    mem, intra, inter, om, ot = _instance(np.random.Generator(np.random.PCG64([L, V])), L, S, V, "each")
+    keys = sorted(om)
+    f0 = np.zeros((V, S))
+
+    def solved():
+        prob = _lib.Problem(mem, intra, inter, V, [om[k] for k in keys], [ot[k] for k in keys], f0=f0)
+        _lib.solve_batch([prob])
+        return prob.total.tobytes(), prob.remaining.tobytes(), prob.res.tobytes()
+    zeros = solved()
+    monkeypatch.setenv("GALVATRON_DP_SCAN_THREADS", threads)
+    assert solved() == zeros
+    f0[50000, 7] = -300.0
+    assert solved()[0] != zeros[0]
