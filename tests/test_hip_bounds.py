@@ -106,6 +106,27 @@ def _work(probs):
     return s.executed / s.relaxations
 
 
+# The limits of the form -- layers, strategies, both together, keys -- and one beyond each; costs that trade memory
+# for time.  Compared with the whole instance, which other tests compare with the oracle.
+@pytest.mark.parametrize("L,S,V,keys,kind,taken", [
+    (512, 24, 6000, 3, "each", True), (513, 24, 6000, 3, "each", False), (512, 80, 3000, 2, "each", True), (320, 128, 3000, 2, "each", True),
+    (321, 128, 3000, 2, "each", False), (12, 128, 4000, 2, "each", True), (12, 129, 4000, 2, "each", False), (16, 40, 4000, 8, "each", True),
+    (16, 40, 4000, 9, "each", False), (16, 40, 8000, 1, "trade", True), (24, 64, 12000, 4, "trade", True), (6, 89, 9000, 3, "trade", True)])
+def test_bounds_take_part_up_to_their_limits(L, S, V, keys, kind, taken, monkeypatch):
+    rng = np.random.Generator(np.random.PCG64([L, S, keys]))
+    mem, intra, inter, _, _ = _instance(rng, L, S, V, kind)
+    om, ot = [V // 3 * k // keys for k in range(keys)], [float(k) for k in range(keys)]
+    probs = [_lib.Problem(mem, intra, inter, V, om, ot) for _ in range(2)]
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "0")
+    whole = _work(probs[:1])
+    assert np.isfinite(probs[0].total).all()
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    done = _work(probs[1:])
+    assert done < 0.6 * whole if taken else done == whole
+    assert probs[0].total.tobytes() == probs[1].total.tobytes()
+    assert np.array_equal(probs[0].remaining, probs[1].remaining) and np.array_equal(probs[0].res, probs[1].res)
+
+
 # instances, L, S, V: on the far side of each term of the rule -- too little work, chains of too many steps, steps of
 # 16 elements, too many transition costs that stay in a batch -- and on the near one
 @pytest.mark.parametrize("shape,kind,bounds", [
