@@ -626,6 +626,27 @@ static bool scan_costs(const double *q, size_t n, double *maxabs)
     return b == 0;
 }
 
+// Whether n doubles hold anything but +0.0.  64 at a time, each block's words ORed in full before the next look at the
+// result: one running OR per word read took 1.4 times as long where the array is in the caches (S = 15, V = 61099,
+// 7 MB: a call 0.11 -> 0.15 ms).
+static bool any_bits(const double *q, size_t n)
+{
+    uint64_t any = 0;
+    size_t k = 0;
+    for (; k + 64 <= n && !any; k += 64)
+        for (int j = 0; j < 64; ++j) {
+            uint64_t w;
+            memcpy(&w, q + k + j, sizeof w);
+            any |= w;
+        }
+    for (; k < n && !any; ++k) {
+        uint64_t w;
+        memcpy(&w, q + k, sizeof w);
+        any |= w;
+    }
+    return any != 0;
+}
+
 // The caller's initial costs (gdp_problem.f0): *live says whether anything but +0.0 is in there (an array of
 // zeros is what every caller of the reference passes, and is treated like no array), *maxabs the largest
 // finite magnitude.  The common case is one pass over the array that ORs its words.
@@ -635,23 +656,10 @@ static int scan_f0(const gdp_problem *p, bool *live, double *maxabs)
     *maxabs = 0;
     if (!p->f0) return 0;
     const size_t n = (size_t)p->V * (size_t)p->S;
-    uint64_t any = 0;
-    size_t k = 0;
-    for (; k + 64 <= n && !any; k += 64)
-        for (int j = 0; j < 64; ++j) {
-            uint64_t w;
-            memcpy(&w, p->f0 + k + j, sizeof w);
-            any |= w;
-        }
-    for (; k < n && !any; ++k) {
-        uint64_t w;
-        memcpy(&w, p->f0 + k, sizeof w);
-        any |= w;
-    }
-    if (!any) return 0;
+    if (!any_bits(p->f0, n)) return 0;
     *live = true;
     double m = 0;
-    for (k = 0; k < n; ++k) {
+    for (size_t k = 0; k < n; ++k) {
         const double x = p->f0[k];
         if (x != x || x == -INFINITY) return 1;
         if (x == 0 && std::signbit(x)) return 2;
@@ -741,13 +749,7 @@ private:
         while (!found()) {
             const size_t k = next_.fetch_add(1, std::memory_order_relaxed);
             if (k >= pieces_.size()) return;
-            uint64_t any = 0;
-            for (size_t j = 0; j < pieces_[k].n; ++j) {
-                uint64_t w;
-                memcpy(&w, pieces_[k].at + j, sizeof w);
-                any |= w;
-            }
-            if (any) found_.store(true, std::memory_order_relaxed);
+            if (any_bits(pieces_[k].at, pieces_[k].n)) found_.store(true, std::memory_order_relaxed);
         }
     }
     void join()
