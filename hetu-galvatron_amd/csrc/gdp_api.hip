@@ -258,7 +258,9 @@ hipError_t lane_take(int device, size_t back_bytes, size_t up_bytes, Lane *out)
         if (e == hipSuccess) e = hipEventCreateWithFlags(&ln.ev_side, hipEventDisableTiming);
     }
     if (e == hipSuccess) e = pinned_reserve(&ln.back, &ln.back_bytes, back_bytes, 65536);
-    if (e == hipSuccess && up_bytes <= UPLOAD_PINNED_MAX) e = pinned_reserve(&ln.up, &ln.up_bytes, up_bytes, (size_t)1 << 20);
+    // (without page-locked memory for them the inputs are laid out in ordinary memory)
+    if (e == hipSuccess && up_bytes <= UPLOAD_PINNED_MAX && pinned_reserve(&ln.up, &ln.up_bytes, up_bytes, (size_t)1 << 20) != hipSuccess)
+        (void)hipGetLastError();
     if (e != hipSuccess) {
         lane_release(ln);
         return e;
@@ -711,6 +713,15 @@ public:
     bool found() const { return found_.load(std::memory_order_relaxed); }
     // bytes that the calling thread has to look through by itself
     size_t alone() const { return helpers_.empty() ? bytes_ : 0; }
+    // Looks through one piece; false: nothing is left, or found.
+    bool step()
+    {
+        if (found()) return false;
+        const size_t k = next_.fetch_add(1, std::memory_order_relaxed);
+        if (k >= pieces_.size()) return false;
+        if (any_bits(pieces_[k].at, pieces_[k].n)) found_.store(true, std::memory_order_relaxed);
+        return true;
+    }
     // true: some array holds more than zeros
     bool finish()
     {
@@ -746,11 +757,7 @@ private:
     }
     void work()
     {
-        while (!found()) {
-            const size_t k = next_.fetch_add(1, std::memory_order_relaxed);
-            if (k >= pieces_.size()) return;
-            if (any_bits(pieces_[k].at, pieces_[k].n)) found_.store(true, std::memory_order_relaxed);
-        }
+        while (step()) {}
     }
     void join()
     {
@@ -1518,7 +1525,7 @@ int PlanBuilder::take_stage()
         const hipError_t e = lane_take(pl->device, pl->back_bytes, small_bytes, &pl->lane);
         if (e == hipErrorOutOfMemory || e == hipErrorMemoryAllocation) {
             (void)hipGetLastError();
-            return fail(GDP_E_NOMEM, "page-locked host memory for inputs and results");
+            return fail(GDP_E_NOMEM, "page-locked host memory for results");
         }
         GDP_HIP(e);
         pl->stream = pl->lane.stream;
@@ -1526,7 +1533,7 @@ int PlanBuilder::take_stage()
         pl->ev_end = pl->lane.ev_end;
     }
     stage.p = pl->lane.up;
-    if (small_bytes > UPLOAD_PINNED_MAX || pl->dry) {
+    if (small_bytes > pl->lane.up_bytes || small_bytes > UPLOAD_PINNED_MAX || pl->dry) {
         try {
             pl->stage.assign(small_bytes, 0);
         } catch (const std::bad_alloc &) {
@@ -2573,6 +2580,8 @@ struct Reduced {
     std::vector<double> intra, inter, total;
     std::vector<int64_t> other_mem, spare;   // per key: budget beyond the cap
     std::vector<int32_t> kept;               // [L][S of q] strategy of the whole instance, -1: padding
+    bool solved = false;                     // total, remaining and res are those of the whole instance already
+    double executed = 0;                     // ... and so many candidates were looked at
 };
 
 static constexpr size_t REDUCE_MAX_BYTES = (size_t)4 << 30;   // of device memory for the bounds of a slice (GALVATRON_DP_ARENA_MB if less)
@@ -2593,7 +2602,7 @@ static bool reducible(const gdp_problem *q, double magnitude)
     return true;
 }
 
-static int bound_multipliers(size_t instances) { return instances <= 4 ? GDP_BOUND_MAX_LAM : GDP_BOUND_MAX_LAM / 2; }
+static int bound_multipliers(size_t instances) { return instances <= 32 ? GDP_BOUND_MAX_LAM : GDP_BOUND_MAX_LAM / 2; }
 
 // Share of the strategies of a layer that are cheaper in time than every one that needs no more memory: most others
 // go.  From one layer each of at most 8 instances (batches of 2 to 1000, share of the relaxations left: random costs
@@ -2661,7 +2670,7 @@ static bool bounds_pay(int32_t n, const gdp_problem *const *p)
     }
     const double dense = work / RATE, save = dense + (std::min(groups, 4) - 1) * std::min(dense, GROUP);
     if (save < FLOOR) return false;
-    const bool wide = gdp_bound_elements(max_S, GDP_BOUND_THREADS) == 16;
+    const bool wide = max_S > 88;
     const double passes = layers * 2 * bound_multipliers((size_t)n) / 1024;
     return save >= std::max(max_L * (wide ? STEP_16 : STEP), passes * (wide ? BUSY_16 : BUSY)) + (n > 1 ? entries * ENTRY * undominated(n, p) : 0.0);
 }
@@ -2780,16 +2789,17 @@ struct BoundEntry {
     int orig, table_of;   // table_of: the entry of the slice whose matrices this one reads
     HostInst h;
     std::vector<int64_t> budget;
-    size_t off_mem, off_intra, off_inter, off_index, off_lam, off_budget, off_inter_t, off_P, off_Q, off_time, off_pmem, off_path, off_ub, off_keep;
+    size_t off_mem, off_intra, off_inter, off_index, off_lam, off_budget, off_inter_f, off_inter_t, off_P, off_Q, off_P_mem, off_Q_mem, off_end,
+        off_window, off_ub, off_keep, off_other_time, off_out, off_res, off_hist, off_hist_mem, off_hist_turns, off_hist_intra;
 };
 
 // Device memory that the bounds of an instance take at most, with matrices of its own.
 static size_t bound_bytes(const gdp_problem *q, const HostInst &h, int n_lam)
 {
     const size_t L = (size_t)q->L, LS = L * q->S, T = (size_t)h.n_inter, K = (size_t)q->n_key, NL = (size_t)n_lam;
-    constexpr size_t ARRAYS = 16;   // aligned to 256 bytes each
-    return sizeof(GdpBoundInst) + T * sizeof(int2) + 13 * LS + 4 * L + 16 * K + 16 * T * (size_t)q->S * q->S +
-           NL * (24 + 16 * LS + L) + 256 * ARRAYS;
+    constexpr size_t ARRAYS = 28;   // aligned to 256 bytes each
+    return sizeof(GdpBoundInst) + T * sizeof(int2) + 13 * LS + 4 * L + 28 * K + 24 * T * (size_t)q->S * q->S +
+           NL * (16 + 24 * LS) + sizeof(GdpFrontierOut) + 4 * K * L + 24 * L * GDP_FRONTIER_LABELS + 12 * GDP_FRONTIER_KEPT + 256 * ARRAYS;
 }
 
 // What the bounds of a slice work with; given back on every way out, the stream idle.
@@ -2810,10 +2820,11 @@ struct BoundLease {
     }
 };
 
-// Bounds of the instances of one slice in one set of launches, and the smaller instances that follow (out[i] stays
-// empty where instance i is solved whole).
+// Bounds of the instances of one slice in one set of launches, and behind them the DP over what stays.  out[i]: the
+// results of instance i; the smaller instance that is left of it where its labels are too many; empty where it is to be
+// solved whole.  The calling thread looks through initial costs while the device works.
 static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &magnitude, BoundEntry *es, int m, int n_lam,
-                        std::vector<std::unique_ptr<Reduced>> &out)
+                        InitialScan &scan, std::vector<std::unique_ptr<Reduced>> &out)
 {
     std::vector<int2> pairs;
     size_t at = 0;
@@ -2829,7 +2840,7 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
             }
         }
     }
-    int max_LS = 0, max_S = 0, max_K = 0, elements = 1, narrow = 1;
+    int max_LS = 0, max_S = 0, max_K = 0;
     // what is uploaded, what is copied back, what stays on the device
     const size_t off_inst = place(sizeof(GdpBoundInst) * (size_t)m);
     for (int j = 0; j < m; ++j) {
@@ -2841,6 +2852,7 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
         e.off_index = place(4 * (size_t)q->L);
         e.off_lam = place(8 * (size_t)n_lam);
         e.off_budget = place(8 * (size_t)q->n_key);
+        e.off_other_time = place(8 * (size_t)q->n_key);
         if (e.table_of == j) {
             e.off_inter = place(8 * (size_t)e.h.n_inter * q->S * q->S);
             for (int t = 0; t < e.h.n_inter; ++t) pairs.push_back(make_int2(j, t));
@@ -2848,33 +2860,38 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
         max_LS = std::max(max_LS, (int)LS);
         max_S = std::max(max_S, q->S);
         max_K = std::max(max_K, q->n_key);
-        const int half = gdp_bound_elements(q->S, GDP_BOUND_THREADS / 2);
-        elements = std::max(elements, gdp_bound_elements(q->S, GDP_BOUND_THREADS));
-        narrow = narrow && half ? std::max(narrow, half) : 0;
     }
-    // With more passes than the device holds at a time what counts is not the chain of a pass but how many run
-    // side by side: half as many threads and few enough registers for
-    // four passes per compute unit (256 instances of S = 44, L = 32: 1.67 -> 0.65 ms).
-    const int threads = narrow && (int64_t)m * n_lam * 2 > 1024 ? GDP_BOUND_THREADS / 2 : GDP_BOUND_THREADS;
     const size_t off_pairs = place(sizeof(int2) * pairs.size());
     const size_t up_bytes = at;
     for (int j = 0; j < m; ++j) {
         BoundEntry &e = es[j];
         const gdp_problem *q = p[e.orig];
-        e.off_ub = place(8 * (size_t)q->n_key);
-        e.off_keep = place((size_t)q->L * q->S);
+        e.off_out = place(sizeof(GdpFrontierOut));
+        e.off_res = place(4 * (size_t)q->n_key * q->L);
     }
-    const size_t back_bytes = at - up_bytes;
+    const size_t back_bytes = at - up_bytes, keep_begin = at;
+    for (int j = 0; j < m; ++j) es[j].off_keep = place((size_t)p[es[j].orig]->L * p[es[j].orig]->S);
+    const size_t keep_bytes = at - keep_begin;
     for (int j = 0; j < m; ++j) {
         BoundEntry &e = es[j];
         const gdp_problem *q = p[e.orig];
         const size_t LS = (size_t)q->L * q->S;
-        if (e.table_of == j) e.off_inter_t = place(8 * (size_t)e.h.n_inter * q->S * q->S);
+        if (e.table_of == j) {
+            e.off_inter_f = place(8 * (size_t)e.h.n_inter * q->S * q->S);
+            e.off_inter_t = place(8 * (size_t)e.h.n_inter * q->S * q->S);
+        }
         e.off_P = place(8 * LS * (size_t)n_lam);
         e.off_Q = place(8 * LS * (size_t)n_lam);
-        e.off_time = place(8 * (size_t)n_lam);
-        e.off_pmem = place(8 * (size_t)n_lam);
-        e.off_path = place((size_t)q->L * (size_t)n_lam);
+        e.off_P_mem = place(4 * LS * (size_t)n_lam);
+        e.off_Q_mem = place(4 * LS * (size_t)n_lam);
+        e.off_end = place(8 * (size_t)n_lam);
+        e.off_window = place(4 * (size_t)q->n_key);
+        e.off_ub = place(8 * (size_t)q->n_key);
+        const size_t labels = (size_t)q->L * GDP_FRONTIER_LABELS;
+        e.off_hist = place(sizeof(GdpFrontierLabel) * labels);
+        e.off_hist_turns = place(8 * labels);
+        e.off_hist_mem = place(4 * GDP_FRONTIER_KEPT);
+        e.off_hist_intra = place(8 * GDP_FRONTIER_KEPT);
     }
 
     // A device or a host that is out of memory solves the instances whole, in the parts that fit; what else may be
@@ -2904,28 +2921,40 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
         for (int l = 0; l < q->L; ++l) reinterpret_cast<int32_t *>(up + e.off_index)[l] = e.h.matrix(q, l);
         multipliers(q, n_lam, reinterpret_cast<double *>(up + e.off_lam));
         memcpy(up + e.off_budget, e.budget.data(), 8 * e.budget.size());
+        memcpy(up + e.off_other_time, q->other_time, 8 * e.budget.size());
         if (e.table_of == j)
             for (int t = 0; t < e.h.n_inter; ++t) memcpy(up + e.off_inter + 8 * SS * (size_t)t, e.h.matrix_at(q, t), 8 * SS);
         GdpBoundInst b;
         b.mem = reinterpret_cast<const int32_t *>(dev + e.off_mem);
         b.intra = reinterpret_cast<const double *>(dev + e.off_intra);
         b.inter = reinterpret_cast<const double *>(dev + te.off_inter);
-        b.inter_t = reinterpret_cast<const double *>(dev + te.off_inter_t);
+        b.inter_f = reinterpret_cast<double *>(dev + te.off_inter_f);
+        b.inter_t = reinterpret_cast<double *>(dev + te.off_inter_t);
         b.index = reinterpret_cast<const int32_t *>(dev + e.off_index);
         b.lam = reinterpret_cast<const double *>(dev + e.off_lam);
         b.budget = reinterpret_cast<const int64_t *>(dev + e.off_budget);
         b.P = reinterpret_cast<double *>(dev + e.off_P);
         b.Q = reinterpret_cast<double *>(dev + e.off_Q);
-        b.path_time = reinterpret_cast<double *>(dev + e.off_time);
-        b.path_mem = reinterpret_cast<int64_t *>(dev + e.off_pmem);
-        b.path = reinterpret_cast<uint8_t *>(dev + e.off_path);
-        b.ub = reinterpret_cast<double *>(dev + e.off_ub);
+        b.P_mem = reinterpret_cast<uint32_t *>(dev + e.off_P_mem);
+        b.Q_mem = reinterpret_cast<uint32_t *>(dev + e.off_Q_mem);
+        b.end = reinterpret_cast<double *>(dev + e.off_end);
+        b.ub = reinterpret_cast<unsigned long long *>(dev + e.off_ub);
+        b.window = reinterpret_cast<int32_t *>(dev + e.off_window);
         b.keep = reinterpret_cast<uint8_t *>(dev + e.off_keep);
+        b.other_time = reinterpret_cast<const double *>(dev + e.off_other_time);
+        b.hist = reinterpret_cast<GdpFrontierLabel *>(dev + e.off_hist);
+        b.hist_mem = reinterpret_cast<int32_t *>(dev + e.off_hist_mem);
+        b.hist_turns = reinterpret_cast<double *>(dev + e.off_hist_turns);
+        b.hist_intra = reinterpret_cast<double *>(dev + e.off_hist_intra);
+        b.out = reinterpret_cast<GdpFrontierOut *>(dev + e.off_out);
+        b.res = reinterpret_cast<int32_t *>(dev + e.off_res);
+        b.n_hist = b.n_hist_turns = q->L * GDP_FRONTIER_LABELS;
         b.magnitude = magnitude[(size_t)e.orig];
         b.L = q->L;
         b.V = q->V;
         b.S = q->S;
         b.K = q->n_key;
+        b.T = te.h.n_inter;
         memcpy(up + off_inst + sizeof b * (size_t)j, &b, sizeof b);
     }
     memcpy(up + off_pairs, pairs.data(), sizeof(int2) * pairs.size());
@@ -2938,12 +2967,21 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
     if (err == hipSuccess && stats) err = hipEventRecord(lane.ev_begin, lane.stream);
     if (err == hipSuccess)
         err = gdp_launch_bounds(reinterpret_cast<const GdpBoundInst *>(dev + off_inst), m, n_lam, max_LS, max_S, max_K,
-                                threads == GDP_BOUND_THREADS ? elements : narrow, threads,
                                 reinterpret_cast<const int2 *>(dev + off_pairs), (int)pairs.size(), lane.stream);
+    if (err == hipSuccess) err = gdp_launch_frontier(reinterpret_cast<const GdpBoundInst *>(dev + off_inst), m, max_K, lane.stream);
     if (err == hipSuccess && stats) err = hipEventRecord(lane.ev_end, lane.stream);
     if (err == hipSuccess) err = hipMemcpyAsync(lane.back, dev + up_bytes, back_bytes, hipMemcpyDeviceToHost, lane.stream);
-    const hipError_t es2 = hipStreamSynchronize(lane.stream);
+    while (scan.step() && hipStreamQuery(lane.stream) == hipErrorNotReady) {}
+    hipError_t es2 = hipStreamSynchronize(lane.stream);
     if (err == hipSuccess) err = es2;
+    std::vector<char> keep;
+    for (int j = 0; j < m && err == hipSuccess && keep.empty(); ++j)
+        if (reinterpret_cast<const GdpFrontierOut *>(lane.back + (es[j].off_out - up_bytes))->status > 1) {
+            keep.resize(keep_bytes);
+            err = hipMemcpyAsync(keep.data(), dev + keep_begin, keep_bytes, hipMemcpyDeviceToHost, lane.stream);
+            es2 = hipStreamSynchronize(lane.stream);
+            if (err == hipSuccess) err = es2;
+        }
     float ms = 0;
     if (err == hipSuccess && stats) err = hipEventElapsedTime(&ms, lane.ev_begin, lane.ev_end);
     if (stats) {
@@ -2955,27 +2993,33 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
     for (int j = 0; j < m; ++j) {
         const BoundEntry &e = es[j];
         const gdp_problem *q = p[e.orig];
-        const double *ub = reinterpret_cast<const double *>(lane.back + (e.off_ub - up_bytes));
-        bool bounded = true;   // a key whose budget no path was found for keeps everything
-        for (int k = 0; k < q->n_key; ++k) bounded = bounded && (e.budget[(size_t)k] < 0 || ub[k] < INFINITY);
-        if (!bounded) continue;
+        const GdpFrontierOut &o = *reinterpret_cast<const GdpFrontierOut *>(lane.back + (e.off_out - up_bytes));
+        if (o.status == 1) continue;   // a key whose budget no path was found for keeps everything
         std::unique_ptr<Reduced> d(new Reduced());
-        if (build_reduced(q, e.h, reinterpret_cast<const uint8_t *>(lane.back + (e.off_keep - up_bytes)), e.budget.data(), *d))
-            out[(size_t)e.orig] = std::move(d);
+        if (o.status == 0) {
+            const int32_t *res = reinterpret_cast<const int32_t *>(lane.back + (e.off_res - up_bytes));
+            d->solved = true;
+            d->executed = o.executed;
+            d->total.assign(o.total, o.total + q->n_key);
+            d->remaining.assign(o.remaining, o.remaining + q->n_key);
+            d->res.assign(res, res + (size_t)q->n_key * q->L);
+        } else if (!build_reduced(q, e.h, reinterpret_cast<const uint8_t *>(keep.data() + (e.off_keep - keep_begin)), e.budget.data(), *d)) {
+            continue;
+        }
+        out[(size_t)e.orig] = std::move(d);
     }
     return GDP_OK;
 }
 
 // Bounds of the instances of a batch that have the form, in consecutive slices of at most `limit` bytes of device
-// memory each; instances that need more by themselves are solved whole.  Initial costs are taken to be zeros; scanned:
-// bytes of them that the calling thread looks through while the device works.
-static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vector<double> &magnitude, size_t scanned,
+// memory each; instances that need more by themselves are solved whole.  Initial costs are taken to be zeros.
+static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vector<double> &magnitude, InitialScan &scan,
                         size_t limit, std::vector<std::unique_ptr<Reduced>> &out)
 {
     const char *env = getenv("GALVATRON_DP_REDUCE"), *skip = getenv("GALVATRON_DP_SKIP");
     const bool forced = env && *env && atoi(env) != 0;
     if ((env && *env && !forced) || (skip && *skip && atoi(skip) == 0)) return GDP_OK;
-    if (!forced && (!bounds_pay(n, p) || !InitialScan::device_bound(dense_work(n, p), scanned))) return GDP_OK;
+    if (!forced && (!bounds_pay(n, p) || !InitialScan::device_bound(dense_work(n, p), scan.alone()))) return GDP_OK;
 
     std::vector<BoundEntry> es;
     for (int i = 0; i < n; ++i) {
@@ -3007,7 +3051,7 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
             bytes += b;
             ++end;
         }
-        if (end > begin) rc = reduce_slice(p, magnitude, es.data() + begin, (int)(end - begin), n_lam, out);
+        if (end > begin) rc = reduce_slice(p, magnitude, es.data() + begin, (int)(end - begin), n_lam, scan, out);
         begin = std::max(end, begin + 1);
     }
     return rc;
@@ -3022,6 +3066,10 @@ static int expand_result(const gdp_problem *q, const Reduced &d, gdp_result *out
         out->total[k] = d.total[(size_t)k];
         out->remaining[k] = d.remaining[(size_t)k];
         if (d.remaining[(size_t)k] == -1) continue;
+        if (d.solved) {
+            memcpy(out->res + (size_t)k * q->L, d.res.data() + (size_t)k * q->L, sizeof(int32_t) * (size_t)q->L);
+            continue;
+        }
         out->remaining[k] += (int32_t)d.spare[(size_t)k];
         for (int l = 0; l < q->L; ++l)
             out->res[(size_t)k * q->L + l] = d.kept[(size_t)l * d.q.S + d.res[(size_t)k * q->L + l]];
@@ -3034,7 +3082,7 @@ static int expand_result(const gdp_problem *q, const Reduced &d, gdp_result *out
 // works on it; *f0_found says afterwards whether any hold more than zeros, in which case nothing has been written
 // to the results, f0_live says which, and a refused one (of the whole instances) is the return code.
 static int solve_parts(int32_t n, const gdp_problem *const *p, gdp_result *const *r, size_t budget, std::vector<char> &f0_live,
-                       InitialScan *scan, const gdp_problem *const *whole, bool *f0_found)
+                       InitialScan *scan, int32_t n_whole, const gdp_problem *const *whole, bool *f0_found)
 {
     int begin = 0, prev_begin = 0;
     gdp_plan *prev = nullptr;
@@ -3100,7 +3148,7 @@ static int solve_parts(int32_t n, const gdp_problem *const *p, gdp_result *const
     int rs = GDP_OK;
     if (found) {
         *f0_found = true;
-        rs = validate_f0_all(n, whole, f0_live);   // this, too, while the device works
+        rs = validate_f0_all(n_whole, whole, f0_live);   // this, too, while the device works
     }
     int rc = finish(prev);
     if (rs != GDP_OK) rc = rs;
@@ -3131,46 +3179,56 @@ int gdp_solve_batch(int32_t n, const gdp_problem *const *p, gdp_result *const *r
         if (any_f0) scan.start(n, p, dense_work(n, p));
         if (scan.found()) {   // no bounds, and nothing to be solved twice (L = 28, S = 40, V = 29493 4.6 -> 2.5 ms)
             const int rv = validate_f0_all(n, p, f0_live);
-            return rv == GDP_OK ? solve_parts(n, p, r, budget, f0_live, nullptr, nullptr, nullptr) : rv;
+            return rv == GDP_OK ? solve_parts(n, p, r, budget, f0_live, nullptr, 0, nullptr, nullptr) : rv;
         }
         std::vector<std::unique_ptr<Reduced>> small((size_t)n);
         int rc = GDP_OK;
         try {
-            rc = reduce_batch(n, p, magnitude, scan.alone(), std::min(budget, REDUCE_MAX_BYTES), small);
+            rc = reduce_batch(n, p, magnitude, scan, std::min(budget, REDUCE_MAX_BYTES), small);
         } catch (const std::bad_alloc &) {   // instances without bounds by then are solved whole, which takes less
         }
         if (rc != GDP_OK) return rc;
-        std::vector<const gdp_problem *> q(p, p + n);
-        std::vector<gdp_result *> qr(r, r + n);
-        for (int i = 0; i < n; ++i)
-            if (small[(size_t)i]) {
-                q[(size_t)i] = &small[(size_t)i]->q;
-                qr[(size_t)i] = &small[(size_t)i]->r;
-            }
+        // what is left to solve: instances whole, and smaller ones
+        std::vector<const gdp_problem *> q;
+        std::vector<gdp_result *> qr;
+        for (int i = 0; i < n; ++i) {
+            Reduced *d = small[(size_t)i].get();
+            if (d && d->solved) continue;
+            q.push_back(d ? &d->q : p[i]);
+            qr.push_back(d ? &d->r : r[i]);
+        }
+        const int32_t m = (int32_t)q.size();
         // Initial costs (gdp_problem.f0) are zeros in every call the reference's own code makes, and looking
         // through V x S doubles takes as long as solving a small instance.  A batch of one part is therefore
         // started as if they were zeros and the arrays are looked through while the device works; should one
         // of them hold anything else, that solve is dropped and the batch solved again with them, whole.
         size_t bytes = 0;
-        for (int i = 0; i < n && bytes <= budget; ++i) bytes += footprint(q[(size_t)i]);
-        const bool late = any_f0 && n <= 65535 && bytes <= budget;
+        for (int i = 0; i < m && bytes <= budget; ++i) bytes += footprint(q[(size_t)i]);
+        const bool late = any_f0 && m > 0 && m <= 65535 && bytes <= budget;
         bool f0_found = any_f0 && !late && scan.finish();
         if (f0_found) {
             rc = validate_f0_all(n, p, f0_live);
-        } else {
-            rc = solve_parts(n, q.data(), qr.data(), budget, f0_live, late ? &scan : nullptr, p, &f0_found);
+        } else if (m > 0) {
+            rc = solve_parts(m, q.data(), qr.data(), budget, f0_live, late ? &scan : nullptr, n, p, &f0_found);
         }
-        if (rc == GDP_OK && f0_found) return solve_parts(n, p, r, budget, f0_live, nullptr, nullptr, nullptr);
-        double left_out = 0;
+        if (rc == GDP_OK && f0_found) return solve_parts(n, p, r, budget, f0_live, nullptr, 0, nullptr, nullptr);
+        double left_out = 0, executed = 0;
+        int64_t solved = 0;
         for (int i = 0; i < n && rc == GDP_OK; ++i)
             if (small[(size_t)i]) {
-                rc = expand_result(p[i], *small[(size_t)i], r[i]);
-                const gdp_problem &d = small[(size_t)i]->q;
-                left_out += (double)p[i]->L * (double)p[i]->V * p[i]->S * p[i]->S - (double)d.L * (double)d.V * d.S * d.S;
+                const Reduced &d = *small[(size_t)i];
+                rc = expand_result(p[i], d, r[i]);
+                left_out += (double)p[i]->L * (double)p[i]->V * p[i]->S * p[i]->S - (double)d.q.L * (double)d.q.V * d.q.S * d.q.S;
+                executed += d.executed;
+                solved += d.solved;
             }
         if (rc == GDP_OK && left_out > 0) {   // statistics count the relaxations of the whole instances
             std::lock_guard<std::mutex> lk(g_stats_mu);
-            if (g_stats_on) g_stats.relaxations += left_out;
+            if (g_stats_on) {
+                g_stats.relaxations += left_out;
+                g_stats.executed += executed;
+                g_stats.instances += solved;
+            }
         }
         return rc;
     } catch (const std::bad_alloc &) {

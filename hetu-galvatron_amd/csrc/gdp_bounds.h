@@ -5,38 +5,77 @@
 
 #include <stdint.h>
 
-constexpr int GDP_BOUND_MAX_S = 128;      // strategies (an argmin is a byte, a matrix at most 16 elements per thread)
-constexpr int GDP_BOUND_MAX_L = 512;      // layers (running sums of four paths in LDS)
-constexpr int GDP_BOUND_MAX_LS = 40960;   // layers x strategies: the argmin table of a pass lives in LDS
+constexpr int GDP_BOUND_MAX_S = 128;      // strategies
+constexpr int GDP_BOUND_MAX_L = 512;      // layers
+constexpr int GDP_BOUND_MAX_LS = 40960;   // layers x strategies
 constexpr int GDP_BOUND_MAX_LAM = 64;     // multipliers
 constexpr int GDP_BOUND_MAX_KEY = 8;
-constexpr int GDP_BOUND_THREADS = 1024;    // at most, per pass; at least GDP_BOUND_MAX_L
-constexpr int GDP_BOUND_PARTS = 32;       // at most this many threads share a target strategy
-constexpr int GDP_BOUND_LOW = 3;          // paths above the budget that are spliced with the one below it
+constexpr int GDP_BOUND_WINDOW = 8;       // multipliers around a key's best one that its upper bound comes from
+constexpr double GDP_BOUND_FAR = 1e200;   // for +inf: 512 of them and the costs of a path (below 1e100) have room above
+constexpr int GDP_BOUND_MEM = 1 << 30;    // memory sums saturate here, above every budget; two of them fit 32 bits
+
+constexpr int GDP_FRONTIER_KEPT = 8192;   // strategies that stay, over all layers of an instance
+constexpr int GDP_FRONTIER_LABELS = 1024; // room in memory for so many labels, and transitions, per layer on average
+
+// What gdp_launch_frontier finds for an instance; the strategies lie in GdpBoundInst.res.
+struct GdpFrontierOut {
+    double total[GDP_BOUND_MAX_KEY];      // +inf: the key has no solution
+    double executed;                      // candidates looked at
+    int32_t remaining[GDP_BOUND_MAX_KEY];
+    int32_t status, pad;                  // 0: solved; otherwise nothing else in here is valid
+};
+
+// From w bins on, strategy s (counted among those of its layer that stay) can be reached at cost c.
+struct GdpFrontierLabel {
+    double c;
+    int32_t w, s;
+};
 
 struct GdpBoundInst {
     const int32_t *mem;      // [L][S]
     const double *intra;     // [L][S]
     const double *inter;     // [T][S][S]
-    const double *inter_t;   // [T][S][S], every matrix transposed
+    double *inter_f;         // [T][S][S], GDP_BOUND_FAR for +inf
+    double *inter_t;         // [T][S][S], the same with every matrix transposed
     const int32_t *index;    // [L] layer -> matrix
     const double *lam;       // [NL] ascending, lam[0] = 0
     const int64_t *budget;   // [K] start row of every key; negative: the key has no solution
     double *P, *Q;           // [NL][L][S] cheapest way from the first layer up to (l, s), and from there to the last
-    double *path_time;       // [NL] of the cheapest path under multiplier i: its time,
-    int64_t *path_mem;       //      its memory
-    uint8_t *path;           // [NL][L] and its strategies
-    double *ub;              // [K] time of the best path found that fits the budget; +inf: none found
+    uint32_t *P_mem, *Q_mem; // [NL][L][S] memory of those ways
+    double *end;             // [NL] cheapest way through all layers
+    unsigned long long *ub;  // [K] time of the best path found that fits the budget, ordered as an unsigned number; ~0: none found
+    int32_t *window;         // [K] first of the multipliers that it comes from
     uint8_t *keep;           // [L][S] 1: (l, s) may lie on a best path of some key
+    const double *other_time;// [K]
+    // of the frontier: the labels of all layers, the transitions between and the costs of what stays, the results
+    GdpFrontierLabel *hist;
+    int32_t *hist_mem;
+    double *hist_turns, *hist_intra;
+    GdpFrontierOut *out;
+    int32_t *res;            // [K][L]
     double magnitude;        // sum over the layers of the largest finite |intra| and |inter|
-    int32_t L, V, S, K;
+    int32_t L, V, S, K, T, n_hist, n_hist_turns;
 };
 
-// Elements of a transition matrix per thread that instances of S strategies need with that many threads per pass (1, 2,
-// 4, 8 or 16; 0: more than that many threads take).
-__attribute__((visibility("hidden"))) int gdp_bound_elements(int S, int threads);
-// Transposes the matrices, runs the passes of all multipliers, finds the upper bounds and marks what stays.
-// pairs: {instance, matrix} of every matrix that is to be transposed.
+// Copies the matrices, runs the passes of all multipliers, finds the upper bounds and marks what stays.
+// pairs: {instance, matrix} of every matrix that is to be copied.
 __attribute__((visibility("hidden")))
-hipError_t gdp_launch_bounds(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K,
-                             int elements, int threads, const int2 *pairs, int n_pairs, hipStream_t stream);
+hipError_t gdp_launch_bounds(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K, const int2 *pairs,
+                             int n_pairs, hipStream_t stream);
+// The DP over what stays (gdp_frontier.hip), after gdp_launch_bounds.
+__attribute__((visibility("hidden"))) hipError_t gdp_launch_frontier(const GdpBoundInst *inst, int n, int max_K, hipStream_t stream);
+
+#ifdef __HIPCC__
+// A double from an unsigned number of the same order.
+__device__ __forceinline__ double gdp_unordered(unsigned long long o)
+{
+    return __longlong_as_double((long long)(o >> 63 ? o & ~(1ull << 63) : ~o));
+}
+
+// Rounding of P and Q under multiplier lam: sums of at most 2 L + 2 terms whose magnitudes add up to no more than
+// magnitude + lam * (L + 1) * V, each rounded, and cut to make room for an index, by no more than 2^-45 of it.
+__device__ __forceinline__ double gdp_bound_margin(int L, int V, double magnitude, double lam)
+{
+    return 4.0 * (double)(L + 4) * 0x1p-45 * (magnitude + lam * ((double)(L + 1) * (double)V));
+}
+#endif

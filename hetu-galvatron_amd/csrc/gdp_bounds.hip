@@ -21,16 +21,11 @@
 
 namespace {
 
-static_assert(GDP_BOUND_MAX_S <= 128, "the cheapest end of a path: two strategies per lane");
-static_assert(GDP_BOUND_MAX_LAM <= 64 && GDP_BOUND_LOW + 1 == 4, "the upper bounds: a multiplier per lane, a path per wave");
+static_assert(GDP_BOUND_MAX_S == 128, "two blocks of 64 targets; a strategy in the low 7 bits of a candidate");
+static_assert(GDP_BOUND_MAX_LAM <= 64, "the best multiplier of a key: one per lane");
 
-__device__ __forceinline__ double lagrangian(int32_t mem, double intra, double lam, int V)
-{
-    return mem < V && intra < INFINITY ? intra + lam * (double)mem : (double)INFINITY;
-}
-
-// inter_t: grid (pairs, 16-row bands of the largest matrix), 256 threads; LDS turns the band around so that both
-// sides are read and written along rows.
+// The matrices as the passes read them: as they are and transposed, +inf replaced by GDP_BOUND_FAR.  grid (pairs, 16-row
+// bands of the largest matrix), 256 threads; LDS turns the band around so that both sides are read and written along rows.
 __global__ __launch_bounds__(256) void gdp_bound_transpose_kernel(const GdpBoundInst *inst, const int2 *pairs)
 {
     __shared__ double tile[16][GDP_BOUND_MAX_S + 1];
@@ -40,261 +35,298 @@ __global__ __launch_bounds__(256) void gdp_bound_transpose_kernel(const GdpBound
     if (r0 >= S) return;
     const int rows = S - r0 < 16 ? S - r0 : 16;
     const double *src = I.inter + (size_t)w.y * S * S;
-    double *dst = const_cast<double *>(I.inter_t) + (size_t)w.y * S * S;
-    for (int e = threadIdx.x; e < rows * S; e += 256) tile[e / S][e % S] = src[(size_t)r0 * S + e];
+    double *fwd = I.inter_f + (size_t)w.y * S * S, *bwd = I.inter_t + (size_t)w.y * S * S;
+    for (int e = threadIdx.x; e < rows * S; e += 256) {
+        const double x = fmin(src[(size_t)r0 * S + e], GDP_BOUND_FAR);
+        tile[e / S][e % S] = x;
+        fwd[(size_t)r0 * S + e] = x;
+    }
     __syncthreads();
     for (int e = threadIdx.x; e < rows * S; e += 256) {
         const int c = e / rows, r = e % rows;
-        dst[(size_t)c * S + r0 + r] = tile[r][c];
+        bwd[(size_t)c * S + r0 + r] = tile[r][c];
     }
 }
 
-// One pass over the layers of one instance under one multiplier: forwards (P, the path and its cost) or backwards
-// (Q).  grid (2 * multipliers, instances): the serial chain of L steps is what takes the time, so everything that
-// does not depend on it runs side by side -- multipliers and directions in workgroups of their own, a step's S*S
-// candidates on up to 1024 threads (thread = target strategy + S * part, its sources part, part + G, ...: loads run
-// along the rows), and the matrices of the next two steps are on their way to registers meanwhile.  A step is then two
-// barriers and the reduction over the parts: L = 80, S = 64 207 -> 132 us, L = 48, S = 88 147 -> 102 us and L = 32,
-// S = 44 79 -> 50 us against loads one step ahead behind comparisons.
-template <int E, int NT>
-__global__ __launch_bounds__(NT, NT == GDP_BOUND_THREADS ? 4 : 8) void gdp_bound_pass_kernel(const GdpBoundInst *inst)
+// Global memory, said so: the compiler takes a pointer that comes from memory for one that may point anywhere, and waits
+// for everything under way around what it may point at.
+typedef const __attribute__((address_space(1))) double *gdouble;
+typedef const __attribute__((address_space(1))) int32_t *gint;
+typedef __attribute__((address_space(1))) double *gout;
+typedef __attribute__((address_space(1))) uint32_t *guint;
+typedef __attribute__((address_space(1))) unsigned long long *gulong;
+
+__device__ __forceinline__ double min_f64(double a, double b)
 {
-    extern __shared__ uint8_t arg_of[];   // [L][S], forwards only
-    __shared__ double X[GDP_BOUND_MAX_S], part_v[GDP_BOUND_THREADS];
-    __shared__ uint8_t part_i[GDP_BOUND_THREADS];
+    double r;   // the bare instruction: no operand is a NaN
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+typedef int int2v __attribute__((ext_vector_type(2)));   // the words of a double, without the shifts of __hiloint2double
+
+// Minimum over the lanes l, l ^ 16, l ^ 32 and l ^ 48, in all four.  (A swap of two copies of x leaves the even rows, or
+// the lower half, twice in one and the others twice in the other.)
+__device__ __forceinline__ double min_of_rows(double x)
+{
+    const uint2v w = __builtin_bit_cast(uint2v, x);
+    const uint2v lo = __builtin_amdgcn_permlane16_swap(w.x, w.x, false, false), hi = __builtin_amdgcn_permlane16_swap(w.y, w.y, false, false);
+    const uint2v a = {lo.x, hi.x}, b = {lo.y, hi.y};
+    x = min_f64(__builtin_bit_cast(double, a), __builtin_bit_cast(double, b));
+    const uint2v v = __builtin_bit_cast(uint2v, x);
+    const uint2v lo2 = __builtin_amdgcn_permlane32_swap(v.x, v.x, false, false), hi2 = __builtin_amdgcn_permlane32_swap(v.y, v.y, false, false);
+    const uint2v c = {lo2.x, hi2.x}, d = {lo2.y, hi2.y};
+    return min_f64(__builtin_bit_cast(double, c), __builtin_bit_cast(double, d));
+}
+
+constexpr int INDEX = GDP_BOUND_MAX_S - 1;   // low bits of a candidate that hold its source strategy
+constexpr int TARGETS = 16;                  // target strategies of a wave: 16 lanes read a line of 128 bytes
+constexpr int PARTS = 64 / TARGETS;          // lanes that share one of them
+
+// x with `index`, a constant, in its low bits; high: ~INDEX, in a register (v_and_or_b32 takes no other constant).
+__device__ __forceinline__ double with_index(double x, int index, int high)
+{
+    int2v w = __builtin_bit_cast(int2v, x);
+    w.x = (w.x & high) | index;
+    return __builtin_bit_cast(double, w);
+}
+
+// An array as the buffer instructions see it: an address is a register of the lane plus one of the wave, no arithmetic.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *p, size_t bytes)
+{
+    const uintptr_t a = (uintptr_t)p;   // the same in all lanes, said so
+    const uintptr_t u = (uintptr_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(a >> 32)) << 32 |
+                        (uint32_t)__builtin_amdgcn_readfirstlane((int)a);
+    return __builtin_amdgcn_make_buffer_rsrc((void *)u, 0, __builtin_amdgcn_readfirstlane((int)(uint32_t)bytes), 0x27000);
+}
+
+__device__ __forceinline__ double load_double(__amdgpu_buffer_rsrc_t b, int lane_bytes, int wave_bytes)
+{
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(b, lane_bytes, wave_bytes, 0));
+}
+
+// One pass over the layers of one instance under one multiplier: forwards (P) or backwards (Q), and the memory of the
+// paths behind them.  grid (2 * multipliers, instances); a wave has 16 target strategies and 4 lanes for each, a lane up to
+// E of the source strategies.  A step is E candidates per lane, two exchanges between the 4 lanes and one barrier, behind
+// which every wave reads all sources back from LDS.  A candidate carries its source in its low bits, so that the
+// minimum is the argmin as well, and what the path behind it needs of memory is one look into LDS beside the chain.
+// The serial chain of L steps is what takes the time, and in it the instructions that a SIMD issues: 4 waves of 16 sources
+// per lane, not 16 of 4, whose reductions and addresses cost as much again each; matrices are AHEAD steps ahead in registers.
+// What it reads is bound by how many lines a load touches: 4 lanes of a target side by side, a line for every 4 lanes, took
+// 151 us where 16 targets side by side take 69.  Against a step of two barriers, 1024 threads and a select per candidate for
+// the argmin: L = 80, S = 64 131 -> 69 us, L = 48, S = 88 102 -> 77, 256 instances of S = 44 635 -> 400.
+template <int E, int AHEAD>
+__global__ __launch_bounds__(64 * GDP_BOUND_MAX_S / TARGETS) void gdp_bound_pass_kernel(const GdpBoundInst *inst)
+{
+    static_assert(E % 2 == 0 && AHEAD % 2 == 0 && E * PARTS <= GDP_BOUND_MAX_S, "");
+    constexpr int STRIDE = E + 2;   // of the sources of a part: 16 bytes at a time from 4 different places in the banks
+    __shared__ __align__(16) double X[2][PARTS * STRIDE];
+    __shared__ uint32_t need[2][GDP_BOUND_MAX_S];    // memory of the path behind each source
     __shared__ int32_t mat[GDP_BOUND_MAX_L];
-    __shared__ uint8_t path[GDP_BOUND_MAX_L];
     const GdpBoundInst &I = inst[blockIdx.y];
     const int L = I.L, S = I.S, V = I.V, t = (int)threadIdx.x, li = (int)blockIdx.x >> 1;
     const bool back = blockIdx.x & 1u;
-    const double lam = I.lam[li];
-    const int G = min(NT / S, GDP_BOUND_PARTS), s = t % S, g = min(t / S, G - 1), c_at = min(t, S - 1);
-    const size_t SS = (size_t)S * S;
-    for (int l = t; l < L; l += NT) mat[l] = I.index[l];
-    if (t < S) X[t] = 0.0;
-    __syncthreads();
-    // Global memory, said so: the compiler takes a pointer that comes from memory for one that may point anywhere.
-    typedef const __attribute__((address_space(1))) double *gdouble;
-    typedef const __attribute__((address_space(1))) int32_t *gint;
-    typedef __attribute__((address_space(1))) double *gout;
-    const gdouble tables = (gdouble)(uintptr_t)(back ? I.inter_t : I.inter), intra = (gdouble)(uintptr_t)I.intra;
-    const gint mem = (gint)(uintptr_t)I.mem;
-    const gout out = (gout)(uintptr_t)((back ? I.Q : I.P) + (size_t)li * L * S);
+    const double lam = ((gdouble)(uintptr_t)I.lam)[li];
+    const int p = (t & 63) / TARGETS, target = (t >> 6) * TARGETS + t % TARGETS, s = min(target, S - 1);
+    for (int l = t; l < L; l += (int)blockDim.x) mat[l] = ((gint)(uintptr_t)I.index)[l];
+    for (int e = t; e < PARTS * STRIDE; e += (int)blockDim.x) X[0][e] = X[1][e] = GDP_BOUND_FAR * 0x1p40;   // sources beyond S
+    if (blockIdx.x == 0 && t < I.K) ((gulong)(uintptr_t)I.ub)[t] = ~0ull;
+    const size_t LS = (size_t)L * S;
+    const __amdgpu_buffer_rsrc_t tables = buffer_of(back ? I.inter_t : I.inter_f, (size_t)I.T * S * S * 8),
+                                 intra = buffer_of(I.intra, LS * 8), mem = buffer_of(I.mem, LS * 4),
+                                 out = buffer_of((back ? I.Q : I.P) + li * LS, LS * 8),
+                                 out_mem = buffer_of((back ? I.Q_mem : I.P_mem) + li * LS, LS * 4);
+    const bool mine = p == 0 && target < S;
+    const int place = target / E * STRIDE + target % E;   // of this target among the sources of the next step
+    int at[E];                                            // of the elements of a matrix, in bytes
+#pragma unroll
+    for (int j = 0; j < E; ++j) at[j] = (min(p * E + j, S - 1) * S + s) * 8;
 
-    // What a step needs from memory: its part of the matrix and the layer's costs of strategy t.  Sources beyond the last
-    // are the last once more, so that nothing here depends on a comparison and the loads of a step leave together.
+    // What a step needs from memory: its part of the matrix and the costs of the layer whose strategies it reaches.
     struct Inputs {
         double m[E], intra;
         int32_t mem;
     };
-    auto from = [&](int k) { return min(g + k * G, S - 1); };
-    constexpr int AHEAD = E <= 8 ? 2 : 1;   // steps: two sets of 16 elements do not fit the registers of 1024 threads
-    auto fetch = [&](int l, Inputs &in) {
-        const gdouble M = tables + (size_t)__builtin_amdgcn_readfirstlane(mat[l]) * SS;
-#pragma unroll
-        for (int k = 0; k < E; ++k) in.m[k] = M[from(k) * S + s];
-        in.mem = mem[l * S + c_at];
-        in.intra = intra[l * S + c_at];
+    // step i: the matrix of layer first + i * step, into the strategies of layer to + i * step
+    const int first = back ? L - 1 : 0, to = back ? L - 2 : 0, step = back ? -1 : 1, steps = back ? L - 1 : L;
+    auto fetch_costs = [&](int l, Inputs &in) {
+        in.mem = __builtin_amdgcn_raw_buffer_load_b32(mem, s * 4, l * S * 4, 0);
+        in.intra = load_double(intra, s * 8, l * S * 8);
     };
-    const int first = back ? L - 1 : 0, step = back ? -1 : 1;
-    // Step i; its registers are filled again for step i + AHEAD as soon as they have been read.
-    auto pass = [&](int i, Inputs &in) {
-        const int l = first + i * step;
-        const double c = lagrangian(in.mem, in.intra, lam, V);
-        if (back) {
-            // X is Q[l]; what lies before layer l sees the cost of (l, s) on top of it
-            if (t < S) {
-                out[(size_t)l * S + t] = X[t];
-                X[t] += c;
-            }
-            if (l == 0) return;
-            __syncthreads();
-        }
-        double best = INFINITY;
-        int arg = 0;
+    auto matrix_of = [&](int i) { return mat[first + min(i, steps - 1) * step]; };
+    auto fetch = [&](int i, int matrix, Inputs &in) {
+        const int M = __builtin_amdgcn_readfirstlane(matrix) * S * S * 8;
 #pragma unroll
-        for (int k = 0; k < E; ++k) {
-            const double v = X[from(k)] + in.m[k];
-            arg = v < best ? from(k) : arg;
-            best = v < best ? v : best;
+        for (int j = 0; j < E; ++j) in.m[j] = load_double(tables, at[j], M);
+        fetch_costs(to + i * step, in);
+    };
+    auto cost = [&](const Inputs &in) {
+        return in.mem < V && in.intra < GDP_BOUND_FAR ? in.intra + lam * (double)in.mem : GDP_BOUND_FAR;
+    };
+    auto more = [](uint32_t m, int32_t by) { return min(m + (uint32_t)by, (uint32_t)GDP_BOUND_MEM); };   // by: <= GDP_BOUND_MEM
+    // What a step found, to be written while the next one computes: the layer, costs, the memory behind them, on its way
+    // from LDS, and what the strategy itself needs.
+    struct Found {
+        int layer;
+        double x;
+        uint32_t m;
+        int32_t by;
+    } found = {0, 0.0, 0, 0};
+    auto write = [&](int i) {   // what step i - 1 found
+        const uint32_t m2 = more(found.m, found.by);
+        const int row = __builtin_amdgcn_readfirstlane(found.layer) * S;
+        if (mine) {
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, found.x), out, s * 8, row * 8, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(back ? found.m : m2, out_mem, s * 4, row * 4, 0);
+            need[i & 1][target] = m2;
         }
-        if (i + AHEAD < L) fetch(l + AHEAD * step, in);
-        if (t < G * S) {
-            part_v[t] = best;
-            part_i[t] = (uint8_t)arg;
+    };
+    __syncthreads();
+    if (back) {
+        Inputs last;
+        fetch_costs(L - 1, last);
+        found.layer = L - 1;
+        found.by = min(last.mem, GDP_BOUND_MEM);
+        if (mine) X[0][place] = cost(last);
+    } else if (mine) {   // (what the first step writes of layer 0 is overwritten by the second)
+        X[0][place] = 0.0;
+    }
+    int next_matrix = matrix_of(AHEAD);
+    int high = ~INDEX;
+    asm volatile("" : "+v"(high));   // in a register
+    const int part = p * E;
+    auto pass = [&](int i, Inputs &in) {
+        write(i);
+        __syncthreads();   // the other half of X and `need` is still being read until the next one
+        const double *from = X[i & 1] + p * STRIDE;
+        double best[2];
+#pragma unroll
+        for (int j = 0; j < E; j += 2) {
+            const double a = with_index(from[j] + in.m[j], j, high), b = with_index(from[j + 1] + in.m[j + 1], j + 1, high);
+            best[0] = j ? min_f64(best[0], a) : a;
+            best[1] = j ? min_f64(best[1], b) : b;
         }
-        __syncthreads();
-        if (t < S) {   // thread t is part 0 of target t
-#pragma unroll 8
-            for (int p = 1; p < G; ++p) {   // no branch: the reads of all parts are in flight together
-                const double v = part_v[p * S + t];
-                const int a = part_i[p * S + t];
-                arg = v < best ? a : arg;
-                best = v < best ? v : best;
-            }
-            if (back) {
-                X[t] = best;
-            } else {
-                X[t] = best + c;
-                out[(size_t)l * S + t] = X[t];
-                arg_of[l * S + t] = (uint8_t)arg;
-            }
-        }
-        __syncthreads();
+        const double c = cost(in);
+        int32_t by = min(in.mem, GDP_BOUND_MEM);
+        asm volatile("" : "+v"(by));   // here, and not as a copy at the top of the loop that waits for every load
+        fetch(min(i + AHEAD, steps - 1), next_matrix, in);   // the last ones once more: no branch
+        next_matrix = matrix_of(i + AHEAD + 1);
+        int2v w = __builtin_bit_cast(int2v, min_f64(best[0], best[1]));
+        w.x += part;
+        double x = __builtin_bit_cast(double, w);
+        x = min_of_rows(x);
+        const double z = x + c;
+        if (mine) X[(i + 1) & 1][place] = z;
+        const uint32_t m = need[i & 1][__builtin_bit_cast(int2v, x).x & INDEX];
+        const bool real = i < steps;
+        found.x = !real ? found.x : back ? x : z;
+        found.m = real ? m : found.m;
+        found.by = real ? by : found.by;
+        found.layer = real ? to + i * step : found.layer;
     };
     Inputs in[AHEAD];
 #pragma unroll
-    for (int a = 0; a < AHEAD; ++a)
-        if (a < L) fetch(first + a * step, in[a]);
-    for (int i = 0; i < L; i += AHEAD)
+    for (int a = 0; a < AHEAD; ++a) {
+        fetch(min(a, steps - 1), matrix_of(a), in[a]);
+        __builtin_amdgcn_sched_barrier(0);   // in this order: the first step waits for the first of them only
+    }
+    // Whole turns of AHEAD steps: a way out in between would make the registers of every turn wait for all loads.  Steps
+    // beyond the last find nothing new.
+    int i = 0;
+    for (; i < steps; i += AHEAD)
 #pragma unroll
-        for (int a = 0; a < AHEAD; ++a)
-            if (i + a < L) pass(i + a, in[a]);
+        for (int a = 0; a < AHEAD; ++a) pass(i + a, in[a]);
+    write(i);
     if (back) return;
-    if (t < 64) {   // the cheapest end: two strategies per lane at most, then across the wave
-        int b = t < S ? t : 0;
-        double least = X[b];
-        if (t + 64 < S && X[t + 64] < least) {
-            b = t + 64;
-            least = X[b];
-        }
+    // the cheapest end
+    __syncthreads();
+    if (mine) X[0][target] = found.x;
+    __syncthreads();
+    if (t >= 64) return;
+    double least = X[0][min(t, S - 1)];
+    least = min_f64(least, X[0][min(t + 64, S - 1)]);
 #pragma unroll
-        for (int w = 32; w > 0; w >>= 1) {
-            const double v = __shfl_xor(least, w);
-            const int a = __shfl_xor(b, w);
-            if (v < least || (v == least && a < b)) {
-                least = v;
-                b = a;
-            }
-        }
-        if (t == 0)
-            for (int l = L - 1; l >= 0; --l) {
-                path[l] = (uint8_t)b;
-                b = arg_of[l * S + b];
-            }
-    }
-    __syncthreads();
-    // what the path costs: one layer per thread (L <= 512), summed in LDS
-    double time = 0.0, memory = 0.0;
-    if (t < L) {
-        const int b = path[t], a = arg_of[t * S + b];
-        I.path[(size_t)li * L + t] = (uint8_t)b;
-        const int32_t m = mem[t * S + b];
-        time = tables[(size_t)mat[t] * SS + (size_t)a * S + b] + (m < V ? intra[t * S + b] : (double)INFINITY);
-        memory = (double)m;   // whole numbers below 2^41: exact
-    }
-    part_v[t] = time;
-    __syncthreads();
-    for (int w = NT / 2; w > 0; w >>= 1) {
-        if (t < w) part_v[t] += part_v[t + w];
-        __syncthreads();
-    }
-    if (t == 0) I.path_time[li] = part_v[0];
-    __syncthreads();
-    part_v[t] = memory;
-    __syncthreads();
-    for (int w = NT / 2; w > 0; w >>= 1) {
-        if (t < w) part_v[t] += part_v[t + w];
-        __syncthreads();
-    }
-    if (t == 0) I.path_mem[li] = (int64_t)part_v[0];
+    for (int w = 32; w > 0; w >>= 1) least = min_f64(least, __shfl_xor(least, w));
+    if (t == 0) ((gout)(uintptr_t)I.end)[li] = least;
 }
 
-// Upper bound of one key: the best of the multipliers' paths that fit, and of the paths that follow one of the
-// last paths that do not fit up to some layer and the first one that does from there on (or the other way round) --
-// where all layers are alike every layer changes its strategy at the same multiplier, and only such a
-// splice comes near the budget.  grid (keys, instances), 256 threads; a candidate per thread from running sums.  Choosing
-// the paths and summing them up are a wave's work instead of one thread's walk through memory (L = 80, S = 64 11.5 ->
-// 7.0 us, 256 instances of S = 44 8.4 -> 6.9 us).
+// Doubles as unsigned numbers of the same order, for atomicMin.
+__device__ __forceinline__ unsigned long long ordered(double x)
+{
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    return b >> 63 ? ~b : b | 1ull << 63;
+}
+
+// Upper bound of one key: the best path that fits among all that go the cheapest way to some (l, s) under one multiplier
+// and the cheapest way on under another, both of the GDP_BOUND_WINDOW around the one whose bound is the best.  Where all
+// layers are alike every layer changes its strategy at the same multiplier, and only such a splice comes near the
+// budget.  grid (256-element groups of the largest table, keys, instances); a (l, s) per thread.
+// Against splices of 4 whole paths the bound leaves half to a fifth of the labels (L = 80, S = 64 68 -> 43 per layer, 30 layers
+// of two kinds that trade memory for time 738 -> 261) in the same 6 us.
 __global__ __launch_bounds__(256) void gdp_bound_upper_kernel(const GdpBoundInst *inst, int n_lam)
 {
-    __shared__ double pt[GDP_BOUND_LOW + 1][GDP_BOUND_MAX_L + 1], pm[GDP_BOUND_LOW + 1][GDP_BOUND_MAX_L + 1];
-    __shared__ uint8_t st[GDP_BOUND_LOW + 1][GDP_BOUND_MAX_L];
-    __shared__ double red[256];
-    __shared__ int which[GDP_BOUND_LOW + 1];
-    const GdpBoundInst &I = inst[blockIdx.y];
-    const int key = (int)blockIdx.x, t = (int)threadIdx.x, L = I.L, S = I.S;
-    if (key >= I.K) return;
+    constexpr int W = GDP_BOUND_WINDOW;
+    __shared__ double red[4];
+    __shared__ int first;
+    const GdpBoundInst &I = inst[blockIdx.z];
+    const int key = (int)blockIdx.y, t = (int)threadIdx.x, LS = I.L * I.S;
+    if (key >= I.K || (int)blockIdx.x * 256 >= LS || I.budget[key] < 0) return;   // the whole workgroup
     const int64_t B = I.budget[key];
-    const size_t SS = (size_t)S * S;
-    double best = INFINITY;
-    if (t < 64) {   // a multiplier per lane: which paths fit, and which there are, are two ballots
-        const double time = t < n_lam ? I.path_time[t] : (double)INFINITY;
-        const bool fits = time < INFINITY && I.path_mem[t] <= B;
-        if (fits) best = time;
-        const unsigned long long fit = __ballot(fits), any = __ballot(time < INFINITY);
-        if (t <= GDP_BOUND_LOW) {
-            const int first = fit ? __ffsll(fit) - 1 : -1;
-            unsigned long long below = first > 0 ? any & ((1ull << first) - 1) : 0;
-            for (int q = 1; q < t && below; ++q) below ^= 1ull << (63 - __clzll(below));
-            which[t] = t == 0 ? first : below ? 63 - __clzll(below) : -1;
-        }
-    }
-    __syncthreads();
-    if (which[0] >= 0 && which[1] >= 0) {   // the same in every thread
-        for (int e = t; e < (GDP_BOUND_LOW + 1) * L; e += 256) {
-            const int q = e / L, l = e % L;
-            if (which[q] < 0) continue;
-            const uint8_t *p = I.path + (size_t)which[q] * L;
-            const int b = p[l];
-            st[q][l] = (uint8_t)b;
-            // the first layer comes from whatever strategy is cheapest: P under lam[0] = 0 is that plus its own cost
-            const double x = l == 0 ? I.P[b]
-                                    : I.inter[(size_t)I.index[l] * SS + (size_t)p[l - 1] * S + b] + I.intra[(size_t)l * S + b];
-            pt[q][l + 1] = x;
-            pm[q][l + 1] = (double)I.mem[(size_t)l * S + b];
-        }
-        __syncthreads();
-        // running sums: a path per wave, 64 layers at a time (their rounding, in whatever order, is within the margin)
-        const int q = t >> 6, lane = t & 63;
-        if (which[q] >= 0) {
-            double time = 0.0, memory = 0.0;   // of the layers before the 64
-            if (lane == 0) pt[q][0] = pm[q][0] = 0.0;
-            for (int l0 = 1; l0 <= L; l0 += 64) {
-                const int l = l0 + lane;
-                double x = l <= L ? pt[q][l] : 0.0, y = l <= L ? pm[q][l] : 0.0;
+    if (t < 64) {
+        const int at = min(t, n_lam - 1);
+        double d = I.end[at] - I.lam[at] * (double)B;
+        int i = at;
 #pragma unroll
-                for (int w = 1; w < 64; w <<= 1) {
-                    const double u = __shfl_up(x, w), v = __shfl_up(y, w);
-                    if (lane >= w) {
-                        x += u;
-                        y += v;
-                    }
-                }
-                x += time;
-                y += memory;
-                if (l <= L) {
-                    pt[q][l] = x;
-                    pm[q][l] = y;
-                }
-                time = __shfl(x, 63);
-                memory = __shfl(y, 63);
+        for (int w = 32; w > 0; w >>= 1) {
+            const double e = __shfl_xor(d, w);
+            const int j = __shfl_xor(i, w);
+            if (e > d || (e == d && j < i)) {
+                d = e;
+                i = j;
             }
         }
-        __syncthreads();
-        for (int e = t; e < 2 * GDP_BOUND_LOW * (L - 1); e += 256) {
-            const int c = 1 + e % (L - 1), d = e / (L - 1), q = 1 + (d >> 1);
-            if (which[q] < 0) continue;
-            const int a = d & 1 ? 0 : q, b = d & 1 ? q : 0;   // a up to layer c, then b
-            if (pm[a][c] + (pm[b][L] - pm[b][c]) > (double)B) continue;
-            const double *M = I.inter + (size_t)I.index[c] * SS;
-            const double turn = M[(size_t)st[a][c - 1] * S + st[b][c]], was = M[(size_t)st[b][c - 1] * S + st[b][c]];
-            const double x = pt[a][c] + (pt[b][L] - pt[b][c]) + (turn - was);
-            if (x < best) best = x;
+        if (t == 0) {
+            first = max(0, min(i - W / 2, n_lam - W));
+            if (blockIdx.x == 0) I.window[key] = first;
         }
     }
-    red[t] = best;
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w && red[t + w] < red[t]) red[t] = red[t + w];
-        __syncthreads();
+    const int e = min((int)blockIdx.x * 256 + t, LS - 1);
+    double p[W], q[W], lam[W];
+    uint32_t pm[W], qm[W];
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+        const size_t at = (size_t)(first + i) * LS + e;
+        p[i] = I.P[at];
+        q[i] = I.Q[at];
+        pm[i] = I.P_mem[at];
+        qm[i] = I.Q_mem[at];
+        lam[i] = I.lam[first + i];
     }
-    if (t == 0) I.ub[key] = red[0];
+    double best = INFINITY;
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+        p[i] -= lam[i] * (double)pm[i];
+        q[i] -= lam[i] * (double)qm[i];
+    }
+#pragma unroll
+    for (int i = 0; i < W; ++i)
+#pragma unroll
+        for (int j = 0; j < W; ++j)
+            if ((int64_t)(pm[i] + qm[j]) <= B) best = fmin(best, p[i] + q[j]);
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1) best = fmin(best, __shfl_xor(best, w));
+    if ((t & 63) == 0) red[t >> 6] = best;
+    __syncthreads();
+    if (t != 0) return;
+    best = fmin(fmin(red[0], red[1]), fmin(red[2], red[3]));
+    if (best < GDP_BOUND_FAR / 2) atomicMin(I.ub + key, ordered(best + gdp_bound_margin(I.L, I.V, I.magnitude, lam[W - 1])));
 }
 
 // What stays: (l, s) is out when for every key some multiplier's bound lies above that key's upper bound.  The
-// margin covers the rounding of the bound, of the upper bound and of the DP's own sums: each is a sum of at most
-// 4 L + 4 terms whose magnitudes add up to no more than `magnitude` + lam * (L + 1) * V.
+// margin covers the rounding of the bound; that of the upper bound is part of it, and that of the DP's own sums is less
+// than either.
 // grid (64-element groups of the largest table, instances), PARTS waves with 8 multipliers at a time each.  What takes
 // the time is the round trips of the loads: with 8 waves all 64 multipliers of an element are asked for at once (L = 80,
 // S = 64 26.8 -> 6.3 us, L = 48, S = 88 25.0 -> 5.7 us).  A batch that fills the device with one wave per 64 elements
@@ -315,14 +347,11 @@ __global__ __launch_bounds__(64 * PARTS) void gdp_bound_keep_kernel(const GdpBou
         budget[k] = 0.0;
         if (k < K && I.budget[k] >= 0) {
             alive |= 1u << k;
-            ub[k] = I.ub[k];
+            ub[k] = gdp_unordered(I.ub[k]);
             budget[k] = (double)I.budget[k];
         }
     }
-    typedef const __attribute__((address_space(1))) double *gdouble;
     const gdouble P = (gdouble)(uintptr_t)I.P, Q = (gdouble)(uintptr_t)I.Q, lams = (gdouble)(uintptr_t)I.lam;
-    const double reach = (double)(I.L + 1) * (double)I.V, magnitude = I.magnitude;
-    const double ulp = 16.0 * (double)(I.L + 4) * 0x1p-53;
     for (int i0 = 8 * part; i0 < n_lam; i0 += 8 * PARTS) {
         double p[8], q[8];
 #pragma unroll
@@ -335,7 +364,7 @@ __global__ __launch_bounds__(64 * PARTS) void gdp_bound_keep_kernel(const GdpBou
         for (int i = 0; i < 8; ++i) {
             const double lam = lams[min(i0 + i, n_lam - 1)];
             const double r = p[i] + q[i];
-            const double margin = ulp * (magnitude + lam * reach);
+            const double margin = gdp_bound_margin(I.L, I.V, I.magnitude, lam);
 #pragma unroll
             for (int k = 0; k < GDP_BOUND_MAX_KEY; ++k)
                 if (k < K && r - lam * budget[k] > ub[k] + margin) alive &= ~(1u << k);
@@ -351,43 +380,28 @@ __global__ __launch_bounds__(64 * PARTS) void gdp_bound_keep_kernel(const GdpBou
 
 }  // namespace
 
-int gdp_bound_elements(int S, int threads)
-{
-    const int G = threads / S < GDP_BOUND_PARTS ? threads / S : GDP_BOUND_PARTS;
-    const int most = threads == GDP_BOUND_THREADS ? 16 : 4;   // S <= 128: with 1024 threads G >= 8, so 16 are enough
-    for (int e = 1; e <= most; e *= 2)
-        if (e * G >= S) return e;
-    return 0;
-}
-
-hipError_t gdp_launch_bounds(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K,
-                             int elements, int threads, const int2 *pairs, int n_pairs, hipStream_t stream)
+hipError_t gdp_launch_bounds(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K, const int2 *pairs,
+                             int n_pairs, hipStream_t stream)
 {
     gdp_bound_transpose_kernel<<<dim3((unsigned)n_pairs, (unsigned)((max_S + 15) / 16)), 256, 0, stream>>>(inst, pairs);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const dim3 grid(2u * (unsigned)n_lam, (unsigned)n);
-    const size_t lds = (size_t)max_LS;
-    auto launch = [&](auto kernel) { kernel<<<grid, threads, lds, stream>>>(inst); };
-    constexpr int WIDE = GDP_BOUND_THREADS, HALF = GDP_BOUND_THREADS / 2;
-    if (threads == WIDE) {
-        switch (elements) {
-        case 1: launch(gdp_bound_pass_kernel<1, WIDE>); break;
-        case 2: launch(gdp_bound_pass_kernel<2, WIDE>); break;
-        case 4: launch(gdp_bound_pass_kernel<4, WIDE>); break;
-        case 8: launch(gdp_bound_pass_kernel<8, WIDE>); break;
-        default: launch(gdp_bound_pass_kernel<16, WIDE>); break;
-        }
-    } else {
-        switch (elements) {
-        case 1: launch(gdp_bound_pass_kernel<1, HALF>); break;
-        case 2: launch(gdp_bound_pass_kernel<2, HALF>); break;
-        default: launch(gdp_bound_pass_kernel<4, HALF>); break;
-        }
-    }
+    const unsigned threads = 64u * (unsigned)((max_S + TARGETS - 1) / TARGETS);
+#define GDP_PASS(E, AHEAD) \
+    if (max_S <= PARTS * E) gdp_bound_pass_kernel<E, AHEAD><<<grid, threads, 0, stream>>>(inst)
+    GDP_PASS(4, 4);
+    else GDP_PASS(6, 4);
+    else GDP_PASS(8, 4);
+    else GDP_PASS(10, 4);
+    else GDP_PASS(12, 4);
+    else GDP_PASS(16, 4);
+    else GDP_PASS(22, 2);
+    else GDP_PASS(32, 2);
+#undef GDP_PASS
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    gdp_bound_upper_kernel<<<dim3((unsigned)max_K, (unsigned)n), 256, 0, stream>>>(inst, n_lam);
+    gdp_bound_upper_kernel<<<dim3((unsigned)((max_LS + 255) / 256), (unsigned)max_K, (unsigned)n), 256, 0, stream>>>(inst, n_lam);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     const dim3 elements64((unsigned)((max_LS + 63) / 64), (unsigned)n);

@@ -1,0 +1,639 @@
+// The DP over what the bounds leave, without the budget axis.
+//
+// f[l][v][s] changes only at a few budgets v: its steps are labels (w, c) -- from w bins on the cost is c -- and a layer's
+// labels follow from those of the layer before: a label (w, c) of strategy s' gives (w + mem[s], (c + inter[s'][s]) +
+// intra[s]) for strategy s, of which those stay that are cheaper than every one that needs no more memory.  The same
+// additions in the same order as in the dense recurrence: rounding is monotone, so that the minimum over the labels up to
+// v is f[l][v][s] bit for bit.  Of these, the ones stay that can be part of a best path: c plus a lower bound on every way
+// on that fits the budget does not exceed the upper bound of some key (gdp_bounds.hip).  What is dropped is on no best path
+// and ties with none, so the walk back finds in every cell of a best path the candidates that tie for it, lowest strategy
+// first, as in the dense table.
+//
+// Of random costs 1 to 200 labels per layer stay whatever the budget (L = 80, S = 64, V = 131072: 40, against 8.4 million
+// cells), of identical layers that trade memory for time up to a few thousand.  An instance is one workgroup: its labels
+// and what it needs of the next layer live in LDS, its layers follow each other at the price of two barriers.  An instance
+// with more labels than fit says so, and is solved as a smaller instance of the dense recurrence.
+#include "gdp_bounds.h"
+
+#include <math.h>
+
+namespace {
+
+constexpr int WORKERS = 8, FETCHERS = 4, THREADS = 64 * (WORKERS + FETCHERS);   // waves
+constexpr int LABELS = 1536;    // of a layer
+constexpr int KEPT = 64;        // strategies of a layer
+constexpr int TURNS = 1024;     // transitions between the strategies of two layers
+constexpr int WINDOW = 4;       // multipliers per key that labels are held against (with 64 in place of 4 a tenth fewer stay)
+constexpr int LINES = 1152;     // doubles: what a layer's strategies are held against, and their costs
+// of the walk back: labels, transitions and strategies of the layers that lie in LDS together
+constexpr int BACK_LABELS = 4096, BACK_TURNS = 4800, BACK_KEPT = 1024;
+static_assert(BACK_LABELS >= LABELS && BACK_TURNS >= TURNS && BACK_KEPT >= KEPT, "a layer fits");
+static_assert(WORKERS >= GDP_BOUND_MAX_KEY, "the walk back: a wave per key");
+
+typedef GdpFrontierLabel Label;
+
+// Keys are whole numbers below 2^53: a double is compared as fast as 32 bits are.
+constexpr double KEY_W = 0x1p17, KEY_S = 0x1p11;
+static_assert(KEPT <= 64 && LABELS <= 2048, "6 bits and 11");
+constexpr int KEY_PAD = 72;   // 8 lanes look at 8 keys at a time each
+
+struct Forward {
+    Label label[LABELS];
+    __align__(16) double lines[2][LINES], turns[2][TURNS];
+    // Of the labels as they are found: w, strategy, number within the strategy in one; +inf behind the last.  Of this layer
+    // and the next.
+    __align__(16) double key[2][LABELS + KEY_PAD];
+    double cost[LABELS];
+};
+
+
+struct Backward {
+    Label label[BACK_LABELS];
+    double turns[BACK_TURNS], intra[BACK_KEPT];
+    int32_t mem[BACK_KEPT];
+};
+
+struct Shared {
+    union {
+        Forward f;
+        Backward b;
+        uint8_t keep[GDP_BOUND_MAX_LS];
+    };
+    // Per layer: strategies that stay, where their list begins, where the transitions into them begin in memory.  One
+    // more at the end for the sums.
+    int4 layer[GDP_BOUND_MAX_L + 1];
+    double lam[GDP_BOUND_MAX_KEY][WINDOW], shift[GDP_BOUND_MAX_KEY][WINDOW], ub[GDP_BOUND_MAX_KEY];
+    int32_t found[3];                    // labels of a layer, of the next one and the one after that
+    int32_t labels_at[GDP_BOUND_MAX_L + 1];
+    int32_t mat[GDP_BOUND_MAX_L];
+    int32_t window[GDP_BOUND_MAX_KEY], budget[GDP_BOUND_MAX_KEY];
+    int32_t lost;
+    uint8_t kept[GDP_FRONTIER_KEPT];
+};
+static_assert(sizeof(Shared) <= 160 * 1024, "LDS of a compute unit");
+
+typedef const __attribute__((address_space(1))) double *gdouble;
+typedef const __attribute__((address_space(1))) int32_t *gint;
+typedef const __attribute__((address_space(1))) uint8_t *gbyte;
+typedef __attribute__((address_space(1))) double *gout;
+typedef __attribute__((address_space(1))) int32_t *giout;
+typedef int int4v __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) int4v *glabel;
+#define GLOBAL(type, p) ((type)(uintptr_t)(p))
+
+typedef int int2v __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ double min_f64(double a, double b)
+{
+    double r;   // the bare instruction: no operand is a NaN
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+__device__ __forceinline__ double max_f64(double a, double b)
+{
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// x of the lane that CTRL names, `other` where there is none.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double moved(double other, double x)
+{
+    const int2v o = __builtin_bit_cast(int2v, other), w = __builtin_bit_cast(int2v, x);
+    const int2v m = {__builtin_amdgcn_update_dpp(o.x, w.x, CTRL, ROWS, 0xf, false), __builtin_amdgcn_update_dpp(o.y, w.y, CTRL, ROWS, 0xf, false)};
+    return __builtin_bit_cast(double, m);
+}
+
+// Minimum over the lanes up to this one, of the first `lanes`.
+__device__ __forceinline__ double prefix_min(double x, int lanes = 64)
+{
+    if (lanes <= 1) return x;
+    x = min_f64(x, moved<0x111, 0xf>(x, x));   // row_shr:1, 2, 4, 8; a lane without a source keeps its own
+    x = min_f64(x, moved<0x112, 0xf>(x, x));
+    x = min_f64(x, moved<0x114, 0xf>(x, x));
+    x = min_f64(x, moved<0x118, 0xf>(x, x));
+    if (lanes <= 16) return x;
+    x = min_f64(x, moved<0x142, 0xa>(x, x));   // row_bcast:15 into rows 1 and 3
+    x = min_f64(x, moved<0x143, 0xc>(x, x));   // row_bcast:31 into rows 2 and 3
+    return x;
+}
+
+__device__ __forceinline__ double lane_of(double x, int lane)
+{
+    const int2v w = __builtin_bit_cast(int2v, x);
+    const int2v r = {__builtin_amdgcn_readlane(w.x, lane), __builtin_amdgcn_readlane(w.y, lane)};
+    return __builtin_bit_cast(double, r);
+}
+
+__device__ __forceinline__ int lanes_min(int x)
+{
+    x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x111, 0xf, 0xf, false));
+    x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x112, 0xf, 0xf, false));
+    x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x114, 0xf, 0xf, false));
+    x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x118, 0xf, 0xf, false));
+    x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x142, 0xa, 0xf, false));
+    x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x143, 0xc, 0xf, false));
+    return __builtin_amdgcn_readlane(x, 63);
+}
+
+// The lowest (value, strategy) of a wave's first `lanes`, +inf in the others: the cheapest, of those the lowest strategy.
+__device__ __forceinline__ void cheapest(double &c, int &s, int lanes)
+{
+    const double least = lane_of(prefix_min(c, lanes), min(lanes, 64) - 1);
+    const unsigned long long at = __builtin_amdgcn_ballot_w64(c == least);
+    s = (at & (at - 1)) == 0 ? __builtin_amdgcn_readlane(s, __builtin_ctzll(at)) : lanes_min(c == least ? s : INT32_MAX);
+    c = least;
+}
+
+// old = *p, *p += n, in LDS, by one lane.
+__device__ __forceinline__ int draw(int32_t *p, int n)
+{
+    int old;
+    asm volatile("ds_add_rtn_u32 %0, %1, %2\n\ts_waitcnt lgkmcnt(0)" : "=&v"(old)
+                 : "v"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) int32_t *)p), "v"(n) : "memory");
+    return old;
+}
+
+// All of a label at a time.
+__device__ __forceinline__ int4v words(const Label &x) { return __builtin_bit_cast(int4v, x); }
+__device__ __forceinline__ Label label_at(const Label *p) { return __builtin_bit_cast(Label, *reinterpret_cast<const int4v *>(p)); }
+__device__ __forceinline__ void put(Label *p, const Label &x) { *reinterpret_cast<int4v *>(p) = words(x); }
+
+// The same in every lane, said so.
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ double uniform(double x) { return lane_of(x, 0); }
+
+// What a wave has on its way from memory for a later layer: transitions, what labels are held against, costs.
+template <int LINE>
+struct Ahead {
+    static constexpr int T = TURNS / 64, N = LINES / 64;
+    double turns[T], lines[N];
+};
+
+// grid (instances).  What a layer takes is latency, so the chain of a layer is kept short: 8 waves take the labels of a
+// strategy each, 64 at a time, and find their order in the next layer by searches in LDS; 4 others in turn have what the
+// next 4 layers need of the matrices on its way and lay it out in LDS, and all meet twice per layer.  KEYS: as many at
+// least, in scalar registers.
+// A dependent instruction takes 9 clocks, a read from LDS 64, a barrier 30, so a layer of few labels is 0.9 us, one of 270
+// labels and 8 strategies 9.  Against the smaller instance of the dense recurrence that the host made of what stays (kernels,
+// without the host's 0.05 to 0.9 ms between them): L = 80, S = 64 311 -> 196 us, L = 48, S = 88 405 -> 111, 256 instances
+// of S = 44 1690 -> 99, 15 stages of a fit 435 -> 329.
+template <int KEYS>
+__global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundInst *inst)
+{
+    constexpr int LINE = KEYS * WINDOW + 2;   // of a strategy: lines, intra, memory
+    extern __shared__ __align__(16) char lds[];
+    Shared &sh = *reinterpret_cast<Shared *>(lds);
+    const GdpBoundInst &I = inst[blockIdx.x];
+    const int L = uniform(I.L), S = uniform(I.S), K = uniform(I.K), LS = L * S;
+    const int t = (int)threadIdx.x, lane = t & 63, wave = uniform(t >> 6);
+    GdpFrontierOut *const out = I.out;
+    auto give_up = [&](int why) {   // by the whole workgroup
+        if (t == 0) out->status = why;
+    };
+
+    // ---- what stays, as lists; the keys ----
+    const gbyte keep = GLOBAL(gbyte, I.keep);
+    for (int e = t; e < LS; e += THREADS) sh.keep[e] = keep[e];
+    for (int l = t; l < L; l += THREADS) sh.mat[l] = GLOBAL(gint, I.index)[l];
+    if (t == 0) sh.lost = 0;
+    if (t < 3) sh.found[t] = 0;
+    __syncthreads();
+    if (t < GDP_BOUND_MAX_KEY) {
+        const bool there = t < K;
+        const int64_t B = there ? GLOBAL(const __attribute__((address_space(1))) int64_t *, I.budget)[t] : -1;
+        const unsigned long long o = there ? GLOBAL(const __attribute__((address_space(1))) unsigned long long *, I.ub)[t] : 0;
+        sh.budget[t] = (int32_t)B;   // a start row; negative: none
+        sh.ub[t] = gdp_unordered(o);
+        const int first = B < 0 ? 0 : GLOBAL(gint, I.window)[t] + (GDP_BOUND_WINDOW - WINDOW) / 2;
+        sh.window[t] = first;
+        for (int i = 0; i < WINDOW; ++i) {
+            const double lam = GLOBAL(gdouble, I.lam)[first + i];
+            sh.lam[t][i] = lam;
+            sh.shift[t][i] = lam * (double)B + gdp_bound_margin(I.L, I.V, I.magnitude, lam);
+        }
+        if (B >= 0 && o == ~0ull) sh.lost = 1;   // no path was found for it
+    }
+    __syncthreads();
+    if (sh.lost) {
+        give_up(1);
+        return;
+    }
+    auto kept_of = [&](int l, unsigned long long &lo, unsigned long long &hi) {
+        const bool a = lane < S && sh.keep[l * S + min(lane, S - 1)], b = lane + 64 < S && sh.keep[l * S + min(lane + 64, S - 1)];
+        lo = __builtin_amdgcn_ballot_w64(a);
+        hi = __builtin_amdgcn_ballot_w64(b);
+    };
+    for (int l = wave; l < L; l += WORKERS + FETCHERS) {
+        unsigned long long lo, hi;
+        kept_of(l, lo, hi);
+        if (lane == 0) sh.layer[l].x = __popcll(lo) + __popcll(hi);
+    }
+    __syncthreads();
+    if (wave == 0) {   // running sums of the numbers and of the transitions, and whether every layer fits
+        int sum = 0, turns = 0, bad = 0, before = 0;
+        for (int l0 = 0; l0 < L; l0 += 64) {
+            const int l = l0 + lane;
+            const int n = l < L ? sh.layer[l].x : 0, up = __shfl_up(n, 1), prev = lane ? up : before;
+            int x = n, y = n * prev;   // none into the first layer
+            bad |= l < L && (n < 1 || n > KEPT || n * LINE > LINES || y > TURNS);
+            before = __shfl(n, 63);
+            const int own = y;
+#pragma unroll
+            for (int w = 1; w < 64; w <<= 1) {
+                const int x2 = __shfl_up(x, w), y2 = __shfl_up(y, w);
+                if (lane >= w) {
+                    x += x2;
+                    y += y2;
+                }
+            }
+            if (l < L) sh.layer[l] = make_int4(n, sum + x - n, turns + y - own, 0);
+            sum += __shfl(x, 63);
+            turns += __shfl(y, 63);
+        }
+        if (lane == 0) sh.layer[L] = make_int4(0, sum, turns, 0);
+        if (__builtin_amdgcn_ballot_w64(bad != 0) != 0 || sum > GDP_FRONTIER_KEPT || turns > I.n_hist_turns) sh.lost = 1;
+    }
+    __syncthreads();
+    if (sh.lost) {
+        give_up(2);
+        return;
+    }
+    for (int l = wave; l < L; l += WORKERS + FETCHERS) {
+        unsigned long long lo, hi;
+        kept_of(l, lo, hi);
+        const unsigned long long below = (1ull << lane) - 1;
+        const int at = sh.layer[l].y;
+        if (lo >> lane & 1) sh.kept[at + __popcll(lo & below)] = (uint8_t)lane;
+        if (hi >> lane & 1) sh.kept[at + __popcll(lo) + __popcll(hi & below)] = (uint8_t)(lane + 64);
+    }
+    __syncthreads();   // the marks themselves are not read any more
+    if (t == 0) sh.labels_at[0] = 0;
+    for (int e = t; e < 2 * (LABELS + KEY_PAD); e += THREADS) sh.f.key[0][e] = INFINITY;   // both
+    __syncthreads();
+
+    const gdouble inter = GLOBAL(gdouble, I.inter), intra = GLOBAL(gdouble, I.intra), Q = GLOBAL(gdouble, I.Q);
+    const gint mem = GLOBAL(gint, I.mem);
+    const giout hist_mem = GLOBAL(giout, I.hist_mem);
+    const gout hist_turns = GLOBAL(gout, I.hist_turns), hist_intra = GLOBAL(gout, I.hist_intra);
+    const glabel hist = GLOBAL(glabel, I.hist);
+    const int n_hist = uniform(I.n_hist);
+
+    if (wave >= WORKERS) {
+        // ---- the waves that fetch: wave f what layers f, f + 4, ... need ----
+        // e / n for e < 2^20 / n
+        auto reciprocal = [](int n) { return ((1u << 20) + (unsigned)n - 1) / (unsigned)n; };
+        auto quotient = [](int e, unsigned r) { return (int)((unsigned)e * r >> 20); };
+        Ahead<LINE> a;
+        auto fetch = [&](int l) {
+            const int n = uniform(sh.layer[l].x), at = uniform(sh.layer[l].y);
+            if (l > 0) {
+                const int before = uniform(sh.layer[l - 1].y), all = n * uniform(sh.layer[l - 1].x);
+                const unsigned r = reciprocal(n);
+                const gdouble M = inter + (size_t)uniform(sh.mat[l]) * S * S;
+#pragma unroll
+                for (int i = 0; i < Ahead<LINE>::T; ++i) {
+                    if (i * 64 >= all) break;
+                    const int e = min(lane + i * 64, all - 1), from = quotient(e, r);
+                    a.turns[i] = M[(uint32_t)(sh.kept[before + from] * S + sh.kept[at + e - from * n])];
+                }
+            }
+            constexpr unsigned r = ((1u << 20) + LINE - 1) / LINE;
+#pragma unroll
+            for (int i = 0; i < Ahead<LINE>::N; ++i) {
+                if (i * 64 >= n * LINE) break;
+                const int e = min(lane + i * 64, n * LINE - 1), b = quotient(e, r), x = e - b * LINE, s = l * S + sh.kept[at + b];
+                const int k = x / WINDOW, j = x % WINDOW;
+                if (x < KEYS * WINDOW)
+                    a.lines[i] = Q[(uint32_t)((sh.window[k] + j) * LS + s)] - sh.shift[k][j];
+                else if (x == KEYS * WINDOW)
+                    a.lines[i] = intra[(uint32_t)s];
+                else
+                    a.lines[i] = __builtin_bit_cast(double, int2v{mem[(uint32_t)s], 0});
+            }
+        };
+        auto place = [&](int l) {
+            const int n = uniform(sh.layer[l].x), at = uniform(sh.layer[l].y), to = l & 1;
+            if (l > 0) {
+                const int all = n * uniform(sh.layer[l - 1].x), turns_at = uniform(sh.layer[l].z);
+#pragma unroll
+                for (int i = 0; i < Ahead<LINE>::T; ++i) {
+                    if (i * 64 >= all) break;
+                    const int e = lane + i * 64;
+                    if (e < all) {
+                        sh.f.turns[to][e] = a.turns[i];
+                        hist_turns[(uint32_t)(turns_at + e)] = a.turns[i];
+                    }
+                }
+            }
+            constexpr unsigned r = ((1u << 20) + LINE - 1) / LINE;
+#pragma unroll
+            for (int i = 0; i < Ahead<LINE>::N; ++i) {
+                if (i * 64 >= n * LINE) break;
+                const int e = lane + i * 64, b = quotient(e, r), x = e - b * LINE;
+                if (e < n * LINE) {
+                    sh.f.lines[to][e] = a.lines[i];
+                    if (x == KEYS * WINDOW) hist_intra[(uint32_t)(at + b)] = a.lines[i];
+                    if (x > KEYS * WINDOW) hist_mem[(uint32_t)(at + b)] = __builtin_bit_cast(int2v, a.lines[i]).x;
+                }
+            }
+        };
+        const int f = wave - WORKERS;
+        if (f < L) fetch(f);
+        if (f == 0) {
+            place(0);
+            if (FETCHERS < L) fetch(FETCHERS);
+        }
+        __syncthreads();
+        int at = 0, sum = 0;
+        for (int l = 0, slot = 0; l < L; ++l, slot = slot == 2 ? 0 : slot + 1) {   // the same barriers, and the same ways out, as the workers'
+            const int n = uniform(sh.layer[l].x);
+            for (int e = t - 64 * WORKERS; e < sum; e += 64 * FETCHERS) sh.f.key[(l + 1) & 1][e] = INFINITY;   // of the layer before
+            if (l + 1 < L && (l + 1) % FETCHERS == f) place(l + 1);
+            if (l % FETCHERS == f && l > 0 && l + FETCHERS < L) fetch(l + FETCHERS);
+            __syncthreads();
+            sum = uniform(sh.found[slot]);
+            if (sum == 0 || sum > LABELS || at + sum > n_hist) return;
+            at += sum;
+            if (n > 1) __syncthreads();
+        }
+    }
+
+    // ---- forwards ----
+    double executed = 0.0, total = INFINITY;
+    int cell = 0;        // strategy of the cell, counted among those that stay
+    int32_t v = -1;      // its budget
+    bool walks = false;
+    if (wave < WORKERS) {
+        double lam[KEYS][WINDOW], ub[KEYS];
+        int32_t budget[KEYS];
+#pragma unroll
+        for (int k = 0; k < KEYS; ++k) {
+#pragma unroll
+            for (int i = 0; i < WINDOW; ++i) lam[k][i] = sh.lam[k][i];
+            ub[k] = sh.ub[k];
+            budget[k] = sh.budget[k];
+        }
+        int before = 1, at = 0;   // labels of the layer before, and where this layer's begin in memory
+        // (before the first layer: one, no memory used, for each strategy the cheapest way in)
+        __syncthreads();
+        int4 here = sh.layer[0];
+        for (int l = 0, slot = 0; l < L; ++l, slot = slot == 2 ? 0 : slot + 1) {
+            const int now = l & 1, n = uniform(here.x), kept_at = uniform(here.y);
+            here = sh.layer[l + 1];
+            // what can still be part of a path that fits and is no worse than the best one known
+            auto alive = [&](const double2 *line, double c, int32_t w) {
+                const double dw = (double)w;
+                bool any = false;
+#pragma unroll
+                for (int k = 0; k < KEYS; ++k) {
+                    const double b0 = __builtin_fma(lam[k][0], dw, line[2 * k].x), b1 = __builtin_fma(lam[k][1], dw, line[2 * k].y),
+                                 b2 = __builtin_fma(lam[k][2], dw, line[2 * k + 1].x), b3 = __builtin_fma(lam[k][3], dw, line[2 * k + 1].y);
+                    const double bound = max_f64(max_f64(b0, b1), max_f64(b2, b3));
+                    any |= w <= budget[k] && c + bound <= ub[k];
+                }
+                return any;
+            };
+            // Of labels that need the same memory the cheapest counts, with the last of them.  c: the least up to each label;
+            // returns the least up to the last label that needs less than this one, `last` for the first ones of a turn, and
+            // moves `last` on.
+            auto step_from = [&](double c, bool ends, double &last) {
+                const unsigned long long goes_on = __builtin_amdgcn_ballot_w64(!ends);
+                double from = moved<0x138, 0xf>(last, c);   // wave_shr:1
+                if (goes_on) {
+                    const unsigned long long starts = ~(goes_on << 1) & ((2ull << lane) - 1);   // up to this lane; bit 0 is set
+                    const int start = 63 - __builtin_clzll(starts | 1);
+                    const int2v w = __builtin_bit_cast(int2v, from);
+                    const int2v f = {__builtin_amdgcn_ds_bpermute(4 * start, w.x), __builtin_amdgcn_ds_bpermute(4 * start, w.y)};
+                    from = __builtin_bit_cast(double, f);
+                }
+                last = goes_on >> 63 ? lane_of(from, 63) : lane_of(c, 63);
+                return from;
+            };
+            // Labels of strategy b, `before_these` of which there are already.
+            auto emit = [&](bool stays, int b, int before_these, double c, int32_t w) {
+                const unsigned long long these = __builtin_amdgcn_ballot_w64(stays);
+                const int count = __popcll(these), number = __builtin_amdgcn_mbcnt_hi((uint32_t)(these >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)these, (uint32_t)before_these));
+                int to = 0;
+                if (lane == 0) to = draw(sh.found + slot, count);
+                to = uniform(to) + number - before_these;
+                if (n == 1) {   // one strategy: these are in order, and none is read any more where they go
+                    const Label label = {c, w, 0};
+                    if (stays && at + to < n_hist) {
+                        put(sh.f.label + to, label);
+                        hist[(uint32_t)(at + to)] = words(label);
+                    }
+                } else if (stays && to < LABELS) {
+                    sh.f.key[now][to] = __builtin_fma((double)w, KEY_W, (double)(b * (int)KEY_S + number));
+                    sh.f.cost[to] = c;
+                }
+                return count;
+            };
+            // the labels of strategy b: from those of the layer before in turn, 64 at a time
+            if (l && before <= 64) {   // a turn is all there is
+                for (int b = wave; b < n; b += WORKERS) {
+                    const Label old = label_at(sh.f.label + min(lane, before - 1));
+                    const int32_t next_w = sh.f.label[min(lane + 1, before - 1)].w;
+                    const double turn = sh.f.turns[now][old.s * n + b];
+                    const double2 *row = reinterpret_cast<const double2 *>(sh.f.lines[now] + b * LINE);
+                    double2 line[KEYS * WINDOW / 2];
+#pragma unroll
+                    for (int i = 0; i < KEYS * WINDOW / 2; ++i) line[i] = row[i];
+                    const double2 costs = row[KEYS * WINDOW / 2];
+                    const int32_t w = old.w + __builtin_bit_cast(int2v, costs.y).x;
+                    const double c = prefix_min(lane < before ? old.c + turn : INFINITY, before) + costs.x;
+                    const bool ends = lane >= before - 1 || next_w != old.w;
+                    double last = INFINITY;
+                    const double from = step_from(c, ends, last);   // (by all lanes)
+                    const bool stays = lane < before && ends && c < from && alive(line, c, w);
+                    emit(stays, b, 0, c, w);
+                }
+            } else {
+                for (int b = wave; b < n; b += WORKERS) {
+                    const double2 *row = reinterpret_cast<const double2 *>(sh.f.lines[now] + b * LINE);
+                    double2 line[KEYS * WINDOW / 2];
+#pragma unroll
+                    for (int i = 0; i < KEYS * WINDOW / 2; ++i) line[i] = row[i];
+                    const double2 costs = row[KEYS * WINDOW / 2];
+                    const double own = costs.x;
+                    const int32_t m = __builtin_bit_cast(int2v, costs.y).x;
+                    double least = INFINITY, last = INFINITY;   // up to the labels before these: of the sums, of the costs
+                    int found = 0;
+                    for (int j0 = 0; j0 < before; j0 += 64) {
+                        const int j = j0 + lane;
+                        double x;
+                        int32_t w = m;
+                        bool ends = true;
+                        if (l) {
+                            const Label old = label_at(sh.f.label + min(j, before - 1));
+                            ends = j >= before - 1 || sh.f.label[min(j + 1, before - 1)].w != old.w;
+                            x = old.c + sh.f.turns[now][old.s * n + b];
+                            w += old.w;
+                        } else {
+                            const gdouble M = inter + (size_t)sh.mat[0] * S * S + sh.kept[kept_at + b];
+                            x = 0.0 + M[(size_t)min(lane, S - 1) * S];
+                            x = min_f64(x, 0.0 + M[(size_t)min(lane + 64, S - 1) * S]);
+                            x = lane_of(prefix_min(x), 63);
+                        }
+                        const double y = min_f64(prefix_min(j < before ? x : INFINITY), least), c = y + own;
+                        const double from = step_from(c, ends, last);   // (by all lanes)
+                        const bool stays = j < before && ends && c < from && alive(line, c, w);
+                        found += emit(stays, b, found, c, w);
+                        least = lane_of(y, 63);
+                    }
+                }
+            }
+            executed += (double)(l ? before : S) * n;
+            __syncthreads();
+            const int sum = uniform(sh.found[slot]);
+            if (sum == 0 || sum > LABELS || at + sum > n_hist) {
+                give_up(sum == 0 ? 3 : 4);
+                return;
+            }
+            before = sum;
+            if (t == 0) {
+                sh.labels_at[l + 1] = at + sum;
+                sh.found[slot == 0 ? 2 : slot - 1] = 0;   // of the layer after the next: all have read what it was
+            }
+            if (n == 1) {
+                at += sum;
+                continue;
+            }
+            // In the order of their memory: a label's place is how many keys are lower.  Up to 8 lanes share them.
+            const int share = sum <= 64 ? 3 : sum <= 128 ? 2 : sum <= 256 ? 1 : 0, lanes = 1 << share;   // (bits)
+            const int part = ((sum + lanes - 1) >> share) + 7 & ~7;
+            for (int e0 = wave << (6 - share); e0 < sum; e0 += WORKERS << (6 - share)) {
+                const int e = e0 + (lane >> share), from = (lane & (lanes - 1)) * part;
+                const double key = sh.f.key[now][min(e, sum - 1)], c = sh.f.cost[min(e, sum - 1)];
+                const double2 *p = reinterpret_cast<const double2 *>(sh.f.key[now] + from);
+                int to[4] = {};
+                for (int i = 0; i < part; i += 8, p += 4) {
+                    const double2 x0 = p[0], x1 = p[1], x2 = p[2], x3 = p[3];
+                    to[0] += x0.x < key;
+                    to[1] += x0.y < key;
+                    to[2] += x1.x < key;
+                    to[3] += x1.y < key;
+                    to[0] += x2.x < key;
+                    to[1] += x2.y < key;
+                    to[2] += x3.x < key;
+                    to[3] += x3.y < key;
+                }
+                int place = to[0] + to[1] + to[2] + to[3];
+                if (share > 0) place += __builtin_amdgcn_mov_dpp(place, 0xb1, 0xf, 0xf, true);    // lane ^ 1
+                if (share > 1) place += __builtin_amdgcn_mov_dpp(place, 0x4e, 0xf, 0xf, true);    // lane ^ 2
+                if (share > 2) place += __builtin_amdgcn_mov_dpp(place, 0x141, 0xf, 0xf, true);   // mirrored within 8
+                if (e < sum && (lane & (lanes - 1)) == 0) {
+                    const long long k = (long long)key;
+                    const Label label = {c, (int32_t)(k >> 17), (int32_t)(k >> 11) & 63};
+                    put(sh.f.label + place, label);
+                    hist[(uint32_t)(at + place)] = words(label);
+                }
+            }
+            at += sum;
+            __syncthreads();
+        }
+        // the start rows: a wave per key
+        walks = wave < K && uniform(sh.budget[min(wave, K - 1)]) >= 0;
+        if (walks) {
+            v = uniform(sh.budget[wave]);
+            double c = INFINITY;
+            int s = INT32_MAX;
+            for (int j = lane; j < before; j += 64) {
+                const Label label = label_at(sh.f.label + j);
+                if (label.w <= v && (label.c < c || (label.c == c && label.s < s))) {
+                    c = label.c;
+                    s = label.s;
+                }
+            }
+            cheapest(c, s, before);
+            total = c;
+            cell = s;
+            if (!(total < INFINITY) && lane == 0) sh.lost = 1;
+        }
+    }
+    __syncthreads();
+    if (sh.lost) {
+        give_up(5);
+        return;
+    }
+
+    // ---- backwards ----
+    const giout res = GLOBAL(giout, I.res) + (size_t)min(wave, K - 1) * L;
+    if (walks && lane == 0) res[L - 1] = sh.kept[sh.layer[L - 1].y + cell];
+    for (int top = L - 1; top >= 0;) {
+        // layers low .. top: their costs, the transitions into them and the labels before them lie in LDS together
+        const int4 end = sh.layer[top + 1];
+        const int low_of_lane = top - lane;
+        const int4 begin = sh.layer[max(low_of_lane, 0)];
+        const bool fits = low_of_lane >= 0 && end.y - begin.y <= BACK_KEPT && end.z - begin.z <= BACK_TURNS &&
+                          sh.labels_at[top] - sh.labels_at[max(low_of_lane - 1, 0)] <= BACK_LABELS;
+        const int low = top + 1 - __popcll(__builtin_amdgcn_ballot_w64(fits));
+        const int kept0 = uniform(sh.layer[low].y), turns0 = uniform(sh.layer[low].z), labels0 = uniform(sh.labels_at[max(low - 1, 0)]);
+        const int labels = uniform(sh.labels_at[top]) - labels0;
+        __syncthreads();   // what lay there is not read any more
+        for (int e = t; e < end.y - kept0; e += THREADS) {
+            sh.b.mem[e] = hist_mem[(uint32_t)(kept0 + e)];
+            sh.b.intra[e] = hist_intra[(uint32_t)(kept0 + e)];
+        }
+        for (int e = t; e < end.z - turns0; e += THREADS) sh.b.turns[e] = hist_turns[(uint32_t)(turns0 + e)];
+        for (int e = t; e < labels; e += THREADS) *reinterpret_cast<int4v *>(sh.b.label + e) = hist[(uint32_t)(labels0 + e)];
+        __syncthreads();
+        if (walks) {
+            // what a step needs beside the cell is fetched a step ahead: the layer, the first 64 labels before it
+            int4 here = sh.layer[top], next = sh.layer[max(top - 1, 0)];
+            int first = uniform(sh.labels_at[max(top - 1, 0)]) - labels0, end_of = labels;
+            Label label = label_at(sh.b.label + min(first + lane, max(end_of, 1) - 1));
+            for (int l = top; l >= low; --l) {
+                const int n = uniform(here.x), kept_at = uniform(here.y) - kept0 + cell, turns_at = uniform(here.z) - turns0 + cell;
+                const int32_t m = sh.b.mem[kept_at];
+                const double own = sh.b.intra[kept_at];
+                if (l == 0) {
+                    v -= uniform(m);
+                    break;
+                }
+                const double turn = sh.b.turns[turns_at + label.s * n];
+                const int begin = first, all = end_of - first, kept_n = uniform(next.x), list = uniform(next.y);
+                here = next;
+                next = sh.layer[max(l - 2, 0)];
+                end_of = first;
+                first = max(uniform(sh.labels_at[max(l - 2, 0)]) - labels0, 0);
+                v -= uniform(m);
+                double c = lane < all && label.w <= v ? (label.c + turn) + own : INFINITY;
+                int s = c < INFINITY ? label.s : INT32_MAX;
+                for (int j = lane + 64; j < all; j += 64) {
+                    const Label other = label_at(sh.b.label + begin + j);
+                    const double x = other.w <= v ? (other.c + sh.b.turns[turns_at + other.s * n]) + own : INFINITY;
+                    if (x < c || (x == c && other.s < s)) {
+                        c = x;
+                        s = other.s;
+                    }
+                }
+                label = label_at(sh.b.label + min(first + lane, max(end_of, 1) - 1));
+                if (all == 1) s = __builtin_amdgcn_readlane(s, 0);
+                else cheapest(c, s, all);
+                cell = min(s, kept_n - 1);   // (there is one: the cell has a cost)
+                if (lane == 0) res[l - 1] = sh.kept[list + cell];
+            }
+        }
+        top = low - 1;
+    }
+    if (wave < K && lane == 0) {
+        out->total[wave] = walks ? total + GLOBAL(gdouble, I.other_time)[wave] : INFINITY;
+        out->remaining[wave] = walks ? v : -1;
+    }
+    if (t == 0) {
+        out->executed = executed;
+        out->status = 0;
+    }
+}
+
+}  // namespace
+
+hipError_t gdp_launch_frontier(const GdpBoundInst *inst, int n, int max_K, hipStream_t stream)
+{
+    if (max_K <= 4) gdp_frontier_kernel<4><<<dim3((unsigned)n), THREADS, sizeof(Shared), stream>>>(inst);
+    else gdp_frontier_kernel<8><<<dim3((unsigned)n), THREADS, sizeof(Shared), stream>>>(inst);
+    return hipGetLastError();
+}
