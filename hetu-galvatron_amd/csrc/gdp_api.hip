@@ -523,8 +523,13 @@ namespace {
 int find_variant(int ts, int r) { return gdp_find_variant(ts, r); }
 }  // namespace
 
+// What a plan holds where its instances are solved by bounds and the DP over what they leave.
+struct PlanBounds;
+static void give_back(PlanBounds *b);
+
 struct gdp_plan {
     int n = 0;
+    PlanBounds *bounds = nullptr;   // null: the launch schemes below
     int device = 0;
     std::vector<HostInst> inst;  // sorted order
     std::vector<Group> groups;
@@ -859,10 +864,12 @@ static int validate_costs(const gdp_problem *p, int i, double *magnitude)
     return GDP_OK;
 }
 
-int gdp_validate(const gdp_problem *p, int i)
+int gdp_validate(const gdp_problem *p, int i, double *magnitude)
 {
-    double magnitude = 0;
-    return validate_costs(p, i, &magnitude);
+    double m = 0;
+    const int rc = validate_costs(p, i, &m);
+    if (magnitude) *magnitude = m;
+    return rc;
 }
 
 namespace {
@@ -884,7 +891,7 @@ int validate_f0_all(int32_t n, const gdp_problem *const *p, std::vector<char> &f
 int validate_all(int32_t n, const gdp_problem *const *p, std::vector<char> &f0_live)
 {
     for (int i = 0; i < n; ++i) {
-        const int rc = gdp_validate(p[i], i);
+        const int rc = gdp_validate(p[i], i, nullptr);
         if (rc != GDP_OK) return rc;
     }
     return validate_f0_all(n, p, f0_live);
@@ -904,6 +911,7 @@ void destroy(gdp_plan *pl)
         pl->holds_fused = false;
         fused_turn_give();
     }
+    give_back(pl->bounds);
     if (pl->dbase) arena_give(pl->device, pl->dbase, pl->dalloc);
     for (hipEvent_t e : pl->ev_relax) (void)hipEventDestroy(e);
     lane_give(pl->lane);
@@ -2436,6 +2444,9 @@ int create_checked(int32_t n, const gdp_problem *const *p, const char *f0_live, 
 
 extern "C" {
 
+static void take_bounds(int32_t n, const gdp_problem *const *p, const std::vector<double> &magnitude, gdp_plan *plan);
+static int run_bounds(gdp_plan *plan, int32_t mode, gdp_timing *t, bool *done);
+
 int gdp_plan_create(int32_t n, const gdp_problem *const *p, gdp_plan **out)
 {
     gdp_clear_error();
@@ -2444,10 +2455,21 @@ int gdp_plan_create(int32_t n, const gdp_problem *const *p, gdp_plan **out)
     if (n < 1 || !p) return fail(GDP_E_BADARG, "need at least one problem");
     if (n > 65535) return fail(GDP_E_BADARG, "at most 65535 instances per plan");
     try {
+        std::vector<double> magnitude((size_t)n, 0.0);
+        for (int i = 0; i < n; ++i) {
+            const int rc = validate_costs(p[i], i, &magnitude[(size_t)i]);
+            if (rc != GDP_OK) return rc;
+        }
         std::vector<char> f0_live;
-        const int rc = validate_all(n, p, f0_live);
-        if (rc != GDP_OK) return rc;
-        return create_checked(n, p, f0_live.data(), out);
+        int rc = validate_f0_all(n, p, f0_live);
+        if (rc == GDP_OK) rc = create_checked(n, p, f0_live.data(), out);
+        if (rc == GDP_OK && std::find(f0_live.begin(), f0_live.end(), 1) == f0_live.end()) {
+            try {
+                take_bounds(n, p, magnitude, *out);
+            } catch (const std::bad_alloc &) {   // without them
+            }
+        }
+        return rc;
     } catch (const std::bad_alloc &) {
         return fail(GDP_E_NOMEM, "host allocation failed");
     }
@@ -2457,7 +2479,13 @@ int gdp_plan_run(gdp_plan *plan, int32_t timing_mode, gdp_timing *timing)
 {
     gdp_clear_error();
     if (!plan) return fail(GDP_E_BADARG, "null plan");
-    return run(plan, timing ? timing_mode : 0, timing);
+    const int32_t mode = timing ? timing_mode : 0;
+    if (plan->bounds && mode < 2) {   // (2 asks what the relaxation kernels take)
+        bool done = false;
+        const int rc = run_bounds(plan, mode, timing, &done);
+        if (rc != GDP_OK || done) return rc;
+    }
+    return run(plan, mode, timing);
 }
 
 int gdp_plan_fetch(gdp_plan *plan, gdp_result *const *r)
@@ -2471,6 +2499,12 @@ int gdp_plan_set_option(gdp_plan *plan, int32_t option, int64_t value)
 {
     gdp_clear_error();
     if (!plan) return fail(GDP_E_BADARG, "null plan");
+    if (plan->bounds && option >= GDP_OPT_FUSED && option <= GDP_OPT_DEBUG_STALL) {   // each of them is about the launch schemes
+        GDP_HIP(hipSetDevice(plan->device));
+        GDP_HIP(hipStreamSynchronize(plan->stream));
+        give_back(plan->bounds);
+        plan->bounds = nullptr;
+    }
     switch (option) {
         case GDP_OPT_FUSED:
             if (value != 0 && !plan->can_fuse)
@@ -2514,7 +2548,7 @@ int gdp_debug_check_layout(int32_t n, const gdp_problem *const *p, int32_t num_c
     if (n > 65535) return fail(GDP_E_BADARG, "at most 65535 instances per plan");
     if (num_cu < 1 || lds_per_cu < 0) return fail(GDP_E_BADARG, "bad device description");
     for (int i = 0; i < n; ++i) {
-        int rc = gdp_validate(p[i], i);
+        int rc = gdp_validate(p[i], i, nullptr);
         if (rc == GDP_OK) rc = gdp_validate_f0(p[i], i, nullptr);
         if (rc != GDP_OK) return rc;
     }
@@ -2586,16 +2620,9 @@ struct Reduced {
 
 static constexpr size_t REDUCE_MAX_BYTES = (size_t)4 << 30;   // of device memory for the bounds of a slice (GALVATRON_DP_ARENA_MB if less)
 
-static bool has_bounds_form(const gdp_problem *q)
-{
-    constexpr uint32_t whole = GDP_EXPORT_F | GDP_EXPORT_MARK | GDP_COMPUTE_ALL | GDP_KEEP_MARKS | GDP_LAUNCH_FUSED | GDP_LAUNCH_PER_LAYER;
-    return !(q->flags & whole) && q->L >= 2 && q->L <= GDP_BOUND_MAX_L && q->S >= 2 && q->S <= GDP_BOUND_MAX_S &&
-           q->n_key >= 1 && q->n_key <= GDP_BOUND_MAX_KEY && q->L * q->S <= GDP_BOUND_MAX_LS;
-}
-
 static bool reducible(const gdp_problem *q, double magnitude)
 {
-    if (!has_bounds_form(q) || !(magnitude < 1e100)) return false;
+    if (!bounds::has_form(q) || !(magnitude < 1e100)) return false;
     // a memory cost of 0 reads the layer's own row: the recurrence is not a path through the layers then
     for (size_t k = 0; k < (size_t)q->L * q->S; ++k)
         if (q->mem[k] == 0) return false;
@@ -2660,7 +2687,7 @@ static bool bounds_pay(int32_t n, const gdp_problem *const *p)
         uint64_t &word = seen[q->S / 64], bit = 1ull << (q->S % 64);
         groups += !(word & bit);
         word |= bit;
-        if (!has_bounds_form(q)) continue;
+        if (!bounds::has_form(q)) continue;
         const double SS = (double)q->S * q->S;
         work += (double)q->L * q->V * SS;
         layers += q->L;
@@ -2673,22 +2700,6 @@ static bool bounds_pay(int32_t n, const gdp_problem *const *p)
     const bool wide = max_S > 88;
     const double passes = layers * 2 * bound_multipliers((size_t)n) / 1024;
     return save >= std::max(max_L * (wide ? STEP_16 : STEP), passes * (wide ? BUSY_16 : BUSY)) + (n > 1 ? entries * ENTRY * undominated(n, p) : 0.0);
-}
-
-// The multipliers of an instance: 0 and a geometric series around (range of times) / (range of memory costs).
-static void multipliers(const gdp_problem *q, int n_lam, double *lam)
-{
-    double t0 = INFINITY, t1 = -INFINITY, m0 = INFINITY, m1 = 0;
-    for (size_t k = 0; k < (size_t)q->L * q->S; ++k) {
-        if (q->mem[k] >= q->V || !(q->intra[k] < INFINITY)) continue;
-        t0 = std::min(t0, q->intra[k]);
-        t1 = std::max(t1, q->intra[k]);
-        m0 = std::min(m0, (double)q->mem[k]);
-        m1 = std::max(m1, (double)q->mem[k]);
-    }
-    const double range = t1 > t0 ? t1 - t0 : 1.0, base = range / std::max(1.0, m1 - m0);
-    lam[0] = 0.0;
-    for (int i = 1; i < n_lam; ++i) lam[i] = base * std::exp2(-6.0 + 12.0 * (i - 1) / (n_lam - 2));
 }
 
 // The smaller instance of q, given what stays ([L][S]); false where it would not be a good deal smaller.
@@ -2820,13 +2831,29 @@ struct BoundLease {
     }
 };
 
-// Bounds of the instances of one slice in one set of launches, and behind them the DP over what stays.  out[i]: the
-// results of instance i; the smaller instance that is left of it where its labels are too many; empty where it is to be
-// solved whole.  The calling thread looks through initial costs while the device works.
-static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &magnitude, BoundEntry *es, int m, int n_lam,
-                        InitialScan &scan, std::vector<std::unique_ptr<Reduced>> &out)
-{
+// The bounds of some instances, and behind them the DP over what stays, in one allocation and one set of launches.
+struct BoundSlice {
+    BoundEntry *es = nullptr;
+    int m = 0, n_lam = 0, max_LS = 0, max_S = 0, max_K = 0;
     std::vector<int2> pairs;
+    // [0, up_bytes): what is uploaded; the results after it; what stays; the rest stays on the device
+    size_t off_inst = 0, off_pairs = 0, up_bytes = 0, back_bytes = 0, keep_begin = 0, keep_bytes = 0, bytes = 0;
+
+    void lay_out(const gdp_problem *const *p, BoundEntry *entries, int count, int multipliers);
+    void fill(const gdp_problem *const *p, const std::vector<double> &magnitude, char *up, char *dev) const;
+    hipError_t enqueue(char *dev, hipStream_t stream) const;
+    const GdpFrontierOut &out_of(const char *back, int j) const
+    {
+        return *reinterpret_cast<const GdpFrontierOut *>(back + (es[j].off_out - up_bytes));
+    }
+    const int32_t *res_of(const char *back, int j) const { return reinterpret_cast<const int32_t *>(back + (es[j].off_res - up_bytes)); }
+};
+
+void BoundSlice::lay_out(const gdp_problem *const *p, BoundEntry *entries, int count, int multipliers)
+{
+    es = entries;
+    m = count;
+    n_lam = multipliers;
     size_t at = 0;
     auto place = [&](size_t bytes) { const size_t o = at; at = align_up(at + bytes, 256); return o; };
     for (int i = 0; i < m; ++i) {   // the stages of one fit and the tasks of one sweep share their matrices
@@ -2840,9 +2867,8 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
             }
         }
     }
-    int max_LS = 0, max_S = 0, max_K = 0;
     // what is uploaded, what is copied back, what stays on the device
-    const size_t off_inst = place(sizeof(GdpBoundInst) * (size_t)m);
+    off_inst = place(sizeof(GdpBoundInst) * (size_t)m);
     for (int j = 0; j < m; ++j) {
         BoundEntry &e = es[j];
         const gdp_problem *q = p[e.orig];
@@ -2861,17 +2887,18 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
         max_S = std::max(max_S, q->S);
         max_K = std::max(max_K, q->n_key);
     }
-    const size_t off_pairs = place(sizeof(int2) * pairs.size());
-    const size_t up_bytes = at;
+    off_pairs = place(sizeof(int2) * pairs.size());
+    up_bytes = at;
     for (int j = 0; j < m; ++j) {
         BoundEntry &e = es[j];
         const gdp_problem *q = p[e.orig];
         e.off_out = place(sizeof(GdpFrontierOut));
         e.off_res = place(4 * (size_t)q->n_key * q->L);
     }
-    const size_t back_bytes = at - up_bytes, keep_begin = at;
+    back_bytes = at - up_bytes;
+    keep_begin = at;
     for (int j = 0; j < m; ++j) es[j].off_keep = place((size_t)p[es[j].orig]->L * p[es[j].orig]->S);
-    const size_t keep_bytes = at - keep_begin;
+    keep_bytes = at - keep_begin;
     for (int j = 0; j < m; ++j) {
         BoundEntry &e = es[j];
         const gdp_problem *q = p[e.orig];
@@ -2893,33 +2920,19 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
         e.off_hist_mem = place(4 * GDP_FRONTIER_KEPT);
         e.off_hist_intra = place(8 * GDP_FRONTIER_KEPT);
     }
+    bytes = at;
+}
 
-    // A device or a host that is out of memory solves the instances whole, in the parts that fit; what else may be
-    // wrong with the device is found, and reported, there.
-    BoundLease lease;
-    if (hipGetDevice(&lease.device) != hipSuccess || lane_take(lease.device, back_bytes, up_bytes, &lease.lane) != hipSuccess ||
-        arena_take(lease.device, at, &lease.dev, &lease.dev_bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        lease.dev = nullptr;
-        return GDP_OK;
-    }
-    const Lane &lane = lease.lane;
-    char *const dev = lease.dev;
-    std::vector<char> pageable;
-    char *up = lane.up;
-    if (lane.up_bytes < up_bytes) {
-        pageable.resize(up_bytes);
-        up = pageable.data();
-    }
+void BoundSlice::fill(const gdp_problem *const *p, const std::vector<double> &magnitude, char *up, char *dev) const
+{
     for (int j = 0; j < m; ++j) {
-        BoundEntry &e = es[j];
-        const BoundEntry &te = es[e.table_of];
+        const BoundEntry &e = es[j], &te = es[e.table_of];
         const gdp_problem *q = p[e.orig];
         const size_t LS = (size_t)q->L * q->S, SS = (size_t)q->S * q->S;
         memcpy(up + e.off_mem, q->mem, 4 * LS);
         memcpy(up + e.off_intra, q->intra, 8 * LS);
         for (int l = 0; l < q->L; ++l) reinterpret_cast<int32_t *>(up + e.off_index)[l] = e.h.matrix(q, l);
-        multipliers(q, n_lam, reinterpret_cast<double *>(up + e.off_lam));
+        bounds::multipliers(q, n_lam, reinterpret_cast<double *>(up + e.off_lam));
         memcpy(up + e.off_budget, e.budget.data(), 8 * e.budget.size());
         memcpy(up + e.off_other_time, q->other_time, 8 * e.budget.size());
         if (e.table_of == j)
@@ -2958,27 +2971,60 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
         memcpy(up + off_inst + sizeof b * (size_t)j, &b, sizeof b);
     }
     memcpy(up + off_pairs, pairs.data(), sizeof(int2) * pairs.size());
+}
+
+hipError_t BoundSlice::enqueue(char *dev, hipStream_t stream) const
+{
+    const GdpBoundInst *inst = reinterpret_cast<const GdpBoundInst *>(dev + off_inst);
+    const hipError_t e = bounds::launch(inst, m, n_lam, max_LS, max_S, max_K, reinterpret_cast<const int2 *>(dev + off_pairs),
+                                           (int)pairs.size(), stream);
+    return e == hipSuccess ? bounds::launch_labels(inst, m, max_K, stream) : e;
+}
+
+// Bounds of the instances of one slice in one set of launches, and behind them the DP over what stays.  out[i]: the
+// results of instance i; the smaller instance that is left of it where its labels are too many; empty where it is to be
+// solved whole.  The calling thread looks through initial costs while the device works.
+static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &magnitude, BoundEntry *es, int m, int n_lam,
+                        InitialScan &scan, std::vector<std::unique_ptr<Reduced>> &out)
+{
+    BoundSlice slice;
+    slice.lay_out(p, es, m, n_lam);
+    // A device or a host that is out of memory solves the instances whole, in the parts that fit; what else may be
+    // wrong with the device is found, and reported, there.
+    BoundLease lease;
+    if (hipGetDevice(&lease.device) != hipSuccess || lane_take(lease.device, slice.back_bytes, slice.up_bytes, &lease.lane) != hipSuccess ||
+        arena_take(lease.device, slice.bytes, &lease.dev, &lease.dev_bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        lease.dev = nullptr;
+        return GDP_OK;
+    }
+    const Lane &lane = lease.lane;
+    char *const dev = lease.dev;
+    std::vector<char> pageable;
+    char *up = lane.up;
+    if (lane.up_bytes < slice.up_bytes) {
+        pageable.resize(slice.up_bytes);
+        up = pageable.data();
+    }
+    slice.fill(p, magnitude, up, dev);
     bool stats = false;
     {
         std::lock_guard<std::mutex> lk(g_stats_mu);
         stats = g_stats_on;
     }
-    hipError_t err = hipMemcpyAsync(dev, up, up_bytes, hipMemcpyHostToDevice, lane.stream);
+    hipError_t err = hipMemcpyAsync(dev, up, slice.up_bytes, hipMemcpyHostToDevice, lane.stream);
     if (err == hipSuccess && stats) err = hipEventRecord(lane.ev_begin, lane.stream);
-    if (err == hipSuccess)
-        err = gdp_launch_bounds(reinterpret_cast<const GdpBoundInst *>(dev + off_inst), m, n_lam, max_LS, max_S, max_K,
-                                reinterpret_cast<const int2 *>(dev + off_pairs), (int)pairs.size(), lane.stream);
-    if (err == hipSuccess) err = gdp_launch_frontier(reinterpret_cast<const GdpBoundInst *>(dev + off_inst), m, max_K, lane.stream);
+    if (err == hipSuccess) err = slice.enqueue(dev, lane.stream);
     if (err == hipSuccess && stats) err = hipEventRecord(lane.ev_end, lane.stream);
-    if (err == hipSuccess) err = hipMemcpyAsync(lane.back, dev + up_bytes, back_bytes, hipMemcpyDeviceToHost, lane.stream);
+    if (err == hipSuccess) err = hipMemcpyAsync(lane.back, dev + slice.up_bytes, slice.back_bytes, hipMemcpyDeviceToHost, lane.stream);
     while (scan.step() && hipStreamQuery(lane.stream) == hipErrorNotReady) {}
     hipError_t es2 = hipStreamSynchronize(lane.stream);
     if (err == hipSuccess) err = es2;
     std::vector<char> keep;
     for (int j = 0; j < m && err == hipSuccess && keep.empty(); ++j)
-        if (reinterpret_cast<const GdpFrontierOut *>(lane.back + (es[j].off_out - up_bytes))->status > 1) {
-            keep.resize(keep_bytes);
-            err = hipMemcpyAsync(keep.data(), dev + keep_begin, keep_bytes, hipMemcpyDeviceToHost, lane.stream);
+        if (slice.out_of(lane.back, j).status > 1) {
+            keep.resize(slice.keep_bytes);
+            err = hipMemcpyAsync(keep.data(), dev + slice.keep_begin, slice.keep_bytes, hipMemcpyDeviceToHost, lane.stream);
             es2 = hipStreamSynchronize(lane.stream);
             if (err == hipSuccess) err = es2;
         }
@@ -2993,17 +3039,17 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
     for (int j = 0; j < m; ++j) {
         const BoundEntry &e = es[j];
         const gdp_problem *q = p[e.orig];
-        const GdpFrontierOut &o = *reinterpret_cast<const GdpFrontierOut *>(lane.back + (e.off_out - up_bytes));
+        const GdpFrontierOut &o = slice.out_of(lane.back, j);
         if (o.status == 1) continue;   // a key whose budget no path was found for keeps everything
         std::unique_ptr<Reduced> d(new Reduced());
         if (o.status == 0) {
-            const int32_t *res = reinterpret_cast<const int32_t *>(lane.back + (e.off_res - up_bytes));
+            const int32_t *res = slice.res_of(lane.back, j);
             d->solved = true;
             d->executed = o.executed;
             d->total.assign(o.total, o.total + q->n_key);
             d->remaining.assign(o.remaining, o.remaining + q->n_key);
             d->res.assign(res, res + (size_t)q->n_key * q->L);
-        } else if (!build_reduced(q, e.h, reinterpret_cast<const uint8_t *>(keep.data() + (e.off_keep - keep_begin)), e.budget.data(), *d)) {
+        } else if (!build_reduced(q, e.h, reinterpret_cast<const uint8_t *>(keep.data() + (e.off_keep - slice.keep_begin)), e.budget.data(), *d)) {
             continue;
         }
         out[(size_t)e.orig] = std::move(d);
@@ -3011,35 +3057,46 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
     return GDP_OK;
 }
 
+static bool bounds_allowed(bool *forced)
+{
+    const char *env = getenv("GALVATRON_DP_REDUCE"), *skip = getenv("GALVATRON_DP_SKIP");
+    *forced = env && *env && atoi(env) != 0;
+    return !(env && *env && !*forced) && !(skip && *skip && atoi(skip) == 0);
+}
+
+// The entry of an instance whose bounds can be taken.
+static bool bound_entry(const gdp_problem *q, int orig, double magnitude, BoundEntry &e)
+{
+    if (!reducible(q, magnitude)) return false;
+    e.orig = orig;
+    int64_t least = 0;
+    for (int l = 0; l < q->L; ++l) least += *std::min_element(q->mem + (size_t)l * q->S, q->mem + (size_t)(l + 1) * q->S);
+    bool any = false;
+    for (int k = 0; k < q->n_key; ++k) {
+        const int64_t b = (int64_t)q->V - 1 - q->other_mem[k];
+        e.budget.push_back(b >= least ? b : -1);
+        any = any || b >= least;
+    }
+    if (!any) return false;
+    e.h.S = q->S;
+    e.h.n_inter = q->inter_index ? q->n_inter : q->L;
+    if (!q->inter_index) share_equal_matrices(q, e.h);
+    return true;
+}
+
 // Bounds of the instances of a batch that have the form, in consecutive slices of at most `limit` bytes of device
 // memory each; instances that need more by themselves are solved whole.  Initial costs are taken to be zeros.
 static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vector<double> &magnitude, InitialScan &scan,
                         size_t limit, std::vector<std::unique_ptr<Reduced>> &out)
 {
-    const char *env = getenv("GALVATRON_DP_REDUCE"), *skip = getenv("GALVATRON_DP_SKIP");
-    const bool forced = env && *env && atoi(env) != 0;
-    if ((env && *env && !forced) || (skip && *skip && atoi(skip) == 0)) return GDP_OK;
+    bool forced = false;
+    if (!bounds_allowed(&forced)) return GDP_OK;
     if (!forced && (!bounds_pay(n, p) || !InitialScan::device_bound(dense_work(n, p), scan.alone()))) return GDP_OK;
 
     std::vector<BoundEntry> es;
     for (int i = 0; i < n; ++i) {
-        if (!reducible(p[i], magnitude[(size_t)i])) continue;
-        const gdp_problem *q = p[i];
         BoundEntry e;
-        e.orig = i;
-        int64_t least = 0;
-        for (int l = 0; l < q->L; ++l) least += *std::min_element(q->mem + (size_t)l * q->S, q->mem + (size_t)(l + 1) * q->S);
-        bool any = false;
-        for (int k = 0; k < q->n_key; ++k) {
-            const int64_t b = (int64_t)q->V - 1 - q->other_mem[k];
-            e.budget.push_back(b >= least ? b : -1);
-            any = any || b >= least;
-        }
-        if (!any) continue;
-        e.h.S = q->S;
-        e.h.n_inter = q->inter_index ? q->n_inter : q->L;
-        if (!q->inter_index) share_equal_matrices(q, e.h);
-        es.push_back(std::move(e));
+        if (bound_entry(p[i], i, magnitude[(size_t)i], e)) es.push_back(std::move(e));
     }
     const int n_lam = bound_multipliers(es.size());
     int rc = GDP_OK;
@@ -3055,6 +3112,90 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
         begin = std::max(end, begin + 1);
     }
     return rc;
+}
+
+struct PlanBounds {
+    std::vector<BoundEntry> es;   // one per instance
+    BoundSlice slice;
+    BoundLease lease;
+    std::vector<GdpDevOut> out;   // as the plan's own results are laid out
+    std::vector<int32_t> res;
+};
+
+static void give_back(PlanBounds *b) { delete b; }
+
+// A plan whose instances all have the form, where it pays: their inputs for the bounds on the device too.  Anything that
+// is missing leaves the plan to its launch schemes.
+static void take_bounds(int32_t n, const gdp_problem *const *p, const std::vector<double> &magnitude, gdp_plan *plan)
+{
+    bool forced = false;
+    if (plan->keep_marks || !bounds_allowed(&forced) || (!forced && !bounds_pay(n, p))) return;
+    std::unique_ptr<PlanBounds> b(new PlanBounds());
+    size_t bytes = 0;
+    const int n_lam = bound_multipliers((size_t)n);
+    for (int i = 0; i < n; ++i) {
+        BoundEntry e;
+        if (!bound_entry(p[i], i, magnitude[(size_t)i], e)) return;
+        bytes += bound_bytes(p[i], e.h, n_lam);
+        if (bytes > REDUCE_MAX_BYTES) return;
+        b->es.push_back(std::move(e));
+    }
+    b->slice.lay_out(p, b->es.data(), n, n_lam);
+    b->out.resize((size_t)plan->n_key_total);
+    b->res.resize(plan->n_res_total);
+    std::vector<char> up(b->slice.up_bytes);
+    b->lease.device = plan->device;
+    if (lane_take(plan->device, b->slice.back_bytes, 0, &b->lease.lane) != hipSuccess ||
+        arena_take(plan->device, b->slice.bytes, &b->lease.dev, &b->lease.dev_bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        b->lease.dev = nullptr;
+        return;
+    }
+    b->slice.fill(p, magnitude, up.data(), b->lease.dev);
+    if (hipMemcpyAsync(b->lease.dev, up.data(), b->slice.up_bytes, hipMemcpyHostToDevice, plan->stream) != hipSuccess ||
+        hipStreamSynchronize(plan->stream) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    plan->bounds = b.release();
+}
+
+// One run by bounds.  *done stays false where an instance has more labels than fit: the plan then runs its launch schemes
+// from here on.
+static int run_bounds(gdp_plan *plan, int32_t mode, gdp_timing *t, bool *done)
+{
+    PlanBounds &b = *plan->bounds;
+    const char *const back = b.lease.lane.back;
+    GDP_HIP(hipSetDevice(plan->device));
+    if (mode >= 1) GDP_HIP(hipEventRecord(plan->ev_begin, plan->stream));
+    GDP_HIP(b.slice.enqueue(b.lease.dev, plan->stream));
+    if (mode >= 1) GDP_HIP(hipEventRecord(plan->ev_end, plan->stream));
+    GDP_HIP(hipMemcpyAsync(b.lease.lane.back, b.lease.dev + b.slice.up_bytes, b.slice.back_bytes, hipMemcpyDeviceToHost, plan->stream));
+    GDP_HIP(hipStreamSynchronize(plan->stream));
+    double executed = 0;
+    for (const HostInst &h : plan->inst) {
+        const GdpFrontierOut &o = b.slice.out_of(back, h.orig);
+        if (o.status != 0) {
+            give_back(plan->bounds);
+            plan->bounds = nullptr;
+            return GDP_OK;
+        }
+        executed += o.executed;
+        const int32_t *res = b.slice.res_of(back, h.orig);
+        for (int k = 0; k < h.n_key; ++k) b.out[(size_t)(h.key_begin + k)] = {o.total[k], o.remaining[k], o.remaining[k] >= 0};
+        memcpy(b.res.data() + h.res_begin, res, sizeof(int32_t) * (size_t)h.n_key * h.L);
+    }
+    plan->h_out = b.out.data();
+    plan->h_res = b.res.data();
+    plan->ran = true;
+    if (t) {
+        memset(t, 0, sizeof *t);
+        t->relaxations = plan->relaxations;
+        t->executed = executed;
+        if (mode >= 1) GDP_HIP(hipEventElapsedTime(&t->total_ms, plan->ev_begin, plan->ev_end));
+    }
+    *done = true;
+    return GDP_OK;
 }
 
 // The results of a smaller instance in the terms of the whole one.

@@ -5,6 +5,8 @@
 
 #include <stdint.h>
 
+#include "../../include/galvatron_dp_hip.h"
+
 constexpr int GDP_BOUND_MAX_S = 128;      // strategies
 constexpr int GDP_BOUND_MAX_L = 512;      // layers
 constexpr int GDP_BOUND_MAX_LS = 40960;   // layers x strategies
@@ -57,13 +59,20 @@ struct GdpBoundInst {
     int32_t L, V, S, K, T, n_hist, n_hist_turns;
 };
 
+// Nothing in here allocates: gdp_solve_static uses it too.
+namespace bounds {
+// Whether an instance has the form, its costs apart (reducible in gdp_api.hip).
+__attribute__((visibility("hidden"))) bool has_form(const gdp_problem *q);
+// The multipliers of an instance: 0 and a geometric series around (range of times) / (range of memory costs).
+__attribute__((visibility("hidden"))) void multipliers(const gdp_problem *q, int n_lam, double *lam);
 // Copies the matrices, runs the passes of all multipliers, finds the upper bounds and marks what stays.
 // pairs: {instance, matrix} of every matrix that is to be copied.
 __attribute__((visibility("hidden")))
-hipError_t gdp_launch_bounds(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K, const int2 *pairs,
-                             int n_pairs, hipStream_t stream);
-// The DP over what stays (gdp_frontier.hip), after gdp_launch_bounds.
-__attribute__((visibility("hidden"))) hipError_t gdp_launch_frontier(const GdpBoundInst *inst, int n, int max_K, hipStream_t stream);
+hipError_t launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K, const int2 *pairs, int n_pairs,
+                  hipStream_t stream);
+// The DP over what stays (gdp_frontier.hip), after it.
+__attribute__((visibility("hidden"))) hipError_t launch_labels(const GdpBoundInst *inst, int n, int max_K, hipStream_t stream);
+}  // namespace bounds
 
 #ifdef __HIPCC__
 // A double from an unsigned number of the same order.

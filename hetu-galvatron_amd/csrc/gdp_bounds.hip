@@ -380,8 +380,30 @@ __global__ __launch_bounds__(64 * PARTS) void gdp_bound_keep_kernel(const GdpBou
 
 }  // namespace
 
-hipError_t gdp_launch_bounds(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K, const int2 *pairs,
-                             int n_pairs, hipStream_t stream)
+bool bounds::has_form(const gdp_problem *q)
+{
+    constexpr uint32_t whole = GDP_EXPORT_F | GDP_EXPORT_MARK | GDP_COMPUTE_ALL | GDP_KEEP_MARKS | GDP_LAUNCH_FUSED | GDP_LAUNCH_PER_LAYER;
+    return !(q->flags & whole) && q->L >= 2 && q->L <= GDP_BOUND_MAX_L && q->S >= 2 && q->S <= GDP_BOUND_MAX_S &&
+           q->n_key >= 1 && q->n_key <= GDP_BOUND_MAX_KEY && q->L * q->S <= GDP_BOUND_MAX_LS;
+}
+
+void bounds::multipliers(const gdp_problem *q, int n_lam, double *lam)
+{
+    double t0 = INFINITY, t1 = -INFINITY, m0 = INFINITY, m1 = 0;
+    for (size_t k = 0; k < (size_t)q->L * q->S; ++k) {
+        if (q->mem[k] >= q->V || !(q->intra[k] < INFINITY)) continue;
+        t0 = fmin(t0, q->intra[k]);
+        t1 = fmax(t1, q->intra[k]);
+        m0 = fmin(m0, (double)q->mem[k]);
+        m1 = fmax(m1, (double)q->mem[k]);
+    }
+    const double range = t1 > t0 ? t1 - t0 : 1.0, base = range / fmax(1.0, m1 - m0);
+    lam[0] = 0.0;
+    for (int i = 1; i < n_lam; ++i) lam[i] = base * exp2(-6.0 + 12.0 * (i - 1) / (n_lam - 2));
+}
+
+hipError_t bounds::launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K, const int2 *pairs, int n_pairs,
+                          hipStream_t stream)
 {
     gdp_bound_transpose_kernel<<<dim3((unsigned)n_pairs, (unsigned)((max_S + 15) / 16)), 256, 0, stream>>>(inst, pairs);
     hipError_t e = hipGetLastError();

@@ -631,7 +631,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
 
 }  // namespace
 
-hipError_t gdp_launch_frontier(const GdpBoundInst *inst, int n, int max_K, hipStream_t stream)
+hipError_t bounds::launch_labels(const GdpBoundInst *inst, int n, int max_K, hipStream_t stream)
 {
     if (max_K <= 4) gdp_frontier_kernel<4><<<dim3((unsigned)n), THREADS, sizeof(Shared), stream>>>(inst);
     else gdp_frontier_kernel<8><<<dim3((unsigned)n), THREADS, sizeof(Shared), stream>>>(inst);

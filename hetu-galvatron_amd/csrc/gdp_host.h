@@ -12,8 +12,9 @@ int gdp_fail_hip(hipError_t e, const char *what);    // GDP_E_NOMEM for an alloc
 
 // Host-side checks of one problem (instance number i is for the message only): sizes, null pointers,
 // mem >= 0, other_mem >= 0, inter_index in range, no NaN / -inf, no possible overflow -- everything but the
-// initial costs.  Allocates nothing.
-int gdp_validate(const gdp_problem *p, int i);
+// initial costs.  *magnitude (may be null): sum over the layers of the largest finite magnitudes of the cost arrays.
+// Allocates nothing.
+int gdp_validate(const gdp_problem *p, int i, double *magnitude);
 // ... and of its initial costs (gdp_problem.f0; GDP_OK when there are none): no NaN / -inf / -0.0, no possible
 // overflow.  *f0_live (may be null): they hold something other than zeros.  Allocates nothing.
 int gdp_validate_f0(const gdp_problem *p, int i, bool *f0_live);

@@ -10,9 +10,10 @@
 // inputs in a fixed host array, runs on the null stream with synchronous copies, and calls no
 // hipMalloc / hipFree / hipHostMalloc / stream or event creation and no host allocator.
 //
-// It uses the kernels of the other entry points in the layout that needs the least memory: two cost
-// buffers used in turn plus the one-byte argmin table (what GDP_KEEP_MARKS selects), one launch per
-// layer, every cell computed.  Results are the same bits as gdp_solve's.
+// An instance that has the form is solved by bounds and the DP over what they leave (gdp_bounds.hip, gdp_frontier.hip).  Any
+// other, and one of which too much stays, by the kernels of the other entry points in the layout that needs the least
+// memory: two cost buffers used in turn plus the one-byte argmin table (what GDP_KEEP_MARKS selects), one launch per layer,
+// every cell computed.  Results are the same bits as gdp_solve's.
 //
 // The array is per process and per device (every device the library's code object is loaded on holds
 // its own copy at its own address) and keeps the contents of the last call; a call rewrites everything
@@ -23,6 +24,7 @@
 #include <cstring>
 #include <mutex>
 
+#include "gdp_bounds.h"
 #include "gdp_host.h"
 #include "gdp_kernels.h"
 
@@ -203,6 +205,109 @@ void build(const gdp_problem *p, const Layout &y, unsigned char *base)
     }
 }
 
+// Solves p by bounds if that is possible: *done.  Initial costs are zeros.
+int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base, gdp_result *r, bool *done)
+{
+    *done = false;
+    gdp_problem form = *p;
+    form.flags = 0;   // (ignored)
+    const int L = p->L, S = p->S, K = p->n_key, T = p->inter_index ? p->n_inter : p->L;
+    if (!bounds::has_form(&form) || !(magnitude < 1e100)) return GDP_OK;
+    int64_t budget[GDP_BOUND_MAX_KEY], least = 0;
+    for (int l = 0; l < L; ++l) {
+        int32_t m = INT32_MAX;
+        for (int s = 0; s < S; ++s) m = std::min(m, p->mem[(size_t)l * S + s]);
+        if (m == 0) return GDP_OK;
+        least += m;
+    }
+    bool any = false;
+    for (int k = 0; k < K; ++k) {
+        const int64_t b = (int64_t)p->V - 1 - p->other_mem[k];
+        budget[k] = b >= least ? b : -1;
+        any = any || b >= least;
+    }
+    if (!any) return GDP_OK;
+    constexpr int NL = GDP_BOUND_MAX_LAM;
+    const size_t LS = (size_t)L * S, SS = (size_t)S * S, labels = (size_t)L * GDP_FRONTIER_LABELS;
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        const size_t o = off;
+        off = align_up(off + bytes, 256);
+        return o;
+    };
+    const size_t off_inst = take(sizeof(GdpBoundInst)), off_pairs = take(sizeof(int2) * (size_t)T), off_mem = take(4 * LS),
+                 off_intra = take(8 * LS), off_inter = take(8 * SS * (size_t)T), off_index = take(4 * (size_t)L),
+                 off_lam = take(8 * NL), off_budget = take(8 * (size_t)K), off_other_time = take(8 * (size_t)K), up_bytes = off,
+                 off_out = take(sizeof(GdpFrontierOut)), off_res = take(4 * (size_t)K * L), back_bytes = off - up_bytes,
+                 off_keep = take(LS), off_inter_f = take(8 * SS * (size_t)T), off_inter_t = take(8 * SS * (size_t)T),
+                 off_P = take(8 * LS * NL), off_Q = take(8 * LS * NL), off_P_mem = take(4 * LS * NL), off_Q_mem = take(4 * LS * NL),
+                 off_end = take(8 * NL), off_window = take(4 * (size_t)K), off_ub = take(8 * (size_t)K),
+                 off_hist = take(sizeof(GdpFrontierLabel) * labels), off_turns = take(8 * labels),
+                 off_hist_mem = take(4 * GDP_FRONTIER_KEPT), off_hist_intra = take(8 * GDP_FRONTIER_KEPT);
+    if (off > (size_t)GDP_STATIC_SCRATCH_BYTES || up_bytes > STAGE_BYTES || back_bytes > STAGE_BYTES) return GDP_OK;
+    memcpy(g_stage + off_mem, p->mem, 4 * LS);
+    memcpy(g_stage + off_intra, p->intra, 8 * LS);
+    memcpy(g_stage + off_inter, p->inter, 8 * SS * (size_t)T);
+    int32_t *index = reinterpret_cast<int32_t *>(g_stage + off_index);
+    for (int l = 0; l < L; ++l) index[l] = p->inter_index ? p->inter_index[l] : l;
+    bounds::multipliers(p, NL, reinterpret_cast<double *>(g_stage + off_lam));
+    memcpy(g_stage + off_budget, budget, 8 * (size_t)K);
+    memcpy(g_stage + off_other_time, p->other_time, 8 * (size_t)K);
+    int2 *pairs = reinterpret_cast<int2 *>(g_stage + off_pairs);
+    for (int t = 0; t < T; ++t) pairs[t] = make_int2(0, t);
+    GdpBoundInst b;
+    memset(&b, 0, sizeof b);
+    b.mem = reinterpret_cast<const int32_t *>(base + off_mem);
+    b.intra = reinterpret_cast<const double *>(base + off_intra);
+    b.inter = reinterpret_cast<const double *>(base + off_inter);
+    b.inter_f = reinterpret_cast<double *>(base + off_inter_f);
+    b.inter_t = reinterpret_cast<double *>(base + off_inter_t);
+    b.index = reinterpret_cast<const int32_t *>(base + off_index);
+    b.lam = reinterpret_cast<const double *>(base + off_lam);
+    b.budget = reinterpret_cast<const int64_t *>(base + off_budget);
+    b.P = reinterpret_cast<double *>(base + off_P);
+    b.Q = reinterpret_cast<double *>(base + off_Q);
+    b.P_mem = reinterpret_cast<uint32_t *>(base + off_P_mem);
+    b.Q_mem = reinterpret_cast<uint32_t *>(base + off_Q_mem);
+    b.end = reinterpret_cast<double *>(base + off_end);
+    b.ub = reinterpret_cast<unsigned long long *>(base + off_ub);
+    b.window = reinterpret_cast<int32_t *>(base + off_window);
+    b.keep = base + off_keep;
+    b.other_time = reinterpret_cast<const double *>(base + off_other_time);
+    b.hist = reinterpret_cast<GdpFrontierLabel *>(base + off_hist);
+    b.hist_mem = reinterpret_cast<int32_t *>(base + off_hist_mem);
+    b.hist_turns = reinterpret_cast<double *>(base + off_turns);
+    b.hist_intra = reinterpret_cast<double *>(base + off_hist_intra);
+    b.out = reinterpret_cast<GdpFrontierOut *>(base + off_out);
+    b.res = reinterpret_cast<int32_t *>(base + off_res);
+    b.magnitude = magnitude;
+    b.L = L; b.V = p->V; b.S = S; b.K = K; b.T = T;
+    b.n_hist = b.n_hist_turns = (int32_t)labels;
+    memcpy(g_stage + off_inst, &b, sizeof b);
+    hipStream_t stream = nullptr;
+    hipError_t e = hipMemcpy(base, g_stage, up_bytes, hipMemcpyHostToDevice);
+    if (e != hipSuccess) return gdp_fail_hip(e, "gdp_solve_static: upload");
+    const GdpBoundInst *inst = reinterpret_cast<const GdpBoundInst *>(base + off_inst);
+    e = bounds::launch(inst, 1, NL, (int)LS, S, K, reinterpret_cast<const int2 *>(base + off_pairs), T, stream);
+    if (e == hipSuccess) e = bounds::launch_labels(inst, 1, K, stream);
+    if (e != hipSuccess) {
+        (void)hipDeviceSynchronize();
+        return gdp_fail_hip(e, "gdp_solve_static: kernel launch");
+    }
+    e = hipMemcpy(g_stage, base + off_out, back_bytes, hipMemcpyDeviceToHost);   // after the kernels, in stream order
+    if (e != hipSuccess) return gdp_fail_hip(e, "gdp_solve_static: download");
+    const GdpFrontierOut *out = reinterpret_cast<const GdpFrontierOut *>(g_stage);
+    if (out->status != 0) return GDP_OK;
+    const int32_t *res = reinterpret_cast<const int32_t *>(g_stage + (off_res - off_out));
+    for (int k = 0; k < K; ++k) {
+        r->total[k] = out->total[k];
+        r->remaining[k] = out->remaining[k];
+        if (out->remaining[k] >= 0) memcpy(r->res + (size_t)k * L, res + (size_t)k * L, sizeof(int32_t) * (size_t)L);
+    }
+    *done = true;
+    return GDP_OK;
+}
+
 }  // namespace
 
 extern "C" int gdp_solve_static(const gdp_problem *p, gdp_result *r)
@@ -210,7 +315,8 @@ extern "C" int gdp_solve_static(const gdp_problem *p, gdp_result *r)
     gdp_clear_error();
     if (!p || !r) return gdp_fail(GDP_E_BADARG, "null problem or result");
     bool f0_live = false;
-    int rc = gdp_validate(p, 0);
+    double magnitude = 0;
+    int rc = gdp_validate(p, 0, &magnitude);
     if (rc == GDP_OK) rc = gdp_validate_f0(p, 0, &f0_live);
     if (rc != GDP_OK) return rc;
     if (p->flags & (GDP_EXPORT_F | GDP_EXPORT_MARK))
@@ -232,6 +338,11 @@ extern "C" int gdp_solve_static(const gdp_problem *p, gdp_result *r)
     unsigned char *base = nullptr;
     const int rs = scratch_of_device(&base);
     if (rs != GDP_OK) return rs;
+    if (!f0_live) {
+        bool done = false;
+        const int rb = solve_by_bounds(p, magnitude, base, r, &done);
+        if (rb != GDP_OK || done) return rb;
+    }
     build(p, y, base);
     hipStream_t stream = nullptr;  // the null stream: nothing is created
     hipError_t e = hipMemcpy(base, g_stage, y.small_bytes, hipMemcpyHostToDevice);
