@@ -2963,6 +2963,7 @@ void BoundSlice::fill(const gdp_problem *const *p, const std::vector<double> &ma
         b.res = reinterpret_cast<int32_t *>(dev + e.off_res);
         b.n_hist = b.n_hist_turns = q->L * GDP_FRONTIER_LABELS;
         b.magnitude = magnitude[(size_t)e.orig];
+        b.limit = 1e30;
         b.L = q->L;
         b.V = q->V;
         b.S = q->S;

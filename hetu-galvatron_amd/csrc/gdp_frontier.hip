@@ -36,6 +36,8 @@ typedef GdpFrontierLabel Label;
 constexpr double KEY_W = 0x1p17, KEY_S = 0x1p11;
 static_assert(KEPT <= 64 && LABELS <= 2048, "6 bits and 11");
 constexpr int KEY_PAD = 72;   // 8 lanes look at 8 keys at a time each
+constexpr int BUCKETS = 64 * WORKERS;
+constexpr int SORTED_FROM = 192;   // labels of a layer; 3 more barriers and 7 reads in a row take as long as looking at that many keys
 
 struct Forward {
     Label label[LABELS];
@@ -44,6 +46,10 @@ struct Forward {
     // and the next.
     __align__(16) double key[2][LABELS + KEY_PAD];
     double cost[LABELS];
+    // where the labels are many: keys by bucket, labels of a bucket and before it, of 64 buckets
+    double sorted[LABELS];
+    int32_t bucket[BUCKETS], bucket_at[BUCKETS];
+    __align__(16) int32_t buckets_of[WORKERS];
 };
 
 
@@ -280,6 +286,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
     const gout hist_turns = GLOBAL(gout, I.hist_turns), hist_intra = GLOBAL(gout, I.hist_intra);
     const glabel hist = GLOBAL(glabel, I.hist);
     const int n_hist = uniform(I.n_hist);
+    const double limit = uniform(I.limit);
 
     if (wave >= WORKERS) {
         // ---- the waves that fetch: wave f what layers f, f + 4, ... need ----
@@ -348,15 +355,23 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
         }
         __syncthreads();
         int at = 0, sum = 0;
+        double executed = 0.0;
         for (int l = 0, slot = 0; l < L; ++l, slot = slot == 2 ? 0 : slot + 1) {   // the same barriers, and the same ways out, as the workers'
             const int n = uniform(sh.layer[l].x);
+            executed += (double)(l ? sum : S) * n;
+            for (int e = t - 64 * WORKERS; e < BUCKETS; e += 64 * FETCHERS) sh.f.bucket[e] = 0;
             for (int e = t - 64 * WORKERS; e < sum; e += 64 * FETCHERS) sh.f.key[(l + 1) & 1][e] = INFINITY;   // of the layer before
             if (l + 1 < L && (l + 1) % FETCHERS == f) place(l + 1);
             if (l % FETCHERS == f && l > 0 && l + FETCHERS < L) fetch(l + FETCHERS);
             __syncthreads();
             sum = uniform(sh.found[slot]);
-            if (sum == 0 || sum > LABELS || at + sum > n_hist) return;
+            if (sum == 0 || sum > LABELS || at + sum > n_hist || executed > limit) return;
             at += sum;
+            if (n > 1 && sum > SORTED_FROM) {
+                __syncthreads();
+                __syncthreads();
+                __syncthreads();
+            }
             if (n > 1) __syncthreads();
         }
     }
@@ -412,13 +427,15 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
                 last = goes_on >> 63 ? lane_of(from, 63) : lane_of(c, 63);
                 return from;
             };
-            // Labels of strategy b, `before_these` of which there are already.
-            auto emit = [&](bool stays, int b, int before_these, double c, int32_t w) {
-                const unsigned long long these = __builtin_amdgcn_ballot_w64(stays);
-                const int count = __popcll(these), number = __builtin_amdgcn_mbcnt_hi((uint32_t)(these >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)these, (uint32_t)before_these));
+            // Labels of strategy b, `before_these` of which there are already: where the next `count` go.
+            auto room = [&](int count) {
                 int to = 0;
                 if (lane == 0) to = draw(sh.found + slot, count);
-                to = uniform(to) + number - before_these;
+                return uniform(to);
+            };
+            auto emit = [&](bool stays, unsigned long long these, int b, int before_these, int to, double c, int32_t w) {
+                const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(these >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)these, 0));
+                to += below;
                 if (n == 1) {   // one strategy: these are in order, and none is read any more where they go
                     const Label label = {c, w, 0};
                     if (stays && at + to < n_hist) {
@@ -426,10 +443,9 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
                         hist[(uint32_t)(at + to)] = words(label);
                     }
                 } else if (stays && to < LABELS) {
-                    sh.f.key[now][to] = __builtin_fma((double)w, KEY_W, (double)(b * (int)KEY_S + number));
+                    sh.f.key[now][to] = __builtin_fma((double)w, KEY_W, (double)(b * (int)KEY_S + before_these + below));
                     sh.f.cost[to] = c;
                 }
-                return count;
             };
             // the labels of strategy b: from those of the layer before in turn, 64 at a time
             if (l && before <= 64) {   // a turn is all there is
@@ -448,7 +464,8 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
                     double last = INFINITY;
                     const double from = step_from(c, ends, last);   // (by all lanes)
                     const bool stays = lane < before && ends && c < from && alive(line, c, w);
-                    emit(stays, b, 0, c, w);
+                    const unsigned long long these = __builtin_amdgcn_ballot_w64(stays);
+                    emit(stays, these, b, 0, room(__popcll(these)), c, w);
                 }
             } else {
                 for (int b = wave; b < n; b += WORKERS) {
@@ -461,37 +478,55 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
                     const int32_t m = __builtin_bit_cast(int2v, costs.y).x;
                     double least = INFINITY, last = INFINITY;   // up to the labels before these: of the sums, of the costs
                     int found = 0;
-                    for (int j0 = 0; j0 < before; j0 += 64) {
-                        const int j = j0 + lane;
-                        double x;
-                        int32_t w = m;
-                        bool ends = true;
-                        if (l) {
-                            const Label old = label_at(sh.f.label + min(j, before - 1));
-                            ends = j >= before - 1 || sh.f.label[min(j + 1, before - 1)].w != old.w;
-                            x = old.c + sh.f.turns[now][old.s * n + b];
-                            w += old.w;
-                        } else {
-                            const gdouble M = inter + (size_t)sh.mat[0] * S * S + sh.kept[kept_at + b];
-                            x = 0.0 + M[(size_t)min(lane, S - 1) * S];
-                            x = min_f64(x, 0.0 + M[(size_t)min(lane + 64, S - 1) * S]);
-                            x = lane_of(prefix_min(x), 63);
+                    // two turns side by side: each is a chain of dependent instructions
+                    for (int j0 = 0; j0 < before; j0 += 128) {
+                        double c[2];
+                        int32_t w[2];
+                        bool ends[2], stays[2];
+                        unsigned long long these[2];
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) {
+                            const int j = j0 + 64 * u + lane;
+                            double x;
+                            w[u] = m;
+                            ends[u] = true;
+                            if (l) {
+                                const Label old = label_at(sh.f.label + min(j, before - 1));
+                                ends[u] = j >= before - 1 || sh.f.label[min(j + 1, before - 1)].w != old.w;
+                                x = old.c + sh.f.turns[now][old.s * n + b];
+                                w[u] += old.w;
+                            } else {
+                                const gdouble M = inter + (size_t)sh.mat[0] * S * S + sh.kept[kept_at + b];
+                                x = 0.0 + M[(size_t)min(lane, S - 1) * S];
+                                x = min_f64(x, 0.0 + M[(size_t)min(lane + 64, S - 1) * S]);
+                                x = lane_of(prefix_min(x), 63);
+                            }
+                            c[u] = prefix_min(j < before ? x : INFINITY);
                         }
-                        const double y = min_f64(prefix_min(j < before ? x : INFINITY), least), c = y + own;
-                        const double from = step_from(c, ends, last);   // (by all lanes)
-                        const bool stays = j < before && ends && c < from && alive(line, c, w);
-                        found += emit(stays, b, found, c, w);
-                        least = lane_of(y, 63);
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) {
+                            c[u] = min_f64(c[u], least);
+                            least = lane_of(c[u], 63);
+                            c[u] += own;
+                            const double from = step_from(c[u], ends[u], last);   // (by all lanes)
+                            stays[u] = j0 + 64 * u + lane < before && ends[u] && c[u] < from && alive(line, c[u], w[u]);
+                            these[u] = __builtin_amdgcn_ballot_w64(stays[u]);
+                        }
+                        const int first = __popcll(these[0]), count = first + __popcll(these[1]), to = room(count);
+                        emit(stays[0], these[0], b, found, to, c[0], w[0]);
+                        emit(stays[1], these[1], b, found + first, to + first, c[1], w[1]);
+                        found += count;
                     }
                 }
             }
             executed += (double)(l ? before : S) * n;
             __syncthreads();
             const int sum = uniform(sh.found[slot]);
-            if (sum == 0 || sum > LABELS || at + sum > n_hist) {
+            if (sum == 0 || sum > LABELS || at + sum > n_hist || executed > limit) {
                 give_up(sum == 0 ? 3 : 4);
                 return;
             }
+            const int32_t first_w = sh.f.label[0].w, last_w = sh.f.label[before - 1].w;   // of the layer before
             before = sum;
             if (t == 0) {
                 sh.labels_at[l + 1] = at + sum;
@@ -501,34 +536,93 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
                 at += sum;
                 continue;
             }
-            // In the order of their memory: a label's place is how many keys are lower.  Up to 8 lanes share them.
-            const int share = sum <= 64 ? 3 : sum <= 128 ? 2 : sum <= 256 ? 1 : 0, lanes = 1 << share;   // (bits)
-            const int part = ((sum + lanes - 1) >> share) + 7 & ~7;
-            for (int e0 = wave << (6 - share); e0 < sum; e0 += WORKERS << (6 - share)) {
-                const int e = e0 + (lane >> share), from = (lane & (lanes - 1)) * part;
-                const double key = sh.f.key[now][min(e, sum - 1)], c = sh.f.cost[min(e, sum - 1)];
-                const double2 *p = reinterpret_cast<const double2 *>(sh.f.key[now] + from);
-                int to[4] = {};
-                for (int i = 0; i < part; i += 8, p += 4) {
-                    const double2 x0 = p[0], x1 = p[1], x2 = p[2], x3 = p[3];
-                    to[0] += x0.x < key;
-                    to[1] += x0.y < key;
-                    to[2] += x1.x < key;
-                    to[3] += x1.y < key;
-                    to[0] += x2.x < key;
-                    to[1] += x2.y < key;
-                    to[2] += x3.x < key;
-                    to[3] += x3.y < key;
+            // In the order of their memory: a label's place is how many keys are lower.
+            auto lay_down = [&](double key, double c, int place) {
+                const long long k = (long long)key;
+                const Label label = {c, (int32_t)(k >> 17), (int32_t)(k >> 11) & 63};
+                put(sh.f.label + place, label);
+                hist[(uint32_t)(at + place)] = words(label);
+            };
+            if (sum > SORTED_FROM) {
+                // Many: into 512 buckets of memory, and among the few of a bucket.  All lie between the lowest and the highest
+                // of the layer before and what the strategies add to them.
+                int32_t most = INT32_MIN, least_m = INT32_MAX;
+                if (lane < n) most = least_m = __builtin_bit_cast(int2v, sh.f.lines[now][lane * LINE + KEYS * WINDOW + 1]).x;
+                least_m = lanes_min(least_m);
+                most = -lanes_min(-max(most, -INT32_MAX));
+                const int32_t low = l ? first_w + least_m : least_m;
+                const float scale = (float)BUCKETS / (float)((l ? last_w + most : most) - low + 1);
+                constexpr int TIMES = (LABELS + 64 * WORKERS - 1) / (64 * WORKERS);
+                double key[TIMES], c[TIMES];
+                int q[TIMES], r[TIMES];
+#pragma unroll
+                for (int i = 0; i < TIMES; ++i) {
+                    const int e = t + i * 64 * WORKERS;
+                    if (e >= sum) continue;
+                    key[i] = sh.f.key[now][e];
+                    c[i] = sh.f.cost[e];
+                    q[i] = min(max((int)((float)((int32_t)((long long)key[i] >> 17) - low) * scale), 0), BUCKETS - 1);
+                    r[i] = atomicAdd(sh.f.bucket + q[i], 1);
                 }
-                int place = to[0] + to[1] + to[2] + to[3];
-                if (share > 0) place += __builtin_amdgcn_mov_dpp(place, 0xb1, 0xf, 0xf, true);    // lane ^ 1
-                if (share > 1) place += __builtin_amdgcn_mov_dpp(place, 0x4e, 0xf, 0xf, true);    // lane ^ 2
-                if (share > 2) place += __builtin_amdgcn_mov_dpp(place, 0x141, 0xf, 0xf, true);   // mirrored within 8
-                if (e < sum && (lane & (lanes - 1)) == 0) {
-                    const long long k = (long long)key;
-                    const Label label = {c, (int32_t)(k >> 17), (int32_t)(k >> 11) & 63};
-                    put(sh.f.label + place, label);
-                    hist[(uint32_t)(at + place)] = words(label);
+                __syncthreads();
+                {
+                    const int own = sh.f.bucket[t];
+                    int x = own;
+#pragma unroll
+                    for (int w = 1; w < 64; w <<= 1) {
+                        const int y = __shfl_up(x, w);
+                        if (lane >= w) x += y;
+                    }
+                    sh.f.bucket_at[t] = x - own;
+                    if (lane == 63) sh.f.buckets_of[wave] = x;
+                }
+                __syncthreads();
+                int of[WORKERS];
+#pragma unroll
+                for (int w = 0; w < WORKERS; ++w) of[w] = sh.f.buckets_of[w];
+#pragma unroll
+                for (int i = 0; i < TIMES; ++i) {
+                    if (t + i * 64 * WORKERS >= sum) continue;
+                    int base = sh.f.bucket_at[q[i]];
+#pragma unroll
+                    for (int w = 0; w < WORKERS - 1; ++w) base += w < q[i] >> 6 ? of[w] : 0;
+                    sh.f.sorted[base + r[i]] = key[i];
+                    r[i] = base;
+                }
+                __syncthreads();
+#pragma unroll
+                for (int i = 0; i < TIMES; ++i) {
+                    if (t + i * 64 * WORKERS >= sum) continue;
+                    const int have = sh.f.bucket[q[i]];
+                    int place = r[i];
+                    for (int k = 0; k < have; ++k) place += sh.f.sorted[r[i] + k] < key[i];
+                    lay_down(key[i], c[i], place);
+                }
+            } else {
+                // Few: up to 8 lanes share the keys.
+                const int share = sum <= 64 ? 3 : sum <= 128 ? 2 : sum <= 256 ? 1 : 0, lanes = 1 << share;   // (bits)
+                const int part = ((sum + lanes - 1) >> share) + 7 & ~7;
+                for (int e0 = wave << (6 - share); e0 < sum; e0 += WORKERS << (6 - share)) {
+                    const int e = e0 + (lane >> share), from = (lane & (lanes - 1)) * part;
+                    const double key = sh.f.key[now][min(e, sum - 1)], c = sh.f.cost[min(e, sum - 1)];
+                    const double2 *p = reinterpret_cast<const double2 *>(sh.f.key[now] + from);
+                    int to[4] = {};
+                    for (int i = 0; i < part; i += 8, p += 4) {
+                        const double2 x0 = p[0], x1 = p[1], x2 = p[2], x3 = p[3];
+                        to[0] += x0.x < key;
+                        to[1] += x0.y < key;
+                        to[2] += x1.x < key;
+                        to[3] += x1.y < key;
+                        to[0] += x2.x < key;
+                        to[1] += x2.y < key;
+                        to[2] += x3.x < key;
+                        to[3] += x3.y < key;
+                    }
+                    int place = to[0] + to[1] + to[2] + to[3];
+                    if (share > 0) place += __builtin_amdgcn_mov_dpp(place, 0xb1, 0xf, 0xf, true);    // lane ^ 1
+                    if (share > 1) place += __builtin_amdgcn_mov_dpp(place, 0x4e, 0xf, 0xf, true);    // lane ^ 2
+                    if (share > 2) place += __builtin_amdgcn_mov_dpp(place, 0x141, 0xf, 0xf, true);   // mirrored within 8
+                    if (e < sum && (lane & (lanes - 1)) == 0) lay_down(key, c, place);
                 }
             }
             at += sum;
@@ -633,7 +727,10 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
 
 hipError_t bounds::launch_labels(const GdpBoundInst *inst, int n, int max_K, hipStream_t stream)
 {
-    if (max_K <= 4) gdp_frontier_kernel<4><<<dim3((unsigned)n), THREADS, sizeof(Shared), stream>>>(inst);
-    else gdp_frontier_kernel<8><<<dim3((unsigned)n), THREADS, sizeof(Shared), stream>>>(inst);
+    const dim3 grid((unsigned)n);
+    if (max_K <= 2) gdp_frontier_kernel<2><<<grid, THREADS, sizeof(Shared), stream>>>(inst);
+    else if (max_K <= 4) gdp_frontier_kernel<4><<<grid, THREADS, sizeof(Shared), stream>>>(inst);
+    else if (max_K == 5) gdp_frontier_kernel<5><<<grid, THREADS, sizeof(Shared), stream>>>(inst);
+    else gdp_frontier_kernel<8><<<grid, THREADS, sizeof(Shared), stream>>>(inst);
     return hipGetLastError();
 }

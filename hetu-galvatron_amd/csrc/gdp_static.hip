@@ -281,6 +281,7 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     b.out = reinterpret_cast<GdpFrontierOut *>(base + off_out);
     b.res = reinterpret_cast<int32_t *>(base + off_res);
     b.magnitude = magnitude;
+    b.limit = 1e30;
     b.L = L; b.V = p->V; b.S = S; b.K = K; b.T = T;
     b.n_hist = b.n_hist_turns = (int32_t)labels;
     memcpy(g_stage + off_inst, &b, sizeof b);
