@@ -278,6 +278,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
     __syncthreads();   // the marks themselves are not read any more
     if (t == 0) sh.labels_at[0] = 0;
     for (int e = t; e < 2 * (LABELS + KEY_PAD); e += THREADS) sh.f.key[0][e] = INFINITY;   // both
+    for (int e = t; e < BUCKETS; e += THREADS) sh.f.bucket[e] = 0;
     __syncthreads();
 
     const gdouble inter = GLOBAL(gdouble, I.inter), intra = GLOBAL(gdouble, I.intra), Q = GLOBAL(gdouble, I.Q);
@@ -314,7 +315,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
                 const int e = min(lane + i * 64, n * LINE - 1), b = quotient(e, r), x = e - b * LINE, s = l * S + sh.kept[at + b];
                 const int k = x / WINDOW, j = x % WINDOW;
                 if (x < KEYS * WINDOW)
-                    a.lines[i] = Q[(uint32_t)((sh.window[k] + j) * LS + s)] - sh.shift[k][j];
+                    a.lines[i] = Q[(uint32_t)((sh.window[k] + j) * LS + s)];   // (nothing here waits for what it loads)
                 else if (x == KEYS * WINDOW)
                     a.lines[i] = intra[(uint32_t)s];
                 else
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
                 if (i * 64 >= n * LINE) break;
                 const int e = lane + i * 64, b = quotient(e, r), x = e - b * LINE;
                 if (e < n * LINE) {
-                    sh.f.lines[to][e] = a.lines[i];
+                    sh.f.lines[to][e] = x < KEYS * WINDOW ? a.lines[i] - sh.shift[x / WINDOW][x % WINDOW] : a.lines[i];
                     if (x == KEYS * WINDOW) hist_intra[(uint32_t)(at + b)] = a.lines[i];
                     if (x > KEYS * WINDOW) hist_mem[(uint32_t)(at + b)] = __builtin_bit_cast(int2v, a.lines[i]).x;
                 }
@@ -359,14 +360,15 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
         for (int l = 0, slot = 0; l < L; ++l, slot = slot == 2 ? 0 : slot + 1) {   // the same barriers, and the same ways out, as the workers'
             const int n = uniform(sh.layer[l].x);
             executed += (double)(l ? sum : S) * n;
-            for (int e = t - 64 * WORKERS; e < BUCKETS; e += 64 * FETCHERS) sh.f.bucket[e] = 0;
+            if (sum > SORTED_FROM)
+                for (int e = t - 64 * WORKERS; e < BUCKETS; e += 64 * FETCHERS) sh.f.bucket[e] = 0;
             for (int e = t - 64 * WORKERS; e < sum; e += 64 * FETCHERS) sh.f.key[(l + 1) & 1][e] = INFINITY;   // of the layer before
             if (l + 1 < L && (l + 1) % FETCHERS == f) place(l + 1);
-            if (l % FETCHERS == f && l > 0 && l + FETCHERS < L) fetch(l + FETCHERS);
             __syncthreads();
             sum = uniform(sh.found[slot]);
             if (sum == 0 || sum > LABELS || at + sum > n_hist || executed > limit) return;
             at += sum;
+            if (l % FETCHERS == f && l > 0 && l + FETCHERS < L) fetch(l + FETCHERS);
             if (n > 1 && sum > SORTED_FROM) {
                 __syncthreads();
                 __syncthreads();
@@ -407,7 +409,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
                     const double b0 = __builtin_fma(lam[k][0], dw, line[2 * k].x), b1 = __builtin_fma(lam[k][1], dw, line[2 * k].y),
                                  b2 = __builtin_fma(lam[k][2], dw, line[2 * k + 1].x), b3 = __builtin_fma(lam[k][3], dw, line[2 * k + 1].y);
                     const double bound = max_f64(max_f64(b0, b1), max_f64(b2, b3));
-                    any |= w <= budget[k] && c + bound <= ub[k];
+                    any |= (w <= budget[k]) & (c + bound <= ub[k]);
                 }
                 return any;
             };
@@ -463,7 +465,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
                     const bool ends = lane >= before - 1 || next_w != old.w;
                     double last = INFINITY;
                     const double from = step_from(c, ends, last);   // (by all lanes)
-                    const bool stays = lane < before && ends && c < from && alive(line, c, w);
+                    const bool stays = (lane < before) & ends & (c < from) & alive(line, c, w);
                     const unsigned long long these = __builtin_amdgcn_ballot_w64(stays);
                     emit(stays, these, b, 0, room(__popcll(these)), c, w);
                 }
@@ -509,7 +511,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
                             least = lane_of(c[u], 63);
                             c[u] += own;
                             const double from = step_from(c[u], ends[u], last);   // (by all lanes)
-                            stays[u] = j0 + 64 * u + lane < before && ends[u] && c[u] < from && alive(line, c[u], w[u]);
+                            stays[u] = (j0 + 64 * u + lane < before) & ends[u] & (c[u] < from) & alive(line, c[u], w[u]);
                             these[u] = __builtin_amdgcn_ballot_w64(stays[u]);
                         }
                         const int first = __popcll(these[0]), count = first + __popcll(these[1]), to = room(count);
