@@ -230,5 +230,7 @@ hipError_t gdp_launch_epilogue(bool marks, const GdpDevInst *insts, const GdpDev
                                int32_t *res, hipStream_t stream);
 // Debug exports in the reference's layouts.
 hipError_t gdp_launch_export_f(const GdpDevInst *inst, double *f_out, int V, int S, hipStream_t stream);
-hipError_t gdp_launch_export_mark(const GdpDevInst *inst, int layer, int32_t *mark_out, int V, int S,
-                                  hipStream_t stream);
+// layers layer0 .. layer0+layers-1 of the argmin table (layers <= 65535): bytes with GDP_EXPORT_NONE for -1 where S <= 255, else
+// int32.
+constexpr int GDP_EXPORT_NONE = 255;
+hipError_t gdp_launch_export_mark(const GdpDevInst *inst, int layer0, int layers, void *mark_out, int V, int S, hipStream_t stream);

@@ -18,6 +18,8 @@
 // hoisted form.)
 #include "gdp_kernels.h"
 
+#include <algorithm>
+
 #include <math.h>
 
 namespace {
@@ -1455,19 +1457,22 @@ __global__ __launch_bounds__(256) void gdp_export_f_kernel(const GdpDevInst *__r
     }
 }
 
-// One layer of the argmin table in the reference's [V][S] int32 layout (-1 where v < mem).
-__global__ __launch_bounds__(256) void gdp_export_mark_kernel(const GdpDevInst *__restrict__ I, int layer,
-                                                              int32_t *__restrict__ mark)
+// Layers of the argmin table in the reference's [V][S] order, a byte per entry as it is stored, GDP_EXPORT_NONE where
+// v < mem: a quarter of what crosses to the host, which widens it while it writes the caller's array.  T: int32 where
+// S needs all 256 values.  grid (V * S / 1024, layers).
+template <typename T>
+__global__ __launch_bounds__(256) void gdp_export_mark_kernel(const GdpDevInst *__restrict__ I, int layer0, T *__restrict__ mark)
 {
-    const int V = I->V, S = I->S;
+    const int V = I->V, S = I->S, layer = layer0 + (int)blockIdx.y;
     const int32_t *mem = I->mem + (int64_t)layer * S;
     const uint8_t *M = I->M + (int64_t)layer * S * I->ldm;
     const int64_t n = (int64_t)V * S;
+    T *out = mark + (int64_t)blockIdx.y * n;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         const int64_t v = i / S;
         const int s = (int)(i - v * S);
         const int64_t u = v - mem[s];
-        mark[i] = (u < 0) ? -1 : (int32_t)M[(int64_t)s * I->ldm + u];
+        out[i] = (u < 0) ? (T)(sizeof(T) == 1 ? GDP_EXPORT_NONE : -1) : (T)M[(int64_t)s * I->ldm + u];
     }
 }
 
@@ -1698,12 +1703,13 @@ hipError_t gdp_launch_export_f(const GdpDevInst *inst, double *f_out, int V, int
     return hipGetLastError();
 }
 
-hipError_t gdp_launch_export_mark(const GdpDevInst *inst, int layer, int32_t *mark_out, int V, int S,
-                                  hipStream_t stream)
+hipError_t gdp_launch_export_mark(const GdpDevInst *inst, int layer0, int layers, void *mark_out, int V, int S, hipStream_t stream)
 {
     const int64_t n = (int64_t)V * S;
-    unsigned nb = (unsigned)((n + 1023) / 1024);
-    if (nb > 65535u * 16u) nb = 65535u * 16u;
-    hipLaunchKernelGGL(gdp_export_mark_kernel, dim3(nb), dim3(256), 0, stream, inst, layer, mark_out);
+    const dim3 grid((unsigned)std::min<int64_t>((n + 1023) / 1024, 65535 * 16), (unsigned)layers);
+    if (S <= GDP_EXPORT_NONE)
+        hipLaunchKernelGGL(gdp_export_mark_kernel<uint8_t>, grid, dim3(256), 0, stream, inst, layer0, (uint8_t *)mark_out);
+    else
+        hipLaunchKernelGGL(gdp_export_mark_kernel<int32_t>, grid, dim3(256), 0, stream, inst, layer0, (int32_t *)mark_out);
     return hipGetLastError();
 }

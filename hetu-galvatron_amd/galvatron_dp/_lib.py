@@ -173,7 +173,7 @@ class Problem:
 
     def __init__(self, mem, intra, inter, V: int, other_mem: Sequence[int], other_time: Sequence[float], *,
                  inter_index=None, export_f: bool = False, export_mark: bool = False, launch: str | None = None,
-                 compute_all: bool = False, keep_marks: bool = False, f0=None):
+                 compute_all: bool = False, keep_marks: bool = False, f0=None, f_out=None, mark_out=None):
         self.mem = np.ascontiguousarray(mem, dtype=np.int32)
         if self.mem.ndim != 2:
             raise ValueError("mem must be [L,S]")
@@ -219,8 +219,12 @@ class Problem:
         self.remaining.fill(-1)
         self.res = np.empty((self.n_key, self.L), dtype=np.int32)
         self.res.fill(-1)
-        self.f_out = np.empty((self.V, self.S), dtype=np.float64) if export_f else None
-        self.mark_out = np.empty((self.L, self.V, self.S), dtype=np.int32) if export_mark else None
+        # (f_out, mark_out: C-contiguous arrays of these sizes to be written instead of new ones)
+        self.f_out = self.mark_out = None
+        if export_f:
+            self.f_out = np.empty((self.V, self.S), dtype=np.float64) if f_out is None else f_out
+        if export_mark:
+            self.mark_out = np.empty((self.L, self.V, self.S), dtype=np.int32) if mark_out is None else mark_out
         addr = _addr
         self._c_problem = gdp_problem(
             self.L, self.V, self.S, addr(self.mem), addr(self.intra), addr(self.inter), addr(self.inter_index),

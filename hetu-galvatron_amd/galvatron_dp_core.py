@@ -63,20 +63,33 @@ class SharedInter:
         return self.dense()[item]
 
 
+def _own(a, dtype, shape):
+    """``a`` if the library can write it directly: a plain array of that type and shape in C order."""
+    fits = type(a) is np.ndarray and a.dtype == dtype and a.shape == shape and a.flags.carray
+    return a if fits else None
+
+
 def _problem(layer_num, max_mem, strategy_num, v_data, _f, inter_cost, intra_cost, other_mem_cost, other_time_cost,
-             export):
+             export, _mark=None):
+    """``_mark``: given where the exported tables may be written into the caller's arrays without a copy in between."""
     L, V, S = int(layer_num), int(max_mem), int(strategy_num)
     mem = np.ascontiguousarray(v_data, dtype=np.int32).reshape(L, S)
     intra = np.ascontiguousarray(intra_cost, dtype=np.float64).reshape(L, S)
+    f_out = mark_out = None
+    if export and _mark is not None:
+        f_out, mark_out = _own(_f, np.float64, (V, S)), _own(_mark, np.int32, (L, V, S))
+        if f_out is not None and mark_out is not None and np.may_share_memory(f_out, mark_out):
+            f_out = mark_out = None
     keys = sorted(int(k) for k in other_mem_cost)          # std::map iterates in ascending key order
     om = [int(other_mem_cost[k]) for k in keys]
     ot = [float(other_time_cost[k]) if k in other_time_cost else 0.0 for k in keys]  # map::operator[] default
     if isinstance(inter_cost, SharedInter):
         return keys, _lib.Problem(mem, intra, inter_cost.tables.reshape(-1, S, S), V, om, ot,
                                   inter_index=inter_cost.index.reshape(L), export_f=export, export_mark=export,
-                                  f0=_f)
+                                  f0=_f, f_out=f_out, mark_out=mark_out)
     inter = np.ascontiguousarray(inter_cost, dtype=np.float64).reshape(L, S, S)
-    return keys, _lib.Problem(mem, intra, inter, V, om, ot, export_f=export, export_mark=export, f0=_f)
+    return keys, _lib.Problem(mem, intra, inter, V, om, ot, export_f=export, export_mark=export, f0=_f, f_out=f_out,
+                              mark_out=mark_out)
 
 
 def _finish(keys, prob, _mark, _f, res_list, export):
@@ -86,8 +99,9 @@ def _finish(keys, prob, _mark, _f, res_list, export):
         remaining_mem[k] = int(prob.remaining[i])
         if prob.remaining[i] != -1:
             res_list[k][...] = prob.res[i]                    # feasible keys only (csrc/dp_core.cpp:103-113)
-    if export:
+    if export and prob.f_out is not _f:
         np.asarray(_f)[...] = prob.f_out
+    if export and prob.mark_out is not _mark:
         np.asarray(_mark)[...] = prob.mark_out
     return total_cost, remaining_mem
 
@@ -99,7 +113,7 @@ def dynamic_programming_core(layer_num, max_mem, strategy_num, v_data, _mark, _f
     pre-filled with -1 by the caller) is written in place for feasible keys."""
     export = export_enabled()
     keys, prob = _problem(layer_num, max_mem, strategy_num, v_data, _f, inter_cost, intra_cost, other_mem_cost,
-                          other_time_cost, export)
+                          other_time_cost, export, _mark)
     _lib.solve_batch([prob])
     return _finish(keys, prob, _mark, _f, res_list, export)
 

@@ -1,0 +1,30 @@
+"""The exported tables through the plugin signature: pieces and widths of the copy, and the caller's arrays that are
+written directly or through a copy."""
+import numpy as np
+import pytest
+
+import galvatron_dp_core as shim
+from galvatron_dp import workloads as W
+from oracle import dp_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+# S = 255: a byte per entry of the argmin table, 256: four; 1 MB pieces: less than one, one and a bit, several
+@pytest.mark.parametrize("L,S,V", [(2, 1, 40), (3, 255, 60), (3, 256, 60), (3, 22, 16000), (9, 7, 40000)])
+@pytest.mark.parametrize("direct", [True, False])
+def test_exported_tables(L, S, V, direct):
+    inst = W.random_instance(np.random.Generator(np.random.PCG64([L, S, V])), L, S, V, mem_hi=max(2, V // L), inf_frac=0.1, n_keys=2)
+    want = O.solve(inst.mem, inst.intra, inst.inter, V, inst.other_mem, inst.other_time, keep=True)
+    f, mark = np.zeros((V, S)), np.full((L, V, S), -1, dtype=np.int32)
+    if not direct:                                   # other strides and another type: written through a copy
+        f, mark = np.zeros((S, V)).T, mark.astype(np.int64)
+    res = {k: np.full(L, -1, dtype=np.int32) for k in inst.other_mem}
+    shim.set_export(True)
+    try:
+        total, left = shim.dynamic_programming_core(L, V, S, inst.mem, mark, f, inst.inter, inst.intra, inst.other_mem, inst.other_time, res)
+    finally:
+        shim.set_export(False)
+    assert np.array_equal(mark, want[4]) and np.ascontiguousarray(f).tobytes() == want[3].tobytes()
+    for k in want[0]:
+        assert np.float64(total[k]).tobytes() == np.float64(want[0][k]).tobytes() and left[k] == want[2][k]
