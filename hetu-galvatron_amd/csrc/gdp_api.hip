@@ -2884,6 +2884,7 @@ struct BoundLease {
 struct BoundSlice {
     BoundEntry *es = nullptr;
     int m = 0, n_lam = 0, max_LS = 0, max_S = 0, max_K = 0;
+    int64_t layers = 0, changes = 0;   // ... and how often a layer has another matrix than the one before
     std::vector<int2> pairs;
     // [0, up_bytes): what is uploaded; the results after it; what stays; the rest stays on the device
     size_t off_inst = 0, off_pairs = 0, up_bytes = 0, back_bytes = 0, keep_begin = 0, keep_bytes = 0, bytes = 0;
@@ -2932,6 +2933,8 @@ void BoundSlice::lay_out(const gdp_problem *const *p, BoundEntry *entries, int c
             e.off_inter = place(8 * (size_t)e.h.n_inter * q->S * q->S);
             for (int t = 0; t < e.h.n_inter; ++t) pairs.push_back(make_int2(j, t));
         }
+        layers += q->L;
+        for (int l = 1; l < q->L; ++l) changes += e.h.matrix(q, l) != e.h.matrix(q, l - 1);
         max_LS = std::max(max_LS, (int)LS);
         max_S = std::max(max_S, q->S);
         max_K = std::max(max_K, q->n_key);
@@ -3026,7 +3029,7 @@ void BoundSlice::fill(const gdp_problem *const *p, const std::vector<double> &ma
 hipError_t BoundSlice::enqueue(char *dev, hipStream_t stream) const
 {
     const GdpBoundInst *inst = reinterpret_cast<const GdpBoundInst *>(dev + off_inst);
-    const hipError_t e = bounds::launch(inst, m, n_lam, max_LS, max_S, max_K, reinterpret_cast<const int2 *>(dev + off_pairs),
+    const hipError_t e = bounds::launch(inst, m, n_lam, max_LS, max_S, max_K, changes * 4 <= layers, reinterpret_cast<const int2 *>(dev + off_pairs),
                                            (int)pairs.size(), stream);
     return e == hipSuccess ? bounds::launch_labels(inst, m, max_K, stream) : e;
 }

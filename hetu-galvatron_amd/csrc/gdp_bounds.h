@@ -67,10 +67,10 @@ __attribute__((visibility("hidden"))) bool has_form(const gdp_problem *q);
 // The multipliers of an instance: 0 and a geometric series around (range of times) / (range of memory costs).
 __attribute__((visibility("hidden"))) void multipliers(const gdp_problem *q, int n_lam, double *lam);
 // Copies the matrices, runs the passes of all multipliers, finds the upper bounds and marks what stays.
-// pairs: {instance, matrix} of every matrix that is to be copied.
+// pairs: {instance, matrix} of every matrix that is to be copied.  held: most layers have the matrix of the one before.
 __attribute__((visibility("hidden")))
-hipError_t launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K, const int2 *pairs, int n_pairs,
-                  hipStream_t stream);
+hipError_t launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K, bool held, const int2 *pairs,
+                  int n_pairs, hipStream_t stream);
 // The DP over what stays (gdp_frontier.hip), after it.
 __attribute__((visibility("hidden"))) hipError_t launch_labels(const GdpBoundInst *inst, int n, int max_K, hipStream_t stream);
 }  // namespace bounds

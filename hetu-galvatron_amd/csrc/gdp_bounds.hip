@@ -116,7 +116,11 @@ __device__ __forceinline__ double load_double(__amdgpu_buffer_rsrc_t b, int lane
 // What it reads is bound by how many lines a load touches: 4 lanes of a target side by side, a line for every 4 lanes, took
 // 151 us where 16 targets side by side take 69.  Against a step of two barriers, 1024 threads and a select per candidate for
 // the argmin: L = 80, S = 64 131 -> 69 us, L = 48, S = 88 102 -> 77, 256 instances of S = 44 635 -> 400.
-template <int E, int AHEAD>
+// HELD: for instances whose layers mostly have the matrix of the layer before.  It stays in registers, and is waited for
+// where it changes: what a compute unit reads, 16 bytes a clock, is what bounds the pass otherwise.
+// L = 48, S = 88 77 -> 39 us, 256 instances of S = 44 400 -> 140; where every layer has a matrix of its own (L = 80, S = 64,
+// 70 us) there is nothing to hold.
+template <int E, int AHEAD, bool HELD>
 __global__ __launch_bounds__(64 * GDP_BOUND_MAX_S / TARGETS) void gdp_bound_pass_kernel(const GdpBoundInst *inst)
 {
     static_assert(E % 2 == 0 && AHEAD % 2 == 0 && E * PARTS <= GDP_BOUND_MAX_S, "");
@@ -145,9 +149,11 @@ __global__ __launch_bounds__(64 * GDP_BOUND_MAX_S / TARGETS) void gdp_bound_pass
 
     // What a step needs from memory: its part of the matrix and the costs of the layer whose strategies it reaches.
     struct Inputs {
-        double m[E], intra;
+        double m[HELD ? 1 : E], intra;
         int32_t mem;
     };
+    double m[HELD ? E : 1];
+    int held = -1;
     // step i: the matrix of layer first + i * step, into the strategies of layer to + i * step
     const int first = back ? L - 1 : 0, to = back ? L - 2 : 0, step = back ? -1 : 1, steps = back ? L - 1 : L;
     auto fetch_costs = [&](int l, Inputs &in) {
@@ -155,10 +161,12 @@ __global__ __launch_bounds__(64 * GDP_BOUND_MAX_S / TARGETS) void gdp_bound_pass
         in.intra = load_double(intra, s * 8, l * S * 8);
     };
     auto matrix_of = [&](int i) { return mat[first + min(i, steps - 1) * step]; };
-    auto fetch = [&](int i, int matrix, Inputs &in) {
-        const int M = __builtin_amdgcn_readfirstlane(matrix) * S * S * 8;
+    auto fetch_matrix = [&](int matrix, double *into) {
 #pragma unroll
-        for (int j = 0; j < E; ++j) in.m[j] = load_double(tables, at[j], M);
+        for (int j = 0; j < E; ++j) into[j] = load_double(tables, at[j], matrix * S * S * 8);
+    };
+    auto fetch = [&](int i, int matrix, Inputs &in) {
+        if constexpr (!HELD) fetch_matrix(__builtin_amdgcn_readfirstlane(matrix), in.m);
         fetch_costs(to + i * step, in);
     };
     auto cost = [&](const Inputs &in) {
@@ -192,18 +200,25 @@ __global__ __launch_bounds__(64 * GDP_BOUND_MAX_S / TARGETS) void gdp_bound_pass
     } else if (mine) {   // (what the first step writes of layer 0 is overwritten by the second)
         X[0][place] = 0.0;
     }
-    int next_matrix = matrix_of(AHEAD);
+    constexpr int LOOK = HELD ? 0 : AHEAD;   // steps from one that looks a matrix up to the one that uses it
+    int next_matrix = matrix_of(LOOK);
     int high = ~INDEX;
     asm volatile("" : "+v"(high));   // in a register
     const int part = p * E;
     auto pass = [&](int i, Inputs &in) {
         write(i);
+        if constexpr (HELD) {
+            const int matrix = __builtin_amdgcn_readfirstlane(next_matrix);
+            if (matrix != held) fetch_matrix(matrix, m);
+            held = matrix;
+        }
+        const double *const M = HELD ? m : in.m;
         __syncthreads();   // the other half of X and `need` is still being read until the next one
         const double *from = X[i & 1] + p * STRIDE;
         double best[2];
 #pragma unroll
         for (int j = 0; j < E; j += 2) {
-            const double a = with_index(from[j] + in.m[j], j, high), b = with_index(from[j + 1] + in.m[j + 1], j + 1, high);
+            const double a = with_index(from[j] + M[j], j, high), b = with_index(from[j + 1] + M[j + 1], j + 1, high);
             best[0] = j ? min_f64(best[0], a) : a;
             best[1] = j ? min_f64(best[1], b) : b;
         }
@@ -211,7 +226,7 @@ __global__ __launch_bounds__(64 * GDP_BOUND_MAX_S / TARGETS) void gdp_bound_pass
         int32_t by = min(in.mem, GDP_BOUND_MEM);
         asm volatile("" : "+v"(by));   // here, and not as a copy at the top of the loop that waits for every load
         fetch(min(i + AHEAD, steps - 1), next_matrix, in);   // the last ones once more: no branch
-        next_matrix = matrix_of(i + AHEAD + 1);
+        next_matrix = matrix_of(i + LOOK + 1);
         int2v w = __builtin_bit_cast(int2v, min_f64(best[0], best[1]));
         w.x += part;
         double x = __builtin_bit_cast(double, w);
@@ -402,8 +417,8 @@ void bounds::multipliers(const gdp_problem *q, int n_lam, double *lam)
     for (int i = 1; i < n_lam; ++i) lam[i] = base * exp2(-6.0 + 12.0 * (i - 1) / (n_lam - 2));
 }
 
-hipError_t bounds::launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K, const int2 *pairs, int n_pairs,
-                          hipStream_t stream)
+hipError_t bounds::launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K, bool held, const int2 *pairs,
+                          int n_pairs, hipStream_t stream)
 {
     gdp_bound_transpose_kernel<<<dim3((unsigned)n_pairs, (unsigned)((max_S + 15) / 16)), 256, 0, stream>>>(inst, pairs);
     hipError_t e = hipGetLastError();
@@ -411,7 +426,8 @@ hipError_t bounds::launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS
     const dim3 grid(2u * (unsigned)n_lam, (unsigned)n);
     const unsigned threads = 64u * (unsigned)((max_S + TARGETS - 1) / TARGETS);
 #define GDP_PASS(E, AHEAD) \
-    if (max_S <= PARTS * E) gdp_bound_pass_kernel<E, AHEAD><<<grid, threads, 0, stream>>>(inst)
+    if (max_S <= PARTS * E && held) gdp_bound_pass_kernel<E, 4, true><<<grid, threads, 0, stream>>>(inst); \
+    else if (max_S <= PARTS * E) gdp_bound_pass_kernel<E, AHEAD, false><<<grid, threads, 0, stream>>>(inst)
     GDP_PASS(4, 4);
     else GDP_PASS(6, 4);
     else GDP_PASS(8, 4);

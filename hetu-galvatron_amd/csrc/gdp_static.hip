@@ -249,7 +249,11 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     memcpy(g_stage + off_intra, p->intra, 8 * LS);
     memcpy(g_stage + off_inter, p->inter, 8 * SS * (size_t)T);
     int32_t *index = reinterpret_cast<int32_t *>(g_stage + off_index);
-    for (int l = 0; l < L; ++l) index[l] = p->inter_index ? p->inter_index[l] : l;
+    int changes = 0;
+    for (int l = 0; l < L; ++l) {
+        index[l] = p->inter_index ? p->inter_index[l] : l;
+        changes += l > 0 && index[l] != index[l - 1];
+    }
     bounds::multipliers(p, NL, reinterpret_cast<double *>(g_stage + off_lam));
     memcpy(g_stage + off_budget, budget, 8 * (size_t)K);
     memcpy(g_stage + off_other_time, p->other_time, 8 * (size_t)K);
@@ -289,7 +293,7 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     hipError_t e = hipMemcpy(base, g_stage, up_bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) return gdp_fail_hip(e, "gdp_solve_static: upload");
     const GdpBoundInst *inst = reinterpret_cast<const GdpBoundInst *>(base + off_inst);
-    e = bounds::launch(inst, 1, NL, (int)LS, S, K, reinterpret_cast<const int2 *>(base + off_pairs), T, stream);
+    e = bounds::launch(inst, 1, NL, (int)LS, S, K, changes * 4 <= L, reinterpret_cast<const int2 *>(base + off_pairs), T, stream);
     if (e == hipSuccess) e = bounds::launch_labels(inst, 1, K, stream);
     if (e != hipSuccess) {
         (void)hipDeviceSynchronize();
