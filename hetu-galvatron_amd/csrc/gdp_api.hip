@@ -2884,6 +2884,7 @@ struct BoundLease {
 struct BoundSlice {
     BoundEntry *es = nullptr;
     int m = 0, n_lam = 0, max_LS = 0, max_S = 0, max_K = 0;
+    double limit_ns = 0;               // of the DP over what stays
     int64_t layers = 0, changes = 0;   // ... and how often a layer has another matrix than the one before
     std::vector<int2> pairs;
     // [0, up_bytes): what is uploaded; the results after it; what stays; the rest stays on the device
@@ -2904,6 +2905,8 @@ void BoundSlice::lay_out(const gdp_problem *const *p, BoundEntry *entries, int c
     es = entries;
     m = count;
     n_lam = multipliers;
+    double relaxations = 0;
+    int max_L = 0;
     size_t at = 0;
     auto place = [&](size_t bytes) { const size_t o = at; at = align_up(at + bytes, 256); return o; };
     for (int i = 0; i < m; ++i) {   // the stages of one fit and the tasks of one sweep share their matrices
@@ -2934,11 +2937,16 @@ void BoundSlice::lay_out(const gdp_problem *const *p, BoundEntry *entries, int c
             for (int t = 0; t < e.h.n_inter; ++t) pairs.push_back(make_int2(j, t));
         }
         layers += q->L;
+        relaxations += (double)q->L * q->V * (double)q->S * q->S;
+        max_L = std::max(max_L, q->L);
         for (int l = 1; l < q->L; ++l) changes += e.h.matrix(q, l) != e.h.matrix(q, l - 1);
         max_LS = std::max(max_LS, (int)LS);
         max_S = std::max(max_S, q->S);
         max_K = std::max(max_K, q->n_key);
     }
+    // what the instances take as dense ones, smaller or whole: 10^13 relaxations a second, a layer's latency, and the second
+    // round trip
+    limit_ns = relaxations / 1e4 + max_L * 5e3 + 100e3;
     off_pairs = place(sizeof(int2) * pairs.size());
     up_bytes = at;
     for (int j = 0; j < m; ++j) {
@@ -3015,7 +3023,7 @@ void BoundSlice::fill(const gdp_problem *const *p, const std::vector<double> &ma
         b.res = reinterpret_cast<int32_t *>(dev + e.off_res);
         b.n_hist = b.n_hist_turns = q->L * GDP_FRONTIER_LABELS;
         b.magnitude = magnitude[(size_t)e.orig];
-        b.limit = 1e30;
+        b.limit = limit_ns;
         b.L = q->L;
         b.V = q->V;
         b.S = q->S;

@@ -56,7 +56,7 @@ struct GdpBoundInst {
     GdpFrontierOut *out;
     int32_t *res;            // [K][L]
     double magnitude;        // sum over the layers of the largest finite |intra| and |inter|
-    double limit;            // candidates that the DP may look at
+    double limit;            // ns that the DP over what stays may take, by its own account
     int32_t L, V, S, K, T, n_hist, n_hist_turns;
 };
 

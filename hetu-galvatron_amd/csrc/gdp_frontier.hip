@@ -288,6 +288,21 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
     const glabel hist = GLOBAL(glabel, I.hist);
     const int n_hist = uniform(I.n_hist);
     const double limit = uniform(I.limit);
+    // What a layer takes, in ns: its barriers, the order of many labels, and a wave's turns of 128 labels for every 8th strategy.
+    // An instance that would take longer than the dense recurrence is left to that one, and early: of identical layers that
+    // trade memory for time the labels of a layer grow towards L / 2 about as they do at the start, and are half of what that
+    // comes to in the mean.  (24 inputs of L = 27, S = 37: 17 come through, in 70 to 430 us by this account, the others are told
+    // at layer 2 or 3, 20 us, but for two that grow late.)
+    auto layer_ns = [](int n, int before) {
+        return (before > SORTED_FROM ? 3000 : 900) + ((n + WORKERS - 1) / WORKERS) * ((before + 127) / 128) * (600 + 200 * KEYS);
+    };
+    auto hopeless = [&](int ns, int l, int n, int labels) {
+        if ((double)ns * (double)L > limit * (double)(l + 1)) return true;
+        if (l < max(2, L / 16) || l >= L / 2) return false;
+        const int half = (l - 1) / 2, grown = labels - uniform(sh.labels_at[half + 1] - sh.labels_at[half]);
+        const int top = labels + max(grown, 0) * (L / 2 - l) / (l - half);
+        return top > 2 * LABELS || (double)ns + (double)(L - l) * layer_ns(n, top / 2) > 0.9 * limit;
+    };
 
     if (wave >= WORKERS) {
         // ---- the waves that fetch: wave f what layers f, f + 4, ... need ----
@@ -356,17 +371,17 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
         }
         __syncthreads();
         int at = 0, sum = 0;
-        double executed = 0.0;
+        int ns = 0;
         for (int l = 0, slot = 0; l < L; ++l, slot = slot == 2 ? 0 : slot + 1) {   // the same barriers, and the same ways out, as the workers'
             const int n = uniform(sh.layer[l].x);
-            executed += (double)(l ? sum : S) * n;
+            ns += layer_ns(n, l ? sum : 1);
             if (sum > SORTED_FROM)
                 for (int e = t - 64 * WORKERS; e < BUCKETS; e += 64 * FETCHERS) sh.f.bucket[e] = 0;
             for (int e = t - 64 * WORKERS; e < sum; e += 64 * FETCHERS) sh.f.key[(l + 1) & 1][e] = INFINITY;   // of the layer before
             if (l + 1 < L && (l + 1) % FETCHERS == f) place(l + 1);
             __syncthreads();
             sum = uniform(sh.found[slot]);
-            if (sum == 0 || sum > LABELS || at + sum > n_hist || executed > limit) return;
+            if (sum == 0 || sum > LABELS || at + sum > n_hist || hopeless(ns, l, n, sum)) return;
             at += sum;
             if (l % FETCHERS == f && l > 0 && l + FETCHERS < L) fetch(l + FETCHERS);
             if (n > 1 && sum > SORTED_FROM) {
@@ -393,7 +408,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
             ub[k] = sh.ub[k];
             budget[k] = sh.budget[k];
         }
-        int before = 1, at = 0;   // labels of the layer before, and where this layer's begin in memory
+        int before = 1, at = 0, ns = 0;   // labels of the layer before, and where this layer's begin in memory
         // (before the first layer: one, no memory used, for each strategy the cheapest way in)
         __syncthreads();
         int4 here = sh.layer[0];
@@ -524,7 +539,8 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
             executed += (double)(l ? before : S) * n;
             __syncthreads();
             const int sum = uniform(sh.found[slot]);
-            if (sum == 0 || sum > LABELS || at + sum > n_hist || executed > limit) {
+            ns += layer_ns(n, before);
+            if (sum == 0 || sum > LABELS || at + sum > n_hist || hopeless(ns, l, n, sum)) {
                 give_up(sum == 0 ? 3 : 4);
                 return;
             }

@@ -213,6 +213,11 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     form.flags = 0;   // (ignored)
     const int L = p->L, S = p->S, K = p->n_key, T = p->inter_index ? p->n_inter : p->L;
     if (!bounds::has_form(&form) || !(magnitude < 1e100)) return GDP_OK;
+    // The dense recurrence is one launch per layer, that takes 4 us and 0.35 for each strategy in turn (V = 5437, S = 9 7.3 us,
+    // V = 18405, S = 26 13.3, V = 12602, S = 41 20); the bounds take 35 us at least (L = 5: S = 8 58 us whole, 60 with them,
+    // S = 11 79 and 60).
+    const double dense_ns = L * (4000.0 + 350.0 * S);
+    if (dense_ns < 36e3) return GDP_OK;
     int64_t budget[GDP_BOUND_MAX_KEY], least = 0;
     for (int l = 0; l < L; ++l) {
         int32_t m = INT32_MAX;
@@ -285,7 +290,7 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     b.out = reinterpret_cast<GdpFrontierOut *>(base + off_out);
     b.res = reinterpret_cast<int32_t *>(base + off_res);
     b.magnitude = magnitude;
-    b.limit = 1e30;
+    b.limit = dense_ns;
     b.L = L; b.V = p->V; b.S = S; b.K = K; b.T = T;
     b.n_hist = b.n_hist_turns = (int32_t)labels;
     memcpy(g_stage + off_inst, &b, sizeof b);
