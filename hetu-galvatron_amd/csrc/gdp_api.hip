@@ -549,6 +549,8 @@ struct gdp_plan {
     size_t back_bytes = 0;
     const GdpDevOut *h_out = nullptr;
     const int32_t *h_res = nullptr;
+    std::vector<GdpDevOut> bounds_out;   // of a run by bounds, laid out as those of the other runs
+    std::vector<int32_t> bounds_res;
     std::vector<char> stage;     // host copy of the inputs' device layout when it is too large for lane.up;
                                  // the upload reads it asynchronously
     double relaxations = 0, relax_bytes = 0;
@@ -3179,8 +3181,6 @@ struct PlanBounds {
     std::vector<BoundEntry> es;   // one per instance
     BoundSlice slice;
     BoundLease lease;
-    std::vector<GdpDevOut> out;   // as the plan's own results are laid out
-    std::vector<int32_t> res;
 };
 
 static void give_back(PlanBounds *b) { delete b; }
@@ -3202,8 +3202,8 @@ static void take_bounds(int32_t n, const gdp_problem *const *p, const std::vecto
         b->es.push_back(std::move(e));
     }
     b->slice.lay_out(p, b->es.data(), n, n_lam);
-    b->out.resize((size_t)plan->n_key_total);
-    b->res.resize(plan->n_res_total);
+    plan->bounds_out.resize((size_t)plan->n_key_total);
+    plan->bounds_res.resize(plan->n_res_total);
     std::vector<char> up(b->slice.up_bytes);
     b->lease.device = plan->device;
     if (lane_take(plan->device, b->slice.back_bytes, 0, &b->lease.lane) != hipSuccess ||
@@ -3243,11 +3243,11 @@ static int run_bounds(gdp_plan *plan, int32_t mode, gdp_timing *t, bool *done)
         }
         executed += o.executed;
         const int32_t *res = b.slice.res_of(back, h.orig);
-        for (int k = 0; k < h.n_key; ++k) b.out[(size_t)(h.key_begin + k)] = {o.total[k], o.remaining[k], o.remaining[k] >= 0};
-        memcpy(b.res.data() + h.res_begin, res, sizeof(int32_t) * (size_t)h.n_key * h.L);
+        for (int k = 0; k < h.n_key; ++k) plan->bounds_out[(size_t)(h.key_begin + k)] = {o.total[k], o.remaining[k], o.remaining[k] >= 0};
+        memcpy(plan->bounds_res.data() + h.res_begin, res, sizeof(int32_t) * (size_t)h.n_key * h.L);
     }
-    plan->h_out = b.out.data();
-    plan->h_res = b.res.data();
+    plan->h_out = plan->bounds_out.data();
+    plan->h_res = plan->bounds_res.data();
     plan->ran = true;
     if (t) {
         memset(t, 0, sizeof *t);

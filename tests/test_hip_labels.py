@@ -1,0 +1,146 @@
+"""The DP over what the bounds leave, as labels: numbers of keys, labels and strategies around which the kernels branch,
+in batches, plans and static calls; against the C oracle, which sees the whole instance."""
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+from galvatron_dp import _lib
+from oracle import dp_oracle as O
+
+
+def _instance(rng, L, S, V, kind, n_keys):
+    """kind: 'each' random costs per layer; 'trade' equal layers that trade memory for time, whose labels are many;
+    'narrow' layers in which one strategy is the best by far, between random ones."""
+    per = V // L
+    n = 1 if kind == "trade" else L
+    mem = rng.integers(max(1, per // 4), max(2, 3 * per), size=(n, S)).astype(np.int32)
+    intra, inter = rng.lognormal(2.5, 0.5, size=(n, S)), rng.uniform(0, 5, size=(n, S, S))
+    if kind == "trade":
+        intra, inter = 40.0 * per / mem * rng.uniform(0.98, 1.02, size=mem.shape), inter * 0.05
+        mem, intra, inter = np.repeat(mem, L, 0), np.repeat(intra, L, 0), np.repeat(inter, L, 0)
+    if kind == "narrow":
+        intra[::3] += 1e4
+        intra[::3, S // 2], mem[::3, S // 2] = 1.0, 1
+    om = [int(V * f) for f in (0.3, 0.1, 0.0, 0.45, 0.2, 0.999, 0.25, 2.0)[:n_keys]]
+    return mem, intra, inter, om, [k / 3 for k in range(n_keys)]
+
+
+def _problem(x, V):
+    return _lib.Problem(x[0], x[1], x[2], V, x[3], x[4])
+
+
+def _want(x, V):
+    keys = range(len(x[3]))
+    return O.solve(x[0], x[1], x[2], V, dict(zip(keys, x[3])), dict(zip(keys, x[4])))[:3]
+
+
+def _check(prob, want, tag):
+    total, res, left = want
+    for k in total:
+        assert np.float64(prob.total[k]).tobytes() == np.float64(total[k]).tobytes(), f"{tag} key {k}: {prob.total[k]} {total[k]}"
+        assert int(prob.remaining[k]) == left[k], f"{tag} key {k}"
+        if left[k] >= 0:
+            assert [int(v) for v in prob.res[k]] == [int(v) for v in res[k]], f"{tag} key {k}"
+
+
+def _solved_by_labels(probs):
+    _lib.batch_stats_begin()
+    _lib.solve_batch(probs)
+    s = _lib.batch_stats_end()
+    return s.executed < 0.01 * s.relaxations
+
+
+# Labels of the layers that have the most: 1 to 64 (a turn), to 128 and 192 (lanes share the keys), more (buckets), more
+# than fit (the smaller instance, or the whole one)
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,L,S,V,labels", [("each", 9, 12, 6000, True), ("narrow", 20, 16, 9000, True), ("trade", 6, 7, 3000, True),
+                                               ("trade", 10, 8, 6000, True), ("trade", 16, 9, 9000, True), ("trade", 24, 24, 12000, None),
+                                               ("each", 40, 64, 9000, True), ("each", 64, 17, 9000, True), ("narrow", 512, 4, 20000, None)])
+@pytest.mark.parametrize("n_keys", [1, 2, 3, 5, 8])
+def test_batches_by_labels(kind, L, S, V, labels, n_keys, monkeypatch):
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    x = _instance(np.random.Generator(np.random.PCG64([L, S, n_keys])), L, S, V, kind, n_keys)
+    prob = _problem(x, V)
+    by_labels = _solved_by_labels([prob])
+    _check(prob, _want(x, V), f"{kind} {L} {S} {V}")
+    assert labels is None or by_labels == labels
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [2, 16, 17, 24, 25, 32, 33, 40, 41, 48, 49, 64, 65, 88, 89, 128])
+def test_passes_over_one_matrix_some_and_many(S, monkeypatch):
+    """Matrices: the same for all layers, another from the middle on (both held), another for every second layer."""
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    rng, L, V, probs, xs = np.random.Generator(np.random.PCG64(S)), 9, 2000, [], []
+    for index in ([0] * L, [0] * 5 + [1] * 4, [l // 2 for l in range(L)]):
+        x = _instance(rng, L, S, V, "each", 3)
+        x = (x[0], x[1], np.ascontiguousarray(x[2][index]), x[3], x[4])
+        xs.append(x)
+        probs.append(_problem(x, V))
+    for x, prob in zip(xs, probs):
+        _lib.solve_batch([prob])
+        _check(prob, _want(x, V), f"S {S}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["each", "trade"])
+def test_plans_by_labels(kind, monkeypatch):
+    """Runs in turn, what is fetched after the bounds were given back, and the launch schemes after it."""
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    V, rng = 5000, np.random.Generator(np.random.PCG64(8))
+    xs = [_instance(rng, L, 12, V, kind, 3) for L in (12, 5)] + [_instance(rng, 30, 30, V, kind, 2)]
+    want, probs = [_want(x, V) for x in xs], [_problem(x, V) for x in xs]
+
+    def fetched(plan):
+        for p in probs:
+            p.total[:], p.remaining[:], p.res[:] = 0, 0, 0
+        plan.fetch()
+        for i, (p, w) in enumerate(zip(probs, want)):
+            _check(p, w, f"{kind} instance {i}")
+    with _lib.Plan(probs) as plan:
+        by_labels = plan.run().relax_launches == 0
+        assert by_labels or kind == "trade"
+        fetched(plan)
+        t = plan.run(1)
+        assert t.total_ms > 0 and (t.relax_launches == 0) == by_labels
+        fetched(plan)
+        assert plan.run(2).relax_launches > 0
+        fetched(plan)
+        plan.run()
+        plan.set_option(1, 0)              # GDP_OPT_FUSED: about the launch schemes, which run from here on
+        fetched(plan)
+        assert plan.run(1).relax_launches > 0
+        fetched(plan)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,L,S,V,n_keys", [("each", 2, 3, 200, 2), ("each", 5, 8, 3000, 3), ("each", 5, 11, 3000, 3), ("each", 30, 30, 5000, 8),
+                                               ("trade", 10, 8, 6000, 2), ("trade", 30, 30, 9000, 1), ("narrow", 21, 16, 6000, 5)])
+def test_static_calls_by_labels(kind, L, S, V, n_keys):
+    x = _instance(np.random.Generator(np.random.PCG64([L, S])), L, S, V, kind, n_keys)
+    prob = _problem(x, V)
+    for _ in range(2):
+        prob.total[:], prob.remaining[:], prob.res[:] = 0, 0, 0
+        _lib.solve_static(prob)
+        _check(prob, _want(x, V), f"{kind} {L} {S}")
+
+
+@pytest.mark.parametrize("source", ["gdp_bounds.hip", "gdp_frontier.hip"])
+def test_the_kernels_launchers_allocate_nothing(source, tmp_path):
+    """gdp_solve_static calls them: no allocator, no stream or event, and no function of the library beside them."""
+    from galvatron_dp import _build
+    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    if shutil.which(hipcc) is None:
+        pytest.skip("no hipcc")
+    obj = str(tmp_path / "o.o")
+    flags = [f for f in _build.HIPCC_FLAGS if f != "-shared"]
+    subprocess.run([hipcc] + flags + ["-c", os.path.join(_build.CSRC, source), "-o", obj], check=True, capture_output=True)
+    undefined = subprocess.run(["nm", "-u", "-C", obj], stdout=subprocess.PIPE, text=True, check=True).stdout
+    names = [ln.split(None, 1)[1].strip() for ln in undefined.splitlines() if ln.strip().startswith("U ")]
+    assert any(n.startswith("hipLaunchKernel") for n in names), names
+    for n in names:
+        assert not n.startswith(("hipMalloc", "hipHost", "hipExtMalloc", "hipMem", "hipStream", "hipEvent", "hipFree", "operator", "gdp_",
+                                 "malloc", "calloc", "realloc", "posix_memalign", "aligned_alloc", "std::__throw")), n
