@@ -2299,6 +2299,20 @@ int run_enqueue(gdp_plan *pl, int32_t mode)
     return GDP_OK;
 }
 
+// How the plan was laid out, also where a run did without.
+void tell_layout(const gdp_plan *pl, gdp_timing *t)
+{
+    if (!pl->groups.empty()) {
+        const Group &g0 = pl->groups.front();
+        t->tile_ts = GDP_VARIANTS[g0.variant].ts;
+        t->tile_r = GDP_VARIANTS[g0.variant].r;
+        t->chunk = (pl->fused && g0.chunk < g0.count) ? g0.chunk : 0;
+        t->latency_variant = pl->fused || (!pl->run_flow && !g0.lat_ok) ? 0 : g0.latency;
+        t->fused_split = pl->fused ? g0.split : 1;
+    }
+    t->keep_marks = pl->keep_marks ? 1 : 0;
+}
+
 // Waits for what run_enqueue started; repeats the run with one launch per layer if a fused launch gave up.
 int run_finish(gdp_plan *pl, int32_t mode, gdp_timing *t)
 {
@@ -2337,15 +2351,7 @@ int run_finish(gdp_plan *pl, int32_t mode, gdp_timing *t)
         t->relax_launches = (int32_t)launches;
         t->fused = pl->fused ? 1 : 0;
         t->flow = pl->run_flow ? 1 : 0;
-        if (!pl->groups.empty()) {
-            const Group &g0 = pl->groups.front();
-            t->tile_ts = GDP_VARIANTS[g0.variant].ts;
-            t->tile_r = GDP_VARIANTS[g0.variant].r;
-            t->chunk = (pl->fused && g0.chunk < g0.count) ? g0.chunk : 0;
-            t->latency_variant = pl->fused || (!pl->run_flow && !g0.lat_ok) ? 0 : g0.latency;
-            t->fused_split = pl->fused ? g0.split : 1;
-        }
-        t->keep_marks = pl->keep_marks ? 1 : 0;
+        tell_layout(pl, t);
         if (mode >= 1) GDP_HIP(hipEventElapsedTime(&t->total_ms, pl->ev_begin, pl->ev_end));
         if (mode >= 2) {
             float sum = 0;
@@ -3080,7 +3086,7 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
     if (err == hipSuccess) err = slice.enqueue(dev, lane.stream);
     if (err == hipSuccess && stats) err = hipEventRecord(lane.ev_end, lane.stream);
     if (err == hipSuccess) err = hipMemcpyAsync(lane.back, dev + slice.up_bytes, slice.back_bytes, hipMemcpyDeviceToHost, lane.stream);
-    while (scan.step() && hipStreamQuery(lane.stream) == hipErrorNotReady) {}
+    while (scan.step() && hipStreamQuery(lane.stream) == hipErrorNotReady) (void)hipGetLastError();   // not one of a launch
     hipError_t es2 = hipStreamSynchronize(lane.stream);
     if (err == hipSuccess) err = es2;
     std::vector<char> keep;
@@ -3253,6 +3259,7 @@ static int run_bounds(gdp_plan *plan, int32_t mode, gdp_timing *t, bool *done)
         memset(t, 0, sizeof *t);
         t->relaxations = plan->relaxations;
         t->executed = executed;
+        tell_layout(plan, t);
         if (mode >= 1) GDP_HIP(hipEventElapsedTime(&t->total_ms, plan->ev_begin, plan->ev_end));
     }
     *done = true;

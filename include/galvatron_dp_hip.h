@@ -110,7 +110,7 @@ typedef struct gdp_result {
 typedef struct gdp_timing {
     float total_ms;        /* first kernel to last kernel (relaxation layers + epilogue)      */
     float relax_ms;        /* sum of the per-launch durations of the relaxation kernel         */
-    int32_t relax_launches;
+    int32_t relax_launches; /* 0: a run by bounds (see gdp_plan_run)                           */
     int32_t fused;         /* 1: all layers in one launch, 0: one launch per layer             */
     double relaxations;    /* sum over instances of L*V*S*S                                    */
     double executed;       /* relaxations actually carried out: cells whose sources are all +inf, and cells
@@ -138,8 +138,9 @@ int gdp_solve(const gdp_problem *p, gdp_result *r);
  * search_engine.py:477-498) with one launch grid per layer index.  A batch whose cost buffers would
  * exceed GALVATRON_DP_ARENA_MB (default 8192) of device memory is solved in consecutive parts that
  * reuse one allocation.
- * Where it pays, strategies that no best path can use are taken out of an instance by lower bounds before it is
- * solved (GALVATRON_DP_REDUCE=0: never); the results are those of the whole instance, bit for bit.
+ * Where it pays, strategies that no best path can use are taken out of an instance by lower bounds, and what is left
+ * is solved without the budget axis, or as a smaller instance where that would take longer (GALVATRON_DP_REDUCE=0:
+ * never); the results are those of the whole instance, bit for bit.
  * f0 arrays of 64 MB or more in all may be read by up to 7 threads that the call starts and joins before it
  * returns, on every path (GALVATRON_DP_SCAN_THREADS=n: at most n, 0: only the calling thread reads them). */
 int gdp_solve_batch(int32_t n, const gdp_problem *const *p, gdp_result *const *r);
@@ -153,7 +154,8 @@ int gdp_solve_batch(int32_t n, const gdp_problem *const *p, gdp_result *const *r
  * its cost buffers, argmin table, tables and results live in one static device array of
  * GDP_STATIC_SCRATCH_BYTES that every device the library runs on holds until the process ends, the
  * inputs' device layout is built in a fixed host array, and the work runs on the null stream with
- * synchronous copies.  It keeps two cost buffers and the one-byte argmin table (the layout of
+ * synchronous copies.  Instances that have the form are solved by bounds and what they leave, as in
+ * gdp_solve_batch; any other with two cost buffers and the one-byte argmin table (the layout of
  * GDP_KEEP_MARKS), one launch per layer, every cell computed.
  *   - An instance that needs more than the array (roughly 17*(V + max mem)*(S+1) + L*S*V bytes, or
  *     tables above 8 MiB) is refused with GDP_E_NOMEM and a message that gives both sizes; so are
@@ -170,7 +172,9 @@ int gdp_solve_static(const gdp_problem *p, gdp_result *r);
  * device memory and run the device part repeatedly:
  *   create  -- validate + allocate + copy inputs to the device
  *   run     -- layer kernels + on-device backtrack; timing may be NULL.
- *              timing_mode 0: none, 1: total_ms only, 2: also per-launch relaxation events
+ *              timing_mode 0: none, 1: total_ms only, 2: also per-launch relaxation events.
+ *              Where it pays (as in gdp_solve_batch), bounds and the DP over what they leave run instead of the layer
+ *              kernels, relax_launches is 0 then.  Not in mode 2, after gdp_plan_set_option or with GDP_COMPUTE_ALL.
  *   fetch   -- copy results of the last run to the caller's arrays
  *   destroy -- release everything                                              */
 int gdp_plan_create(int32_t n, const gdp_problem *const *p, gdp_plan **out);
@@ -238,7 +242,7 @@ typedef struct gdp_batch_stats {
     double relaxations;   /* sum over the solved instances of L*V*S*S, as the caller gave them; what initial costs
                              that were found late made the call solve again counts again    */
     double executed;      /* of those, carried out (see gdp_timing.executed); where strategies were taken out by
-                             bounds, those of the smaller instance that was solved          */
+                             bounds, those of the smaller instance or of the labels that were solved */
     double device_ms;     /* sum over the parts of first kernel -> last kernel, and of the bounds' kernels */
     int64_t instances;
     int64_t parts;        /* plans (a batch above GALVATRON_DP_ARENA_MB is solved in parts) */

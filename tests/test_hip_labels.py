@@ -144,3 +144,19 @@ def test_the_kernels_launchers_allocate_nothing(source, tmp_path):
     for n in names:
         assert not n.startswith(("hipMalloc", "hipHost", "hipExtMalloc", "hipMem", "hipStream", "hipEvent", "hipFree", "operator", "gdp_",
                                  "malloc", "calloc", "realloc", "posix_memalign", "aligned_alloc", "std::__throw")), n
+
+
+@pytest.mark.gpu
+def test_what_is_given_up_goes_on_after_the_initial_costs_were_begun(monkeypatch):
+    """The calling thread looks through initial costs while the bounds run, and asks between pieces whether they are done;
+    the launches of the smaller instance come after that."""
+    L, S, V = 40, 24, 200000
+    x = _instance(np.random.Generator(np.random.PCG64(3)), L, S, V, "trade", 2)
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "0")
+    whole = _problem(x, V)
+    _lib.solve_batch([whole])
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    prob = _lib.Problem(x[0], x[1], x[2], V, x[3], x[4], f0=np.zeros((V, S)))
+    assert not _solved_by_labels([prob])
+    assert prob.total.tobytes() == whole.total.tobytes() and np.array_equal(prob.remaining, whole.remaining)
+    assert np.array_equal(prob.res, whole.res)
