@@ -325,7 +325,14 @@ def main() -> int:
 
     def measure(workload, steps, warmup, compute_all=True, keep_marks=False, host_leg=False, check=False):
         insts, probs = _problems(workload, compute_all, keep_marks)
-        with _lib.Plan(probs) as plan:
+        # the recurrence itself is what is measured, not what bounds would leave of it
+        preset = os.environ.get("GALVATRON_DP_REDUCE")
+        os.environ["GALVATRON_DP_REDUCE"] = "0"
+        made = _lib.Plan(probs)
+        del os.environ["GALVATRON_DP_REDUCE"]
+        if preset is not None:
+            os.environ["GALVATRON_DP_REDUCE"] = preset
+        with made as plan:
             for _ in range(warmup):
                 plan.run(0)
             device_sync()
