@@ -2691,25 +2691,30 @@ static int bound_multipliers(size_t instances) { return instances <= 32 ? GDP_BO
 // Share of the strategies of a layer that are cheaper in time than every one that needs no more memory: most others
 // go.  From one layer each of at most 8 instances (batches of 2 to 1000, share of the relaxations left: random costs
 // 0.15 on average and 0.06; costs where memory is traded for time 0.44 and 0.40).
+static double undominated(const gdp_problem *q, int32_t layer, std::vector<std::pair<int32_t, double>> &sorted)
+{
+    const size_t row = (size_t)layer * q->S;
+    sorted.clear();
+    for (int s = 0; s < q->S; ++s) sorted.emplace_back(q->mem[row + s], q->intra[row + s]);
+    std::sort(sorted.begin(), sorted.end());
+    double least = INFINITY;
+    int stay = 0;
+    for (const auto &s : sorted) {
+        stay += s.first < q->V && s.second < least;
+        least = s.first < q->V ? std::min(least, s.second) : least;
+    }
+    return (double)stay / q->S;
+}
+
 static double undominated(int32_t n, const gdp_problem *const *p)
 {
     constexpr int32_t LOOKED_AT = 8;
-    std::vector<std::pair<int32_t, double>> layer;
+    std::vector<std::pair<int32_t, double>> sorted;
     double share = 0;
     const int32_t m = std::min(n, LOOKED_AT);
     for (int32_t k = 0; k < m; ++k) {
         const gdp_problem *q = p[(int64_t)n * k / m];
-        const size_t row = (size_t)(q->L / 2) * q->S;
-        layer.clear();
-        for (int s = 0; s < q->S; ++s) layer.emplace_back(q->mem[row + s], q->intra[row + s]);
-        std::sort(layer.begin(), layer.end());
-        double least = INFINITY;
-        int stay = 0;
-        for (const auto &s : layer) {
-            stay += s.first < q->V && s.second < least;
-            least = s.first < q->V ? std::min(least, s.second) : least;
-        }
-        share += (double)stay / q->S;
+        share += undominated(q, q->L / 2, sorted);
     }
     return share / m;
 }
@@ -2757,6 +2762,40 @@ static bool bounds_pay(int32_t n, const gdp_problem *const *p)
     const bool wide = max_S > 88;
     const double passes = layers * 2 * bound_multipliers((size_t)n) / 1024;
     return save >= std::max(max_L * (wide ? STEP_16 : STEP), passes * (wide ? BUSY_16 : BUSY)) + (n > 1 ? entries * ENTRY * undominated(n, p) : 0.0);
+}
+
+// The same for a call of one instance, below bounds_pay's floor: where its labels stay few, the whole call is one round
+// trip of 55 us + L * (2.3 + 0.06 S) us, host included, against 60 us + L * (2.8 + 0.085 S) us of the launch schemes and
+// their relaxations.  How many labels there will be is not known before; what tells it best is how many strategies of a
+// layer no other one dominates, times the layers (4 of them are looked at), unless layers are alike: then whatever trades
+// memory for time does so in every one.  Whole / by labels, us, means of 5 inputs each:
+//   layers of their own, random costs (2 to 8 of S undominated)   L = 6, S = 24, 3e7 81 / 77    L = 12, S = 24, 1e8 108 / 94
+//     L = 28, S = 40, 3e8 221 / 168    L = 28, S = 88, 2e8 419 / 310    L = 60, S = 20, 2e8 304 / 240    L = 128, S = 8, 2e8 502 / 497
+//   ... that follow a layout (5 to 24)  L = 8, S = 44, 2e8 113 / 103   L = 28, S = 44, 2e8 229 / 263   L = 60, S = 20, 2e8 305 / 369
+//   layers alike, a layout  L = 6, S = 40, 1e8 93 / 97; 3e8 108 / 96   L = 12, S = 40, 3e8 136 / 144; 7e8 165 / 142
+//     L = 28, S = 40, 7e8 232 / 278; 1.5e9 312 / 259   L = 60, S = 24, 7e8 330 / 389; 1.5e9 514 / 406; S = 40, 1.5e9 491 / 495
+// So few of a layer and layers of their own take them from 3e7 relaxations on -- below 80 over all layers none of 150 inputs lost more
+// than 8 %, from 84 on some do, up to a third --, everything else from 5e7 a layer, as in bounds_pay.  Initial
+// costs are looked through while the device works; where that takes longer than the chain of layers nothing is gained.
+static bool labels_pay(const gdp_problem *q, size_t scanned)
+{
+    constexpr double LEAST = 3e7, MANY = 3e8, MANY_LAYER = 5e7, FEW = 80;
+    if (!bounds::has_form(q) || q->S > 88) return false;
+    const double work = (double)q->L * q->V * q->S * q->S;
+    if (work < LEAST) return false;
+    if (work >= std::max(MANY, MANY_LAYER * q->L) && InitialScan::device_bound(work, scanned)) return true;
+    if ((double)scanned / 35e9 > q->L * (2.8e-6 + 0.085e-6 * q->S)) return false;
+    int alike = 0;
+    for (int l = 1; l < q->L; ++l) {
+        const size_t at = (size_t)l * q->S, before = at - q->S;
+        alike += memcmp(q->mem + at, q->mem + before, sizeof(int32_t) * q->S) == 0 && memcmp(q->intra + at, q->intra + before, sizeof(double) * q->S) == 0;
+    }
+    if (alike * 4 > q->L) return false;
+    std::vector<std::pair<int32_t, double>> sorted;
+    const int m = std::min(q->L, 4);
+    double share = 0;
+    for (int k = 0; k < m; ++k) share += undominated(q, (int)((int64_t)q->L * (2 * k + 1) / (2 * m)), sorted);
+    return share / m * q->S * q->L <= FEW;
 }
 
 // The smaller instance of q, given what stays ([L][S]); false where it would not be a good deal smaller.
@@ -3160,7 +3199,8 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
 {
     bool forced = false;
     if (!bounds_allowed(&forced)) return GDP_OK;
-    if (!forced && (!bounds_pay(n, p) || !InitialScan::device_bound(dense_work(n, p), scan.alone()))) return GDP_OK;
+    if (!forced && !(bounds_pay(n, p) && InitialScan::device_bound(dense_work(n, p), scan.alone())) && !(n == 1 && labels_pay(p[0], scan.alone())))
+        return GDP_OK;
 
     std::vector<BoundEntry> es;
     for (int i = 0; i < n; ++i) {

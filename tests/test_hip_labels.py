@@ -160,3 +160,20 @@ def test_what_is_given_up_goes_on_after_the_initial_costs_were_begun(monkeypatch
     assert not _solved_by_labels([prob])
     assert prob.total.tobytes() == whole.total.tobytes() and np.array_equal(prob.remaining, whole.remaining)
     assert np.array_equal(prob.res, whole.res)
+
+
+# The line of a single call: 3e7 relaxations where layers are their own and few strategies undominated, 5e7 a layer (3e8 at
+# least) otherwise; initial costs that take longer than the chain of layers
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,L,S,V,zeros,labels", [("each", 10, 20, 7400, False, False), ("each", 10, 20, 7600, False, True),
+                                                     ("each", 10, 20, 7600, True, True), ("each", 10, 20, 60000, True, False),
+                                                     ("each", 3, 89, 7600, False, False), ("trade", 6, 20, 20000, False, False),
+                                                     ("trade", 3, 20, 250100, False, True), ("each", 256, 8, 9000, False, False)])
+def test_single_calls_around_the_rule(kind, L, S, V, zeros, labels):
+    if "GALVATRON_DP_REDUCE" in os.environ or "GALVATRON_DP_SKIP" in os.environ:
+        pytest.skip("the environment presets the rule")
+    x = _instance(np.random.Generator(np.random.PCG64([L, S])), L, S, V, kind, 3)
+    prob = _lib.Problem(x[0], x[1], x[2], V, x[3], x[4], f0=np.zeros((V, S)) if zeros else None)
+    by_labels = _solved_by_labels([prob])
+    _check(prob, _want(x, V), f"{kind} {L} {S} {V}")
+    assert by_labels == labels
