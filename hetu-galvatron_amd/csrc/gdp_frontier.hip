@@ -184,8 +184,8 @@ struct Ahead {
 // least, in scalar registers.
 // A dependent instruction takes 9 clocks, a read from LDS 64, a barrier 30, so a layer of few labels is 0.9 us, one of 270
 // labels and 8 strategies 9.  Against the smaller instance of the dense recurrence that the host made of what stays (kernels,
-// without the host's 0.05 to 0.9 ms between them): L = 80, S = 64 311 -> 196 us, L = 48, S = 88 405 -> 111, 256 instances
-// of S = 44 1690 -> 99, 15 stages of a fit 435 -> 329.
+// without the host's 0.05 to 0.9 ms between them): L = 80, S = 64 311 -> 216 to 255 us by input, L = 48, S = 88 405 -> 90 to 124,
+// 256 instances of S = 44 1690 -> 118, 15 stages of a fit 435 -> 217 to 260.
 template <int KEYS>
 __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundInst *inst)
 {
