@@ -169,20 +169,25 @@ size_t cache_cap(int device)
 void arena_give(int device, char *ptr, size_t bytes)
 {
     const size_t cap = cache_cap(device);
+    bool kept = false;
     std::vector<Arena> drop;
-    if (bytes > cap) {
-        drop.push_back({device, ptr, bytes});
-    } else {
-        std::lock_guard<std::mutex> lk(g_arena_mu);
-        g_arenas.push_back({device, ptr, bytes});
-        size_t total = 0;
-        for (const Arena &a : g_arenas) total += a.bytes;
-        while (total > cap) {  // the one given back longest ago first (they are kept in that order)
-            total -= g_arenas.front().bytes;
-            drop.push_back(g_arenas.front());
-            g_arenas.erase(g_arenas.begin());
+    try {
+        if (bytes <= cap) {
+            std::lock_guard<std::mutex> lk(g_arena_mu);
+            drop.reserve(g_arenas.size() + 1);
+            g_arenas.push_back({device, ptr, bytes});
+            kept = true;
+            size_t total = 0;
+            for (const Arena &a : g_arenas) total += a.bytes;
+            while (total > cap) {  // the one given back longest ago first (they are kept in that order)
+                total -= g_arenas.front().bytes;
+                drop.push_back(g_arenas.front());
+                g_arenas.erase(g_arenas.begin());
+            }
         }
+    } catch (const std::bad_alloc &) {   // no host memory to note it in
     }
+    if (!kept) (void)hipFree(ptr);
     for (const Arena &a : drop) (void)hipFree(a.ptr);  // same device as the caller's plan
 }
 
@@ -2382,31 +2387,27 @@ int run(gdp_plan *pl, int32_t mode, gdp_timing *t)
     return rc == GDP_OK ? run_finish(pl, mode, t) : rc;
 }
 
-// Copies `bytes` from the device to the host a piece at a time over the plan's two streams: one piece is taken out of
-// page-locked memory -- take(piece, offset, bytes) -- while the next one is on its way.  What lies on the device is
-// complete on the plan's stream.  (Without page-locked memory the piece is an ordinary array: each then waits.)
+constexpr size_t EXPORT_PIECE = (size_t)1 << 20;
+
+// Copies `bytes` from the device to the host a piece at a time over the plan's two streams: one of the two pieces that lie
+// at `piece` is handed out -- take(piece, offset, bytes) -- while the other is on its way.  What lies on the device is complete on
+// the plan's stream.  (Pieces of ordinary memory each wait for their copy.)
 template <typename Take>
-hipError_t copy_out(gdp_plan *pl, const char *from, size_t bytes, Take take)
+hipError_t copy_out(gdp_plan *pl, char *piece, const char *from, size_t bytes, Take take)
 {
-    constexpr size_t PIECE = (size_t)1 << 20;
     const hipStream_t streams[2] = {pl->stream, pl->lane.side};
-    std::vector<char> pageable;
-    char *piece = pl->lane.up;
-    if (pl->lane.up_bytes < 2 * PIECE) {
-        pageable.resize(2 * PIECE);
-        piece = pageable.data();
-    }
     hipError_t e = hipStreamSynchronize(pl->stream);
     auto ask = [&](size_t k) {
-        if (k * PIECE < bytes && e == hipSuccess)
-            e = hipMemcpyAsync(piece + (k & 1) * PIECE, from + k * PIECE, std::min(PIECE, bytes - k * PIECE), hipMemcpyDeviceToHost, streams[k & 1]);
+        if (k * EXPORT_PIECE < bytes && e == hipSuccess)
+            e = hipMemcpyAsync(piece + (k & 1) * EXPORT_PIECE, from + k * EXPORT_PIECE, std::min(EXPORT_PIECE, bytes - k * EXPORT_PIECE),
+                               hipMemcpyDeviceToHost, streams[k & 1]);
     };
     ask(0);
-    for (size_t k = 0; k * PIECE < bytes && e == hipSuccess; ++k) {
+    for (size_t k = 0; k * EXPORT_PIECE < bytes && e == hipSuccess; ++k) {
         ask(k + 1);
         const hipError_t w = hipStreamSynchronize(streams[k & 1]);
         if (e == hipSuccess) e = w;
-        if (e == hipSuccess) take(piece + (k & 1) * PIECE, k * PIECE, std::min(PIECE, bytes - k * PIECE));
+        if (e == hipSuccess) take(piece + (k & 1) * EXPORT_PIECE, k * EXPORT_PIECE, std::min(EXPORT_PIECE, bytes - k * EXPORT_PIECE));
     }
     for (hipStream_t s : streams) (void)hipStreamSynchronize(s);   // nothing is on its way into `piece` any more
     return e;
@@ -2416,6 +2417,8 @@ hipError_t copy_out(gdp_plan *pl, const char *from, size_t bytes, Take take)
 // device memory holds, in one launch each.  (L = 12, S = 22, V = 8192,
 // against a launch, a copy to pageable memory and a wait per layer and a second copy into the caller's arrays: a call 1105 ->
 // 581 us.)
+// What can run short is taken before anything is written, and the costs are written last: they may be the array that
+// the caller hands in as initial costs, and a call that failed can be made again with it.
 int fetch_tables(gdp_plan *pl, const HostInst &h, const GdpDevInst *d_inst, gdp_result *out)
 {
     constexpr size_t PART = (size_t)256 << 20;
@@ -2423,22 +2426,24 @@ int fetch_tables(gdp_plan *pl, const HostInst &h, const GdpDevInst *d_inst, gdp_
     const bool f = (h.flags & GDP_EXPORT_F) && out->f_out, mark = (h.flags & GDP_EXPORT_MARK) && out->mark_out;
     const size_t layers = mark ? std::min<size_t>(std::min<size_t>((size_t)h.L, 65535), std::max<size_t>(1, PART / (cells * width))) : 0;
     // (the inputs that were laid out in lane.up are on the device: a run has been waited for)
-    if (pinned_reserve(&pl->lane.up, &pl->lane.up_bytes, (size_t)2 << 20, (size_t)1 << 20) != hipSuccess) (void)hipGetLastError();
+    if (pinned_reserve(&pl->lane.up, &pl->lane.up_bytes, 2 * EXPORT_PIECE, (size_t)1 << 20) != hipSuccess) (void)hipGetLastError();
+    std::unique_ptr<char[]> pageable;
+    char *piece = pl->lane.up;
+    if (pl->lane.up_bytes < 2 * EXPORT_PIECE) {
+        pageable.reset(new (std::nothrow) char[2 * EXPORT_PIECE]);
+        if (!pageable) return fail(GDP_E_NOMEM, "host memory for the exported tables");
+        piece = pageable.get();
+    }
     char *tmp = nullptr;
     size_t tmp_bytes = 0;
     hipError_t e = arena_take(pl->device, std::max(f ? cells * sizeof(double) : 0, layers * cells * width), &tmp, &tmp_bytes);
     if (e != hipSuccess) return fail_hip(e, "export");
-    if (f) {
-        e = gdp_launch_export_f(d_inst, reinterpret_cast<double *>(tmp), h.V, h.S, pl->stream);
-        if (e == hipSuccess)
-            e = copy_out(pl, tmp, cells * sizeof(double), [&](const char *p, size_t at, size_t n) { memcpy(reinterpret_cast<char *>(out->f_out) + at, p, n); });
-    }
     for (size_t l = 0; mark && l < (size_t)h.L && e == hipSuccess; l += layers) {
         const size_t m = std::min(layers, (size_t)h.L - l);
         e = gdp_launch_export_mark(d_inst, (int)l, (int)m, tmp, h.V, h.S, pl->stream);
         int32_t *to = out->mark_out + l * cells;
         if (e == hipSuccess)
-            e = copy_out(pl, tmp, m * cells * width, [&](const char *p, size_t at, size_t n) {
+            e = copy_out(pl, piece, tmp, m * cells * width, [&](const char *p, size_t at, size_t n) {
                 if (width != 1) {
                     memcpy(reinterpret_cast<char *>(to) + at, p, n);
                     return;
@@ -2447,6 +2452,11 @@ int fetch_tables(gdp_plan *pl, const HostInst &h, const GdpDevInst *d_inst, gdp_
                 int32_t *w = to + at;
                 for (size_t k = 0; k < n; ++k) w[k] = b[k] == GDP_EXPORT_NONE ? -1 : (int32_t)b[k];
             });
+    }
+    if (f && e == hipSuccess) {
+        e = gdp_launch_export_f(d_inst, reinterpret_cast<double *>(tmp), h.V, h.S, pl->stream);
+        if (e == hipSuccess)
+            e = copy_out(pl, piece, tmp, cells * sizeof(double), [&](const char *p, size_t at, size_t n) { memcpy(reinterpret_cast<char *>(out->f_out) + at, p, n); });
     }
     arena_give(pl->device, tmp, tmp_bytes);
     return e == hipSuccess ? GDP_OK : fail_hip(e, "export");

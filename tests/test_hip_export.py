@@ -1,10 +1,14 @@
 """The exported tables through the plugin signature: pieces and widths of the copy, and the caller's arrays that are
 written directly or through a copy."""
+import os
+import shutil
+import subprocess
+
 import numpy as np
 import pytest
 
 import galvatron_dp_core as shim
-from galvatron_dp import workloads as W
+from galvatron_dp import _build, workloads as W
 from oracle import dp_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -28,3 +32,14 @@ def test_exported_tables(L, S, V, direct):
     assert np.array_equal(mark, want[4]) and np.ascontiguousarray(f).tobytes() == want[3].tobytes()
     for k in want[0]:
         assert np.float64(total[k]).tobytes() == np.float64(want[0][k]).tobytes() and left[k] == want[2][k]
+
+
+def test_no_host_memory_for_the_pieces(tmp_path):
+    """An error code, and nothing written to the costs, where the pieces of the copy cannot be had."""
+    here, exe = os.path.dirname(os.path.abspath(__file__)), str(tmp_path / "export_check")
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    subprocess.run(["g++", "-O1", "-std=c++17", os.path.join(here, "sanitize", "export_check.cpp"), _build.LIB_PATH, "-Wl,-rpath," + _build.LIB_DIR,
+                    "-Wl,--allow-shlib-undefined", "-o", exe], check=True, capture_output=True)
+    run = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
+    assert run.returncode == 0 and "fetched" in run.stdout, run.stdout
