@@ -2414,7 +2414,7 @@ hipError_t copy_out(gdp_plan *pl, char *piece, const char *from, size_t bytes, T
 }
 
 // The final costs and the argmin table of one instance in the reference's layout: as many layers at a time as a part of
-// device memory holds, in one launch each.  (L = 12, S = 22, V = 8192,
+// device memory holds, fewer where that much cannot be had, in one launch each.  (L = 12, S = 22, V = 8192,
 // against a launch, a copy to pageable memory and a wait per layer and a second copy into the caller's arrays: a call 1105 ->
 // 581 us.)
 // What can run short is taken before anything is written, and the costs are written last: they may be the array that
@@ -2424,7 +2424,7 @@ int fetch_tables(gdp_plan *pl, const HostInst &h, const GdpDevInst *d_inst, gdp_
     constexpr size_t PART = (size_t)256 << 20;
     const size_t cells = (size_t)h.V * h.S, width = h.S <= GDP_EXPORT_NONE ? 1 : sizeof(int32_t);
     const bool f = (h.flags & GDP_EXPORT_F) && out->f_out, mark = (h.flags & GDP_EXPORT_MARK) && out->mark_out;
-    const size_t layers = mark ? std::min<size_t>(std::min<size_t>((size_t)h.L, 65535), std::max<size_t>(1, PART / (cells * width))) : 0;
+    size_t layers = mark ? std::min<size_t>(std::min<size_t>((size_t)h.L, 65535), std::max<size_t>(1, PART / (cells * width))) : 0;
     // (the inputs that were laid out in lane.up are on the device: a run has been waited for)
     if (pinned_reserve(&pl->lane.up, &pl->lane.up_bytes, 2 * EXPORT_PIECE, (size_t)1 << 20) != hipSuccess) (void)hipGetLastError();
     std::unique_ptr<char[]> pageable;
@@ -2436,8 +2436,12 @@ int fetch_tables(gdp_plan *pl, const HostInst &h, const GdpDevInst *d_inst, gdp_
     }
     char *tmp = nullptr;
     size_t tmp_bytes = 0;
-    hipError_t e = arena_take(pl->device, std::max(f ? cells * sizeof(double) : 0, layers * cells * width), &tmp, &tmp_bytes);
-    if (e != hipSuccess) return fail_hip(e, "export");
+    hipError_t e;
+    while ((e = arena_take(pl->device, std::max(f ? cells * sizeof(double) : 0, layers * cells * width), &tmp, &tmp_bytes)) != hipSuccess) {
+        if ((e != hipErrorOutOfMemory && e != hipErrorMemoryAllocation) || layers <= 1) return fail_hip(e, "export");
+        (void)hipGetLastError();
+        layers = (layers + 1) / 2;   // a layer at a time is enough
+    }
     for (size_t l = 0; mark && l < (size_t)h.L && e == hipSuccess; l += layers) {
         const size_t m = std::min(layers, (size_t)h.L - l);
         e = gdp_launch_export_mark(d_inst, (int)l, (int)m, tmp, h.V, h.S, pl->stream);

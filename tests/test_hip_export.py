@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 import galvatron_dp_core as shim
-from galvatron_dp import _build, workloads as W
+from galvatron_dp import _build, _lib, workloads as W
 from oracle import dp_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -32,6 +32,23 @@ def test_exported_tables(L, S, V, direct):
     assert np.array_equal(mark, want[4]) and np.ascontiguousarray(f).tobytes() == want[3].tobytes()
     for k in want[0]:
         assert np.float64(total[k]).tobytes() == np.float64(want[0][k]).tobytes() and left[k] == want[2][k]
+
+
+# 12 layers as twice 6, 11 as 6 and 5, 3 (four bytes an entry) as 2 and 1, 5 one at a time
+@pytest.mark.parametrize("L,S,V,limit_mb", [(12, 8, 12000, 1), (11, 16, 7000, 1), (3, 256, 1000, 2), (5, 10, 100000, 1)])
+def test_exported_tables_in_what_memory_there_is(L, S, V, limit_mb, monkeypatch):
+    """The device grants less than all layers take after the run: the table comes in several parts."""
+    inst = W.random_instance(np.random.Generator(np.random.PCG64([L, S])), L, S, V, mem_hi=V // L, n_keys=1)
+    want = O.solve(inst.mem, inst.intra, inst.inter, V, inst.other_mem, inst.other_time, keep=True)
+    keys = sorted(inst.other_mem)
+    prob = _lib.Problem(inst.mem, inst.intra, inst.inter, V, [inst.other_mem[k] for k in keys], [inst.other_time[k] for k in keys],
+                        export_f=V * S * 8 <= limit_mb << 20, export_mark=True)
+    with _lib.Plan([prob]) as plan:
+        plan.run()
+        monkeypatch.setenv("GALVATRON_DP_DEVICE_LIMIT_MB", str(limit_mb))
+        plan.fetch()
+    assert np.array_equal(prob.mark_out, want[4])
+    assert prob.f_out is None or prob.f_out.tobytes() == want[3].tobytes()
 
 
 def test_no_host_memory_for_the_pieces(tmp_path):
