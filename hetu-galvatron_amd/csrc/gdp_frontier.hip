@@ -181,7 +181,7 @@ struct Ahead {
 // grid (instances).  What a layer takes is latency, so the chain of a layer is kept short: 8 waves take the labels of a
 // strategy each, 64 at a time, and find their order in the next layer by searches in LDS; 4 others in turn have what the
 // next 4 layers need of the matrices on its way and lay it out in LDS, and all meet twice per layer.  KEYS: as many at
-// least, in scalar registers.
+// least.
 // A dependent instruction takes 9 clocks, a read from LDS 64, a barrier 30, so a layer of few labels is 0.9 us, one of 270
 // labels and 8 strategies 9.  Against the smaller instance of the dense recurrence that the host made of what stays (kernels,
 // without the host's 0.05 to 0.9 ms between them): L = 80, S = 64 311 -> 216 to 255 us by input, L = 48, S = 88 405 -> 90 to 124,
@@ -190,6 +190,11 @@ template <int KEYS>
 __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundInst *inst)
 {
     constexpr int LINE = KEYS * WINDOW + 2;   // of a strategy: lines, intra, memory
+    // Keys whose lines, and whose multipliers, are held in registers; the others' are read from LDS.  All where there is room for
+    // them: no kernel here may need scratch memory, which the runtime would have to obtain for the launch, and gdp_solve_static
+    // promises that nothing is obtained.  (8 keys with all of them held took 252 bytes a lane and longer: L = 80, S = 64 408 -> 377 us;
+    // 5 keys 16 bytes, 296 -> 298.)
+    constexpr int LINES_HELD = KEYS <= 4 ? KEYS : 2, KEYS_HELD = KEYS <= 5 ? KEYS : 0;
     extern __shared__ __align__(16) char lds[];
     Shared &sh = *reinterpret_cast<Shared *>(lds);
     const GdpBoundInst &I = inst[blockIdx.x];
@@ -399,10 +404,10 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
     int32_t v = -1;      // its budget
     bool walks = false;
     if (wave < WORKERS) {
-        double lam[KEYS][WINDOW], ub[KEYS];
-        int32_t budget[KEYS];
+        double lam[KEYS_HELD ? KEYS_HELD : 1][WINDOW], ub[KEYS_HELD ? KEYS_HELD : 1];
+        int32_t budget[KEYS_HELD ? KEYS_HELD : 1];
 #pragma unroll
-        for (int k = 0; k < KEYS; ++k) {
+        for (int k = 0; k < KEYS_HELD; ++k) {
 #pragma unroll
             for (int i = 0; i < WINDOW; ++i) lam[k][i] = sh.lam[k][i];
             ub[k] = sh.ub[k];
@@ -416,15 +421,18 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
             const int now = l & 1, n = uniform(here.x), kept_at = uniform(here.y);
             here = sh.layer[l + 1];
             // what can still be part of a path that fits and is no worse than the best one known
-            auto alive = [&](const double2 *line, double c, int32_t w) {
+            auto alive = [&](const double2 *line, const double2 *row, double c, int32_t w) {
                 const double dw = (double)w;
                 bool any = false;
 #pragma unroll
                 for (int k = 0; k < KEYS; ++k) {
-                    const double b0 = __builtin_fma(lam[k][0], dw, line[2 * k].x), b1 = __builtin_fma(lam[k][1], dw, line[2 * k].y),
-                                 b2 = __builtin_fma(lam[k][2], dw, line[2 * k + 1].x), b3 = __builtin_fma(lam[k][3], dw, line[2 * k + 1].y);
+                    const bool held = k < KEYS_HELD;
+                    const double *const by = held ? lam[held ? k : 0] : sh.lam[k];
+                    const double2 *const at = k < LINES_HELD ? line : row;
+                    const double b0 = __builtin_fma(by[0], dw, at[2 * k].x), b1 = __builtin_fma(by[1], dw, at[2 * k].y),
+                                 b2 = __builtin_fma(by[2], dw, at[2 * k + 1].x), b3 = __builtin_fma(by[3], dw, at[2 * k + 1].y);
                     const double bound = max_f64(max_f64(b0, b1), max_f64(b2, b3));
-                    any |= (w <= budget[k]) & (c + bound <= ub[k]);
+                    any |= (w <= (held ? budget[held ? k : 0] : sh.budget[k])) & (c + bound <= (held ? ub[held ? k : 0] : sh.ub[k]));
                 }
                 return any;
             };
@@ -471,25 +479,25 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
                     const int32_t next_w = sh.f.label[min(lane + 1, before - 1)].w;
                     const double turn = sh.f.turns[now][old.s * n + b];
                     const double2 *row = reinterpret_cast<const double2 *>(sh.f.lines[now] + b * LINE);
-                    double2 line[KEYS * WINDOW / 2];
+                    double2 line[LINES_HELD ? LINES_HELD * WINDOW / 2 : 1];
 #pragma unroll
-                    for (int i = 0; i < KEYS * WINDOW / 2; ++i) line[i] = row[i];
+                    for (int i = 0; i < LINES_HELD * WINDOW / 2; ++i) line[i] = row[i];
                     const double2 costs = row[KEYS * WINDOW / 2];
                     const int32_t w = old.w + __builtin_bit_cast(int2v, costs.y).x;
                     const double c = prefix_min(lane < before ? old.c + turn : INFINITY, before) + costs.x;
                     const bool ends = lane >= before - 1 || next_w != old.w;
                     double last = INFINITY;
                     const double from = step_from(c, ends, last);   // (by all lanes)
-                    const bool stays = (lane < before) & ends & (c < from) & alive(line, c, w);
+                    const bool stays = (lane < before) & ends & (c < from) & alive(line, row, c, w);
                     const unsigned long long these = __builtin_amdgcn_ballot_w64(stays);
                     emit(stays, these, b, 0, room(__popcll(these)), c, w);
                 }
             } else {
                 for (int b = wave; b < n; b += WORKERS) {
                     const double2 *row = reinterpret_cast<const double2 *>(sh.f.lines[now] + b * LINE);
-                    double2 line[KEYS * WINDOW / 2];
+                    double2 line[LINES_HELD ? LINES_HELD * WINDOW / 2 : 1];
 #pragma unroll
-                    for (int i = 0; i < KEYS * WINDOW / 2; ++i) line[i] = row[i];
+                    for (int i = 0; i < LINES_HELD * WINDOW / 2; ++i) line[i] = row[i];
                     const double2 costs = row[KEYS * WINDOW / 2];
                     const double own = costs.x;
                     const int32_t m = __builtin_bit_cast(int2v, costs.y).x;
@@ -526,7 +534,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
                             least = lane_of(c[u], 63);
                             c[u] += own;
                             const double from = step_from(c[u], ends[u], last);   // (by all lanes)
-                            stays[u] = (j0 + 64 * u + lane < before) & ends[u] & (c[u] < from) & alive(line, c[u], w[u]);
+                            stays[u] = (j0 + 64 * u + lane < before) & ends[u] & (c[u] < from) & alive(line, row, c[u], w[u]);
                             these[u] = __builtin_amdgcn_ballot_w64(stays[u]);
                         }
                         const int first = __popcll(these[0]), count = first + __popcll(these[1]), to = room(count);
@@ -746,6 +754,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
 hipError_t bounds::launch_labels(const GdpBoundInst *inst, int n, int max_K, hipStream_t stream)
 {
     const dim3 grid((unsigned)n);
+    // 5 keys have a kernel of their own: its registers hold what that of 8 reads from LDS (L = 80, S = 64 298 us against 370)
     if (max_K <= 2) gdp_frontier_kernel<2><<<grid, THREADS, sizeof(Shared), stream>>>(inst);
     else if (max_K <= 4) gdp_frontier_kernel<4><<<grid, THREADS, sizeof(Shared), stream>>>(inst);
     else if (max_K == 5) gdp_frontier_kernel<5><<<grid, THREADS, sizeof(Shared), stream>>>(inst);

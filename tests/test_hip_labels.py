@@ -1,6 +1,7 @@
 """The DP over what the bounds leave, as labels: numbers of keys, labels and strategies around which the kernels branch,
 in batches, plans and static calls; against the C oracle, which sees the whole instance."""
 import os
+import re
 import shutil
 import subprocess
 
@@ -144,6 +145,23 @@ def test_the_kernels_launchers_allocate_nothing(source, tmp_path):
     for n in names:
         assert not n.startswith(("hipMalloc", "hipHost", "hipExtMalloc", "hipMem", "hipStream", "hipEvent", "hipFree", "operator", "gdp_",
                                  "malloc", "calloc", "realloc", "posix_memalign", "aligned_alloc", "std::__throw")), n
+
+
+@pytest.mark.parametrize("source,kernels", [("gdp_bounds.hip", ("pass", "upper", "keep", "transpose")), ("gdp_frontier.hip", ("frontier",)),
+                                            ("gdp_kernels.hip", ("gdp_relax_kernel", "init", "zero_pass", "epilogue"))])
+def test_kernels_of_static_calls_have_no_scratch_memory(source, kernels):
+    """Scratch memory is device memory that the runtime may have to obtain for a launch: the kernels of gdp_solve_static spill nothing."""
+    from galvatron_dp import _build
+    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    if shutil.which(hipcc) is None:
+        pytest.skip("no hipcc")
+    flags = [f for f in _build.HIPCC_FLAGS if f != "-shared"]
+    log = subprocess.run([hipcc] + flags + ["-c", "--offload-device-only", "-Rpass-analysis=kernel-resource-usage",
+                                            os.path.join(_build.CSRC, source), "-o", os.devnull], check=True, capture_output=True, text=True).stderr
+    found = re.findall(r"Function Name: (\S+).*?ScratchSize \[bytes/lane\]: (\d+)", log, re.S)
+    for part in kernels:
+        own = [(name, int(size)) for name, size in found if part in name]
+        assert own and all(size == 0 for _, size in own), (part, own)
 
 
 @pytest.mark.gpu
