@@ -2655,6 +2655,19 @@ void gdp_debug_shared_device(int32_t seems_shared)
     g_last_give_up_ms.store(seems_shared ? steady_ms() : -1, std::memory_order_relaxed);
 }
 
+}  // extern "C"
+
+void stats::count(double relaxations, double executed)
+{
+    std::lock_guard<std::mutex> lk(g_stats_mu);
+    if (!g_stats_on) return;
+    g_stats.relaxations += relaxations;
+    g_stats.executed += executed;
+    g_stats.instances += 1;
+}
+
+extern "C" {
+
 void gdp_batch_stats_begin(void)
 {
     std::lock_guard<std::mutex> lk(g_stats_mu);
@@ -3187,13 +3200,6 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
     return GDP_OK;
 }
 
-static bool bounds_allowed(bool *forced)
-{
-    const char *env = getenv("GALVATRON_DP_REDUCE"), *skip = getenv("GALVATRON_DP_SKIP");
-    *forced = env && *env && atoi(env) != 0;
-    return !(env && *env && !*forced) && !(skip && *skip && atoi(skip) == 0);
-}
-
 // The entry of an instance whose bounds can be taken.
 static bool bound_entry(const gdp_problem *q, int orig, double magnitude, BoundEntry &e)
 {
@@ -3220,7 +3226,7 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
                         size_t limit, std::vector<std::unique_ptr<Reduced>> &out)
 {
     bool forced = false;
-    if (!bounds_allowed(&forced)) return GDP_OK;
+    if (!bounds::allowed(&forced)) return GDP_OK;
     if (!forced && !(bounds_pay(n, p) && InitialScan::device_bound(dense_work(n, p), scan.alone())) && !(n == 1 && labels_pay(p[0], scan.alone())))
         return GDP_OK;
 
@@ -3258,7 +3264,7 @@ static void give_back(PlanBounds *b) { delete b; }
 static void take_bounds(int32_t n, const gdp_problem *const *p, const std::vector<double> &magnitude, gdp_plan *plan)
 {
     bool forced = false;
-    if (plan->keep_marks || !bounds_allowed(&forced) || (!forced && !bounds_pay(n, p))) return;
+    if (plan->keep_marks || !bounds::allowed(&forced) || (!forced && !bounds_pay(n, p))) return;
     std::unique_ptr<PlanBounds> b(new PlanBounds());
     size_t bytes = 0;
     const int n_lam = bound_multipliers((size_t)n);

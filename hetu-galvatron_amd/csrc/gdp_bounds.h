@@ -64,6 +64,9 @@ struct GdpBoundInst {
 namespace bounds {
 // Whether an instance has the form, its costs apart (reducible in gdp_api.hip).
 __attribute__((visibility("hidden"))) bool has_form(const gdp_problem *q);
+// What the environment says of bounds: false with GALVATRON_DP_REDUCE=0 and with GALVATRON_DP_SKIP=0 (every cell is asked for);
+// *forced: with GALVATRON_DP_REDUCE=1 (every instance that has the form takes them).
+__attribute__((visibility("hidden"))) bool allowed(bool *forced);
 // The multipliers of an instance: 0 and a geometric series around (range of times) / (range of memory costs).
 __attribute__((visibility("hidden"))) void multipliers(const gdp_problem *q, int n_lam, double *lam);
 // Copies the matrices, runs the passes of all multipliers, finds the upper bounds and marks what stays.

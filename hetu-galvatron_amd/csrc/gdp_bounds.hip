@@ -18,6 +18,7 @@
 #include "gdp_bounds.h"
 
 #include <math.h>
+#include <stdlib.h>
 
 namespace {
 
@@ -400,6 +401,13 @@ bool bounds::has_form(const gdp_problem *q)
     constexpr uint32_t whole = GDP_EXPORT_F | GDP_EXPORT_MARK | GDP_COMPUTE_ALL | GDP_KEEP_MARKS | GDP_LAUNCH_FUSED | GDP_LAUNCH_PER_LAYER;
     return !(q->flags & whole) && q->L >= 2 && q->L <= GDP_BOUND_MAX_L && q->S >= 2 && q->S <= GDP_BOUND_MAX_S &&
            q->n_key >= 1 && q->n_key <= GDP_BOUND_MAX_KEY && q->L * q->S <= GDP_BOUND_MAX_LS;
+}
+
+bool bounds::allowed(bool *forced)
+{
+    const char *env = getenv("GALVATRON_DP_REDUCE"), *skip = getenv("GALVATRON_DP_SKIP");
+    *forced = env && *env && atoi(env) != 0;
+    return !(env && *env && !*forced) && !(skip && *skip && atoi(skip) == 0);
 }
 
 void bounds::multipliers(const gdp_problem *q, int n_lam, double *lam)

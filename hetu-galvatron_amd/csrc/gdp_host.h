@@ -19,5 +19,10 @@ int gdp_validate(const gdp_problem *p, int i, double *magnitude);
 // overflow.  *f0_live (may be null): they hold something other than zeros.  Allocates nothing.
 int gdp_validate_f0(const gdp_problem *p, int i, bool *f0_live);
 
+namespace stats {
+// Counts one solved instance in the statistics of gdp_batch_stats_begin() while they are on.  Allocates nothing.
+__attribute__((visibility("hidden"))) void count(double relaxations, double executed);
+}  // namespace stats
+
 // Index into GDP_VARIANTS of the register tile ts x r, or -1.
 int gdp_find_variant(int ts, int r);

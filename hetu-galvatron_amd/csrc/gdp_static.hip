@@ -205,19 +205,23 @@ void build(const gdp_problem *p, const Layout &y, unsigned char *base)
     }
 }
 
+double work(const gdp_problem *p) { return (double)p->L * p->V * (double)p->S * p->S; }
+
 // Solves p by bounds if that is possible: *done.  Initial costs are zeros.
 int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base, gdp_result *r, bool *done)
 {
     *done = false;
+    bool forced = false;
+    if (!bounds::allowed(&forced)) return GDP_OK;
     gdp_problem form = *p;
-    form.flags = 0;   // (ignored)
+    form.flags = p->flags & GDP_COMPUTE_ALL;   // (the others are ignored)
     const int L = p->L, S = p->S, K = p->n_key, T = p->inter_index ? p->n_inter : p->L;
     if (!bounds::has_form(&form) || !(magnitude < 1e100)) return GDP_OK;
     // The dense recurrence is one launch per layer, that takes 4 us and 0.35 for each strategy in turn (V = 5437, S = 9 7.3 us,
     // V = 18405, S = 26 13.3, V = 12602, S = 41 20); the bounds take 35 us at least (L = 5: S = 8 58 us whole, 60 with them,
     // S = 11 79 and 60).
     const double dense_ns = L * (4000.0 + 350.0 * S);
-    if (dense_ns < 36e3) return GDP_OK;
+    if (dense_ns < 36e3 && !forced) return GDP_OK;
     int64_t budget[GDP_BOUND_MAX_KEY], least = 0;
     for (int l = 0; l < L; ++l) {
         int32_t m = INT32_MAX;
@@ -314,6 +318,7 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
         r->remaining[k] = out->remaining[k];
         if (out->remaining[k] >= 0) memcpy(r->res + (size_t)k * L, res + (size_t)k * L, sizeof(int32_t) * (size_t)L);
     }
+    stats::count(work(p), out->executed);
     *done = true;
     return GDP_OK;
 }
@@ -398,5 +403,6 @@ extern "C" int gdp_solve_static(const gdp_problem *p, gdp_result *r)
         r->remaining[k] = out[k].remaining;
         if (out[k].feasible) memcpy(r->res + (size_t)k * y.L, res + (size_t)k * y.L, sizeof(int32_t) * (size_t)y.L);
     }
+    stats::count(work(p), work(p));
     return GDP_OK;
 }

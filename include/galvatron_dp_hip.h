@@ -155,11 +155,11 @@ int gdp_solve_batch(int32_t n, const gdp_problem *const *p, gdp_result *const *r
  * GDP_STATIC_SCRATCH_BYTES that every device the library runs on holds until the process ends, the
  * inputs' device layout is built in a fixed host array, and the work runs on the null stream with
  * synchronous copies.  Instances that have the form are solved by bounds and what they leave, as in
- * gdp_solve_batch; any other with two cost buffers and the one-byte argmin table (the layout of
- * GDP_KEEP_MARKS), one launch per layer, every cell computed.
+ * gdp_solve_batch (with GALVATRON_DP_REDUCE=0, GALVATRON_DP_SKIP=0 or GDP_COMPUTE_ALL none is); any other with two cost
+ * buffers and the one-byte argmin table (the layout of GDP_KEEP_MARKS), one launch per layer, every cell computed.
  *   - An instance that needs more than the array (roughly 17*(V + max mem)*(S+1) + L*S*V bytes, or
  *     tables above 8 MiB) is refused with GDP_E_NOMEM and a message that gives both sizes; so are
- *     S > GDP_MAX_S_MARKS and the export flags (GDP_E_BADARG).  Other flags are ignored.
+ *     S > GDP_MAX_S_MARKS and the export flags (GDP_E_BADARG).  The flags that choose a launch scheme or a layout are ignored.
  *   - All calls of a process share the array of their device, which keeps what the last call left; a
  *     call rewrites everything it reads, and calls take a process-wide lock, so they run one after the
  *     other.  Work that other code queues on the null stream is ordered with it as usual. */
@@ -234,7 +234,8 @@ int gdp_debug_check_layout(int32_t n, const gdp_problem *const *p, int32_t num_c
 void gdp_debug_shared_device(int32_t seems_shared);
 
 /* Benchmark aid (no counterpart in the reference): what the gdp_solve_batch calls of the whole process did
- * between gdp_batch_stats_begin() and gdp_batch_stats_end().  While it is on, every part of a batch is
+ * between gdp_batch_stats_begin() and gdp_batch_stats_end(); of gdp_solve_static calls relaxations, executed and
+ * instances.  While it is on, every part of a batch is
  * bracketed by two HIP events on its stream; device_ms is the sum of those intervals (first kernel of the
  * part to its last one: relaxation launches and backtrack), so the host's share of a sweep's wall time is
  * what is left of the wall clock. */

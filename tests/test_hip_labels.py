@@ -195,3 +195,30 @@ def test_single_calls_around_the_rule(kind, L, S, V, zeros, labels):
     by_labels = _solved_by_labels([prob])
     _check(prob, _want(x, V), f"{kind} {L} {S} {V}")
     assert by_labels == labels
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,L,S,V", [("each", 30, 30, 5000), ("each", 24, 16, 6000), ("trade", 10, 8, 6000)])
+def test_static_calls_do_without_bounds_where_told(kind, L, S, V, monkeypatch):
+    """By labels unless the environment or the caller asks for every cell; told by the statistics."""
+    monkeypatch.delenv("GALVATRON_DP_REDUCE", raising=False)
+    monkeypatch.delenv("GALVATRON_DP_SKIP", raising=False)
+    x = _instance(np.random.Generator(np.random.PCG64([L, S])), L, S, V, kind, 3)
+    want = _want(x, V)
+
+    def share(**flags):
+        prob = _lib.Problem(x[0], x[1], x[2], V, x[3], x[4], **flags)
+        _lib.batch_stats_begin()
+        _lib.solve_static(prob)
+        s = _lib.batch_stats_end()
+        _check(prob, want, f"{kind} {flags}")
+        assert s.instances == 1 and s.relaxations == prob.relaxations
+        return s.executed / s.relaxations
+    assert share() < 0.01 and share(launch="fused") < 0.01
+    assert share(compute_all=True) == 1
+    monkeypatch.setenv("GALVATRON_DP_SKIP", "0")
+    assert share() == 1
+    monkeypatch.setenv("GALVATRON_DP_SKIP", "1")
+    assert share() < 0.01
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "0")
+    assert share() == 1
