@@ -2840,7 +2840,6 @@ static bool build_reduced(const gdp_problem *q, const HostInst &h, const uint8_t
     int most = 0;
     int64_t base = 0, span = 0;   // memory that every path needs beyond 1 per layer, and what a path can need on top
     std::vector<int32_t> low((size_t)L);
-    std::vector<int> count((size_t)L);
     for (int l = 0; l < L; ++l) {
         int n = 0, lo = INT32_MAX, hi = 0;
         for (int s = 0; s < S; ++s) {
@@ -2853,7 +2852,6 @@ static bool build_reduced(const gdp_problem *q, const HostInst &h, const uint8_t
         }
         if (n == 0) return false;
         most = std::max(most, n);
-        count[(size_t)l] = n;
         low[(size_t)l] = lo;
         base += lo - 1;
         span += hi - lo + 1;
@@ -2872,32 +2870,13 @@ static bool build_reduced(const gdp_problem *q, const HostInst &h, const uint8_t
     d.q.n_key = q->n_key;
     d.q.other_time = q->other_time;
     d.q.flags = q->flags;
-    d.kept.assign((size_t)L * R, -1);
+    d.kept.resize((size_t)L * R);
     d.mem.resize((size_t)L * R);
     d.intra.assign((size_t)L * R, INFINITY);
     d.inter.assign((size_t)L * R * R, 0.0);
-    for (int l = 0; l < L; ++l) {
-        int32_t *kept = d.kept.data() + (size_t)l * R;
-        int n = 0;
-        for (int s = 0; s < S; ++s)
-            if (keep[(size_t)l * S + s]) kept[n++] = s;
-        const double *M = h.matrix_at(q, h.matrix(q, l));
-        double *to = d.inter.data() + (size_t)l * R * R;
-        for (int j = 0; j < R; ++j) {
-            const int s = kept[std::min(j, n - 1)];
-            d.mem[(size_t)l * R + j] = q->mem[(size_t)l * S + s] - low[(size_t)l] + 1;
-            if (j >= n) continue;
-            d.intra[(size_t)l * R + j] = q->intra[(size_t)l * S + s];
-            if (l == 0) {   // the zeros before the first layer are reached from every strategy: its cheapest transition
-                double c = INFINITY;
-                for (int sp = 0; sp < S; ++sp) c = std::min(c, 0.0 + M[(size_t)sp * S + s]);
-                for (int i = 0; i < R; ++i) to[(size_t)i * R + j] = c;
-            } else {
-                const int32_t *from = d.kept.data() + (size_t)(l - 1) * R;
-                for (int i = 0; i < count[(size_t)l - 1]; ++i) to[(size_t)i * R + j] = M[(size_t)from[i] * S + s];
-            }
-        }
-    }
+    for (int32_t &m : low) m -= 1;   // every memory cost stays above 0
+    bounds::fill_kept(q, keep, R, [&](int l) { return h.matrix_at(q, h.matrix(q, l)); }, low.data(), d.kept.data(), d.mem.data(), d.intra.data(),
+                      d.inter.data());
     d.other_mem.resize((size_t)q->n_key);
     d.spare.assign((size_t)q->n_key, 0);
     for (int k = 0; k < q->n_key; ++k) {

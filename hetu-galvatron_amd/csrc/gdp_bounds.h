@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <math.h>
 #include <stdint.h>
 
 #include "../../include/galvatron_dp_hip.h"
@@ -76,6 +77,42 @@ hipError_t launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int ma
                   int n_pairs, hipStream_t stream);
 // The DP over what stays (gdp_frontier.hip), after it.
 __attribute__((visibility("hidden"))) hipError_t launch_labels(const GdpBoundInst *inst, int n, int max_K, hipStream_t stream);
+// What stays of q, given the marks ([L][S]), as arrays of R strategies a layer: kept[L][R] is the strategy of q, or -1 for
+// padding, which costs +inf; memory costs less cut[l] (may be null).  matrix(l): that of layer l of q.  R: the most that
+// stay of a layer, at least; at least one stays of every layer.  inter [L][R][R] and intra hold zeros and +inf before.
+template <class Matrix>
+void fill_kept(const gdp_problem *q, const uint8_t *keep, int R, Matrix matrix, const int32_t *cut, int32_t *kept_of, int32_t *mem, double *intra,
+               double *inter)
+{
+    const int L = q->L, S = q->S;
+    int before = 0;
+    for (int l = 0; l < L; ++l) {
+        int32_t *kept = kept_of + (size_t)l * R;
+        int n = 0;
+        for (int s = 0; s < S; ++s)
+            if (keep[(size_t)l * S + s]) kept[n++] = s;
+        for (int j = n; j < R; ++j) kept[j] = -1;
+        const double *M = matrix(l);
+        double *to = inter + (size_t)l * R * R;
+        for (int j = 0; j < R; ++j) {
+            const int s = kept[j < n ? j : n - 1];
+            mem[(size_t)l * R + j] = q->mem[(size_t)l * S + s] - (cut ? cut[l] : 0);
+            if (j >= n) continue;
+            intra[(size_t)l * R + j] = q->intra[(size_t)l * S + s];
+            if (l == 0) {   // the zeros before the first layer are reached from every strategy: its cheapest transition
+                double c = INFINITY;
+                for (int sp = 0; sp < S; ++sp) {
+                    const double x = 0.0 + M[(size_t)sp * S + s];
+                    c = x < c ? x : c;
+                }
+                for (int i = 0; i < R; ++i) to[(size_t)i * R + j] = c;
+            } else {
+                for (int i = 0; i < before; ++i) to[(size_t)i * R + j] = M[(size_t)kept_of[(size_t)(l - 1) * R + i] * S + s];
+            }
+        }
+        before = n;
+    }
+}
 }  // namespace bounds
 
 #ifdef __HIPCC__

@@ -11,9 +11,9 @@
 // hipMalloc / hipFree / hipHostMalloc / stream or event creation and no host allocator.
 //
 // An instance that has the form is solved by bounds and the DP over what they leave (gdp_bounds.hip, gdp_frontier.hip).  Any
-// other, and one of which too much stays, by the kernels of the other entry points in the layout that needs the least
-// memory: two cost buffers used in turn plus the one-byte argmin table (what GDP_KEEP_MARKS selects), one launch per layer,
-// every cell computed.  Results are the same bits as gdp_solve's.
+// other, and what stays of one that is left with too many labels, by the kernels of the other entry points in the layout
+// that needs the least memory: two cost buffers used in turn plus the one-byte argmin table (what GDP_KEEP_MARKS selects), one
+// launch per layer, every cell computed.  Results are the same bits as gdp_solve's.
 //
 // The array is per process and per device (every device the library's code object is loaded on holds
 // its own copy at its own address) and keeps the contents of the last call; a call rewrites everything
@@ -43,6 +43,11 @@ unsigned char *g_scratch_ptr[MAX_DEVICES];  // device address of `scratch` on de
 constexpr size_t STAGE_BYTES = (size_t)8 << 20;
 alignas(256) unsigned char g_stage[STAGE_BYTES];
 
+// What stays of an instance: the marks that the device found, and the smaller instance they leave.
+uint8_t g_keep[GDP_BOUND_MAX_LS];
+constexpr size_t KEPT_BYTES = (size_t)4 << 20;
+alignas(256) unsigned char g_kept[KEPT_BYTES];
+
 inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 // The address of `scratch` on the current device; asked for once per device, with that device current.
@@ -71,6 +76,10 @@ struct Layout {
     size_t off_out, off_res, back_bytes, off_H, off_M, total_bytes;
 };
 
+// Strategies of S in register tiles of those built with the argmin table (11 or 8 wide, 64 rows): the least padding, then the
+// wider one.
+int padded(int S) { return (int)std::min(align_up((size_t)S, 11), align_up((size_t)S, 8)); }
+
 // Shapes and offsets (bytes from the start of `scratch`); the same rules as a plan laid out with
 // GDP_KEEP_MARKS and one launch per layer.
 void lay_out(const gdp_problem *p, Layout *y)
@@ -78,12 +87,9 @@ void lay_out(const gdp_problem *p, Layout *y)
     y->L = p->L; y->V = p->V; y->S = p->S;
     y->T = p->inter_index ? p->n_inter : p->L;
     y->n_key = p->n_key;
-    // register tile among those built with the argmin table (11 or 8 wide, 64 rows): least padding of S,
-    // then the wider one
-    const size_t sp11 = align_up((size_t)p->S, 11), sp8 = align_up((size_t)p->S, 8);
-    y->ts = sp11 <= sp8 ? 11 : 8;
+    y->SP = padded(p->S);
+    y->ts = y->SP % 11 == 0 ? 11 : 8;
     y->variant = gdp_find_variant(y->ts, 1);
-    y->SP = (int)(y->ts == 11 ? sp11 : sp8);
     y->SU = (int)align_up((size_t)p->S, GDP_SRC_UNROLL);
     y->rows = y->SU + GDP_SRC_PAD;
     int maxm = 1;
@@ -207,21 +213,23 @@ void build(const gdp_problem *p, const Layout &y, unsigned char *base)
 
 double work(const gdp_problem *p) { return (double)p->L * p->V * (double)p->S * p->S; }
 
-// Solves p by bounds if that is possible: *done.  Initial costs are zeros.
-int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base, gdp_result *r, bool *done)
+// What the dense recurrence takes: one launch per layer, 4 us and 0.35 for each strategy in turn (V = 5437, S = 9 7.3 us,
+// V = 18405, S = 26 13.3, V = 12602, S = 41 20).
+double dense_ns(int L, int S) { return L * (4000.0 + 350.0 * S); }
+
+// Solves p by bounds if that is possible: *done.  Initial costs are zeros.  *marked: that is left to the dense recurrence, and
+// g_keep says which strategies can matter to it.
+int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base, gdp_result *r, bool *done, bool *marked)
 {
-    *done = false;
+    *done = *marked = false;
     bool forced = false;
     if (!bounds::allowed(&forced)) return GDP_OK;
     gdp_problem form = *p;
     form.flags = p->flags & GDP_COMPUTE_ALL;   // (the others are ignored)
     const int L = p->L, S = p->S, K = p->n_key, T = p->inter_index ? p->n_inter : p->L;
     if (!bounds::has_form(&form) || !(magnitude < 1e100)) return GDP_OK;
-    // The dense recurrence is one launch per layer, that takes 4 us and 0.35 for each strategy in turn (V = 5437, S = 9 7.3 us,
-    // V = 18405, S = 26 13.3, V = 12602, S = 41 20); the bounds take 35 us at least (L = 5: S = 8 58 us whole, 60 with them,
-    // S = 11 79 and 60).
-    const double dense_ns = L * (4000.0 + 350.0 * S);
-    if (dense_ns < 36e3 && !forced) return GDP_OK;
+    // The bounds take 35 us at least (L = 5: S = 8 58 us whole, 60 with them, S = 11 79 and 60).
+    if (dense_ns(L, S) < 36e3 && !forced) return GDP_OK;
     int64_t budget[GDP_BOUND_MAX_KEY], least = 0;
     for (int l = 0; l < L; ++l) {
         int32_t m = INT32_MAX;
@@ -294,7 +302,7 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     b.out = reinterpret_cast<GdpFrontierOut *>(base + off_out);
     b.res = reinterpret_cast<int32_t *>(base + off_res);
     b.magnitude = magnitude;
-    b.limit = dense_ns;
+    b.limit = dense_ns(L, S);
     b.L = L; b.V = p->V; b.S = S; b.K = K; b.T = T;
     b.n_hist = b.n_hist_turns = (int32_t)labels;
     memcpy(g_stage + off_inst, &b, sizeof b);
@@ -311,6 +319,11 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     e = hipMemcpy(g_stage, base + off_out, back_bytes, hipMemcpyDeviceToHost);   // after the kernels, in stream order
     if (e != hipSuccess) return gdp_fail_hip(e, "gdp_solve_static: download");
     const GdpFrontierOut *out = reinterpret_cast<const GdpFrontierOut *>(g_stage);
+    if (out->status > 1) {
+        e = hipMemcpy(g_keep, base + off_keep, LS, hipMemcpyDeviceToHost);
+        if (e != hipSuccess) return gdp_fail_hip(e, "gdp_solve_static: download");
+        *marked = true;
+    }
     if (out->status != 0) return GDP_OK;
     const int32_t *res = reinterpret_cast<const int32_t *>(g_stage + (off_res - off_out));
     for (int k = 0; k < K; ++k) {
@@ -323,41 +336,44 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     return GDP_OK;
 }
 
-}  // namespace
-
-extern "C" int gdp_solve_static(const gdp_problem *p, gdp_result *r)
+// What stays of p (g_keep) as an instance of its own in g_kept, and its layout; false where it would not be a good deal
+// smaller, or does not fit.  (L = 27, S = 37, V = 20011, two kinds of layers that trade memory for time, calls left with too
+// many labels, us: without bounds 541; after them whole 642 to 790, what stays 360 to 480.)
+bool lay_out_kept(const gdp_problem *p, const Layout &whole, gdp_problem *small, Layout *y)
 {
-    gdp_clear_error();
-    if (!p || !r) return gdp_fail(GDP_E_BADARG, "null problem or result");
-    bool f0_live = false;
-    double magnitude = 0;
-    int rc = gdp_validate(p, 0, &magnitude);
-    if (rc == GDP_OK) rc = gdp_validate_f0(p, 0, &f0_live);
-    if (rc != GDP_OK) return rc;
-    if (p->flags & (GDP_EXPORT_F | GDP_EXPORT_MARK))
-        return gdp_fail(GDP_E_BADARG, "gdp_solve_static does not export f / mark");
-    if (p->S > GDP_MAX_S_MARKS) return gdp_fail(GDP_E_BADARG, "gdp_solve_static: S exceeds GDP_MAX_S_MARKS");
-    if (p->n_key > 0 && (!r->total || !r->remaining || !r->res)) return gdp_fail(GDP_E_BADARG, "null result array");
-    Layout y;
-    lay_out(p, &y);
-    if (y.variant < 0) return gdp_fail(GDP_E_HIP, "gdp_solve_static: register tile not built");
-    if (y.total_bytes > (size_t)GDP_STATIC_SCRATCH_BYTES || y.small_bytes > STAGE_BYTES || y.back_bytes > STAGE_BYTES) {
-        char buf[256];
-        snprintf(buf, sizeof buf,
-                 "gdp_solve_static: this instance needs %zu bytes of device working memory (tables %zu, results %zu); "
-                 "the static array holds %zu (tables and results up to %zu each): use gdp_solve",
-                 y.total_bytes, y.small_bytes, y.back_bytes, (size_t)GDP_STATIC_SCRATCH_BYTES, STAGE_BYTES);
-        return gdp_fail(GDP_E_NOMEM, buf);
+    int most = 0;
+    for (int l = 0; l < p->L; ++l) {
+        int n = 0;
+        for (int s = 0; s < p->S; ++s) n += g_keep[(size_t)l * p->S + s];
+        if (n == 0) return false;
+        most = std::max(most, n);
     }
-    std::lock_guard<std::mutex> lk(g_mu);
-    unsigned char *base = nullptr;
-    const int rs = scratch_of_device(&base);
-    if (rs != GDP_OK) return rs;
-    if (!f0_live) {
-        bool done = false;
-        const int rb = solve_by_bounds(p, magnitude, base, r, &done);
-        if (rb != GDP_OK || done) return rb;
-    }
+    const int R = most;
+    if (!(dense_ns(p->L, padded(R)) < 0.85 * dense_ns(p->L, whole.SP))) return false;
+    const size_t LR = (size_t)p->L * R;
+    const size_t off_mem = align_up(4 * LR, 256), off_intra = off_mem + align_up(4 * LR, 256), off_inter = off_intra + align_up(8 * LR, 256),
+                 bytes = off_inter + 8 * LR * (size_t)R;
+    if (bytes > KEPT_BYTES) return false;
+    int32_t *kept = reinterpret_cast<int32_t *>(g_kept), *mem = reinterpret_cast<int32_t *>(g_kept + off_mem);
+    double *intra = reinterpret_cast<double *>(g_kept + off_intra), *inter = reinterpret_cast<double *>(g_kept + off_inter);
+    std::fill(intra, intra + LR, INFINITY);
+    std::fill(inter, inter + LR * (size_t)R, 0.0);
+    bounds::fill_kept(p, g_keep, R, [&](int l) { return p->inter + (size_t)(p->inter_index ? p->inter_index[l] : l) * p->S * p->S; }, nullptr, kept,
+                      mem, intra, inter);
+    *small = *p;
+    small->S = R;
+    small->mem = mem;
+    small->intra = intra;
+    small->inter = inter;
+    small->inter_index = nullptr;
+    small->n_inter = p->L;
+    lay_out(small, y);
+    return y->variant >= 0 && y->total_bytes <= (size_t)GDP_STATIC_SCRATCH_BYTES && y->small_bytes <= STAGE_BYTES && y->back_bytes <= STAGE_BYTES;
+}
+
+// The dense recurrence.  kept: what to say for a strategy of a layer ([L][S] of p), null: itself.
+int solve_dense(const gdp_problem *p, const Layout &y, unsigned char *base, bool f0_live, const int32_t *kept, gdp_result *r)
+{
     build(p, y, base);
     hipStream_t stream = nullptr;  // the null stream: nothing is created
     hipError_t e = hipMemcpy(base, g_stage, y.small_bytes, hipMemcpyHostToDevice);
@@ -401,8 +417,56 @@ extern "C" int gdp_solve_static(const gdp_problem *p, gdp_result *r)
     for (int k = 0; k < y.n_key; ++k) {
         r->total[k] = out[k].total;
         r->remaining[k] = out[k].remaining;
-        if (out[k].feasible) memcpy(r->res + (size_t)k * y.L, res + (size_t)k * y.L, sizeof(int32_t) * (size_t)y.L);
+        if (!out[k].feasible) continue;
+        memcpy(r->res + (size_t)k * y.L, res + (size_t)k * y.L, sizeof(int32_t) * (size_t)y.L);
+        for (int l = 0; kept && l < y.L; ++l) {
+            int32_t &strategy = r->res[(size_t)k * y.L + l];
+            strategy = kept[(size_t)l * y.S + strategy];
+        }
     }
-    stats::count(work(p), work(p));
     return GDP_OK;
+}
+
+}  // namespace
+
+extern "C" int gdp_solve_static(const gdp_problem *p, gdp_result *r)
+{
+    gdp_clear_error();
+    if (!p || !r) return gdp_fail(GDP_E_BADARG, "null problem or result");
+    bool f0_live = false;
+    double magnitude = 0;
+    int rc = gdp_validate(p, 0, &magnitude);
+    if (rc == GDP_OK) rc = gdp_validate_f0(p, 0, &f0_live);
+    if (rc != GDP_OK) return rc;
+    if (p->flags & (GDP_EXPORT_F | GDP_EXPORT_MARK))
+        return gdp_fail(GDP_E_BADARG, "gdp_solve_static does not export f / mark");
+    if (p->S > GDP_MAX_S_MARKS) return gdp_fail(GDP_E_BADARG, "gdp_solve_static: S exceeds GDP_MAX_S_MARKS");
+    if (p->n_key > 0 && (!r->total || !r->remaining || !r->res)) return gdp_fail(GDP_E_BADARG, "null result array");
+    Layout y;
+    lay_out(p, &y);
+    if (y.variant < 0) return gdp_fail(GDP_E_HIP, "gdp_solve_static: register tile not built");
+    if (y.total_bytes > (size_t)GDP_STATIC_SCRATCH_BYTES || y.small_bytes > STAGE_BYTES || y.back_bytes > STAGE_BYTES) {
+        char buf[256];
+        snprintf(buf, sizeof buf,
+                 "gdp_solve_static: this instance needs %zu bytes of device working memory (tables %zu, results %zu); "
+                 "the static array holds %zu (tables and results up to %zu each): use gdp_solve",
+                 y.total_bytes, y.small_bytes, y.back_bytes, (size_t)GDP_STATIC_SCRATCH_BYTES, STAGE_BYTES);
+        return gdp_fail(GDP_E_NOMEM, buf);
+    }
+    std::lock_guard<std::mutex> lk(g_mu);
+    unsigned char *base = nullptr;
+    const int rs = scratch_of_device(&base);
+    if (rs != GDP_OK) return rs;
+    bool marked = false;
+    if (!f0_live) {
+        bool done = false;
+        const int rb = solve_by_bounds(p, magnitude, base, r, &done, &marked);
+        if (rb != GDP_OK || done) return rb;
+    }
+    gdp_problem small;
+    Layout ys;
+    const bool less = marked && lay_out_kept(p, y, &small, &ys);
+    rc = less ? solve_dense(&small, ys, base, false, reinterpret_cast<const int32_t *>(g_kept), r) : solve_dense(p, y, base, f0_live, nullptr, r);
+    if (rc == GDP_OK) stats::count(work(p), work(less ? &small : p));
+    return rc;
 }

@@ -222,3 +222,29 @@ def test_static_calls_do_without_bounds_where_told(kind, L, S, V, monkeypatch):
     assert share() < 0.01
     monkeypatch.setenv("GALVATRON_DP_REDUCE", "0")
     assert share() == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,S,V,n_keys,shared", [(30, 37, 9000, 2, False), (24, 30, 8000, 8, False), (40, 16, 9000, 3, True), (24, 40, 5000, 6, True)])
+def test_static_calls_left_with_many_labels(L, S, V, n_keys, shared):
+    """Every layer trades memory for time and has other strategies, a third of them, that cannot pay: what stays is solved by
+    the dense recurrence, and said in the terms of the whole instance; `shared`: matrices behind an index."""
+    if "GALVATRON_DP_REDUCE" in os.environ or "GALVATRON_DP_SKIP" in os.environ:
+        pytest.skip("the environment presets the rule")
+    rng = np.random.Generator(np.random.PCG64([L, S, n_keys]))
+    mem, intra, inter, om, ot = _instance(rng, L, S, V, "trade", n_keys)
+    for l in range(L):
+        order = rng.permutation(S)
+        mem[l], intra[l] = mem[l][order], intra[l][order]
+        intra[l][rng.permutation(S)[:S // 3 + l % 3]] += 1e4
+    if shared:
+        tables, index = inter[:3], (np.arange(L) % 3).astype(np.int32)
+        prob = _lib.Problem(mem, intra, tables, V, om, ot, inter_index=index)
+        inter = np.ascontiguousarray(tables[index])
+    else:
+        prob = _lib.Problem(mem, intra, inter, V, om, ot)
+    _lib.batch_stats_begin()
+    _lib.solve_static(prob)
+    s = _lib.batch_stats_end()
+    _check(prob, _want((mem, intra, inter, om, ot), V), f"{L} {S} {V}")
+    assert 0.1 < s.executed / s.relaxations < 0.75
