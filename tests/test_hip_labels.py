@@ -248,3 +248,25 @@ def test_static_calls_left_with_many_labels(L, S, V, n_keys, shared):
     s = _lib.batch_stats_end()
     _check(prob, _want((mem, intra, inter, om, ot), V), f"{L} {S} {V}")
     assert 0.1 < s.executed / s.relaxations < 0.75
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,S,V,n_keys,kinds,seed", [(39, 9, 5072, 5, 2, 167), (31, 11, 4894, 4, 1, 346), (23, 13, 6952, 5, 23, 654), (42, 20, 3016, 2, 2, 887)])
+def test_labels_are_not_given_up_near_the_last_layer(L, S, V, n_keys, kinds, seed):
+    """Labels that are many, and late: what they have taken counts no more than what is ahead.  `kinds` of layers that trade
+    memory for time."""
+    if "GALVATRON_DP_REDUCE" in os.environ or "GALVATRON_DP_SKIP" in os.environ:
+        pytest.skip("the environment presets the rule")
+    rng = np.random.Generator(np.random.PCG64(seed))
+    rng.integers(12, 48), rng.integers(8, 24), rng.integers(1, 6), rng.integers(1500, 7000)
+    per, which = V // L, np.arange(L) * kinds // L
+    mem = rng.integers(max(1, per // 4), max(2, 3 * per), size=(kinds, S)).astype(np.int32)
+    intra, inter = 40.0 * per / mem * rng.uniform(0.98, 1.02, size=(kinds, S)), rng.uniform(0, 0.25, size=(kinds, S, S))
+    om = [int(V * f) for f in (0.3, 0.1, 0.0, 0.45, 0.2)[:n_keys]]
+    x = mem[which], intra[which], inter[which], om, [k / 3 for k in range(n_keys)]
+    prob = _problem(x, V)
+    _lib.batch_stats_begin()
+    _lib.solve_static(prob)
+    s = _lib.batch_stats_end()
+    _check(prob, _want(x, V), f"{L} {S} {V}")
+    assert s.executed < 0.01 * s.relaxations
