@@ -106,16 +106,11 @@ void arena_trim(int device /* -1: every device */)
     (void)hipSetDevice(cur);
 }
 
-// Test aid: requests above GALVATRON_DP_DEVICE_LIMIT_MB are answered like a device that is full.
-bool device_refuses(size_t need)
-{
-    return getenv("GALVATRON_DP_DEVICE_LIMIT_MB") && need > env_mb("GALVATRON_DP_DEVICE_LIMIT_MB", 0);
-}
-
 // The smallest kept allocation of `device` that holds `need` bytes, or a fresh one.
 hipError_t arena_take(int device, size_t need, char **ptr, size_t *bytes)
 {
-    if (device_refuses(need)) {
+    // test aid: requests above GALVATRON_DP_DEVICE_LIMIT_MB are answered like a device that is full
+    if (getenv("GALVATRON_DP_DEVICE_LIMIT_MB") && need > env_mb("GALVATRON_DP_DEVICE_LIMIT_MB", 0)) {
         *ptr = nullptr;
         return hipErrorOutOfMemory;
     }
@@ -2815,9 +2810,6 @@ static bool labels_pay(const gdp_problem *q, size_t scanned)
     if (!bounds::has_form(q) || q->S > 88) return false;
     const double work = (double)q->L * q->V * q->S * q->S;
     if (work < LEAST) return false;
-    // where its labels are too many it is solved whole, with two cost buffers and the argmin table at least: whether a call
-    // is refused for that does not depend on its costs
-    if (device_refuses((size_t)q->V * q->S * (2 * sizeof(double) + q->L))) return false;
     if (work >= std::max(MANY, MANY_LAYER * q->L) && InitialScan::device_bound(work, scanned)) return true;
     if ((double)scanned / 35e9 > q->L * (2.8e-6 + 0.085e-6 * q->S)) return false;
     int alike = 0;

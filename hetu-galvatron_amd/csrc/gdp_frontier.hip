@@ -299,7 +299,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
     // first half: of identical layers that trade memory for time the labels of a layer grow towards L / 2 about as they do
     // at the start, and are half of what that comes to in the mean.  In the second half they become fewer again.  Where
     // layers differ the labels may also grow late: then what the layers so far took tells.
-    // (Static calls, 800 inputs of L = 3 to 80, S = 5 to 44, us in all: dense 217, by labels where they pass 141 with either account; one that
+    // (Static calls, 800 inputs of L = 3 to 80, S = 5 to 44, ms in all: dense 217, by labels where they come through 141 with either account; one that
     // counts what has been taken, too, and grows no labels in the second half gives up as late as in the last layer: the worst
     // call 2.05 times the dense one, now 1.6; most that are left early lose the 80 us of the bounds.)
     auto layer_ns = [](int n, int before) {

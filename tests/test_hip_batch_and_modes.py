@@ -307,9 +307,11 @@ def test_device_memory_short_for_one_buffer_per_layer(golden, monkeypatch):
     assert H.sha(prob.f_out) == rec["f_sha256"]
     assert t.relax_bytes == float(inst.L) * inst.V * inst.S * 17 and not t.fused
     monkeypatch.setenv("GALVATRON_DP_DEVICE_LIMIT_MB", "4")
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "0")     # (by labels it needs 3 MB)
     with pytest.raises(MemoryError):
         _lib.solve_batch([_problem(inst)])
     monkeypatch.delenv("GALVATRON_DP_DEVICE_LIMIT_MB")
+    monkeypatch.delenv("GALVATRON_DP_REDUCE")
     prob = _problem(inst)
     _lib.solve_batch([prob])
     _check_against_golden(prob, rec, "cfg2_small afterwards")

@@ -270,3 +270,25 @@ def test_labels_are_not_given_up_near_the_last_layer(L, S, V, n_keys, kinds, see
     s = _lib.batch_stats_end()
     _check(prob, _want(x, V), f"{L} {S} {V}")
     assert s.executed < 0.01 * s.relaxations
+
+
+@pytest.mark.gpu
+def test_a_call_by_labels_needs_no_dense_buffers(monkeypatch):
+    """A device too full for the dense recurrence, but not for the bounds and the labels: solved by them,
+    below the line of batches and above it; refused where they are switched off, or where the labels are too many."""
+    for name in ("GALVATRON_DP_REDUCE", "GALVATRON_DP_SKIP"):
+        monkeypatch.delenv(name, raising=False)
+    _lib.cache_trim()
+    monkeypatch.setenv("GALVATRON_DP_DEVICE_LIMIT_MB", "4")
+    for L, S, V in ((12, 40, 12000), (8, 40, 200000)):     # 2.3e8 relaxations, 2.6e9; 8 MB and 130 at least
+        x = _instance(np.random.Generator(np.random.PCG64([L, S])), L, S, V, "each", 3)
+        prob = _problem(x, V)
+        assert _solved_by_labels([prob])
+        _check(prob, _want(x, V), f"{L} {S} {V}")
+        monkeypatch.setenv("GALVATRON_DP_REDUCE", "0")
+        with pytest.raises(MemoryError):
+            _lib.solve_batch([_problem(x, V)])
+        monkeypatch.delenv("GALVATRON_DP_REDUCE")
+    x = _instance(np.random.Generator(np.random.PCG64(3)), 40, 24, 200000, "trade", 2)
+    with pytest.raises(MemoryError):
+        _lib.solve_batch([_problem(x, 200000)])
