@@ -83,6 +83,9 @@ size_t env_mb(const char *name, size_t dflt_mb)
     return v <= 0 ? 0 : (size_t)v << 20;
 }
 
+// Device memory that a batch works in at a time.
+size_t arena_budget() { return std::max<size_t>(env_mb("GALVATRON_DP_ARENA_MB", 8192), (size_t)1 << 20); }
+
 void arena_trim(int device /* -1: every device */)
 {
     std::vector<Arena> drop;
@@ -2702,7 +2705,7 @@ struct Reduced {
     double executed = 0;                     // ... and so many candidates were looked at
 };
 
-static constexpr size_t REDUCE_MAX_BYTES = (size_t)4 << 30;   // of device memory for the bounds of a slice (GALVATRON_DP_ARENA_MB if less)
+static constexpr size_t REDUCE_MAX_BYTES = (size_t)4 << 30;   // of device memory for the bounds of a slice or plan (GALVATRON_DP_ARENA_MB if less)
 
 static bool reducible(const gdp_problem *q, double magnitude)
 {
@@ -3238,12 +3241,13 @@ static void take_bounds(int32_t n, const gdp_problem *const *p, const std::vecto
     if (plan->keep_marks || !bounds::allowed(&forced) || (!forced && !bounds_pay(n, p))) return;
     std::unique_ptr<PlanBounds> b(new PlanBounds());
     size_t bytes = 0;
+    const size_t limit = std::min(arena_budget(), REDUCE_MAX_BYTES);
     const int n_lam = bound_multipliers((size_t)n);
     for (int i = 0; i < n; ++i) {
         BoundEntry e;
         if (!bound_entry(p[i], i, magnitude[(size_t)i], e)) return;
         bytes += bound_bytes(p[i], e.h, n_lam);
-        if (bytes > REDUCE_MAX_BYTES) return;
+        if (bytes > limit) return;
         b->es.push_back(std::move(e));
     }
     b->slice.lay_out(p, b->es.data(), n, n_lam);
@@ -3421,7 +3425,7 @@ int gdp_solve_batch(int32_t n, const gdp_problem *const *p, gdp_result *const *r
         // A batch whose cost buffers would take more than GALVATRON_DP_ARENA_MB (default 8192) of device
         // memory is solved in consecutive parts that reuse one allocation: the time to obtain device
         // memory grows with its size, the time to solve a part does not grow faster than its share.
-        const size_t budget = std::max<size_t>(env_mb("GALVATRON_DP_ARENA_MB", 8192), (size_t)1 << 20);
+        const size_t budget = arena_budget();
         std::vector<char> f0_live((size_t)n, 0);
         InitialScan scan;
         if (any_f0) scan.start(n, p, dense_work(n, p));

@@ -292,3 +292,21 @@ def test_a_call_by_labels_needs_no_dense_buffers(monkeypatch):
     x = _instance(np.random.Generator(np.random.PCG64(3)), 40, 24, 200000, "trade", 2)
     with pytest.raises(MemoryError):
         _lib.solve_batch([_problem(x, 200000)])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("limit_mb", [None, 8, 2])
+def test_plans_hold_no_more_for_their_bounds_than_a_batch_works_in(limit_mb, monkeypatch):
+    """4 instances whose bounds take 1 MB each."""
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    if limit_mb is not None:
+        monkeypatch.setenv("GALVATRON_DP_ARENA_MB", str(limit_mb))
+    L, S, V, rng = 12, 24, 3000, np.random.Generator(np.random.PCG64(12))
+    xs = [_instance(rng, L, S, V, "each", 2) for _ in range(4)]
+    probs = [_problem(x, V) for x in xs]
+    with _lib.Plan(probs) as plan:
+        by_labels = plan.run().relax_launches == 0
+        plan.fetch()
+    for x, prob in zip(xs, probs):
+        _check(prob, _want(x, V), f"limit {limit_mb}")
+    assert by_labels == (limit_mb != 2)
