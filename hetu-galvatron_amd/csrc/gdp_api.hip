@@ -3102,10 +3102,18 @@ hipError_t BoundSlice::enqueue(char *dev, hipStream_t stream) const
 // results of instance i; the smaller instance that is left of it where its labels are too many; empty where it is to be
 // solved whole.  The calling thread looks through initial costs while the device works.
 static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &magnitude, BoundEntry *es, int m, int n_lam,
-                        InitialScan &scan, std::vector<std::unique_ptr<Reduced>> &out)
+                        bool forced, InitialScan &scan, std::vector<std::unique_ptr<Reduced>> &out)
 {
     BoundSlice slice;
     slice.lay_out(p, es, m, n_lam);
+    if (m == 1 && !forced) {
+        // What stays of one instance as a smaller one: mostly half of what the whole one takes (labels_pay, 1.2 10^13 relaxations a
+        // second), and a second layout and round trip.  245 calls above the rule's line and 300 others, L = 3 to 128, S = 5 to 88,
+        // ms in all, whole / with the limit of batches / this one: 156 / 82.0 / 77.1 (more than 10 % slower than whole: 9, now
+        // 2), 140 / 95.2 / 91.9.  (0.75 times and nothing: 78.4, 92.9; 0.4 and 60 us 76.8, 92.7; 0.5 and 100 us 76.9, 91.5, one more slower.)
+        const gdp_problem *q = p[es[0].orig];
+        slice.limit_ns = 0.5 * ((double)q->L * q->V * (double)q->S * q->S / 1.2e4 + q->L * (2800.0 + 85.0 * q->S)) + 60e3;
+    }
     // A device or a host that is out of memory solves the instances whole, in the parts that fit; what else may be
     // wrong with the device is found, and reported, there.
     BoundLease lease;
@@ -3219,7 +3227,7 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
             bytes += b;
             ++end;
         }
-        if (end > begin) rc = reduce_slice(p, magnitude, es.data() + begin, (int)(end - begin), n_lam, scan, out);
+        if (end > begin) rc = reduce_slice(p, magnitude, es.data() + begin, (int)(end - begin), n_lam, forced, scan, out);
         begin = std::max(end, begin + 1);
     }
     return rc;

@@ -310,3 +310,25 @@ def test_plans_hold_no_more_for_their_bounds_than_a_batch_works_in(limit_mb, mon
     for x, prob in zip(xs, probs):
         _check(prob, _want(x, V), f"limit {limit_mb}")
     assert by_labels == (limit_mb != 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,S,n_keys,V,seed", [(8, 48, 5, 44101, 203), (10, 52, 3, 35964, 205)])
+def test_single_calls_whose_labels_take_longer_than_what_stays(L, S, n_keys, V, seed, monkeypatch):
+    """Equal layers that trade memory for time: their labels fit (GALVATRON_DP_REDUCE=1 waits for them), but the smaller instance
+    takes less."""
+    for name in ("GALVATRON_DP_REDUCE", "GALVATRON_DP_SKIP"):
+        monkeypatch.delenv(name, raising=False)
+    rng = np.random.Generator(np.random.PCG64(seed))
+    rng.integers(5, 16), rng.integers(20, 56), rng.integers(1, 6), rng.integers(20000, 90000)
+    per = V // L
+    mem = rng.integers(max(1, per // 4), max(2, 3 * per), size=(1, S)).astype(np.int32)
+    intra, inter = 40.0 * per / mem * rng.uniform(0.98, 1.02, size=(1, S)), rng.uniform(0, 0.25, size=(1, S, S))
+    om = [int(V * f) for f in (0.3, 0.1, 0.0, 0.45, 0.2)[:n_keys]]
+    x = np.repeat(mem, L, 0), np.repeat(intra, L, 0), np.repeat(inter, L, 0), om, [k / 3 for k in range(n_keys)]
+    prob, want = _problem(x, V), _want(x, V)
+    assert not _solved_by_labels([prob])
+    _check(prob, want, f"{L} {S}")
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    assert _solved_by_labels([prob])
+    _check(prob, want, f"{L} {S} by labels")
