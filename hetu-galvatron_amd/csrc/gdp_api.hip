@@ -2939,7 +2939,8 @@ struct BoundLease {
 // The bounds of some instances, and behind them the DP over what stays, in one allocation and one set of launches.
 struct BoundSlice {
     BoundEntry *es = nullptr;
-    int m = 0, n_lam = 0, max_LS = 0, max_S = 0, max_K = 0;
+    int m = 0, n_lam = 0, max_L = 0, max_LS = 0, max_S = 0, max_K = 0;
+    double relaxations = 0;            // of the whole instances
     double limit_ns = 0;               // of the DP over what stays
     int64_t layers = 0, changes = 0;   // ... and how often a layer has another matrix than the one before
     std::vector<int2> pairs;
@@ -2961,8 +2962,6 @@ void BoundSlice::lay_out(const gdp_problem *const *p, BoundEntry *entries, int c
     es = entries;
     m = count;
     n_lam = multipliers;
-    double relaxations = 0;
-    int max_L = 0;
     size_t at = 0;
     auto place = [&](size_t bytes) { const size_t o = at; at = align_up(at + bytes, 256); return o; };
     for (int i = 0; i < m; ++i) {   // the stages of one fit and the tasks of one sweep share their matrices
@@ -3106,14 +3105,13 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
 {
     BoundSlice slice;
     slice.lay_out(p, es, m, n_lam);
-    if (m == 1 && !forced) {
-        // What stays of one instance as a smaller one: mostly half of what the whole one takes (labels_pay, 1.2 10^13 relaxations a
-        // second), and a second layout and round trip.  245 calls above the rule's line and 300 others, L = 3 to 128, S = 5 to 88,
-        // ms in all, whole / with the limit of batches / this one: 156 / 82.0 / 77.1 (more than 10 % slower than whole: 9, now
-        // 2), 140 / 95.2 / 91.9.  (0.75 times and nothing: 78.4, 92.9; 0.4 and 60 us 76.8, 92.7; 0.5 and 100 us 76.9, 91.5, one more slower.)
-        const gdp_problem *q = p[es[0].orig];
-        slice.limit_ns = 0.5 * ((double)q->L * q->V * (double)q->S * q->S / 1.2e4 + q->L * (2800.0 + 85.0 * q->S)) + 60e3;
-    }
+    // What stays as smaller instances takes about half of what the whole ones take (labels_pay, 1.2 10^13 relaxations a second),
+    // and a second layout and round trip.  ms in all, whole / with limit_ns as it is / with this one:
+    //   245 calls above the rule's line, L = 3 to 128, S = 5 to 88  156 / 82.0 / 77.1 (more than 10 % slower than whole: 9, now 2)
+    //   300 calls on either side of it  140 / 95.2 / 91.9
+    //   255 batches of 2 to 128 that the rule takes  484 / 221 / 216 (10, now 6)
+    // (of single calls 0.75 times and nothing: 78.4, 92.9; 0.4 and 60 us 76.8, 92.7; 0.5 and 100 us 76.9, 91.5, one more of them slower.)
+    if (!forced) slice.limit_ns = 0.5 * (slice.relaxations / 1.2e4 + slice.max_L * (2800.0 + 85.0 * slice.max_S)) + (m == 1 ? 60e3 : 100e3);
     // A device or a host that is out of memory solves the instances whole, in the parts that fit; what else may be
     // wrong with the device is found, and reported, there.
     BoundLease lease;
