@@ -55,11 +55,11 @@ def _solved_by_labels(probs):
 
 
 # Labels of the layers that have the most: 1 to 64 (a turn), to 128 and 192 (lanes share the keys), more (buckets), more
-# than fit (the smaller instance, or the whole one)
+# than fit (the smaller instance, or the whole one); a set: with so many keys they fit
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind,L,S,V,labels", [("each", 9, 12, 6000, True), ("narrow", 20, 16, 9000, True), ("trade", 6, 7, 3000, True),
-                                               ("trade", 10, 8, 6000, True), ("trade", 16, 9, 9000, True), ("trade", 24, 24, 12000, None),
-                                               ("each", 40, 64, 9000, True), ("each", 64, 17, 9000, True), ("narrow", 512, 4, 20000, None)])
+                                               ("trade", 10, 8, 6000, True), ("trade", 16, 9, 9000, True), ("trade", 24, 24, 12000, {1, 5}),
+                                               ("each", 40, 64, 9000, True), ("each", 64, 17, 9000, True), ("narrow", 512, 4, 20000, False)])
 @pytest.mark.parametrize("n_keys", [1, 2, 3, 5, 8])
 def test_batches_by_labels(kind, L, S, V, labels, n_keys, monkeypatch):
     monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
@@ -67,7 +67,7 @@ def test_batches_by_labels(kind, L, S, V, labels, n_keys, monkeypatch):
     prob = _problem(x, V)
     by_labels = _solved_by_labels([prob])
     _check(prob, _want(x, V), f"{kind} {L} {S} {V}")
-    assert labels is None or by_labels == labels
+    assert by_labels == (n_keys in labels if isinstance(labels, set) else labels)
 
 
 @pytest.mark.gpu
@@ -82,7 +82,7 @@ def test_passes_over_one_matrix_some_and_many(S, monkeypatch):
         xs.append(x)
         probs.append(_problem(x, V))
     for x, prob in zip(xs, probs):
-        _lib.solve_batch([prob])
+        assert _solved_by_labels([prob])     # (bounds of no use leave too many of them)
         _check(prob, _want(x, V), f"S {S}")
 
 
@@ -118,15 +118,22 @@ def test_plans_by_labels(kind, monkeypatch):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("kind,L,S,V,n_keys", [("each", 2, 3, 200, 2), ("each", 5, 8, 3000, 3), ("each", 5, 11, 3000, 3), ("each", 30, 30, 5000, 8),
-                                               ("trade", 10, 8, 6000, 2), ("trade", 30, 30, 9000, 1), ("narrow", 21, 16, 6000, 5)])
-def test_static_calls_by_labels(kind, L, S, V, n_keys):
+@pytest.mark.parametrize("kind,L,S,V,n_keys,labels", [("each", 2, 3, 200, 2, False), ("each", 5, 8, 3000, 3, False), ("each", 5, 11, 3000, 3, True),
+                                                      ("each", 30, 30, 5000, 8, True), ("trade", 10, 8, 6000, 2, True), ("trade", 30, 30, 9000, 1, True),
+                                                      ("narrow", 21, 16, 6000, 5, False)])
+def test_static_calls_by_labels(kind, L, S, V, n_keys, labels):
+    """labels: False below the 36 us of layer launches from which bounds are taken, and where the labels are too many."""
+    if "GALVATRON_DP_REDUCE" in os.environ or "GALVATRON_DP_SKIP" in os.environ:
+        pytest.skip("the environment presets the rule")
     x = _instance(np.random.Generator(np.random.PCG64([L, S])), L, S, V, kind, n_keys)
     prob = _problem(x, V)
     for _ in range(2):
         prob.total[:], prob.remaining[:], prob.res[:] = 0, 0, 0
+        _lib.batch_stats_begin()
         _lib.solve_static(prob)
+        s = _lib.batch_stats_end()
         _check(prob, _want(x, V), f"{kind} {L} {S}")
+        assert (s.executed < 0.01 * s.relaxations) == labels
 
 
 @pytest.mark.parametrize("source", ["gdp_bounds.hip", "gdp_frontier.hip"])
