@@ -297,15 +297,15 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
     // An instance whose other layers would take longer than the dense recurrence (`limit`) is left to that one; what its
     // labels have taken by then does not come back either way, so that only what is ahead counts.  Ahead, as from layer 2 on, in the
     // first half: of identical layers that trade memory for time the labels of a layer grow towards L / 2 about as they do
-    // at the start, and are half of what that comes to in the mean.  In the second half they become fewer again.  Where
-    // layers differ the labels may also grow late: then what the layers so far took tells.
-    // (Static calls, 800 inputs of L = 3 to 80, S = 5 to 44, ms in all: dense 217, by labels where they come through 141 with either account; one that
-    // counts what has been taken, too, and grows no labels in the second half gives up as late as in the last layer: the worst
-    // call 2.05 times the dense one, now 1.6; most that are left early lose the 80 us of the bounds.)
+    // at the start, and are half of what that comes to in the mean.  In the second half they become fewer again.
+    // (Static calls, 2000 inputs of L = 3 to 80, S = 5 to 44, ms in all: dense 521, by labels where they come through 335; 114 take more than 1.1
+    // times what they take dense, mostly by the 80 us of bounds whose labels are left at layer 2 or 3, the worst two 1.6 and 2.1.  An account that counts what has been taken, too, and nothing ahead in the second half gives up as late as in the last layer.
+    // Growth in the second half is no better guide: it takes layers of two kinds in turn for growing ones.)
     auto layer_ns = [](int n, int before) {
         return (before > SORTED_FROM ? 3000 : 900) + ((n + WORKERS - 1) / WORKERS) * ((before + 127) / 128) * (600 + 200 * KEYS);
     };
     auto hopeless = [&](int ns, int l, int n, int labels) {
+        if (labels <= 64) return false;   // (less than a dense layer takes, and these tests lie in the chain)
         const int ahead = L - 1 - l;
         if ((double)ns * (double)ahead > limit * (double)(l + 1)) return true;
         if (l >= L / 2) return (double)ahead * layer_ns(n, labels / 2) > limit;
