@@ -3109,9 +3109,11 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
     // and a second layout and round trip.  ms in all, whole / with limit_ns as it is / with this one:
     //   245 calls above the rule's line, L = 3 to 128, S = 5 to 88  156 / 82.0 / 77.1 (more than 10 % slower than whole: 9, now 2)
     //   300 calls on either side of it  140 / 95.2 / 91.9
-    //   255 batches of 2 to 128 that the rule takes  484 / 221 / 216 (10, now 6)
+    //   201 batches of 2 to 128 that the rule takes  379 / 171 / 169
+    //   120 fits of up to 15 stages  92.1 / 66.9 / 65.4 (none more than 3 % slower than whole; with 100 us 64.9, but 3 of them 1.2 to
+    //   1.3 times the former limit's)
     // (of single calls 0.75 times and nothing: 78.4, 92.9; 0.4 and 60 us 76.8, 92.7; 0.5 and 100 us 76.9, 91.5, one more of them slower.)
-    if (!forced) slice.limit_ns = 0.5 * (slice.relaxations / 1.2e4 + slice.max_L * (2800.0 + 85.0 * slice.max_S)) + (m == 1 ? 60e3 : 100e3);
+    if (!forced) slice.limit_ns = 0.5 * (slice.relaxations / 1.2e4 + slice.max_L * (2800.0 + 85.0 * slice.max_S)) + (m == 1 ? 60e3 : 200e3);
     // A device or a host that is out of memory solves the instances whole, in the parts that fit; what else may be
     // wrong with the device is found, and reported, there.
     BoundLease lease;
