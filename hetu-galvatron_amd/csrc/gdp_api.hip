@@ -2749,25 +2749,28 @@ static double undominated(int32_t n, const gdp_problem *const *p)
     return share / m;
 }
 
-// Whether the bounds of a batch are worth their time (GALVATRON_DP_REDUCE=1 takes them for every instance that has the
+// Whether the bounds of a batch or plan are worth their time (GALVATRON_DP_REDUCE=1 takes them for every instance that has the
 // form, =0 for none).  What they can save is the dense recurrence, 10^13 relaxations a second; where the instances
 // have several S it runs in launches of their own, one after the other, which cost as much again up to 0.1 ms each, and
-// what is left of them mostly runs in one.  They cost
-// * a round trip, 0.1 ms, and two chains of max L steps -- the passes, then the DP on what is left --, whatever V is:
-//   5 us a step, 25 us where a thread of a pass has 16 elements (S > 88: 16 us a step of the passes instead of 1.65);
-// * from 1024 passes (2 per multiplier and instance) on the device's time for all steps instead, 1.5 and 13 us;
-// * in batches the host's: layout, matrices of what stays and their upload, 3 ns per transition cost times the share of
-//   strategies that stay at least (undominated); the arrays of a single instance stay in its caches.
-// How much is left is not known before: random costs leave a tenth, 128 equal layers four fifths.  So the line lies
-// where the calls on it gain on average.  Of 4500 calls tried on either side of it 1500 gain, to 0.55 on average, and 250 lose
-// more than 8 % -- those that are not thinned out, mostly a fifth, up to a half, single ones more.  Some of them, ms whole / with bounds, random costs; costs that follow a layout, all layers alike:
-//   L = 24, S = 64   1.0e9 0.25 / 0.26; 0.24 / 0.30    2.0e9 0.38 / 0.29; 0.35 / 0.34    1.0e10 0.92 / 0.33; 0.83 / 0.63
-//   L = 64, S = 64   2.0e9 0.62 / 0.56; 0.57 / 0.67    4.0e9 0.81 / 0.58; 0.80 / 0.93    1.0e10 1.37 / 0.57; 1.43 / 1.00
-//   L = 256, S = 32  4.0e9 1.66 / 1.50; 1.59 / 2.03    1.0e10 2.64 / 1.53; 2.56 / 2.99
-//   L = 32, S = 128  4.0e9 0.90 / 0.95; 0.78 / 1.26    1.0e10 1.51 / 0.96; 1.56 / 1.81
-//   32 x L = 14, S = 40  V = 8000 0.75 / 0.62; 0.76 / 1.08    V = 30000 2.11 / 0.82; 2.23 / 1.73
-//   64 x L = 28, S = 64  V = 8000 5.0 / 2.7; 5.3 / 8.0        16 x L = 28, S = 40, V = 30000 2.02 / 1.19; 2.05 / 2.07
-//   15 stages of a fit, L = 8 to 1, S = 60 to 8, V = 16583 (6.5e8) -; 0.44 / 0.37
+// what is left of them mostly runs in one.  The line asks for 0.2 ms of that at least, and for
+// * 5 us per layer, 25 us above 88 strategies;
+// * from 1024 passes (2 per multiplier and instance) on 1.5 and 13 us per 1024 of their steps instead;
+// * in batches, for what the host does, 3 ns per transition cost times the share of strategies that no other one dominates.
+// That is more than bounds take: a step of a pass takes 0.9 us (S = 64), a layer of the labels 1 to 9, the round trip 0.1 ms.
+// How much is left is not known before -- random costs leave few labels, equal layers that trade memory for time more than fit --, and
+// where it is much, all of that comes on top of a smaller instance that takes half to four fifths of the whole one.  Of 245 single
+// calls that this line or that of labels_pay took 2 were more than 1.1 times as slow as whole (1.13), of 201 batches 5 (1.33), of 120
+// fits none.  On the far side random costs would gain, most others lose.  ms whole / with bounds, means of 5 (batches: 2) inputs, random
+// costs, layers of their own; costs that follow a layout, all layers alike (*: taken):
+//   L = 24, S = 64   1.0e9 0.27 / 0.19; 0.27 / 0.31    2.0e9 * 0.33 / 0.19; 0.33 / 0.30     1.0e10 * 0.93 / 0.19; 0.76 / 0.47
+//   L = 64, S = 64   2.0e9 0.61 / 0.42; 0.55 / 0.60    4.0e9 * 0.81 / 0.42; 0.77 / 0.69     1.0e10 * 1.39 / 0.44; 1.35 / 0.81
+//   L = 256, S = 32  4.0e9 1.63 / 1.42; 1.55 / 1.63    1.0e10 2.56 / 1.86; 2.45 / 2.17      2.0e10 * 3.33 / 1.70; 3.18 / 3.04
+//   L = 32, S = 128  1.0e9 0.72 / 0.56; 0.58 / 0.57    4.0e9 0.91 / 0.53; 0.81 / 0.60       8.0e9 1.28 / 0.53; 1.21 / 0.61
+//   8 x L = 28, S = 40   V = 8000 * 0.73 / 0.43, not taken 0.71 / 1.03    V = 16000 * 1.22 / 0.43; 0.83 / 1.05
+//   16 x L = 28, S = 40, V = 30000 * 2.60 / 0.73; 2.53 / 2.02             16 x L = 20, S = 104, V = 6000 * 6.00 / 3.88; 3.64 / 3.72
+//   32 x L = 14, S = 40  V = 8000 * 1.33 / 0.71, not taken 1.08 / 1.13    V = 30000 * 2.79 / 0.71; 2.61 / 1.29
+//   64 x L = 28, S = 64, V = 8000 * 24.6 / 18.5; 9.3 / 10.6
+// (Single calls are taken earlier where labels_pay says so.)
 static bool bounds_pay(int32_t n, const gdp_problem *const *p)
 {
     constexpr double RATE = 1e13, FLOOR = 0.2e-3, STEP = 5e-6, STEP_16 = 25e-6, BUSY = 1.5e-6, BUSY_16 = 13e-6, ENTRY = 3e-9, GROUP = 0.1e-3;
@@ -2798,12 +2801,13 @@ static bool bounds_pay(int32_t n, const gdp_problem *const *p)
 // trip of 55 us + L * (2.3 + 0.06 S) us, host included, against 60 us + L * (2.8 + 0.085 S) us of the launch schemes and
 // their relaxations.  How many labels there will be is not known before; what tells it best is how many strategies of a
 // layer no other one dominates, times the layers (4 of them are looked at), unless layers are alike: then whatever trades
-// memory for time does so in every one.  Whole / by labels, us, means of 5 inputs each:
-//   layers of their own, random costs (2 to 8 of S undominated)   L = 6, S = 24, 3e7 81 / 77    L = 12, S = 24, 1e8 108 / 94
+// memory for time does so in every one.  Whole / by labels, us, means of 5 inputs each (*: taken):
+//   layers of their own, random costs (2 to 8 of S undominated)   * L = 6, S = 24, 3e7 81 / 77    * L = 12, S = 24, 1e8 108 / 94
 //     L = 28, S = 40, 3e8 221 / 168    L = 28, S = 88, 2e8 419 / 310    L = 60, S = 20, 2e8 304 / 240    L = 128, S = 8, 2e8 502 / 497
+//     (these four have more than 80 undominated strategies over all layers)
 //   ... that follow a layout (5 to 24)  L = 8, S = 44, 2e8 113 / 103   L = 28, S = 44, 2e8 229 / 263   L = 60, S = 20, 2e8 305 / 369
-//   layers alike, a layout  L = 6, S = 40, 1e8 93 / 97; 3e8 108 / 96   L = 12, S = 40, 3e8 136 / 144; 7e8 165 / 142
-//     L = 28, S = 40, 7e8 232 / 278; 1.5e9 312 / 259   L = 60, S = 24, 7e8 330 / 389; 1.5e9 514 / 406; S = 40, 1.5e9 491 / 495
+//   layers alike, a layout  L = 6, S = 40, 1e8 93 / 97; * 3e8 108 / 96   L = 12, S = 40, 3e8 136 / 144; * 7e8 165 / 142
+//     L = 28, S = 40, 7e8 232 / 278; * 1.5e9 312 / 259   L = 60, S = 24, 7e8 330 / 389; 1.5e9 514 / 406; S = 40, 1.5e9 491 / 495
 // So few of a layer and layers of their own take them from 3e7 relaxations on -- below 80 over all layers none of 150 inputs lost more
 // than 8 %, from 84 on some do, up to a third --, everything else from 5e7 a layer, as in bounds_pay.  Initial
 // costs are looked through while the device works; where that takes longer than the chain of layers nothing is gained.

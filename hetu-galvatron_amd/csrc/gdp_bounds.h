@@ -20,7 +20,7 @@ constexpr int GDP_BOUND_MEM = 1 << 30;    // memory sums saturate here, above ev
 constexpr int GDP_FRONTIER_KEPT = 8192;   // strategies that stay, over all layers of an instance
 constexpr int GDP_FRONTIER_LABELS = 1024; // room in memory for so many labels, and transitions, per layer on average
 
-// What gdp_launch_frontier finds for an instance; the strategies lie in GdpBoundInst.res.
+// What bounds::launch_labels finds for an instance; the strategies lie in GdpBoundInst.res.
 struct GdpFrontierOut {
     double total[GDP_BOUND_MAX_KEY];      // +inf: the key has no solution
     double executed;                      // candidates looked at
@@ -57,7 +57,7 @@ struct GdpBoundInst {
     GdpFrontierOut *out;
     int32_t *res;            // [K][L]
     double magnitude;        // sum over the layers of the largest finite |intra| and |inter|
-    double limit;            // ns that the DP over what stays may take, by its own account
+    double limit;            // ns that the layers ahead of the DP over what stays may take, by its own account
     int32_t L, V, S, K, T, n_hist, n_hist_turns;
 };
 

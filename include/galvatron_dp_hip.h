@@ -173,8 +173,10 @@ int gdp_solve_static(const gdp_problem *p, gdp_result *r);
  *   create  -- validate + allocate + copy inputs to the device
  *   run     -- layer kernels + on-device backtrack; timing may be NULL.
  *              timing_mode 0: none, 1: total_ms only, 2: also per-launch relaxation events.
- *              Where it pays (as in gdp_solve_batch), bounds and the DP over what they leave run instead of the layer
- *              kernels, relax_launches is 0 then.  Not in mode 2, after gdp_plan_set_option or with GDP_COMPUTE_ALL.
+ *              Where it pays (by the rule that gdp_solve_batch has for batches, also for a single instance, and if every
+ *              instance has the form), bounds and the DP over what they leave run instead of the layer kernels,
+ *              relax_launches is 0 then; where the labels are too many the layer kernels follow, in that run and
+ *              all later ones.  Not in mode 2, after gdp_plan_set_option or with GDP_COMPUTE_ALL.
  *   fetch   -- copy results of the last run to the caller's arrays
  *   destroy -- release everything                                              */
 int gdp_plan_create(int32_t n, const gdp_problem *const *p, gdp_plan **out);

@@ -127,8 +127,8 @@ def test_bounds_take_part_up_to_their_limits(L, S, V, keys, kind, taken, monkeyp
     assert np.array_equal(probs[0].remaining, probs[1].remaining) and np.array_equal(probs[0].res, probs[1].res)
 
 
-# instances, L, S, V: on the far side of each term of the rule -- too little work, chains of too many steps, steps of
-# 16 elements, too many transition costs that stay in a batch -- and on the near one
+# instances, L, S, V: on the far side of each term of the rule -- too little work, too many layers, more than 88
+# strategies, too many transition costs that stay in a batch -- and on the near one
 @pytest.mark.parametrize("shape,kind,bounds", [
     ((1, 24, 40, 30000), "each", False), ((1, 16, 64, 40000), "each", True), ((1, 256, 16, 33000), "each", False),
     ((1, 40, 64, 30000), "each", True), ((1, 24, 96, 12000), "each", False), ((1, 4, 96, 80000), "each", True),
@@ -201,7 +201,7 @@ def test_initial_costs_that_are_not_zeros(monkeypatch):
 
 @pytest.mark.parametrize("strategies", [(22,), (23, 32), (33, 44, 9), (45, 8)])
 def test_batches_with_narrow_passes(strategies, monkeypatch):
-    """From 17 instances on a pass has 512 threads where 4 elements per thread are enough (up to 44 strategies)."""
+    """18 instances of up to 9, 22, 32, 44 and 45 strategies in one set of launches: passes as wide as the widest of them needs."""
     monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
     rng = np.random.Generator(np.random.PCG64([7, *strategies]))
     V, xs = 400, []
