@@ -2716,37 +2716,31 @@ static bool reducible(const gdp_problem *q, double magnitude)
     return true;
 }
 
-static int bound_multipliers(size_t instances) { return instances <= 32 ? GDP_BOUND_MAX_LAM : GDP_BOUND_MAX_LAM / 2; }
+// (GDP_BOUND_MAX_LAM for a single instance that many labels are to be expected of: bounds::key_multipliers)
+static int bound_multipliers(size_t instances) { return instances <= 32 ? 64 : 32; }
 
-// Share of the strategies of a layer that are cheaper in time than every one that needs no more memory: most others
-// go.  From one layer each of at most 8 instances (batches of 2 to 1000, share of the relaxations left: random costs
-// 0.15 on average and 0.06; costs where memory is traded for time 0.44 and 0.40).
-static double undominated(const gdp_problem *q, int32_t layer, std::vector<std::pair<int32_t, double>> &sorted)
-{
-    const size_t row = (size_t)layer * q->S;
-    sorted.clear();
-    for (int s = 0; s < q->S; ++s) sorted.emplace_back(q->mem[row + s], q->intra[row + s]);
-    std::sort(sorted.begin(), sorted.end());
-    double least = INFINITY;
-    int stay = 0;
-    for (const auto &s : sorted) {
-        stay += s.first < q->V && s.second < least;
-        least = s.first < q->V ? std::min(least, s.second) : least;
-    }
-    return (double)stay / q->S;
-}
-
+// Share of the strategies that no other one dominates: most others go.  From one layer each of at most 8 instances (batches of 2 to
+// 1000, share of the relaxations left: random costs 0.15 on average and 0.06; costs where memory is traded for time 0.44 and 0.40).
 static double undominated(int32_t n, const gdp_problem *const *p)
 {
     constexpr int32_t LOOKED_AT = 8;
-    std::vector<std::pair<int32_t, double>> sorted;
+    if (n == 1) return bounds::undominated(p[0]);
     double share = 0;
     const int32_t m = std::min(n, LOOKED_AT);
     for (int32_t k = 0; k < m; ++k) {
         const gdp_problem *q = p[(int64_t)n * k / m];
-        share += undominated(q, q->L / 2, sorted);
+        share += bounds::undominated(q, q->L / 2);
     }
     return share / m;
+}
+
+// Whether the keys of these instances have a workgroup each (gdp_key_labels.hip).  Not where next to no strategy is dominated by another:
+// labels are many either way then, and most such calls are given up as they were.
+static bool keys_alone(int32_t n, const gdp_problem *const *p)
+{
+    for (int32_t i = 0; i < n; ++i)
+        if (p[i]->L > GDP_KEY_LABELS_MAX_L) return false;
+    return undominated(n, p) <= GDP_KEY_LABELS_MOST;
 }
 
 // Whether the bounds of a batch or plan are worth their time (GALVATRON_DP_REDUCE=1 takes them for every instance that has the
@@ -2825,11 +2819,7 @@ static bool labels_pay(const gdp_problem *q, size_t scanned)
         alike += memcmp(q->mem + at, q->mem + before, sizeof(int32_t) * q->S) == 0 && memcmp(q->intra + at, q->intra + before, sizeof(double) * q->S) == 0;
     }
     if (alike * 4 > q->L) return false;
-    std::vector<std::pair<int32_t, double>> sorted;
-    const int m = std::min(q->L, 4);
-    double share = 0;
-    for (int k = 0; k < m; ++k) share += undominated(q, (int)((int64_t)q->L * (2 * k + 1) / (2 * m)), sorted);
-    return share / m * q->S * q->L <= FEW;
+    return bounds::undominated(q) * q->S * q->L <= FEW;
 }
 
 // The smaller instance of q, given what stays ([L][S]); false where it would not be a good deal smaller.
@@ -2910,16 +2900,17 @@ struct BoundEntry {
     HostInst h;
     std::vector<int64_t> budget;
     size_t off_mem, off_intra, off_inter, off_index, off_lam, off_budget, off_inter_f, off_inter_t, off_P, off_Q, off_P_mem, off_Q_mem, off_end,
-        off_window, off_ub, off_keep, off_other_time, off_out, off_res, off_hist, off_hist_mem, off_hist_turns, off_hist_intra;
+        off_best, off_ub, off_keep, off_marks, off_other_time, off_out, off_res, off_hist, off_hist_mem, off_hist_turns, off_hist_intra;
 };
 
 // Device memory that the bounds of an instance take at most, with matrices of its own.
-static size_t bound_bytes(const gdp_problem *q, const HostInst &h, int n_lam)
+static size_t bound_bytes(const gdp_problem *q, const HostInst &h, int n_lam, bool alone)
 {
     const size_t L = (size_t)q->L, LS = L * q->S, T = (size_t)h.n_inter, K = (size_t)q->n_key, NL = (size_t)n_lam;
-    constexpr size_t ARRAYS = 28;   // aligned to 256 bytes each
+    constexpr size_t ARRAYS = 29;   // aligned to 256 bytes each
     return sizeof(GdpBoundInst) + T * sizeof(int2) + 13 * LS + 4 * L + 28 * K + 24 * T * (size_t)q->S * q->S +
-           NL * (16 + 24 * LS) + sizeof(GdpFrontierOut) + 4 * K * L + 24 * L * GDP_FRONTIER_LABELS + 12 * GDP_FRONTIER_KEPT + 256 * ARRAYS;
+           NL * (16 + 24 * LS) + sizeof(GdpFrontierOut) + 20 * K * L +
+           (alone ? 16 * K * L * GDP_KEY_LABELS : 24 * L * GDP_FRONTIER_LABELS + 12 * GDP_FRONTIER_KEPT) + 256 * ARRAYS;
 }
 
 // What the bounds of a slice work with; given back on every way out, the stream idle.
@@ -2943,7 +2934,8 @@ struct BoundLease {
 // The bounds of some instances, and behind them the DP over what stays, in one allocation and one set of launches.
 struct BoundSlice {
     BoundEntry *es = nullptr;
-    int m = 0, n_lam = 0, max_L = 0, max_LS = 0, max_S = 0, max_K = 0;
+    int m = 0, n_lam = 0, max_L = 0, max_LS = 0, max_rows = 0, max_S = 0, max_K = 0;
+    bool alone = false;                // a workgroup per key
     double relaxations = 0;            // of the whole instances
     double limit_ns = 0;               // of the DP over what stays
     int64_t layers = 0, changes = 0;   // ... and how often a layer has another matrix than the one before
@@ -2951,20 +2943,22 @@ struct BoundSlice {
     // [0, up_bytes): what is uploaded; the results after it; what stays; the rest stays on the device
     size_t off_inst = 0, off_pairs = 0, up_bytes = 0, back_bytes = 0, keep_begin = 0, keep_bytes = 0, bytes = 0;
 
-    void lay_out(const gdp_problem *const *p, BoundEntry *entries, int count, int multipliers);
+    void lay_out(const gdp_problem *const *p, BoundEntry *entries, int count, int multipliers, bool key_alone);
     void fill(const gdp_problem *const *p, const std::vector<double> &magnitude, char *up, char *dev) const;
     hipError_t enqueue(char *dev, hipStream_t stream) const;
     const GdpFrontierOut &out_of(const char *back, int j) const
     {
         return *reinterpret_cast<const GdpFrontierOut *>(back + (es[j].off_out - up_bytes));
     }
+    size_t labels_of(const gdp_problem *q) const { return (size_t)q->L * (alone ? GDP_KEY_LABELS : GDP_FRONTIER_LABELS); }
     const int32_t *res_of(const char *back, int j) const { return reinterpret_cast<const int32_t *>(back + (es[j].off_res - up_bytes)); }
 };
 
-void BoundSlice::lay_out(const gdp_problem *const *p, BoundEntry *entries, int count, int multipliers)
+void BoundSlice::lay_out(const gdp_problem *const *p, BoundEntry *entries, int count, int multipliers, bool key_alone)
 {
     es = entries;
     m = count;
+    alone = key_alone;
     n_lam = multipliers;
     size_t at = 0;
     auto place = [&](size_t bytes) { const size_t o = at; at = align_up(at + bytes, 256); return o; };
@@ -3000,6 +2994,7 @@ void BoundSlice::lay_out(const gdp_problem *const *p, BoundEntry *entries, int c
         max_L = std::max(max_L, q->L);
         for (int l = 1; l < q->L; ++l) changes += e.h.matrix(q, l) != e.h.matrix(q, l - 1);
         max_LS = std::max(max_LS, (int)LS);
+        max_rows = std::max(max_rows, q->L * ((q->S + 63) / 64));
         max_S = std::max(max_S, q->S);
         max_K = std::max(max_K, q->n_key);
     }
@@ -3026,18 +3021,19 @@ void BoundSlice::lay_out(const gdp_problem *const *p, BoundEntry *entries, int c
             e.off_inter_f = place(8 * (size_t)e.h.n_inter * q->S * q->S);
             e.off_inter_t = place(8 * (size_t)e.h.n_inter * q->S * q->S);
         }
+        e.off_marks = place(16 * (size_t)q->n_key * q->L);
         e.off_P = place(8 * LS * (size_t)n_lam);
         e.off_Q = place(8 * LS * (size_t)n_lam);
         e.off_P_mem = place(4 * LS * (size_t)n_lam);
         e.off_Q_mem = place(4 * LS * (size_t)n_lam);
         e.off_end = place(8 * (size_t)n_lam);
-        e.off_window = place(4 * (size_t)q->n_key);
+        e.off_best = place(4 * (size_t)q->n_key);
         e.off_ub = place(8 * (size_t)q->n_key);
-        const size_t labels = (size_t)q->L * GDP_FRONTIER_LABELS;
+        const size_t keys = alone ? (size_t)q->n_key : 1, labels = keys * labels_of(q);
         e.off_hist = place(sizeof(GdpFrontierLabel) * labels);
-        e.off_hist_turns = place(8 * labels);
-        e.off_hist_mem = place(4 * GDP_FRONTIER_KEPT);
-        e.off_hist_intra = place(8 * GDP_FRONTIER_KEPT);
+        e.off_hist_turns = place(alone ? 0 : 8 * labels);
+        e.off_hist_mem = place(alone ? 0 : 4 * GDP_FRONTIER_KEPT);
+        e.off_hist_intra = place(alone ? 0 : 8 * GDP_FRONTIER_KEPT);
     }
     bytes = at;
 }
@@ -3071,8 +3067,9 @@ void BoundSlice::fill(const gdp_problem *const *p, const std::vector<double> &ma
         b.Q_mem = reinterpret_cast<uint32_t *>(dev + e.off_Q_mem);
         b.end = reinterpret_cast<double *>(dev + e.off_end);
         b.ub = reinterpret_cast<unsigned long long *>(dev + e.off_ub);
-        b.window = reinterpret_cast<int32_t *>(dev + e.off_window);
+        b.best = reinterpret_cast<int32_t *>(dev + e.off_best);
         b.keep = reinterpret_cast<uint8_t *>(dev + e.off_keep);
+        b.marks = reinterpret_cast<unsigned long long *>(dev + e.off_marks);
         b.other_time = reinterpret_cast<const double *>(dev + e.off_other_time);
         b.hist = reinterpret_cast<GdpFrontierLabel *>(dev + e.off_hist);
         b.hist_mem = reinterpret_cast<int32_t *>(dev + e.off_hist_mem);
@@ -3080,7 +3077,8 @@ void BoundSlice::fill(const gdp_problem *const *p, const std::vector<double> &ma
         b.hist_intra = reinterpret_cast<double *>(dev + e.off_hist_intra);
         b.out = reinterpret_cast<GdpFrontierOut *>(dev + e.off_out);
         b.res = reinterpret_cast<int32_t *>(dev + e.off_res);
-        b.n_hist = b.n_hist_turns = q->L * GDP_FRONTIER_LABELS;
+        b.n_hist = b.n_hist_turns = (int32_t)labels_of(q);
+        b.n_lam = n_lam;
         b.magnitude = magnitude[(size_t)e.orig];
         b.limit = limit_ns;
         b.L = q->L;
@@ -3096,19 +3094,20 @@ void BoundSlice::fill(const gdp_problem *const *p, const std::vector<double> &ma
 hipError_t BoundSlice::enqueue(char *dev, hipStream_t stream) const
 {
     const GdpBoundInst *inst = reinterpret_cast<const GdpBoundInst *>(dev + off_inst);
-    const hipError_t e = bounds::launch(inst, m, n_lam, max_LS, max_S, max_K, changes * 4 <= layers, reinterpret_cast<const int2 *>(dev + off_pairs),
+    const hipError_t e = bounds::launch(inst, m, n_lam, max_LS, max_rows, max_S, max_K, changes * 4 <= layers, reinterpret_cast<const int2 *>(dev + off_pairs),
                                            (int)pairs.size(), stream);
-    return e == hipSuccess ? bounds::launch_labels(inst, m, max_K, stream) : e;
+    if (e != hipSuccess) return e;
+    return alone ? bounds::launch_key_labels(inst, m, max_K, stream) : bounds::launch_labels(inst, m, max_K, stream);
 }
 
 // Bounds of the instances of one slice in one set of launches, and behind them the DP over what stays.  out[i]: the
 // results of instance i; the smaller instance that is left of it where its labels are too many; empty where it is to be
 // solved whole.  The calling thread looks through initial costs while the device works.
 static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &magnitude, BoundEntry *es, int m, int n_lam,
-                        bool forced, InitialScan &scan, std::vector<std::unique_ptr<Reduced>> &out)
+                        bool alone, bool forced, InitialScan &scan, std::vector<std::unique_ptr<Reduced>> &out)
 {
     BoundSlice slice;
-    slice.lay_out(p, es, m, n_lam);
+    slice.lay_out(p, es, m, n_lam, alone);
     // What stays as smaller instances takes about half of what the whole ones take (labels_pay, 1.2 10^13 relaxations a second),
     // and a second layout and round trip.  ms in all, whole / with limit_ns as it is / with this one:
     //   245 calls above the rule's line, L = 3 to 128, S = 5 to 88  156 / 82.0 / 77.1 (more than 10 % slower than whole: 9, now 2)
@@ -3151,7 +3150,7 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
     if (err == hipSuccess) err = es2;
     std::vector<char> keep;
     for (int j = 0; j < m && err == hipSuccess && keep.empty(); ++j)
-        if (slice.out_of(lane.back, j).status > 1) {
+        if (bounds::status_of(slice.out_of(lane.back, j), p[es[j].orig]->n_key) > 1) {
             keep.resize(slice.keep_bytes);
             err = hipMemcpyAsync(keep.data(), dev + slice.keep_begin, slice.keep_bytes, hipMemcpyDeviceToHost, lane.stream);
             es2 = hipStreamSynchronize(lane.stream);
@@ -3169,12 +3168,13 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
         const BoundEntry &e = es[j];
         const gdp_problem *q = p[e.orig];
         const GdpFrontierOut &o = slice.out_of(lane.back, j);
-        if (o.status == 1) continue;   // a key whose budget no path was found for keeps everything
+        const int status = bounds::status_of(o, q->n_key);
+        if (status == 1) continue;   // a key whose budget no path was found for keeps everything
         std::unique_ptr<Reduced> d(new Reduced());
-        if (o.status == 0) {
+        if (status == 0) {
             const int32_t *res = slice.res_of(lane.back, j);
             d->solved = true;
-            d->executed = o.executed;
+            d->executed = bounds::executed_of(o, q->n_key);
             d->total.assign(o.total, o.total + q->n_key);
             d->remaining.assign(o.remaining, o.remaining + q->n_key);
             d->res.assign(res, res + (size_t)q->n_key * q->L);
@@ -3221,17 +3221,18 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
         BoundEntry e;
         if (bound_entry(p[i], i, magnitude[(size_t)i], e)) es.push_back(std::move(e));
     }
-    const int n_lam = bound_multipliers(es.size());
+    const bool alone = keys_alone(n, p);
+    const int n_lam = alone && es.size() == 1 ? bounds::key_multipliers(p[es[0].orig]) : bound_multipliers(es.size());
     int rc = GDP_OK;
     for (size_t begin = 0; begin < es.size() && rc == GDP_OK;) {
         size_t end = begin, bytes = 0;
         while (end < es.size() && end - begin < 65535) {
-            const size_t b = bound_bytes(p[es[end].orig], es[end].h, n_lam);
+            const size_t b = bound_bytes(p[es[end].orig], es[end].h, n_lam, alone);
             if (bytes + b > limit) break;
             bytes += b;
             ++end;
         }
-        if (end > begin) rc = reduce_slice(p, magnitude, es.data() + begin, (int)(end - begin), n_lam, forced, scan, out);
+        if (end > begin) rc = reduce_slice(p, magnitude, es.data() + begin, (int)(end - begin), n_lam, alone, forced, scan, out);
         begin = std::max(end, begin + 1);
     }
     return rc;
@@ -3254,15 +3255,22 @@ static void take_bounds(int32_t n, const gdp_problem *const *p, const std::vecto
     std::unique_ptr<PlanBounds> b(new PlanBounds());
     size_t bytes = 0;
     const size_t limit = std::min(arena_budget(), REDUCE_MAX_BYTES);
-    const int n_lam = bound_multipliers((size_t)n);
     for (int i = 0; i < n; ++i) {
         BoundEntry e;
         if (!bound_entry(p[i], i, magnitude[(size_t)i], e)) return;
-        bytes += bound_bytes(p[i], e.h, n_lam);
-        if (bytes > limit) return;
         b->es.push_back(std::move(e));
     }
-    b->slice.lay_out(p, b->es.data(), n, n_lam);
+    bool alone = keys_alone(n, p);
+    int n_lam = 0;
+    auto fits = [&](bool key_alone) {
+        n_lam = key_alone && n == 1 ? bounds::key_multipliers(p[0]) : bound_multipliers((size_t)n);
+        bytes = 0;
+        for (int i = 0; i < n; ++i) bytes += bound_bytes(p[i], b->es[(size_t)i].h, n_lam, key_alone);
+        return bytes <= limit;
+    };
+    if (alone && !fits(true)) alone = false;
+    if (!fits(alone)) return;
+    b->slice.lay_out(p, b->es.data(), n, n_lam, alone);
     plan->bounds_out.resize((size_t)plan->n_key_total);
     plan->bounds_res.resize(plan->n_res_total);
     std::vector<char> up(b->slice.up_bytes);
@@ -3297,12 +3305,12 @@ static int run_bounds(gdp_plan *plan, int32_t mode, gdp_timing *t, bool *done)
     double executed = 0;
     for (const HostInst &h : plan->inst) {
         const GdpFrontierOut &o = b.slice.out_of(back, h.orig);
-        if (o.status != 0) {
+        if (bounds::status_of(o, h.n_key) != 0) {
             give_back(plan->bounds);
             plan->bounds = nullptr;
             return GDP_OK;
         }
-        executed += o.executed;
+        executed += bounds::executed_of(o, h.n_key);
         const int32_t *res = b.slice.res_of(back, h.orig);
         for (int k = 0; k < h.n_key; ++k) plan->bounds_out[(size_t)(h.key_begin + k)] = {o.total[k], o.remaining[k], o.remaining[k] >= 0};
         memcpy(plan->bounds_res.data() + h.res_begin, res, sizeof(int32_t) * (size_t)h.n_key * h.L);

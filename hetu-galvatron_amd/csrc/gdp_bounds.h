@@ -11,7 +11,7 @@
 constexpr int GDP_BOUND_MAX_S = 128;      // strategies
 constexpr int GDP_BOUND_MAX_L = 512;      // layers
 constexpr int GDP_BOUND_MAX_LS = 40960;   // layers x strategies
-constexpr int GDP_BOUND_MAX_LAM = 64;     // multipliers
+constexpr int GDP_BOUND_MAX_LAM = 128;    // multipliers
 constexpr int GDP_BOUND_MAX_KEY = 8;
 constexpr int GDP_BOUND_WINDOW = 8;       // multipliers around a key's best one that its upper bound comes from
 constexpr double GDP_BOUND_FAR = 1e200;   // for +inf: 512 of them and the costs of a path (below 1e100) have room above
@@ -19,13 +19,16 @@ constexpr int GDP_BOUND_MEM = 1 << 30;    // memory sums saturate here, above ev
 
 constexpr int GDP_FRONTIER_KEPT = 8192;   // strategies that stay, over all layers of an instance
 constexpr int GDP_FRONTIER_LABELS = 1024; // room in memory for so many labels, and transitions, per layer on average
+constexpr int GDP_KEY_LABELS = 512;       // ... so many labels of a key with a workgroup of its own
+constexpr int GDP_KEY_LABELS_MAX_L = 128; // its layers
+constexpr double GDP_KEY_LABELS_MOST = 0.8;   // share of the strategies that no other one dominates
 
 // What bounds::launch_labels finds for an instance; the strategies lie in GdpBoundInst.res.
 struct GdpFrontierOut {
     double total[GDP_BOUND_MAX_KEY];      // +inf: the key has no solution
-    double executed;                      // candidates looked at
+    double executed[GDP_BOUND_MAX_KEY];   // candidates looked at
     int32_t remaining[GDP_BOUND_MAX_KEY];
-    int32_t status, pad;                  // 0: solved; otherwise nothing else in here is valid
+    int32_t status[GDP_BOUND_MAX_KEY];    // 0: solved; otherwise nothing else of the key is valid; 1: no path was found for it
 };
 
 // From w bins on, strategy s (counted among those of its layer that stay) can be reached at cost c.
@@ -47,10 +50,12 @@ struct GdpBoundInst {
     uint32_t *P_mem, *Q_mem; // [NL][L][S] memory of those ways
     double *end;             // [NL] cheapest way through all layers
     unsigned long long *ub;  // [K] time of the best path found that fits the budget, ordered as an unsigned number; ~0: none found
-    int32_t *window;         // [K] first of the multipliers that it comes from
-    uint8_t *keep;           // [L][S] 1: (l, s) may lie on a best path of some key
+    int32_t *best;           // [K] the multiplier whose bound is the best
+    uint8_t *keep;           // [L][S] bit k: (l, s) may lie on a best path of key k
+    unsigned long long *marks;   // [K][L][2] the same by key, strategies 0 to 63 and from 64 on; 16-byte aligned
     const double *other_time;// [K]
-    // of the frontier: the labels of all layers, the transitions between and the costs of what stays, the results
+    // of the frontier: the labels of all layers, the transitions between and the costs of what stays, the results; of keys with a
+    // workgroup of their own one after the other
     GdpFrontierLabel *hist;
     int32_t *hist_mem;
     double *hist_turns, *hist_intra;
@@ -58,7 +63,7 @@ struct GdpBoundInst {
     int32_t *res;            // [K][L]
     double magnitude;        // sum over the layers of the largest finite |intra| and |inter|
     double limit;            // ns that the layers ahead of the DP over what stays may take, by its own account
-    int32_t L, V, S, K, T, n_hist, n_hist_turns;
+    int32_t L, V, S, K, T, n_hist, n_hist_turns, n_lam;
 };
 
 // Nothing in here allocates: gdp_solve_static uses it too.
@@ -68,15 +73,37 @@ __attribute__((visibility("hidden"))) bool has_form(const gdp_problem *q);
 // What the environment says of bounds: false with GALVATRON_DP_REDUCE=0 and with GALVATRON_DP_SKIP=0 (every cell is asked for);
 // *forced: with GALVATRON_DP_REDUCE=1 (every instance that has the form takes them).
 __attribute__((visibility("hidden"))) bool allowed(bool *forced);
+// Share of the strategies of a layer, and on average of 4 layers, that are cheaper in time than every one that needs no more memory.
+__attribute__((visibility("hidden"))) double undominated(const gdp_problem *q, int layer);
+__attribute__((visibility("hidden"))) double undominated(const gdp_problem *q);
+// How many multipliers an instance takes whose keys have a workgroup each.
+__attribute__((visibility("hidden"))) int key_multipliers(const gdp_problem *q);
 // The multipliers of an instance: 0 and a geometric series around (range of times) / (range of memory costs).
 __attribute__((visibility("hidden"))) void multipliers(const gdp_problem *q, int n_lam, double *lam);
 // Copies the matrices, runs the passes of all multipliers, finds the upper bounds and marks what stays.
-// pairs: {instance, matrix} of every matrix that is to be copied.  held: most layers have the matrix of the one before.
+// max_rows: layers times (strategies / 64, rounded up).  pairs: {instance, matrix} of every matrix that is to be copied.  held: most layers have the matrix of the one before.
 __attribute__((visibility("hidden")))
-hipError_t launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K, bool held, const int2 *pairs,
+hipError_t launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_rows, int max_S, int max_K, bool held, const int2 *pairs,
                   int n_pairs, hipStream_t stream);
-// The DP over what stays (gdp_frontier.hip), after it.
+// The DP over what stays, after it: a workgroup per instance (gdp_frontier.hip), or per key of each (gdp_key_labels.hip; up to
+// GDP_KEY_LABELS_MAX_L layers).
 __attribute__((visibility("hidden"))) hipError_t launch_labels(const GdpBoundInst *inst, int n, int max_K, hipStream_t stream);
+__attribute__((visibility("hidden"))) hipError_t launch_key_labels(const GdpBoundInst *inst, int n, int max_K, hipStream_t stream);
+// Of all keys of an instance: 0 solved, 1 no path was found for one, otherwise given up; candidates looked at.
+inline int status_of(const GdpFrontierOut &o, int K)
+{
+    int status = 0;
+    for (int k = 0; k < K; ++k)
+        if (o.status[k] == 1) return 1;
+        else if (o.status[k] != 0) status = o.status[k];
+    return status;
+}
+inline double executed_of(const GdpFrontierOut &o, int K)
+{
+    double sum = 0;
+    for (int k = 0; k < K; ++k) sum += o.executed[k];
+    return sum;
+}
 // What stays of q, given the marks ([L][S]), as arrays of R strategies a layer: kept[L][R] is the strategy of q, or -1 for
 // padding, which costs +inf; memory costs less cut[l] (may be null).  matrix(l): that of layer l of q.  R: the most that
 // stay of a layer, at least; at least one stays of every layer.  inter [L][R][R] and intra hold zeros and +inf before.

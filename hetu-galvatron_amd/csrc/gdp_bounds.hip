@@ -19,11 +19,13 @@
 
 #include <math.h>
 #include <stdlib.h>
+#include <string.h>
+
+#include <algorithm>
 
 namespace {
 
 static_assert(GDP_BOUND_MAX_S == 128, "two blocks of 64 targets; a strategy in the low 7 bits of a candidate");
-static_assert(GDP_BOUND_MAX_LAM <= 64, "the best multiplier of a key: one per lane");
 
 // The matrices as the passes read them: as they are and transposed, +inf replaced by GDP_BOUND_FAR.  grid (pairs, 16-row
 // bands of the largest matrix), 256 threads; LDS turns the band around so that both sides are read and written along rows.
@@ -290,9 +292,15 @@ __global__ __launch_bounds__(256) void gdp_bound_upper_kernel(const GdpBoundInst
     if (key >= I.K || (int)blockIdx.x * 256 >= LS || I.budget[key] < 0) return;   // the whole workgroup
     const int64_t B = I.budget[key];
     if (t < 64) {
-        const int at = min(t, n_lam - 1);
-        double d = I.end[at] - I.lam[at] * (double)B;
-        int i = at;
+        double d = -INFINITY;
+        int i = n_lam;
+        for (int at = t; at < n_lam; at += 64) {
+            const double e = I.end[at] - I.lam[at] * (double)B;
+            if (e > d) {
+                d = e;
+                i = at;
+            }
+        }
 #pragma unroll
         for (int w = 32; w > 0; w >>= 1) {
             const double e = __shfl_xor(d, w);
@@ -304,7 +312,7 @@ __global__ __launch_bounds__(256) void gdp_bound_upper_kernel(const GdpBoundInst
         }
         if (t == 0) {
             first = max(0, min(i - W / 2, n_lam - W));
-            if (blockIdx.x == 0) I.window[key] = first;
+            if (blockIdx.x == 0) I.best[key] = i;
         }
     }
     __syncthreads();
@@ -343,18 +351,22 @@ __global__ __launch_bounds__(256) void gdp_bound_upper_kernel(const GdpBoundInst
 // What stays: (l, s) is out when for every key some multiplier's bound lies above that key's upper bound.  The
 // margin covers the rounding of the bound; that of the upper bound is part of it, and that of the DP's own sums is less
 // than either.
-// grid (64-element groups of the largest table, instances), PARTS waves with 8 multipliers at a time each.  What takes
+// grid (ROWS times 64 strategies of a layer, instances), PARTS waves for each with 8 multipliers at a time.  What takes
 // the time is the round trips of the loads: with 8 waves all 64 multipliers of an element are asked for at once (L = 80,
 // S = 64 26.8 -> 6.3 us, L = 48, S = 88 25.0 -> 5.7 us).  A batch that fills the device with one wave per 64 elements
-// hides them by itself and would only start more waves (256 instances of S = 44 23.6 us with 1 wave, 40 with 8).
-template <int PARTS>
-__global__ __launch_bounds__(64 * PARTS) void gdp_bound_keep_kernel(const GdpBoundInst *inst, int n_lam)
+// hides them by itself and would only start more waves, and what it does wait for is the start of its workgroups, so that one has
+// 4 layers (256 instances of S = 44 44 us with a layer each, 32 with 4).
+template <int PARTS, int ROWS>
+__global__ __launch_bounds__(64 * PARTS * ROWS) void gdp_bound_keep_kernel(const GdpBoundInst *inst, int n_lam)
 {
+    static_assert(PARTS == 1 || ROWS == 1, "waves that meet at the barrier all get there");
     __shared__ unsigned left[PARTS][64];
     const GdpBoundInst &I = inst[blockIdx.y];
-    const int LS = I.L * I.S, K = I.K, lane = (int)threadIdx.x & 63, part = (int)threadIdx.x >> 6;
-    if ((int)blockIdx.x * 64 >= LS) return;   // the whole workgroup
-    const int e = (int)blockIdx.x * 64 + lane, at = min(e, LS - 1);
+    const int L = I.L, S = I.S, LS = L * S, K = I.K, lane = (int)threadIdx.x & 63, part = PARTS == 1 ? 0 : (int)threadIdx.x >> 6;
+    const int halves = (S + 63) / 64, row = (int)blockIdx.x * ROWS + (ROWS == 1 ? 0 : (int)threadIdx.x >> 6), l = row / halves, half = row - l * halves,
+              s = 64 * half + lane;
+    if (l >= L) return;   // the whole workgroup, or a wave that meets no other
+    const int at = l * S + min(s, S - 1);
     unsigned alive = 0;
     double ub[GDP_BOUND_MAX_KEY], budget[GDP_BOUND_MAX_KEY];
 #pragma unroll
@@ -368,6 +380,8 @@ __global__ __launch_bounds__(64 * PARTS) void gdp_bound_keep_kernel(const GdpBou
         }
     }
     const gdouble P = (gdouble)(uintptr_t)I.P, Q = (gdouble)(uintptr_t)I.Q, lams = (gdouble)(uintptr_t)I.lam;
+    const gulong marks = (gulong)(uintptr_t)I.marks;   // (here: behind a store the compiler would fetch it again)
+    __attribute__((address_space(1))) uint8_t *const keep = (__attribute__((address_space(1))) uint8_t *)(uintptr_t)I.keep;
     for (int i0 = 8 * part; i0 < n_lam; i0 += 8 * PARTS) {
         double p[8], q[8];
 #pragma unroll
@@ -386,12 +400,21 @@ __global__ __launch_bounds__(64 * PARTS) void gdp_bound_keep_kernel(const GdpBou
                 if (k < K && r - lam * budget[k] > ub[k] + margin) alive &= ~(1u << k);
         }
     }
-    left[part][lane] = alive;
-    __syncthreads();
-    if (part != 0 || e >= LS) return;
+    if constexpr (PARTS > 1) {
+        left[part][lane] = alive;
+        __syncthreads();
+        if (part != 0) return;
 #pragma unroll
-    for (int w = 1; w < PARTS; ++w) alive &= left[w][lane];
-    I.keep[e] = alive != 0;
+        for (int w = 1; w < PARTS; ++w) alive &= left[w][lane];
+    }
+    if (s < S) keep[at] = (uint8_t)alive;
+    else alive = 0;
+    for (int k = 0; k < K; ++k) {
+        const unsigned long long these = __builtin_amdgcn_ballot_w64(alive >> k & 1);
+        const gulong mark = marks + 2 * ((size_t)k * L + l);
+        if (lane == 0) mark[half] = these;
+        if (lane == 0 && halves == 1) mark[1] = 0;
+    }
 }
 
 }  // namespace
@@ -410,6 +433,46 @@ bool bounds::allowed(bool *forced)
     return !(env && *env && !*forced) && !(skip && *skip && atoi(skip) == 0);
 }
 
+double bounds::undominated(const gdp_problem *q, int layer)
+{
+    const int32_t *const mem = q->mem + (size_t)layer * q->S;
+    const double *const time = q->intra + (size_t)layer * q->S;
+    int16_t order[GDP_MAX_S];
+    for (int s = 0; s < q->S; ++s) order[s] = (int16_t)s;
+    std::sort(order, order + q->S, [&](int a, int b) { return mem[a] != mem[b] ? mem[a] < mem[b] : time[a] < time[b]; });   // allocates nothing
+    double least = INFINITY;
+    int stay = 0;
+    for (int i = 0; i < q->S && mem[order[i]] < q->V; ++i) {
+        stay += time[order[i]] < least;
+        least = fmin(least, time[order[i]]);
+    }
+    return (double)stay / q->S;
+}
+
+double bounds::undominated(const gdp_problem *q)
+{
+    const int m = q->L < 4 ? q->L : 4;
+    const size_t S = (size_t)q->S;
+    double share = 0, last = 0;
+    for (int k = 0, before = -1; k < m; ++k) {
+        const int l = (int)((int64_t)q->L * (2 * k + 1) / (2 * m));
+        if (before < 0 || memcmp(q->mem + l * S, q->mem + before * S, sizeof(int32_t) * S) != 0 || memcmp(q->intra + l * S, q->intra + before * S, sizeof(double) * S) != 0)
+            last = undominated(q, l);
+        share += last;
+        before = l;
+    }
+    return share / m;
+}
+
+// Twice as many leave fewer labels where those are many, which the undominated strategies of all layers tell best, and take 3 us longer (a
+// wave of passes on every compute unit instead of every second).  110 calls of random inputs, us with 64 / 128: up to 250 of these strategies 64 is as fast or up to
+// 4 us faster; above 183 / 172, 190 / 153, 228 / 140, 235 / 219, 351 / 269, 1263 / 424.  256 are slower in nearly all.
+int bounds::key_multipliers(const gdp_problem *q)
+{
+    constexpr double MANY = 250;
+    return undominated(q) * q->S * q->L <= MANY ? 64 : GDP_BOUND_MAX_LAM;
+}
+
 void bounds::multipliers(const gdp_problem *q, int n_lam, double *lam)
 {
     double t0 = INFINITY, t1 = -INFINITY, m0 = INFINITY, m1 = 0;
@@ -425,7 +488,7 @@ void bounds::multipliers(const gdp_problem *q, int n_lam, double *lam)
     for (int i = 1; i < n_lam; ++i) lam[i] = base * exp2(-6.0 + 12.0 * (i - 1) / (n_lam - 2));
 }
 
-hipError_t bounds::launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_S, int max_K, bool held, const int2 *pairs,
+hipError_t bounds::launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_rows, int max_S, int max_K, bool held, const int2 *pairs,
                           int n_pairs, hipStream_t stream)
 {
     gdp_bound_transpose_kernel<<<dim3((unsigned)n_pairs, (unsigned)((max_S + 15) / 16)), 256, 0, stream>>>(inst, pairs);
@@ -450,10 +513,9 @@ hipError_t bounds::launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS
     gdp_bound_upper_kernel<<<dim3((unsigned)((max_LS + 255) / 256), (unsigned)max_K, (unsigned)n), 256, 0, stream>>>(inst, n_lam);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const dim3 elements64((unsigned)((max_LS + 63) / 64), (unsigned)n);
-    if ((int64_t)elements64.x * n <= 1024)   // 8 waves of each are on the device at a time
-        gdp_bound_keep_kernel<8><<<elements64, 512, 0, stream>>>(inst, n_lam);
+    if ((int64_t)max_rows * n <= 1024)   // 8 waves of each are on the device at a time
+        gdp_bound_keep_kernel<8, 1><<<dim3((unsigned)max_rows, (unsigned)n), 512, 0, stream>>>(inst, n_lam);
     else
-        gdp_bound_keep_kernel<1><<<elements64, 64, 0, stream>>>(inst, n_lam);
+        gdp_bound_keep_kernel<1, 4><<<dim3((unsigned)(max_rows + 3) / 4, (unsigned)n), 256, 0, stream>>>(inst, n_lam);
     return hipGetLastError();
 }

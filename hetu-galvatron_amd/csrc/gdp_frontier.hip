@@ -14,6 +14,7 @@
 // and what it needs of the next layer live in LDS, its layers follow each other at the price of two barriers.  An instance
 // with more labels than fit says so, and is solved as a smaller instance of the dense recurrence.
 #include "gdp_bounds.h"
+#include "gdp_label_ops.h"
 
 #include <math.h>
 
@@ -29,8 +30,6 @@ constexpr int LINES = 1152;     // doubles: what a layer's strategies are held a
 constexpr int BACK_LABELS = 4096, BACK_TURNS = 4800, BACK_KEPT = 1024;
 static_assert(BACK_LABELS >= LABELS && BACK_TURNS >= TURNS && BACK_KEPT >= KEPT, "a layer fits");
 static_assert(WORKERS >= GDP_BOUND_MAX_KEY, "the walk back: a wave per key");
-
-typedef GdpFrontierLabel Label;
 
 // Keys are whole numbers below 2^53: a double is compared as fast as 32 bits are.
 constexpr double KEY_W = 0x1p17, KEY_S = 0x1p11;
@@ -78,99 +77,6 @@ struct Shared {
 };
 static_assert(sizeof(Shared) <= 160 * 1024, "LDS of a compute unit");
 
-typedef const __attribute__((address_space(1))) double *gdouble;
-typedef const __attribute__((address_space(1))) int32_t *gint;
-typedef const __attribute__((address_space(1))) uint8_t *gbyte;
-typedef __attribute__((address_space(1))) double *gout;
-typedef __attribute__((address_space(1))) int32_t *giout;
-typedef int int4v __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(1))) int4v *glabel;
-#define GLOBAL(type, p) ((type)(uintptr_t)(p))
-
-typedef int int2v __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ double min_f64(double a, double b)
-{
-    double r;   // the bare instruction: no operand is a NaN
-    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-
-__device__ __forceinline__ double max_f64(double a, double b)
-{
-    double r;
-    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-
-// x of the lane that CTRL names, `other` where there is none.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double moved(double other, double x)
-{
-    const int2v o = __builtin_bit_cast(int2v, other), w = __builtin_bit_cast(int2v, x);
-    const int2v m = {__builtin_amdgcn_update_dpp(o.x, w.x, CTRL, ROWS, 0xf, false), __builtin_amdgcn_update_dpp(o.y, w.y, CTRL, ROWS, 0xf, false)};
-    return __builtin_bit_cast(double, m);
-}
-
-// Minimum over the lanes up to this one, of the first `lanes`.
-__device__ __forceinline__ double prefix_min(double x, int lanes = 64)
-{
-    if (lanes <= 1) return x;
-    x = min_f64(x, moved<0x111, 0xf>(x, x));   // row_shr:1, 2, 4, 8; a lane without a source keeps its own
-    x = min_f64(x, moved<0x112, 0xf>(x, x));
-    x = min_f64(x, moved<0x114, 0xf>(x, x));
-    x = min_f64(x, moved<0x118, 0xf>(x, x));
-    if (lanes <= 16) return x;
-    x = min_f64(x, moved<0x142, 0xa>(x, x));   // row_bcast:15 into rows 1 and 3
-    x = min_f64(x, moved<0x143, 0xc>(x, x));   // row_bcast:31 into rows 2 and 3
-    return x;
-}
-
-__device__ __forceinline__ double lane_of(double x, int lane)
-{
-    const int2v w = __builtin_bit_cast(int2v, x);
-    const int2v r = {__builtin_amdgcn_readlane(w.x, lane), __builtin_amdgcn_readlane(w.y, lane)};
-    return __builtin_bit_cast(double, r);
-}
-
-__device__ __forceinline__ int lanes_min(int x)
-{
-    x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x111, 0xf, 0xf, false));
-    x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x112, 0xf, 0xf, false));
-    x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x114, 0xf, 0xf, false));
-    x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x118, 0xf, 0xf, false));
-    x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x142, 0xa, 0xf, false));
-    x = min(x, __builtin_amdgcn_update_dpp(x, x, 0x143, 0xc, 0xf, false));
-    return __builtin_amdgcn_readlane(x, 63);
-}
-
-// The lowest (value, strategy) of a wave's first `lanes`, +inf in the others: the cheapest, of those the lowest strategy.
-__device__ __forceinline__ void cheapest(double &c, int &s, int lanes)
-{
-    const double least = lane_of(prefix_min(c, lanes), min(lanes, 64) - 1);
-    const unsigned long long at = __builtin_amdgcn_ballot_w64(c == least);
-    s = (at & (at - 1)) == 0 ? __builtin_amdgcn_readlane(s, __builtin_ctzll(at)) : lanes_min(c == least ? s : INT32_MAX);
-    c = least;
-}
-
-// old = *p, *p += n, in LDS, by one lane.
-__device__ __forceinline__ int draw(int32_t *p, int n)
-{
-    int old;
-    asm volatile("ds_add_rtn_u32 %0, %1, %2\n\ts_waitcnt lgkmcnt(0)" : "=&v"(old)
-                 : "v"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) int32_t *)p), "v"(n) : "memory");
-    return old;
-}
-
-// All of a label at a time.
-__device__ __forceinline__ int4v words(const Label &x) { return __builtin_bit_cast(int4v, x); }
-__device__ __forceinline__ Label label_at(const Label *p) { return __builtin_bit_cast(Label, *reinterpret_cast<const int4v *>(p)); }
-__device__ __forceinline__ void put(Label *p, const Label &x) { *reinterpret_cast<int4v *>(p) = words(x); }
-
-// The same in every lane, said so.
-__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
-__device__ __forceinline__ double uniform(double x) { return lane_of(x, 0); }
-
 // What a wave has on its way from memory for a later layer: transitions, what labels are held against, costs.
 template <int LINE>
 struct Ahead {
@@ -194,7 +100,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
     // them: no kernel here may need scratch memory, which the runtime would have to obtain for the launch, and gdp_solve_static
     // promises that nothing is obtained.  (8 keys with all of them held took 252 bytes a lane and longer: L = 80, S = 64 408 -> 377 us;
     // 5 keys with two lines held 12 to 16 bytes, 522 -> 517 us.)
-    constexpr int LINES_HELD = KEYS <= 4 ? KEYS : KEYS == 5 ? 1 : 2, KEYS_HELD = KEYS <= 5 ? KEYS : 0;
+    constexpr int LINES_HELD = KEYS <= 4 ? KEYS : KEYS == 5 ? 0 : 2, KEYS_HELD = KEYS <= 5 ? KEYS : 0;
     extern __shared__ __align__(16) char lds[];
     Shared &sh = *reinterpret_cast<Shared *>(lds);
     const GdpBoundInst &I = inst[blockIdx.x];
@@ -202,7 +108,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
     const int t = (int)threadIdx.x, lane = t & 63, wave = uniform(t >> 6);
     GdpFrontierOut *const out = I.out;
     auto give_up = [&](int why) {   // by the whole workgroup
-        if (t == 0) out->status = why;
+        if (t < K) out->status[t] = why;
     };
 
     // ---- what stays, as lists; the keys ----
@@ -218,7 +124,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
         const unsigned long long o = there ? GLOBAL(const __attribute__((address_space(1))) unsigned long long *, I.ub)[t] : 0;
         sh.budget[t] = (int32_t)B;   // a start row; negative: none
         sh.ub[t] = gdp_unordered(o);
-        const int first = B < 0 ? 0 : GLOBAL(gint, I.window)[t] + (GDP_BOUND_WINDOW - WINDOW) / 2;
+        const int first = B < 0 ? 0 : max(0, min(GLOBAL(gint, I.best)[t] - GDP_BOUND_WINDOW / 2, I.n_lam - GDP_BOUND_WINDOW)) + (GDP_BOUND_WINDOW - WINDOW) / 2;
         sh.window[t] = first;
         for (int i = 0; i < WINDOW; ++i) {
             const double lam = GLOBAL(gdouble, I.lam)[first + i];
@@ -748,10 +654,8 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
     if (wave < K && lane == 0) {
         out->total[wave] = walks ? total + GLOBAL(gdouble, I.other_time)[wave] : INFINITY;
         out->remaining[wave] = walks ? v : -1;
-    }
-    if (t == 0) {
-        out->executed = executed;
-        out->status = 0;
+        out->executed[wave] = wave == 0 ? executed : 0.0;
+        out->status[wave] = 0;
     }
 }
 

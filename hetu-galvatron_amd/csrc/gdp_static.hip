@@ -230,6 +230,8 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     if (!bounds::has_form(&form) || !(magnitude < 1e100)) return GDP_OK;
     // The bounds take 35 us at least (L = 5: S = 8 58 us whole, 60 with them, S = 11 79 and 60).
     if (dense_ns(L, S) < 36e3 && !forced) return GDP_OK;
+    // (calls of more keys go the way they went, and end it where they did)
+    constexpr int MOST_ALONE = 4;
     int64_t budget[GDP_BOUND_MAX_KEY], least = 0;
     for (int l = 0; l < L; ++l) {
         int32_t m = INT32_MAX;
@@ -244,8 +246,9 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
         any = any || b >= least;
     }
     if (!any) return GDP_OK;
-    constexpr int NL = GDP_BOUND_MAX_LAM;
-    const size_t LS = (size_t)L * S, SS = (size_t)S * S, labels = (size_t)L * GDP_FRONTIER_LABELS;
+    const bool alone = K <= MOST_ALONE && L <= GDP_KEY_LABELS_MAX_L && bounds::undominated(p) <= GDP_KEY_LABELS_MOST;
+    const size_t NL = alone ? (size_t)bounds::key_multipliers(p) : 64, keys = alone ? (size_t)K : 1;
+    const size_t LS = (size_t)L * S, SS = (size_t)S * S, labels = (size_t)L * (alone ? GDP_KEY_LABELS : GDP_FRONTIER_LABELS);
     size_t off = 0;
     auto take = [&](size_t bytes) {
         const size_t o = off;
@@ -256,10 +259,10 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
                  off_intra = take(8 * LS), off_inter = take(8 * SS * (size_t)T), off_index = take(4 * (size_t)L),
                  off_lam = take(8 * NL), off_budget = take(8 * (size_t)K), off_other_time = take(8 * (size_t)K), up_bytes = off,
                  off_out = take(sizeof(GdpFrontierOut)), off_res = take(4 * (size_t)K * L), back_bytes = off - up_bytes,
-                 off_keep = take(LS), off_inter_f = take(8 * SS * (size_t)T), off_inter_t = take(8 * SS * (size_t)T),
+                 off_keep = take(LS), off_marks = take(16 * (size_t)K * L), off_inter_f = take(8 * SS * (size_t)T), off_inter_t = take(8 * SS * (size_t)T),
                  off_P = take(8 * LS * NL), off_Q = take(8 * LS * NL), off_P_mem = take(4 * LS * NL), off_Q_mem = take(4 * LS * NL),
-                 off_end = take(8 * NL), off_window = take(4 * (size_t)K), off_ub = take(8 * (size_t)K),
-                 off_hist = take(sizeof(GdpFrontierLabel) * labels), off_turns = take(8 * labels),
+                 off_end = take(8 * NL), off_best = take(4 * (size_t)K), off_ub = take(8 * (size_t)K),
+                 off_hist = take(sizeof(GdpFrontierLabel) * labels * keys), off_turns = take(alone ? 0 : 8 * labels),
                  off_hist_mem = take(4 * GDP_FRONTIER_KEPT), off_hist_intra = take(8 * GDP_FRONTIER_KEPT);
     if (off > (size_t)GDP_STATIC_SCRATCH_BYTES || up_bytes > STAGE_BYTES || back_bytes > STAGE_BYTES) return GDP_OK;
     memcpy(g_stage + off_mem, p->mem, 4 * LS);
@@ -271,7 +274,7 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
         index[l] = p->inter_index ? p->inter_index[l] : l;
         changes += l > 0 && index[l] != index[l - 1];
     }
-    bounds::multipliers(p, NL, reinterpret_cast<double *>(g_stage + off_lam));
+    bounds::multipliers(p, (int)NL, reinterpret_cast<double *>(g_stage + off_lam));
     memcpy(g_stage + off_budget, budget, 8 * (size_t)K);
     memcpy(g_stage + off_other_time, p->other_time, 8 * (size_t)K);
     int2 *pairs = reinterpret_cast<int2 *>(g_stage + off_pairs);
@@ -292,8 +295,9 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     b.Q_mem = reinterpret_cast<uint32_t *>(base + off_Q_mem);
     b.end = reinterpret_cast<double *>(base + off_end);
     b.ub = reinterpret_cast<unsigned long long *>(base + off_ub);
-    b.window = reinterpret_cast<int32_t *>(base + off_window);
+    b.best = reinterpret_cast<int32_t *>(base + off_best);
     b.keep = base + off_keep;
+    b.marks = reinterpret_cast<unsigned long long *>(base + off_marks);
     b.other_time = reinterpret_cast<const double *>(base + off_other_time);
     b.hist = reinterpret_cast<GdpFrontierLabel *>(base + off_hist);
     b.hist_mem = reinterpret_cast<int32_t *>(base + off_hist_mem);
@@ -305,13 +309,14 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     b.limit = dense_ns(L, S);
     b.L = L; b.V = p->V; b.S = S; b.K = K; b.T = T;
     b.n_hist = b.n_hist_turns = (int32_t)labels;
+    b.n_lam = (int32_t)NL;
     memcpy(g_stage + off_inst, &b, sizeof b);
     hipStream_t stream = nullptr;
     hipError_t e = hipMemcpy(base, g_stage, up_bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) return gdp_fail_hip(e, "gdp_solve_static: upload");
     const GdpBoundInst *inst = reinterpret_cast<const GdpBoundInst *>(base + off_inst);
-    e = bounds::launch(inst, 1, NL, (int)LS, S, K, changes * 4 <= L, reinterpret_cast<const int2 *>(base + off_pairs), T, stream);
-    if (e == hipSuccess) e = bounds::launch_labels(inst, 1, K, stream);
+    e = bounds::launch(inst, 1, (int)NL, (int)LS, L * ((S + 63) / 64), S, K, changes * 4 <= L, reinterpret_cast<const int2 *>(base + off_pairs), T, stream);
+    if (e == hipSuccess) e = alone ? bounds::launch_key_labels(inst, 1, K, stream) : bounds::launch_labels(inst, 1, K, stream);
     if (e != hipSuccess) {
         (void)hipDeviceSynchronize();
         return gdp_fail_hip(e, "gdp_solve_static: kernel launch");
@@ -319,19 +324,20 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     e = hipMemcpy(g_stage, base + off_out, back_bytes, hipMemcpyDeviceToHost);   // after the kernels, in stream order
     if (e != hipSuccess) return gdp_fail_hip(e, "gdp_solve_static: download");
     const GdpFrontierOut *out = reinterpret_cast<const GdpFrontierOut *>(g_stage);
-    if (out->status > 1) {
+    const int status = bounds::status_of(*out, K);
+    if (status > 1) {
         e = hipMemcpy(g_keep, base + off_keep, LS, hipMemcpyDeviceToHost);
         if (e != hipSuccess) return gdp_fail_hip(e, "gdp_solve_static: download");
         *marked = true;
     }
-    if (out->status != 0) return GDP_OK;
+    if (status != 0) return GDP_OK;
     const int32_t *res = reinterpret_cast<const int32_t *>(g_stage + (off_res - off_out));
     for (int k = 0; k < K; ++k) {
         r->total[k] = out->total[k];
         r->remaining[k] = out->remaining[k];
         if (out->remaining[k] >= 0) memcpy(r->res + (size_t)k * L, res + (size_t)k * L, sizeof(int32_t) * (size_t)L);
     }
-    stats::count(work(p), out->executed);
+    stats::count(work(p), bounds::executed_of(*out, K));
     *done = true;
     return GDP_OK;
 }
@@ -344,7 +350,7 @@ bool lay_out_kept(const gdp_problem *p, const Layout &whole, gdp_problem *small,
     int most = 0;
     for (int l = 0; l < p->L; ++l) {
         int n = 0;
-        for (int s = 0; s < p->S; ++s) n += g_keep[(size_t)l * p->S + s];
+        for (int s = 0; s < p->S; ++s) n += g_keep[(size_t)l * p->S + s] != 0;
         if (n == 0) return false;
         most = std::max(most, n);
     }

@@ -1,0 +1,113 @@
+"""The DP over labels with a workgroup for every key of an instance: at the numbers of labels, strategies, layers and keys around which
+its kernel branches, against the C oracle, which sees the whole instance."""
+import os
+import re
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+from galvatron_dp import _lib
+from oracle import dp_oracle as O
+
+
+def _instance(L, S, V, kind, n_keys):
+    """Two thirds of the strategies are dominated by another ('each', 'alike': random costs; 'trade': what is left trades memory for
+    time and is the same in all layers, so that labels are many; 'ties': small whole numbers; 'runs': one strategy is the best by
+    far in most layers)."""
+    rng = np.random.Generator(np.random.PCG64([L, S, V, n_keys]))
+    per, n = max(2, V // L), 1 if kind in ("trade", "alike") else L
+    mem = rng.integers(max(1, per // 4), 3 * per, size=(n, S)).astype(np.int32)
+    intra, inter = rng.lognormal(2.5, 0.5, size=(n, S)), rng.uniform(0, 5, size=(n, S, S))
+    if kind == "trade":
+        intra, inter = 40.0 * per / mem * rng.uniform(0.98, 1.02, size=mem.shape), inter * 0.05
+        worse = rng.permutation(S)[:2 * S // 3]
+        intra[:, worse] = intra.max() + 1.0 + worse
+    if kind == "ties":
+        mem, intra, inter = (mem // max(1, per // 4) + 1).astype(np.int32), rng.integers(1, 5, size=(n, S)).astype(float), rng.integers(0, 3, size=(n, S, S)).astype(float)
+    if kind == "runs":
+        for l in range(L):
+            if l % 7 != 3:
+                intra[l, rng.integers(S)] = 1e-3
+                mem[l, np.argmin(intra[l])] = 1
+    if n == 1:
+        mem, intra, inter = np.repeat(mem, L, 0), np.repeat(intra, L, 0), np.repeat(inter, L, 0)
+    om = [int(V * f) for f in (0.1, 0.3, 0.0, 0.45, 0.2, 0.999, 0.25, 2.0)[:n_keys]]
+    return mem, intra, inter, om, [k / 3 for k in range(n_keys)]
+
+
+def _same(prob, x, V, tag):
+    keys = range(len(x[3]))
+    total, res, left = O.solve(x[0], x[1], x[2], V, dict(zip(keys, x[3])), dict(zip(keys, x[4])))[:3]
+    for k in keys:
+        assert np.float64(prob.total[k]).tobytes() == np.float64(total[k]).tobytes(), f"{tag} key {k}: {prob.total[k]} {total[k]}"
+        assert int(prob.remaining[k]) == left[k], f"{tag} key {k}"
+        if left[k] >= 0:
+            assert [int(v) for v in prob.res[k]] == [int(v) for v in res[k]], f"{tag} key {k}"
+
+
+# Layers: 2, around 64 (a word of marks), 128, and one more, which has a workgroup per instance; strategies: 2, around 64 (the
+# words of a layer's marks), 128; labels: one (runs of layers with one strategy), up to 16, 32 and 64 beside each other, more (trade)
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,L,S,V", [("each", 2, 2, 60), ("each", 9, 12, 3000), ("each", 20, 63, 4000), ("each", 20, 64, 4000), ("each", 20, 65, 4000),
+                                        ("each", 6, 128, 2000), ("each", 63, 7, 6000), ("each", 64, 7, 6000), ("each", 65, 7, 6000), ("runs", 127, 6, 4000),
+                                        ("runs", 128, 6, 4000), ("runs", 129, 6, 4000), ("runs", 40, 20, 5000), ("alike", 30, 24, 5000),
+                                        ("trade", 8, 9, 2000), ("trade", 12, 24, 5000), ("trade", 16, 33, 9000), ("trade", 24, 48, 12000), ("ties", 12, 24, 300),
+                                        ("ties", 30, 40, 900), ("ties", 70, 9, 1000)])
+@pytest.mark.parametrize("n_keys", [1, 3, 4, 8])
+def test_calls_against_the_oracle(kind, L, S, V, n_keys, monkeypatch):
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    x = _instance(L, S, V, kind, n_keys)
+    prob = _lib.Problem(x[0], x[1], x[2], V, x[3], x[4])
+    _lib.batch_stats_begin()
+    _lib.solve_batch([prob])
+    s = _lib.batch_stats_end()
+    _same(prob, x, V, f"{kind} {L} {S} {V}")
+    if kind in ("each", "runs") and V > 1000:
+        assert s.executed < 0.01 * s.relaxations
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("many", [2, 60, 130])
+def test_batches_of_different_shapes(many, monkeypatch):
+    """More keys than compute units, more layers than the shortest of them has, strategies on both sides of 64."""
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    V, xs = 1500, [_instance(3 + i % 9, 5 + 11 * (i % 7), 1500 + i, ("each", "ties")[i % 2], 1 + i % 6) for i in range(many)]
+    probs = [_lib.Problem(x[0], x[1], x[2], V, x[3], x[4]) for x in xs]
+    _lib.solve_batch(probs)
+    for i, (x, prob) in enumerate(zip(xs, probs)):
+        _same(prob, x, V, f"instance {i}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,L,S,V,n_keys", [("each", 30, 24, 5000, 4), ("trade", 20, 30, 6000, 2), ("runs", 60, 9, 6000, 3), ("ties", 20, 30, 600, 4)])
+def test_static_calls_and_plans(kind, L, S, V, n_keys, monkeypatch):
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    x = _instance(L, S, V, kind, n_keys)
+    prob = _lib.Problem(x[0], x[1], x[2], V, x[3], x[4])
+    _lib.solve_static(prob)
+    _same(prob, x, V, f"static {kind}")
+    prob.total[:], prob.remaining[:], prob.res[:] = 0, 0, 0
+    with _lib.Plan([prob]) as plan:
+        for _ in range(2):
+            plan.run()
+            plan.fetch()
+            _same(prob, x, V, f"plan {kind}")
+
+
+def test_the_kernel_needs_nothing_obtained_for_a_launch(tmp_path):
+    """It is one of gdp_solve_static's: no scratch memory, and a launcher that calls no allocator."""
+    from galvatron_dp import _build
+    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    if shutil.which(hipcc) is None:
+        pytest.skip("no hipcc")
+    flags = [f for f in _build.HIPCC_FLAGS if f != "-shared"]
+    source, obj = os.path.join(_build.CSRC, "gdp_key_labels.hip"), str(tmp_path / "o.o")
+    log = subprocess.run([hipcc] + flags + ["-c", "-Rpass-analysis=kernel-resource-usage", source, "-o", obj], check=True, capture_output=True,
+                         text=True).stderr
+    found = re.findall(r"Function Name: (\S+).*?ScratchSize \[bytes/lane\]: (\d+)", log, re.S)
+    assert [int(size) for name, size in found if "key_labels" in name] == [0]
+    undefined = subprocess.run(["nm", "-u", "-C", obj], stdout=subprocess.PIPE, text=True, check=True).stdout
+    for name in (ln.split(None, 1)[1].strip() for ln in undefined.splitlines() if ln.strip().startswith("U ")):
+        assert not name.startswith(("hipMalloc", "hipHost", "hipMem", "hipStream", "hipEvent", "hipFree", "operator", "malloc", "calloc", "std::__throw")), name
