@@ -2899,7 +2899,7 @@ struct BoundEntry {
     int orig, table_of;   // table_of: the entry of the slice whose matrices this one reads
     HostInst h;
     std::vector<int64_t> budget;
-    size_t off_mem, off_intra, off_inter, off_index, off_lam, off_budget, off_inter_f, off_inter_t, off_P, off_Q, off_P_mem, off_Q_mem, off_end,
+    size_t off_mem, off_intra, off_index, off_inter, off_lam, off_budget, off_inter_f, off_inter_t, off_P, off_Q, off_P_mem, off_Q_mem, off_end,
         off_best, off_ub, off_keep, off_marks, off_other_time, off_out, off_res, off_hist, off_hist_mem, off_hist_turns, off_hist_intra;
 };
 
@@ -2908,7 +2908,7 @@ static size_t bound_bytes(const gdp_problem *q, const HostInst &h, int n_lam, bo
 {
     const size_t L = (size_t)q->L, LS = L * q->S, T = (size_t)h.n_inter, K = (size_t)q->n_key, NL = (size_t)n_lam;
     constexpr size_t ARRAYS = 29;   // aligned to 256 bytes each
-    return sizeof(GdpBoundInst) + T * sizeof(int2) + 13 * LS + 4 * L + 28 * K + 24 * T * (size_t)q->S * q->S +
+    return sizeof(GdpBoundInst) + T * sizeof(GdpBoundMatrix) + 13 * LS + 4 * L + 28 * K + 24 * T * (size_t)q->S * q->S +
            NL * (16 + 24 * LS) + sizeof(GdpFrontierOut) + 20 * K * L +
            (alone ? 16 * K * L * GDP_KEY_LABELS : 24 * L * GDP_FRONTIER_LABELS + 12 * GDP_FRONTIER_KEPT) + 256 * ARRAYS;
 }
@@ -2939,19 +2939,19 @@ struct BoundSlice {
     double relaxations = 0;            // of the whole instances
     double limit_ns = 0;               // of the DP over what stays
     int64_t layers = 0, changes = 0;   // ... and how often a layer has another matrix than the one before
-    std::vector<int2> pairs;
-    // [0, up_bytes): what is uploaded; the results after it; what stays; the rest stays on the device
-    size_t off_inst = 0, off_pairs = 0, up_bytes = 0, back_bytes = 0, keep_begin = 0, keep_bytes = 0, bytes = 0;
+    int matrices = 0;
+    // [0, up_bytes): what is uploaded, the matrices from head_bytes on; what stays; the rest stays on the device.  The results go to
+    // page-locked host memory.
+    size_t off_inst = 0, off_matrices = 0, head_bytes = 0, up_bytes = 0, back_bytes = 0, keep_begin = 0, keep_bytes = 0, bytes = 0;
 
     void lay_out(const gdp_problem *const *p, BoundEntry *entries, int count, int multipliers, bool key_alone);
-    void fill(const gdp_problem *const *p, const std::vector<double> &magnitude, char *up, char *dev) const;
-    hipError_t enqueue(char *dev, hipStream_t stream) const;
-    const GdpFrontierOut &out_of(const char *back, int j) const
-    {
-        return *reinterpret_cast<const GdpFrontierOut *>(back + (es[j].off_out - up_bytes));
-    }
+    // read_from: where the launches find the matrices, the upload or what was made of it on the device
+    void fill(const gdp_problem *const *p, const std::vector<double> &magnitude, char *up, const char *read_from, char *dev, char *back) const;
+    // up: page-locked memory that the launches bring to the device themselves, or null, where it is there already
+    hipError_t enqueue(const char *up, char *dev, hipStream_t stream) const;
+    const GdpFrontierOut &out_of(const char *back, int j) const { return *reinterpret_cast<const GdpFrontierOut *>(back + es[j].off_out); }
     size_t labels_of(const gdp_problem *q) const { return (size_t)q->L * (alone ? GDP_KEY_LABELS : GDP_FRONTIER_LABELS); }
-    const int32_t *res_of(const char *back, int j) const { return reinterpret_cast<const int32_t *>(back + (es[j].off_res - up_bytes)); }
+    const int32_t *res_of(const char *back, int j) const { return reinterpret_cast<const int32_t *>(back + es[j].off_res); }
 };
 
 void BoundSlice::lay_out(const gdp_problem *const *p, BoundEntry *entries, int count, int multipliers, bool key_alone)
@@ -2985,10 +2985,7 @@ void BoundSlice::lay_out(const gdp_problem *const *p, BoundEntry *entries, int c
         e.off_lam = place(8 * (size_t)n_lam);
         e.off_budget = place(8 * (size_t)q->n_key);
         e.off_other_time = place(8 * (size_t)q->n_key);
-        if (e.table_of == j) {
-            e.off_inter = place(8 * (size_t)e.h.n_inter * q->S * q->S);
-            for (int t = 0; t < e.h.n_inter; ++t) pairs.push_back(make_int2(j, t));
-        }
+        if (e.table_of == j) matrices += e.h.n_inter;
         layers += q->L;
         relaxations += (double)q->L * q->V * (double)q->S * q->S;
         max_L = std::max(max_L, q->L);
@@ -3001,15 +2998,11 @@ void BoundSlice::lay_out(const gdp_problem *const *p, BoundEntry *entries, int c
     // what the instances take as dense ones, smaller or whole: 10^13 relaxations a second, a layer's latency, and the second
     // round trip
     limit_ns = relaxations / 1e4 + max_L * 5e3 + 100e3;
-    off_pairs = place(sizeof(int2) * pairs.size());
+    off_matrices = place(sizeof(GdpBoundMatrix) * (size_t)matrices);
+    head_bytes = at;
+    for (int j = 0; j < m; ++j)
+        if (es[j].table_of == j) es[j].off_inter = place(8 * (size_t)es[j].h.n_inter * p[es[j].orig]->S * p[es[j].orig]->S);
     up_bytes = at;
-    for (int j = 0; j < m; ++j) {
-        BoundEntry &e = es[j];
-        const gdp_problem *q = p[e.orig];
-        e.off_out = place(sizeof(GdpFrontierOut));
-        e.off_res = place(4 * (size_t)q->n_key * q->L);
-    }
-    back_bytes = at - up_bytes;
     keep_begin = at;
     for (int j = 0; j < m; ++j) es[j].off_keep = place((size_t)p[es[j].orig]->L * p[es[j].orig]->S);
     keep_bytes = at - keep_begin;
@@ -3036,10 +3029,19 @@ void BoundSlice::lay_out(const gdp_problem *const *p, BoundEntry *entries, int c
         e.off_hist_intra = place(alone ? 0 : 8 * GDP_FRONTIER_KEPT);
     }
     bytes = at;
+    at = 0;
+    for (int j = 0; j < m; ++j) {
+        BoundEntry &e = es[j];
+        const gdp_problem *q = p[e.orig];
+        e.off_out = place(sizeof(GdpFrontierOut));
+        e.off_res = place(4 * (size_t)q->n_key * q->L);
+    }
+    back_bytes = at;
 }
 
-void BoundSlice::fill(const gdp_problem *const *p, const std::vector<double> &magnitude, char *up, char *dev) const
+void BoundSlice::fill(const gdp_problem *const *p, const std::vector<double> &magnitude, char *up, const char *read_from, char *dev, char *back) const
 {
+    GdpBoundMatrix *matrix = reinterpret_cast<GdpBoundMatrix *>(up + off_matrices);
     for (int j = 0; j < m; ++j) {
         const BoundEntry &e = es[j], &te = es[e.table_of];
         const gdp_problem *q = p[e.orig];
@@ -3051,11 +3053,15 @@ void BoundSlice::fill(const gdp_problem *const *p, const std::vector<double> &ma
         memcpy(up + e.off_budget, e.budget.data(), 8 * e.budget.size());
         memcpy(up + e.off_other_time, q->other_time, 8 * e.budget.size());
         if (e.table_of == j)
-            for (int t = 0; t < e.h.n_inter; ++t) memcpy(up + e.off_inter + 8 * SS * (size_t)t, e.h.matrix_at(q, t), 8 * SS);
+            for (int t = 0; t < e.h.n_inter; ++t) {
+                const size_t at = 8 * SS * (size_t)t;
+                memcpy(up + e.off_inter + at, e.h.matrix_at(q, t), 8 * SS);
+                *matrix++ = {reinterpret_cast<const double *>(read_from + e.off_inter + at), reinterpret_cast<double *>(dev + e.off_inter_f + at),
+                             reinterpret_cast<double *>(dev + e.off_inter_t + at), q->S, 0};
+            }
         GdpBoundInst b;
         b.mem = reinterpret_cast<const int32_t *>(dev + e.off_mem);
         b.intra = reinterpret_cast<const double *>(dev + e.off_intra);
-        b.inter = reinterpret_cast<const double *>(dev + te.off_inter);
         b.inter_f = reinterpret_cast<double *>(dev + te.off_inter_f);
         b.inter_t = reinterpret_cast<double *>(dev + te.off_inter_t);
         b.index = reinterpret_cast<const int32_t *>(dev + e.off_index);
@@ -3075,8 +3081,8 @@ void BoundSlice::fill(const gdp_problem *const *p, const std::vector<double> &ma
         b.hist_mem = reinterpret_cast<int32_t *>(dev + e.off_hist_mem);
         b.hist_turns = reinterpret_cast<double *>(dev + e.off_hist_turns);
         b.hist_intra = reinterpret_cast<double *>(dev + e.off_hist_intra);
-        b.out = reinterpret_cast<GdpFrontierOut *>(dev + e.off_out);
-        b.res = reinterpret_cast<int32_t *>(dev + e.off_res);
+        b.out = reinterpret_cast<GdpFrontierOut *>(back + e.off_out);
+        b.res = reinterpret_cast<int32_t *>(back + e.off_res);
         b.n_hist = b.n_hist_turns = (int32_t)labels_of(q);
         b.n_lam = n_lam;
         b.magnitude = magnitude[(size_t)e.orig];
@@ -3088,14 +3094,13 @@ void BoundSlice::fill(const gdp_problem *const *p, const std::vector<double> &ma
         b.T = te.h.n_inter;
         memcpy(up + off_inst + sizeof b * (size_t)j, &b, sizeof b);
     }
-    memcpy(up + off_pairs, pairs.data(), sizeof(int2) * pairs.size());
 }
 
-hipError_t BoundSlice::enqueue(char *dev, hipStream_t stream) const
+hipError_t BoundSlice::enqueue(const char *up, char *dev, hipStream_t stream) const
 {
     const GdpBoundInst *inst = reinterpret_cast<const GdpBoundInst *>(dev + off_inst);
-    const hipError_t e = bounds::launch(inst, m, n_lam, max_LS, max_rows, max_S, max_K, changes * 4 <= layers, reinterpret_cast<const int2 *>(dev + off_pairs),
-                                           (int)pairs.size(), stream);
+    const hipError_t e = bounds::launch(inst, m, n_lam, max_LS, max_rows, max_S, max_K, changes * 4 <= layers,
+                                        {reinterpret_cast<const GdpBoundMatrix *>((up ? up : dev) + off_matrices), matrices, up, dev, head_bytes}, stream);
     if (e != hipSuccess) return e;
     return alone ? bounds::launch_key_labels(inst, m, max_K, stream) : bounds::launch_labels(inst, m, max_K, stream);
 }
@@ -3129,22 +3134,19 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
     const Lane &lane = lease.lane;
     char *const dev = lease.dev;
     std::vector<char> pageable;
-    char *up = lane.up;
-    if (lane.up_bytes < slice.up_bytes) {
-        pageable.resize(slice.up_bytes);
-        up = pageable.data();
-    }
-    slice.fill(p, magnitude, up, dev);
+    const bool pinned = lane.up_bytes >= slice.up_bytes;
+    if (!pinned) pageable.resize(slice.up_bytes);
+    char *const up = pinned ? lane.up : pageable.data();
+    slice.fill(p, magnitude, up, pinned ? up : dev, dev, lane.back);
     bool stats = false;
     {
         std::lock_guard<std::mutex> lk(g_stats_mu);
         stats = g_stats_on;
     }
-    hipError_t err = hipMemcpyAsync(dev, up, slice.up_bytes, hipMemcpyHostToDevice, lane.stream);
+    hipError_t err = pinned ? hipSuccess : hipMemcpyAsync(dev, up, slice.up_bytes, hipMemcpyHostToDevice, lane.stream);
     if (err == hipSuccess && stats) err = hipEventRecord(lane.ev_begin, lane.stream);
-    if (err == hipSuccess) err = slice.enqueue(dev, lane.stream);
+    if (err == hipSuccess) err = slice.enqueue(pinned ? up : nullptr, dev, lane.stream);
     if (err == hipSuccess && stats) err = hipEventRecord(lane.ev_end, lane.stream);
-    if (err == hipSuccess) err = hipMemcpyAsync(lane.back, dev + slice.up_bytes, slice.back_bytes, hipMemcpyDeviceToHost, lane.stream);
     while (scan.step() && hipStreamQuery(lane.stream) == hipErrorNotReady) (void)hipGetLastError();   // not one of a launch
     hipError_t es2 = hipStreamSynchronize(lane.stream);
     if (err == hipSuccess) err = es2;
@@ -3281,7 +3283,7 @@ static void take_bounds(int32_t n, const gdp_problem *const *p, const std::vecto
         b->lease.dev = nullptr;
         return;
     }
-    b->slice.fill(p, magnitude, up.data(), b->lease.dev);
+    b->slice.fill(p, magnitude, up.data(), b->lease.dev, b->lease.dev, b->lease.lane.back);
     if (hipMemcpyAsync(b->lease.dev, up.data(), b->slice.up_bytes, hipMemcpyHostToDevice, plan->stream) != hipSuccess ||
         hipStreamSynchronize(plan->stream) != hipSuccess) {
         (void)hipGetLastError();
@@ -3298,9 +3300,8 @@ static int run_bounds(gdp_plan *plan, int32_t mode, gdp_timing *t, bool *done)
     const char *const back = b.lease.lane.back;
     GDP_HIP(hipSetDevice(plan->device));
     if (mode >= 1) GDP_HIP(hipEventRecord(plan->ev_begin, plan->stream));
-    GDP_HIP(b.slice.enqueue(b.lease.dev, plan->stream));
+    GDP_HIP(b.slice.enqueue(nullptr, b.lease.dev, plan->stream));
     if (mode >= 1) GDP_HIP(hipEventRecord(plan->ev_end, plan->stream));
-    GDP_HIP(hipMemcpyAsync(b.lease.lane.back, b.lease.dev + b.slice.up_bytes, b.slice.back_bytes, hipMemcpyDeviceToHost, plan->stream));
     GDP_HIP(hipStreamSynchronize(plan->stream));
     double executed = 0;
     for (const HostInst &h : plan->inst) {

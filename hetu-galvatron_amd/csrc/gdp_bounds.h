@@ -37,10 +37,16 @@ struct GdpFrontierLabel {
     int32_t w, s;
 };
 
+// A matrix on its way to the passes, and what they read of it.
+struct GdpBoundMatrix {
+    const double *src;       // [S][S], device memory or page-locked host memory
+    double *fwd, *bwd;       // the same with GDP_BOUND_FAR for +inf, and transposed
+    int32_t S, pad;
+};
+
 struct GdpBoundInst {
     const int32_t *mem;      // [L][S]
     const double *intra;     // [L][S]
-    const double *inter;     // [T][S][S]
     double *inter_f;         // [T][S][S], GDP_BOUND_FAR for +inf
     double *inter_t;         // [T][S][S], the same with every matrix transposed
     const int32_t *index;    // [L] layer -> matrix
@@ -59,7 +65,7 @@ struct GdpBoundInst {
     GdpFrontierLabel *hist;
     int32_t *hist_mem;
     double *hist_turns, *hist_intra;
-    GdpFrontierOut *out;
+    GdpFrontierOut *out;     // this and `res`: device memory, or page-locked host memory
     int32_t *res;            // [K][L]
     double magnitude;        // sum over the layers of the largest finite |intra| and |inter|
     double limit;            // ns that the layers ahead of the DP over what stays may take, by its own account
@@ -80,11 +86,20 @@ __attribute__((visibility("hidden"))) double undominated(const gdp_problem *q);
 __attribute__((visibility("hidden"))) int key_multipliers(const gdp_problem *q);
 // The multipliers of an instance: 0 and a geometric series around (range of times) / (range of memory costs).
 __attribute__((visibility("hidden"))) void multipliers(const gdp_problem *q, int n_lam, double *lam);
-// Copies the matrices, runs the passes of all multipliers, finds the upper bounds and marks what stays.
-// max_rows: layers times (strategies / 64, rounded up).  pairs: {instance, matrix} of every matrix that is to be copied.  held: most layers have the matrix of the one before.
+// What a set of launches begins with: head_bytes (a multiple of 16) are copied from `head`, if there is one, page-locked host memory,
+// to head_to, and the matrices are laid out.
+struct Inputs {
+    const GdpBoundMatrix *matrices;
+    int n_matrices;
+    const void *head;
+    void *head_to;
+    size_t head_bytes;
+};
+// Lays out the inputs, runs the passes of all multipliers, finds the upper bounds and marks what stays.
+// max_rows: layers times (strategies / 64, rounded up).  held: most layers have the matrix of the one before.
 __attribute__((visibility("hidden")))
-hipError_t launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_rows, int max_S, int max_K, bool held, const int2 *pairs,
-                  int n_pairs, hipStream_t stream);
+hipError_t launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_rows, int max_S, int max_K, bool held, const Inputs &in,
+                  hipStream_t stream);
 // The DP over what stays, after it: a workgroup per instance (gdp_frontier.hip), or per key of each (gdp_key_labels.hip; up to
 // GDP_KEY_LABELS_MAX_L layers).
 __attribute__((visibility("hidden"))) hipError_t launch_labels(const GdpBoundInst *inst, int n, int max_K, hipStream_t stream);

@@ -27,27 +27,48 @@ namespace {
 
 static_assert(GDP_BOUND_MAX_S == 128, "two blocks of 64 targets; a strategy in the low 7 bits of a candidate");
 
-// The matrices as the passes read them: as they are and transposed, +inf replaced by GDP_BOUND_FAR.  grid (pairs, 16-row
-// bands of the largest matrix), 256 threads; LDS turns the band around so that both sides are read and written along rows.
-__global__ __launch_bounds__(256) void gdp_bound_transpose_kernel(const GdpBoundInst *inst, const int2 *pairs)
+// The inputs as the passes read them.  First workgroups of 16 KB of `head` each, which go where they are read from then on; then a
+// 16-row band of a matrix each, as it is and transposed, +inf replaced by GDP_BOUND_FAR; LDS turns the band around so that both
+// sides are read and written along rows.
+// Both may lie in page-locked host memory: what the copy engine would bring in a copy of its own, and the first kernel would wait for
+// through a signal between the two (20 us and more of a call), comes over the bus where it is needed.
+typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+constexpr int HEAD = 1024;   // times 16 bytes
+__global__ __launch_bounds__(256) void gdp_bound_prepare_kernel(const GdpBoundMatrix *matrices, int bands, const uint4v *head, uint4v *head_to, int n_head)
 {
     __shared__ double tile[16][GDP_BOUND_MAX_S + 1];
-    const int2 w = pairs[blockIdx.x];
-    const GdpBoundInst &I = inst[w.x];
-    const int S = I.S, r0 = (int)blockIdx.y * 16;
+    const int head_blocks = (n_head + HEAD - 1) / HEAD, b = (int)blockIdx.x - head_blocks;
+    if (b < 0) {
+        const int first = (int)blockIdx.x * HEAD + (int)threadIdx.x;
+        uint4v x[HEAD / 256];
+#pragma unroll
+        for (int i = 0; i < HEAD / 256; ++i) x[i] = head[min(first + 256 * i, n_head - 1)];
+#pragma unroll
+        for (int i = 0; i < HEAD / 256; ++i)
+            if (first + 256 * i < n_head) head_to[first + 256 * i] = x[i];
+        return;
+    }
+    const GdpBoundMatrix M = matrices[b / bands];
+    const int S = M.S, r0 = b % bands * 16;
     if (r0 >= S) return;
-    const int rows = S - r0 < 16 ? S - r0 : 16;
-    const double *src = I.inter + (size_t)w.y * S * S;
-    double *fwd = I.inter_f + (size_t)w.y * S * S, *bwd = I.inter_t + (size_t)w.y * S * S;
-    for (int e = threadIdx.x; e < rows * S; e += 256) {
-        const double x = fmin(src[(size_t)r0 * S + e], GDP_BOUND_FAR);
-        tile[e / S][e % S] = x;
-        fwd[(size_t)r0 * S + e] = x;
+    const int rows = S - r0 < 16 ? S - r0 : 16, all = rows * S;
+    const double *const src = M.src + (size_t)r0 * S;
+    double x[16 * GDP_BOUND_MAX_S / 256];
+#pragma unroll
+    for (int i = 0; i < 16 * GDP_BOUND_MAX_S / 256; ++i)   // all of them on their way at once
+        if (i * 256 < all) x[i] = src[min((int)threadIdx.x + 256 * i, all - 1)];
+#pragma unroll
+    for (int i = 0; i < 16 * GDP_BOUND_MAX_S / 256; ++i) {
+        const int e = (int)threadIdx.x + 256 * i;
+        if (e >= all) continue;
+        const double y = fmin(x[i], GDP_BOUND_FAR);
+        tile[e / S][e % S] = y;
+        M.fwd[(size_t)r0 * S + e] = y;
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < rows * S; e += 256) {
+    for (int e = threadIdx.x; e < all; e += 256) {
         const int c = e / rows, r = e % rows;
-        bwd[(size_t)c * S + r0 + r] = tile[r][c];
+        M.bwd[(size_t)c * S + r0 + r] = tile[r][c];
     }
 }
 
@@ -488,10 +509,12 @@ void bounds::multipliers(const gdp_problem *q, int n_lam, double *lam)
     for (int i = 1; i < n_lam; ++i) lam[i] = base * exp2(-6.0 + 12.0 * (i - 1) / (n_lam - 2));
 }
 
-hipError_t bounds::launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_rows, int max_S, int max_K, bool held, const int2 *pairs,
-                          int n_pairs, hipStream_t stream)
+hipError_t bounds::launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_rows, int max_S, int max_K, bool held, const Inputs &in,
+                          hipStream_t stream)
 {
-    gdp_bound_transpose_kernel<<<dim3((unsigned)n_pairs, (unsigned)((max_S + 15) / 16)), 256, 0, stream>>>(inst, pairs);
+    const int bands = (max_S + 15) / 16, n_head = in.head ? (int)(in.head_bytes / 16) : 0;
+    gdp_bound_prepare_kernel<<<(unsigned)((n_head + HEAD - 1) / HEAD + in.n_matrices * bands), 256, 0, stream>>>(
+        in.matrices, bands, static_cast<const uint4v *>(in.head), static_cast<uint4v *>(in.head_to), n_head);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const dim3 grid(2u * (unsigned)n_lam, (unsigned)n);

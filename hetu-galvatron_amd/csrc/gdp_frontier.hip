@@ -192,7 +192,7 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
     for (int e = t; e < BUCKETS; e += THREADS) sh.f.bucket[e] = 0;
     __syncthreads();
 
-    const gdouble inter = GLOBAL(gdouble, I.inter), intra = GLOBAL(gdouble, I.intra), Q = GLOBAL(gdouble, I.Q);
+    const gdouble inter = GLOBAL(gdouble, I.inter_f), intra = GLOBAL(gdouble, I.intra), Q = GLOBAL(gdouble, I.Q);
     const gint mem = GLOBAL(gint, I.mem);
     const giout hist_mem = GLOBAL(giout, I.hist_mem);
     const gout hist_turns = GLOBAL(gout, I.hist_turns), hist_intra = GLOBAL(gout, I.hist_intra);

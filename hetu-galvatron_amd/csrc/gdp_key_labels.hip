@@ -67,6 +67,7 @@ struct Shared {
     int32_t labels_at[GDP_KEY_LABELS_MAX_L + 1];     // where the labels of a layer begin in memory; of one strategy: none lie there
     int32_t labels_of[GDP_KEY_LABELS_MAX_L];         // how many there are
     int2 step[GDP_KEY_LABELS_MAX_L + 1];             // strategies of a layer, and how many layers from it on have one behind one
+    int32_t res[GDP_KEY_LABELS_MAX_L];               // the strategies of the best path
     int32_t several_before[GDP_KEY_LABELS_MAX_L];    // the last layer before it of more than one, -1: none
     int32_t found[3];                                // labels of a layer, of the next one of all waves and the one after that
     int32_t lost, unsorted;
@@ -176,7 +177,7 @@ __global__ __launch_bounds__(THREADS) void gdp_key_labels_kernel(const GdpBoundI
     }
     const int32_t budget = uniform((int32_t)B);
     double ub = uniform(gdp_unordered(known));
-    const gdouble Q = GLOBAL(gdouble, I.Q), intra = GLOBAL(gdouble, I.intra), inter = GLOBAL(gdouble, I.inter);
+    const gdouble Q = GLOBAL(gdouble, I.Q), intra = GLOBAL(gdouble, I.intra), inter = GLOBAL(gdouble, I.inter_f);
     const gint Q_mem = GLOBAL(gint, I.Q_mem), mem = GLOBAL(gint, I.mem);
     const glabel hist = GLOBAL(glabel, I.hist) + (size_t)own_key * I.n_hist;
     const int n_hist = uniform(I.n_hist);
@@ -262,8 +263,7 @@ __global__ __launch_bounds__(THREADS) void gdp_key_labels_kernel(const GdpBoundI
         if (l < L) sh.several_before[l] = before;
     }
     if (t == 128) sh.step[128] = make_int2(0, 0);
-    const giout res = GLOBAL(giout, I.res) + (size_t)own_key * L;
-    if (t < L && sh.layer[t].x == 1) res[t] = sh.kept[sh.layer[t].y] & 127;
+    if (t < L && sh.layer[t].x == 1) sh.res[t] = sh.kept[sh.layer[t].y] & 127;
     __syncthreads();
 
     // ---- what the layers need, in LDS ----
@@ -825,7 +825,7 @@ __global__ __launch_bounds__(THREADS) void gdp_key_labels_kernel(const GdpBoundI
 
     // ---- backwards ----
     // Layers with one strategy are passed by in one step; of the others wave 0 looks for the cheapest label that leads to the cell.
-    if (t == 0) res[L - 1] = sh.kept[sh.layer[L - 1].y + cell] & 127;
+    if (t == 0) sh.res[L - 1] = sh.kept[sh.layer[L - 1].y + cell] & 127;
     int walk = L - 1;        // the layer of the cell
     bool paid = false;       // whether its budget is that before it already
     for (int chunk = chunks - 1, top = L - 1; chunk >= 0; --chunk) {
@@ -899,7 +899,7 @@ __global__ __launch_bounds__(THREADS) void gdp_key_labels_kernel(const GdpBoundI
                     walk = step.next;
                     const int4 at_walk = sh.layer[walk];
                     cell = min(s, uniform(at_walk.x) - 1);   // (there is one: the cell has a cost)
-                    if (lane == 0) res[walk] = sh.kept[at_walk.y + cell] & 127;
+                    if (lane == 0) sh.res[walk] = sh.kept[at_walk.y + cell] & 127;
                     row = uniform(at_walk.y) - k0;
                     paid = false;
                     step = after;
@@ -908,6 +908,9 @@ __global__ __launch_bounds__(THREADS) void gdp_key_labels_kernel(const GdpBoundI
             top = lowest - 1;
         }
     }
+    __syncthreads();
+    const giout res = GLOBAL(giout, I.res) + (size_t)own_key * L;
+    if (t < L) res[t] = sh.res[t];
     if (t == 0) {
         out->total[own_key] = total + GLOBAL(gdouble, I.other_time)[own_key];
         out->remaining[own_key] = v;

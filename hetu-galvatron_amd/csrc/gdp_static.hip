@@ -255,7 +255,7 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
         off = align_up(off + bytes, 256);
         return o;
     };
-    const size_t off_inst = take(sizeof(GdpBoundInst)), off_pairs = take(sizeof(int2) * (size_t)T), off_mem = take(4 * LS),
+    const size_t off_inst = take(sizeof(GdpBoundInst)), off_matrices = take(sizeof(GdpBoundMatrix) * (size_t)T), off_mem = take(4 * LS),
                  off_intra = take(8 * LS), off_inter = take(8 * SS * (size_t)T), off_index = take(4 * (size_t)L),
                  off_lam = take(8 * NL), off_budget = take(8 * (size_t)K), off_other_time = take(8 * (size_t)K), up_bytes = off,
                  off_out = take(sizeof(GdpFrontierOut)), off_res = take(4 * (size_t)K * L), back_bytes = off - up_bytes,
@@ -277,13 +277,14 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     bounds::multipliers(p, (int)NL, reinterpret_cast<double *>(g_stage + off_lam));
     memcpy(g_stage + off_budget, budget, 8 * (size_t)K);
     memcpy(g_stage + off_other_time, p->other_time, 8 * (size_t)K);
-    int2 *pairs = reinterpret_cast<int2 *>(g_stage + off_pairs);
-    for (int t = 0; t < T; ++t) pairs[t] = make_int2(0, t);
+    GdpBoundMatrix *matrices = reinterpret_cast<GdpBoundMatrix *>(g_stage + off_matrices);
+    for (int t = 0; t < T; ++t)
+        matrices[t] = {reinterpret_cast<const double *>(base + off_inter) + SS * (size_t)t, reinterpret_cast<double *>(base + off_inter_f) + SS * (size_t)t,
+                       reinterpret_cast<double *>(base + off_inter_t) + SS * (size_t)t, S, 0};
     GdpBoundInst b;
     memset(&b, 0, sizeof b);
     b.mem = reinterpret_cast<const int32_t *>(base + off_mem);
     b.intra = reinterpret_cast<const double *>(base + off_intra);
-    b.inter = reinterpret_cast<const double *>(base + off_inter);
     b.inter_f = reinterpret_cast<double *>(base + off_inter_f);
     b.inter_t = reinterpret_cast<double *>(base + off_inter_t);
     b.index = reinterpret_cast<const int32_t *>(base + off_index);
@@ -315,7 +316,8 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     hipError_t e = hipMemcpy(base, g_stage, up_bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) return gdp_fail_hip(e, "gdp_solve_static: upload");
     const GdpBoundInst *inst = reinterpret_cast<const GdpBoundInst *>(base + off_inst);
-    e = bounds::launch(inst, 1, (int)NL, (int)LS, L * ((S + 63) / 64), S, K, changes * 4 <= L, reinterpret_cast<const int2 *>(base + off_pairs), T, stream);
+    e = bounds::launch(inst, 1, (int)NL, (int)LS, L * ((S + 63) / 64), S, K, changes * 4 <= L,
+                       {reinterpret_cast<const GdpBoundMatrix *>(base + off_matrices), T, nullptr, nullptr, 0}, stream);
     if (e == hipSuccess) e = alone ? bounds::launch_key_labels(inst, 1, K, stream) : bounds::launch_labels(inst, 1, K, stream);
     if (e != hipSuccess) {
         (void)hipDeviceSynchronize();
