@@ -78,6 +78,7 @@ typedef const __attribute__((address_space(1))) double *gdouble;
 typedef const __attribute__((address_space(1))) int32_t *gint;
 typedef __attribute__((address_space(1))) double *gout;
 typedef __attribute__((address_space(1))) uint32_t *guint;
+typedef const __attribute__((address_space(1))) uint32_t *guint_in;
 typedef __attribute__((address_space(1))) unsigned long long *gulong;
 
 __device__ __forceinline__ double min_f64(double a, double b)
@@ -297,6 +298,32 @@ __device__ __forceinline__ unsigned long long ordered(double x)
     return b >> 63 ? ~b : b | 1ull << 63;
 }
 
+__device__ __forceinline__ double of_lane(double x, int lane)
+{
+    const int2v w = __builtin_bit_cast(int2v, x);
+    const int2v r = {__builtin_amdgcn_readlane(w.x, lane), __builtin_amdgcn_readlane(w.y, lane)};
+    return __builtin_bit_cast(double, r);
+}
+
+// Minimum over a wave, in all lanes.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double lower_of_moved(double x)
+{
+    const int2v w = __builtin_bit_cast(int2v, x);   // a lane without a source keeps its own
+    const int2v m = {__builtin_amdgcn_update_dpp(w.x, w.x, CTRL, ROWS, 0xf, false), __builtin_amdgcn_update_dpp(w.y, w.y, CTRL, ROWS, 0xf, false)};
+    return min_f64(x, __builtin_bit_cast(double, m));
+}
+__device__ __forceinline__ double lowest_of(double x)
+{
+    x = lower_of_moved<0x111, 0xf>(x);   // row_shr:1, 2, 4, 8
+    x = lower_of_moved<0x112, 0xf>(x);
+    x = lower_of_moved<0x114, 0xf>(x);
+    x = lower_of_moved<0x118, 0xf>(x);
+    x = lower_of_moved<0x142, 0xa>(x);   // row_bcast:15, 31
+    x = lower_of_moved<0x143, 0xc>(x);
+    return of_lane(x, 63);
+}
+
 // Upper bound of one key: the best path that fits among all that go the cheapest way to some (l, s) under one multiplier
 // and the cheapest way on under another, both of the GDP_BOUND_WINDOW around the one whose bound is the best.  Where all
 // layers are alike every layer changes its strategy at the same multiplier, and only such a splice comes near the
@@ -307,47 +334,40 @@ __global__ __launch_bounds__(256) void gdp_bound_upper_kernel(const GdpBoundInst
 {
     constexpr int W = GDP_BOUND_WINDOW;
     __shared__ double red[4];
-    __shared__ int first;
     const GdpBoundInst &I = inst[blockIdx.z];
-    const int key = (int)blockIdx.y, t = (int)threadIdx.x, LS = I.L * I.S;
-    if (key >= I.K || (int)blockIdx.x * 256 >= LS || I.budget[key] < 0) return;   // the whole workgroup
-    const int64_t B = I.budget[key];
-    if (t < 64) {
-        double d = -INFINITY;
-        int i = n_lam;
-        for (int at = t; at < n_lam; at += 64) {
-            const double e = I.end[at] - I.lam[at] * (double)B;
-            if (e > d) {
-                d = e;
-                i = at;
-            }
-        }
-#pragma unroll
-        for (int w = 32; w > 0; w >>= 1) {
-            const double e = __shfl_xor(d, w);
-            const int j = __shfl_xor(i, w);
-            if (e > d || (e == d && j < i)) {
-                d = e;
-                i = j;
-            }
-        }
-        if (t == 0) {
-            first = max(0, min(i - W / 2, n_lam - W));
-            if (blockIdx.x == 0) I.best[key] = i;
+    const int key = (int)blockIdx.y, t = (int)threadIdx.x, lane = t & 63, LS = I.L * I.S;
+    if (key >= I.K || (int)blockIdx.x * 256 >= LS) return;   // the whole workgroup
+    const gdouble P = (gdouble)(uintptr_t)I.P, Q = (gdouble)(uintptr_t)I.Q, lams = (gdouble)(uintptr_t)I.lam, ends = (gdouble)(uintptr_t)I.end;
+    const guint_in P_mem = (guint_in)(uintptr_t)I.P_mem, Q_mem = (guint_in)(uintptr_t)I.Q_mem;
+    const int64_t B = ((const __attribute__((address_space(1))) int64_t *)(uintptr_t)I.budget)[key];
+    // the best multiplier, every wave for itself
+    double d = -INFINITY;
+    int at_d = 0;
+    for (int at = lane; at < n_lam; at += 64) {
+        const double e = ends[at] - lams[at] * (double)B;
+        if (e > d) {
+            d = e;
+            at_d = at;
         }
     }
-    __syncthreads();
+    if (B < 0) return;   // the whole workgroup
+    const double most = -lowest_of(-d);
+    int best_at = n_lam;
+    for (unsigned long long with = __builtin_amdgcn_ballot_w64(d == most); with; with &= with - 1)
+        best_at = min(best_at, __builtin_amdgcn_readlane(at_d, __builtin_ctzll(with)));
+    const int first = max(0, min(best_at - W / 2, n_lam - W));
+    if (blockIdx.x == 0 && t == 0) I.best[key] = best_at;
     const int e = min((int)blockIdx.x * 256 + t, LS - 1);
     double p[W], q[W], lam[W];
     uint32_t pm[W], qm[W];
 #pragma unroll
     for (int i = 0; i < W; ++i) {
         const size_t at = (size_t)(first + i) * LS + e;
-        p[i] = I.P[at];
-        q[i] = I.Q[at];
-        pm[i] = I.P_mem[at];
-        qm[i] = I.Q_mem[at];
-        lam[i] = I.lam[first + i];
+        p[i] = P[at];
+        q[i] = Q[at];
+        pm[i] = P_mem[at];
+        qm[i] = Q_mem[at];
+        lam[i] = lams[first + i];
     }
     double best = INFINITY;
 #pragma unroll
@@ -360,9 +380,8 @@ __global__ __launch_bounds__(256) void gdp_bound_upper_kernel(const GdpBoundInst
 #pragma unroll
         for (int j = 0; j < W; ++j)
             if ((int64_t)(pm[i] + qm[j]) <= B) best = fmin(best, p[i] + q[j]);
-#pragma unroll
-    for (int w = 32; w > 0; w >>= 1) best = fmin(best, __shfl_xor(best, w));
-    if ((t & 63) == 0) red[t >> 6] = best;
+    best = lowest_of(best);
+    if (lane == 0) red[t >> 6] = best;
     __syncthreads();
     if (t != 0) return;
     best = fmin(fmin(red[0], red[1]), fmin(red[2], red[3]));
@@ -388,37 +407,41 @@ __global__ __launch_bounds__(64 * PARTS * ROWS) void gdp_bound_keep_kernel(const
               s = 64 * half + lane;
     if (l >= L) return;   // the whole workgroup, or a wave that meets no other
     const int at = l * S + min(s, S - 1);
-    unsigned alive = 0;
-    double ub[GDP_BOUND_MAX_KEY], budget[GDP_BOUND_MAX_KEY];
-#pragma unroll
-    for (int k = 0; k < GDP_BOUND_MAX_KEY; ++k) {
-        ub[k] = INFINITY;
-        budget[k] = 0.0;
-        if (k < K && I.budget[k] >= 0) {
-            alive |= 1u << k;
-            ub[k] = gdp_unordered(I.ub[k]);
-            budget[k] = (double)I.budget[k];
-        }
-    }
+    // the keys: a lane each asks for what is known of it, all at once
+    const int own = min(lane, K - 1);
+    const int64_t own_budget = ((const __attribute__((address_space(1))) int64_t *)(uintptr_t)I.budget)[own];
+    const unsigned long long own_ub = ((const __attribute__((address_space(1))) unsigned long long *)(uintptr_t)I.ub)[own];
+    const int V = I.V;
+    const double magnitude = I.magnitude;
     const gdouble P = (gdouble)(uintptr_t)I.P, Q = (gdouble)(uintptr_t)I.Q, lams = (gdouble)(uintptr_t)I.lam;
     const gulong marks = (gulong)(uintptr_t)I.marks;   // (here: behind a store the compiler would fetch it again)
     __attribute__((address_space(1))) uint8_t *const keep = (__attribute__((address_space(1))) uint8_t *)(uintptr_t)I.keep;
+    unsigned alive = (1u << K) - 1;
+    double ub[GDP_BOUND_MAX_KEY], budget[GDP_BOUND_MAX_KEY];
     for (int i0 = 8 * part; i0 < n_lam; i0 += 8 * PARTS) {
-        double p[8], q[8];
+        double p[8], q[8], lam[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {   // beyond the last: the last once more
             const size_t row = (size_t)min(i0 + i, n_lam - 1) * LS + at;
             p[i] = P[row];
             q[i] = Q[row];
+            lam[i] = lams[min(i0 + i, n_lam - 1)];
+        }
+        if (i0 == 8 * part) {
+            const double as_double = (double)own_budget, bound = own_budget >= 0 ? gdp_unordered(own_ub) : -INFINITY;   // (no solution: nothing stays)
+#pragma unroll
+            for (int k = 0; k < GDP_BOUND_MAX_KEY; ++k) {
+                budget[k] = of_lane(as_double, k);
+                ub[k] = of_lane(bound, k);
+            }
         }
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const double lam = lams[min(i0 + i, n_lam - 1)];
             const double r = p[i] + q[i];
-            const double margin = gdp_bound_margin(I.L, I.V, I.magnitude, lam);
+            const double margin = gdp_bound_margin(L, V, magnitude, lam[i]);
 #pragma unroll
             for (int k = 0; k < GDP_BOUND_MAX_KEY; ++k)
-                if (k < K && r - lam * budget[k] > ub[k] + margin) alive &= ~(1u << k);
+                if (k < K && r - lam[i] * budget[k] > ub[k] + margin) alive &= ~(1u << k);
         }
     }
     if constexpr (PARTS > 1) {
