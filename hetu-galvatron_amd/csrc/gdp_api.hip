@@ -2791,35 +2791,34 @@ static bool bounds_pay(int32_t n, const gdp_problem *const *p)
     return save >= std::max(max_L * (wide ? STEP_16 : STEP), passes * (wide ? BUSY_16 : BUSY)) + (n > 1 ? entries * ENTRY * undominated(n, p) : 0.0);
 }
 
-// The same for a call of one instance, below bounds_pay's floor: where its labels stay few, the whole call is one round
-// trip of 55 us + L * (2.3 + 0.06 S) us, host included, against 60 us + L * (2.8 + 0.085 S) us of the launch schemes and
-// their relaxations.  How many labels there will be is not known before; what tells it best is how many strategies of a
-// layer no other one dominates, times the layers (4 of them are looked at), unless layers are alike: then whatever trades
-// memory for time does so in every one.  Whole / by labels, us, means of 5 inputs each (*: taken):
-//   layers of their own, random costs (2 to 8 of S undominated)   * L = 6, S = 24, 3e7 81 / 77    * L = 12, S = 24, 1e8 108 / 94
-//     L = 28, S = 40, 3e8 221 / 168    L = 28, S = 88, 2e8 419 / 310    L = 60, S = 20, 2e8 304 / 240    L = 128, S = 8, 2e8 502 / 497
-//     (these four have more than 80 undominated strategies over all layers)
-//   ... that follow a layout (5 to 24)  L = 8, S = 44, 2e8 113 / 103   L = 28, S = 44, 2e8 229 / 263   L = 60, S = 20, 2e8 305 / 369
-//   layers alike, a layout  L = 6, S = 40, 1e8 93 / 97; * 3e8 108 / 96   L = 12, S = 40, 3e8 136 / 144; * 7e8 165 / 142
-//     L = 28, S = 40, 7e8 232 / 278; * 1.5e9 312 / 259   L = 60, S = 24, 7e8 330 / 389; 1.5e9 514 / 406; S = 40, 1.5e9 491 / 495
-// So few of a layer and layers of their own take them from 3e7 relaxations on -- below 80 over all layers none of 150 inputs lost more
-// than 8 %, from 84 on some do, up to a third --, everything else from 5e7 a layer, as in bounds_pay.  Initial
-// costs are looked through while the device works; where that takes longer than the chain of layers nothing is gained.
+// The same for a call of one instance, below bounds_pay's floor.  The launch schemes take 60 us + L * (2.8 + 0.085 S) us and their
+// relaxations; by labels it is a round trip of 50 us and, where each key has its workgroup, what its labels take: which is not known
+// before, what tells it best is how many strategies no other one dominates, over the layers (4 of them are looked at) and keys -- a
+// key whose labels are too many takes the call back to the launch schemes.  500 of them are taken from 3e7 relaxations on, more where
+// that is 0.5 us each at most.  Of 520 random calls (L = 3 to 80, S = 5 to 88, 1 to 5 keys; layers alike, two sorts, their own) 286
+// go by labels then, in 53.5 of 97 ms; 4 of them are more than 1.05 times as slow as whole.  us, whole / by labels (*: taken):
+//   layers alike, random costs  * L = 24, S = 22, 1.9e8, 4 keys 157 / 70    L = 8, S = 16, 2.9e7 80 / 62
+//   layers of their own  * L = 32, S = 44, 4e9 668 / 150   * L = 27, S = 16, 5.3e7 155 / 113   * L = 53, S = 5, 4.4e7 219 / 294
+//   layers alike that follow a layout (7 to 20 undominated)  * L = 13, S = 18, 3e7 104 / 96    L = 28, S = 40, 1.3e9 282 / 258 to 440
+//     L = 58, S = 12, 4.8e7 251 / 604    L = 28, S = 80, 6.8e8 354 / 389
+// The workgroup that all keys share is slower; for its sake layers of their own with 80 at most, however many keys there are, and
+// everything from 5e7 a layer, as in bounds_pay.  Initial costs are looked through while the device works, at 45 GB/s of
+// memory: where that takes longer than the launch schemes nothing is gained.
 static bool labels_pay(const gdp_problem *q, size_t scanned)
 {
-    constexpr double LEAST = 3e7, MANY = 3e8, MANY_LAYER = 5e7, FEW = 80;
+    constexpr double LEAST = 3e7, MANY = 3e8, MANY_LAYER = 5e7, FEW = 80, FEW_OF_KEYS = 500, EACH = 0.5e-6;
     if (!bounds::has_form(q) || q->S > 88) return false;
-    const double work = (double)q->L * q->V * q->S * q->S;
-    if (work < LEAST) return false;
-    if (work >= std::max(MANY, MANY_LAYER * q->L) && InitialScan::device_bound(work, scanned)) return true;
-    if ((double)scanned / 35e9 > q->L * (2.8e-6 + 0.085e-6 * q->S)) return false;
+    const double work = (double)q->L * q->V * q->S * q->S, chain = q->L * (2.8e-6 + 0.085e-6 * q->S), whole = chain + work / 1.2e13;
+    if (work < LEAST || (double)scanned / 45e9 > whole) return false;
+    if (work >= std::max(MANY, MANY_LAYER * q->L)) return true;
+    const double share = bounds::undominated(q), expected = share * q->S * q->L;
+    if (q->L <= GDP_KEY_LABELS_MAX_L && share <= GDP_KEY_LABELS_MOST && expected * q->n_key <= std::max(FEW_OF_KEYS, whole / EACH)) return true;
     int alike = 0;
     for (int l = 1; l < q->L; ++l) {
         const size_t at = (size_t)l * q->S, before = at - q->S;
         alike += memcmp(q->mem + at, q->mem + before, sizeof(int32_t) * q->S) == 0 && memcmp(q->intra + at, q->intra + before, sizeof(double) * q->S) == 0;
     }
-    if (alike * 4 > q->L) return false;
-    return bounds::undominated(q) * q->S * q->L <= FEW;
+    return alike * 4 <= q->L && expected <= FEW;
 }
 
 // The smaller instance of q, given what stays ([L][S]); false where it would not be a good deal smaller.

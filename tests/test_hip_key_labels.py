@@ -111,3 +111,23 @@ def test_the_kernel_needs_nothing_obtained_for_a_launch(tmp_path):
     undefined = subprocess.run(["nm", "-u", "-C", obj], stdout=subprocess.PIPE, text=True, check=True).stdout
     for name in (ln.split(None, 1)[1].strip() for ln in undefined.splitlines() if ln.strip().startswith("U ")):
         assert not name.startswith(("hipMalloc", "hipHost", "hipMem", "hipStream", "hipEvent", "hipFree", "operator", "malloc", "calloc", "std::__throw")), name
+
+
+# On either side of each term of the rule for a call: 3e7 relaxations, undominated strategies over layers and keys, their share, the
+# layers a workgroup has words for; initial costs that take longer to look through than the launch schemes, and that do not
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,L,S,V,n_keys,zeros,labels", [("alike", 24, 22, 16384, 4, False, True), ("alike", 24, 22, 16384, 8, False, False),
+                                                            ("alike", 24, 22, 2500, 4, False, False), ("trade", 20, 24, 16000, 4, False, False),
+                                                            ("runs", 128, 8, 9000, 1, False, True), ("runs", 129, 8, 9000, 1, False, False),
+                                                            ("alike", 24, 22, 16384, 4, True, True), ("each", 8, 24, 60000, 2, True, False),
+                                                            ("each", 8, 24, 60000, 2, False, True)])
+def test_calls_around_the_rule(kind, L, S, V, n_keys, zeros, labels, monkeypatch):
+    monkeypatch.delenv("GALVATRON_DP_REDUCE", raising=False)
+    monkeypatch.delenv("GALVATRON_DP_SKIP", raising=False)
+    x = _instance(L, S, V, kind, n_keys)
+    prob = _lib.Problem(x[0], x[1], x[2], V, x[3], x[4], f0=np.zeros((V, S)) if zeros else None)
+    _lib.batch_stats_begin()
+    _lib.solve_batch([prob])
+    s = _lib.batch_stats_end()
+    assert (s.executed < 0.01 * s.relaxations) == labels
+    _same(prob, x, V, f"{kind} {L} {S} {V} {n_keys} {zeros}")
