@@ -34,7 +34,7 @@ static_assert(GDP_BOUND_MAX_S == 128, "two blocks of 64 targets; a strategy in t
 // through a signal between the two (20 us and more of a call), comes over the bus where it is needed.
 typedef unsigned uint4v __attribute__((ext_vector_type(4)));
 constexpr int HEAD = 1024;   // times 16 bytes
-__global__ __launch_bounds__(256) void gdp_bound_prepare_kernel(const GdpBoundMatrix *matrices, int bands, const uint4v *head, uint4v *head_to, int n_head)
+__global__ __launch_bounds__(256) void gdp_bound_transpose_kernel(const GdpBoundMatrix *matrices, int bands, const uint4v *head, uint4v *head_to, int n_head)
 {
     __shared__ double tile[16][GDP_BOUND_MAX_S + 1];
     const int head_blocks = (n_head + HEAD - 1) / HEAD, b = (int)blockIdx.x - head_blocks;
@@ -536,7 +536,7 @@ hipError_t bounds::launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS
                           hipStream_t stream)
 {
     const int bands = (max_S + 15) / 16, n_head = in.head ? (int)(in.head_bytes / 16) : 0;
-    gdp_bound_prepare_kernel<<<(unsigned)((n_head + HEAD - 1) / HEAD + in.n_matrices * bands), 256, 0, stream>>>(
+    gdp_bound_transpose_kernel<<<(unsigned)((n_head + HEAD - 1) / HEAD + in.n_matrices * bands), 256, 0, stream>>>(
         in.matrices, bands, static_cast<const uint4v *>(in.head), static_cast<uint4v *>(in.head_to), n_head);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
