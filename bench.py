@@ -79,11 +79,11 @@ PEAK_HBM_GBS = 8000.0
 # bench line carries it only while both still match, null otherwise.
 MEASURED_TRAFFIC = {
     # workload (+ mode): (bytes per launch, kernel sources hash, register tile "TSxR", profile)
-    "cfg2": (12.131e9, "4ed01c2a4281373f", "16x1", "profiles/gdp_relax_fused_kernel_cfg2.txt"),                 # algorithmic 10.737e9
-    "cfg2+row_skipping": (7.651e9, "4ed01c2a4281373f", "16x1", "profiles/gdp_relax_fused_kernel_cfg2_row_skipping.txt"),
-    "cfg2+mark_table": (12.209e9, "4ed01c2a4281373f", "8x2", "profiles/gdp_relax_fused_kernel_cfg2_mark_table.txt"),  # algorithmic 11.409e9
-    "cfg3": (45.82e9, "4ed01c2a4281373f", "15x3", "profiles/gdp_relax_fused_kernel_cfg3.txt"),   # algorithmic 44.3e9; average of the 4 launches of a solve
-    "cfg4": (17.596e9, "4ed01c2a4281373f", "15x3", "profiles/gdp_relax_fused_kernel_cfg4.txt"),                 # algorithmic 17.716e9
+    "cfg2": (12.131e9, "c2bf34df7147a1b8", "16x1", "profiles/gdp_relax_fused_kernel_cfg2.txt"),                 # algorithmic 10.737e9
+    "cfg2+row_skipping": (7.653e9, "c2bf34df7147a1b8", "16x1", "profiles/gdp_relax_fused_kernel_cfg2_row_skipping.txt"),
+    "cfg2+mark_table": (12.212e9, "c2bf34df7147a1b8", "8x2", "profiles/gdp_relax_fused_kernel_cfg2_mark_table.txt"),  # algorithmic 11.409e9
+    "cfg3": (45.75e9, "c2bf34df7147a1b8", "15x3", "profiles/gdp_relax_fused_kernel_cfg3.txt"),   # algorithmic 44.3e9; average of the 4 launches of a solve
+    "cfg4": (17.612e9, "c2bf34df7147a1b8", "15x3", "profiles/gdp_relax_fused_kernel_cfg4.txt"),                 # algorithmic 17.716e9
 }
 KERNEL_SOURCES = ("hetu-galvatron_amd/csrc/gdp_kernels.hip", "hetu-galvatron_amd/csrc/gdp_kernels.h")
 GOLDEN = os.path.join(ROOT, "tests", "golden", "dp_core_golden.json")

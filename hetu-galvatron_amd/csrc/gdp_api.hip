@@ -201,7 +201,7 @@ struct Lane {
     hipEvent_t ev_back = nullptr;  // after the copy of the results (a flow run queues more work behind it)
     hipStream_t side = nullptr;    // second stream: the upload of a small plan's inputs runs beside the kernel that
     hipEvent_t ev_side = nullptr;  // prepares its cost buffers; the event joins it to the main stream
-    char *back = nullptr;  // page-locked host memory the results are copied into
+    char *back = nullptr;  // page-locked host memory the results are written into
     size_t back_bytes = 0;
     char *up = nullptr;    // page-locked host memory the inputs' device layout is built in (may be absent)
     size_t up_bytes = 0;
@@ -552,8 +552,7 @@ struct gdp_plan {
     hipStream_t stream = nullptr;    // = lane.stream
     hipEvent_t ev_begin = nullptr, ev_end = nullptr;
     std::vector<hipEvent_t> ev_relax;  // pairs
-    // What a run copies back in one piece: abort flag, per-key outputs, strategy lists (device offsets
-    // off_abort .. off_res + its size; the same offsets relative to off_abort inside lane.back).
+    // What a run writes into lane.back: abort flag, per-key outputs (off_out), strategy lists (off_res).
     size_t back_bytes = 0;
     const GdpDevOut *h_out = nullptr;
     const int32_t *h_res = nullptr;
@@ -1405,7 +1404,7 @@ PlanBuilder::FlowPick PlanBuilder::flow_pick(const Group &g) const
 }
 
 // Device layout, first part: [tables | per-instance inputs] (uploaded in one copy), then the words every run
-// resets and the results (copied back in one piece).
+// resets.
 int PlanBuilder::lay_out_tables()
 {
     off = 0;
@@ -1485,11 +1484,11 @@ int PlanBuilder::lay_out_tables()
     }
     pl->off_abort = take(sizeof(int32_t));
     pl->zero_words = (off - pl->off_zero) / sizeof(int32_t);
-    // abort flag, per-key outputs and strategy lists lie together: a run copies them back in one piece
-    pl->off_out = take(sizeof(GdpDevOut) * (size_t)std::max(nk, 1));
-    pl->off_res = take(sizeof(int32_t) * std::max<size_t>(nres, 1));
-    pl->back_bytes = off - pl->off_abort;
     fixed_bytes = off;
+    // lane.back, which a run writes its results to: abort flag, per-key outputs, strategy lists
+    pl->off_out = 256;
+    pl->off_res = align_up(pl->off_out + sizeof(GdpDevOut) * (size_t)std::max(nk, 1), 256);
+    pl->back_bytes = pl->off_res + sizeof(int32_t) * std::max<size_t>(nres, 1);
     return GDP_OK;
 }
 
@@ -1864,18 +1863,26 @@ void PlanBuilder::build_group_tables()
 // The tables onto the device, and the parts of the cost buffers that no run ever overwrites.
 int PlanBuilder::upload()
 {
-    // A flow plan (small): the tables go first, the kernel that prepares the cost buffers needs nothing else;
+    // Tables and inputs up to PULLED_MOST are brought over the bus by a kernel on the plan's own stream, at 46 GB/s: the copy
+    // engine takes the host 10 us longer to start, and what comes on a second stream is waited for 20 us after it has ended.  Larger ones
+    // gain more beside the kernel that prepares the cost buffers.  With the results, which the last kernel writes to the host: 70 random calls
+    // under 200 us 9 us less each, L = 4, S = 6, V = 640 66 -> 50 us; L = 28, S = 40, V = 29493 (0.36 MB) 295 us either way.
+    constexpr size_t PULLED_MOST = (size_t)384 << 10;
+    const bool pulled = stage.p == pl->lane.up && small_bytes <= PULLED_MOST;
+    // Of a larger flow plan the tables go first, the kernel that prepares the cost buffers needs nothing else;
     // the per-instance inputs follow on a second stream, beside that kernel.
     size_t tables_bytes = small_bytes;
     bool &split_upload = pl->split_upload;
-    split_upload = turn_free;
-    if (prepared_early) {
+    split_upload = turn_free && !pulled;
+    if (pulled) {
+        GDP_HIP(gdp_launch_pull(stage.data(), pl->dbase, small_bytes, pl->stream));
+    } else if (prepared_early) {
         tables_bytes = 0;      // everything over the second stream, beside the kernel that is already running
     } else if (split_upload) {
         for (const auto &h : inst) tables_bytes = std::min(tables_bytes, h.off_inter);
         split_upload = tables_bytes > 0 && tables_bytes < small_bytes;
     }
-    if (!prepared_early)
+    if (!prepared_early && !pulled)
         GDP_HIP(hipMemcpyAsync(pl->dbase, stage.data(), split_upload ? tables_bytes : small_bytes, hipMemcpyHostToDevice,
                                pl->stream));
     if (split_upload) {
@@ -1889,7 +1896,7 @@ int PlanBuilder::upload()
         // A plan laid out for the flow launch gets NaN into its bands here if the turn is free right now (its
         // first run will most likely flow), else when a run first takes that way: a plan that finds the turn
         // taken every time never pays for it.
-        const bool nan_bands = split_upload;
+        const bool nan_bands = pulled ? turn_free : split_upload;
         for (const Group &g : pl->groups) {
             if (prepared_early) continue;
             if (!nan_bands)   // (one launch instead of three pays only where the three are short)
@@ -1975,8 +1982,6 @@ int audit_sub_allocations(const gdp_plan *pl)
     auto span = [&](size_t lo, size_t bytes) { spans.push_back({lo, lo + bytes}); };
     span(pl->off_insts, sizeof(GdpDevInst) * (size_t)pl->n);
     span(pl->off_keys, sizeof(GdpDevKey) * (size_t)std::max(pl->n_key_total, 1));
-    span(pl->off_out, sizeof(GdpDevOut) * (size_t)std::max(pl->n_key_total, 1));
-    span(pl->off_res, sizeof(int32_t) * std::max<size_t>(pl->n_res_total, 1));
     span(pl->off_abort, sizeof(int32_t));
     for (const Group &g : pl->groups) {
         span(g.off_active, sizeof(int32_t) * (size_t)g.max_L);
@@ -2189,15 +2194,13 @@ size_t relax_launches(const gdp_plan *pl)
     return launches;
 }
 
-// Everything of a run that does not wait: the launches and the copy of the results into the plan's
+// Everything of a run that does not wait: the launches, the last of which writes the results into the plan's
 // page-locked buffer, on the plan's stream.
 int run_enqueue(gdp_plan *pl, int32_t mode)
 {
     GDP_HIP(hipSetDevice(pl->device));
     const GdpDevInst *d_insts = reinterpret_cast<const GdpDevInst *>(pl->dbase + pl->off_insts);
     const GdpDevKey *d_keys = reinterpret_cast<const GdpDevKey *>(pl->dbase + pl->off_keys);
-    GdpDevOut *d_out = reinterpret_cast<GdpDevOut *>(pl->dbase + pl->off_out);
-    int32_t *d_res = reinterpret_cast<int32_t *>(pl->dbase + pl->off_res);
     pl->run_flow = false;
     // A plan that gave a waiting launch up runs with one launch per layer -- until the time has passed for which
     // the library avoids such launches after a give-up; then it is armed again with the scheme it was given.
@@ -2286,10 +2289,10 @@ int run_enqueue(gdp_plan *pl, int32_t mode)
                 ++li;
             }
     }
-    GDP_HIP(gdp_launch_epilogue(pl->keep_marks, d_insts, d_keys, pl->n_key_total, d_out, d_res, pl->stream));
+    GDP_HIP(gdp_launch_epilogue(pl->keep_marks, d_insts, d_keys, pl->n_key_total, reinterpret_cast<GdpDevOut *>(pl->lane.back + pl->off_out),
+                                reinterpret_cast<int32_t *>(pl->lane.back + pl->off_res), reinterpret_cast<const int32_t *>(pl->dbase + pl->off_abort),
+                                reinterpret_cast<int32_t *>(pl->lane.back), pl->stream));
     if (mode >= 1) GDP_HIP(hipEventRecord(pl->ev_end, pl->stream));
-    GDP_HIP(hipMemcpyAsync(pl->lane.back, pl->dbase + pl->off_abort, pl->back_bytes, hipMemcpyDeviceToHost,
-                           pl->stream));
     pl->wait_back = false;
     pl->flow_clean = false;
     bool exports = false;   // gdp_plan_fetch then reads the cost buffers: they are cleaned before the next run instead
@@ -2332,8 +2335,8 @@ int run_finish(gdp_plan *pl, int32_t mode, gdp_timing *t)
         fused_turn_give();
     }
     GDP_HIP(waited);
-    pl->h_out = reinterpret_cast<const GdpDevOut *>(pl->lane.back + (pl->off_out - pl->off_abort));
-    pl->h_res = reinterpret_cast<const int32_t *>(pl->lane.back + (pl->off_res - pl->off_abort));
+    pl->h_out = reinterpret_cast<const GdpDevOut *>(pl->lane.back + pl->off_out);
+    pl->h_res = reinterpret_cast<const int32_t *>(pl->lane.back + pl->off_res);
     // the flag is cleared and written by fused launches only
     const int32_t aborted = (pl->fused || pl->run_flow) ? *reinterpret_cast<const int32_t *>(pl->lane.back) : 0;
     if (aborted) {
@@ -2468,7 +2471,7 @@ int fetch(gdp_plan *pl, gdp_result *const *r)
 {
     if (!pl->ran) return fail(GDP_E_BADARG, "gdp_plan_fetch before gdp_plan_run");
     GDP_HIP(hipSetDevice(pl->device));
-    // the run has already copied the outputs into the plan's page-locked buffer
+    // the run has already written the outputs into the plan's page-locked buffer
     const GdpDevInst *d_insts = reinterpret_cast<const GdpDevInst *>(pl->dbase + pl->off_insts);
     for (int i = 0; i < pl->n; ++i) {
         const HostInst &h = pl->inst[(size_t)i];

@@ -226,8 +226,11 @@ hipError_t gdp_launch_zero_pass(bool marks, const GdpDevInst *insts, const GdpDe
                                 int n_inst, int max_V, int layer, hipStream_t stream);
 // argmin over the last layer's row + backtrack, one wavefront per key (marks: through the stored
 // argmin table; otherwise recomputed from the cost buffers of all layers).
+// flag_out: null, or where the int at `flag` goes as well.
 hipError_t gdp_launch_epilogue(bool marks, const GdpDevInst *insts, const GdpDevKey *keys, int n_key, GdpDevOut *out,
-                               int32_t *res, hipStream_t stream);
+                               int32_t *res, const int32_t *flag, int32_t *flag_out, hipStream_t stream);
+// Copies page-locked host memory to the device (both aligned to 16 bytes, whole 16 bytes).
+hipError_t gdp_launch_pull(const void *from, void *to, size_t bytes, hipStream_t stream);
 // Debug exports in the reference's layouts.
 hipError_t gdp_launch_export_f(const GdpDevInst *inst, double *f_out, int V, int S, hipStream_t stream);
 // layers layer0 .. layer0+layers-1 of the argmin table (layers <= 65535): bytes with GDP_EXPORT_NONE for -1 where S <= 255, else

@@ -1287,12 +1287,17 @@ __device__ __forceinline__ int wave_argmin_by_lane(double val)
 // the one cell per layer that lies on its path, with the arithmetic and the tie-break of the
 // relaxation (csrc/dp_core.cpp:67-73: ascending source strategies, strict '<', so the lowest index
 // among equal candidates, and index 0 when all are +inf).
+// `out` and `res` may be page-locked host memory, then `flag` (whether a bounded wait ran out) goes there as well and the run needs
+// no copy behind it, which began 12 us after this kernel (L = 4, S = 6).  The strategies of 64 layers are collected in the lanes
+// and written at once: one write over the bus instead of 64.
 template <bool MARKS>
 __global__ __launch_bounds__(64) void gdp_epilogue_kernel(const GdpDevInst *__restrict__ insts,
                                                           const GdpDevKey *__restrict__ keys,
-                                                          GdpDevOut *__restrict__ out,
-                                                          int32_t *__restrict__ res)
+                                                          int n_key, GdpDevOut *__restrict__ out,
+                                                          int32_t *__restrict__ res, const int32_t *flag, int32_t *flag_out)
 {
+    if (flag_out && blockIdx.x == 0 && threadIdx.x == 0) *flag_out = *flag;
+    if ((int)blockIdx.x >= n_key) return;
     const GdpDevKey *K = keys + blockIdx.x;
     const GdpDevInst *I = insts + uload(&K->inst);
     const int lane = threadIdx.x;
@@ -1329,7 +1334,12 @@ __global__ __launch_bounds__(64) void gdp_epilogue_kernel(const GdpDevInst *__re
     const int32_t *mem = uload(&I->mem);
     int32_t *path = res + uload(&K->res_off);
     int64_t v = v0;
-    if (lane == 0) path[L - 1] = idx;
+    int collected = 0;   // lane j: the strategy of layer j of the 64 that are under way
+    auto step_to = [&](int layer) {
+        if (lane == (layer & 63)) collected = idx;
+        if ((layer & 63) == 0 && layer + lane < L) path[layer + lane] = collected;
+    };
+    step_to(L - 1);
     if constexpr (MARKS) {
         const uint8_t *M = uload(&I->M);
         const int64_t ldm = uload(&I->ldm);
@@ -1339,7 +1349,7 @@ __global__ __launch_bounds__(64) void gdp_epilogue_kernel(const GdpDevInst *__re
             if (v < 0) break;  // cannot happen on a finite path; keeps a damaged table from being indexed
             idx = __builtin_amdgcn_readfirstlane((int)M[((int64_t)i * S + cur) * ldm + v]);
             if (idx >= S) { v = -1; break; }
-            if (lane == 0) path[i - 1] = idx;
+            step_to(i - 1);
         }
     } else {
         const int SP = uload(&I->SP);
@@ -1399,7 +1409,7 @@ __global__ __launch_bounds__(64) void gdp_epilogue_kernel(const GdpDevInst *__re
                 }
                 idx = wave_argmin_by_lane(bv);
                 if (idx >= S) { v = -1; break; }
-                if (lane == 0) path[i - 1] = idx;
+                step_to(i - 1);
                 if (--b < 0) {
                     b = nbuf - 1;
                     src = H + (int64_t)b * hstride;
@@ -1429,7 +1439,7 @@ __global__ __launch_bounds__(64) void gdp_epilogue_kernel(const GdpDevInst *__re
             wave_argmin(bv, bi);
             idx = __builtin_amdgcn_readfirstlane(bi);
             if (idx >= S) { v = -1; break; }
-            if (lane == 0) path[i - 1] = idx;
+            step_to(i - 1);
         }
     }
     if (lane != 0) return;
@@ -1684,13 +1694,37 @@ hipError_t gdp_launch_zero_pass(bool marks, const GdpDevInst *insts, const GdpDe
 }
 
 hipError_t gdp_launch_epilogue(bool marks, const GdpDevInst *insts, const GdpDevKey *keys, int n_key, GdpDevOut *out,
-                               int32_t *res, hipStream_t stream)
+                               int32_t *res, const int32_t *flag, int32_t *flag_out, hipStream_t stream)
 {
-    if (n_key <= 0) return hipSuccess;
+    if (n_key <= 0 && !flag_out) return hipSuccess;
+    const dim3 grid((unsigned)(n_key > 0 ? n_key : 1));
     if (marks)
-        hipLaunchKernelGGL(gdp_epilogue_kernel<true>, dim3((unsigned)n_key), dim3(64), 0, stream, insts, keys, out, res);
+        hipLaunchKernelGGL(gdp_epilogue_kernel<true>, grid, dim3(64), 0, stream, insts, keys, n_key, out, res, flag, flag_out);
     else
-        hipLaunchKernelGGL(gdp_epilogue_kernel<false>, dim3((unsigned)n_key), dim3(64), 0, stream, insts, keys, out, res);
+        hipLaunchKernelGGL(gdp_epilogue_kernel<false>, grid, dim3(64), 0, stream, insts, keys, n_key, out, res, flag, flag_out);
+    return hipGetLastError();
+}
+
+// 16 bytes a thread and step, 4 steps a thread, all asked for before the first is written.
+__global__ __launch_bounds__(256) void gdp_pull_kernel(const uint4 *__restrict__ from, uint4 *__restrict__ to, int64_t n)
+{
+    constexpr int STEPS = 4;
+    const int64_t at = (int64_t)blockIdx.x * 256 * STEPS + threadIdx.x;
+    uint4 x[STEPS];
+#pragma unroll
+    for (int j = 0; j < STEPS; ++j)
+        if (at + 256 * j < n) x[j] = from[at + 256 * j];
+#pragma unroll
+    for (int j = 0; j < STEPS; ++j)
+        if (at + 256 * j < n) to[at + 256 * j] = x[j];
+}
+
+hipError_t gdp_launch_pull(const void *from, void *to, size_t bytes, hipStream_t stream)
+{
+    const int64_t n = (int64_t)(bytes / 16);
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(gdp_pull_kernel, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, stream, static_cast<const uint4 *>(from),
+                       static_cast<uint4 *>(to), n);
     return hipGetLastError();
 }
 

@@ -413,7 +413,7 @@ int solve_dense(const gdp_problem *p, const Layout &y, unsigned char *base, bool
     if (e == hipSuccess)
         e = gdp_launch_epilogue(true, d_inst, reinterpret_cast<const GdpDevKey *>(base + y.off_keys), y.n_key,
                                 reinterpret_cast<GdpDevOut *>(base + y.off_out),
-                                reinterpret_cast<int32_t *>(base + y.off_res), stream);
+                                reinterpret_cast<int32_t *>(base + y.off_res), nullptr, nullptr, stream);
     if (e != hipSuccess) {
         (void)hipDeviceSynchronize();
         return gdp_fail_hip(e, "gdp_solve_static: kernel launch");
