@@ -131,3 +131,24 @@ def test_calls_around_the_rule(kind, L, S, V, n_keys, zeros, labels, monkeypatch
     s = _lib.batch_stats_end()
     assert (s.executed < 0.01 * s.relaxations) == labels
     _same(prob, x, V, f"{kind} {L} {S} {V} {n_keys} {zeros}")
+
+
+# One key with many labels among keys with few: what it is given up for takes the others along, and the next run starts from bounds of its own
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 6])
+def test_a_key_that_is_given_up_takes_the_others_along(n, monkeypatch):
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    L, S, V = 24, 64, 12000
+    xs = []
+    for k in range(n):
+        rng = np.random.Generator(np.random.PCG64([L, S, k]))
+        per = V // L
+        mem = np.repeat(rng.integers(per // 4, 3 * per, size=(1, S)), L, 0).astype(np.int32)
+        intra = 40.0 * per / mem
+        intra[:, ::3] += 1e3                       # a third is dominated
+        xs.append((mem, intra, np.repeat(rng.uniform(0, 0.05, size=(1, S, S)), L, 0), [0, V // 2, 6 * V // 10], [0.0, 0.5, 1.0]))
+    probs = [_lib.Problem(x[0], x[1], x[2], V, x[3], x[4]) for x in xs]
+    for _ in range(3):
+        _lib.solve_batch(probs)
+    for x, prob in zip(xs, probs):
+        _same(prob, x, V, f"{n}")
