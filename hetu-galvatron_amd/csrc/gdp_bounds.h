@@ -86,7 +86,7 @@ __attribute__((visibility("hidden"))) double undominated(const gdp_problem *q);
 __attribute__((visibility("hidden"))) int key_multipliers(const gdp_problem *q);
 // The multipliers of an instance: 0 and a geometric series around (range of times) / (range of memory costs).
 __attribute__((visibility("hidden"))) void multipliers(const gdp_problem *q, int n_lam, double *lam);
-// What a set of launches begins with: head_bytes (a multiple of 16) are copied from `head`, if there is one, page-locked host memory,
+// What is laid out before a set of launches: head_bytes (a multiple of 16) are copied from `head`, if there is one, page-locked host memory,
 // to head_to, and the matrices are laid out.
 struct Inputs {
     const GdpBoundMatrix *matrices;
@@ -95,10 +95,11 @@ struct Inputs {
     void *head_to;
     size_t head_bytes;
 };
-// Lays out the inputs, runs the passes of all multipliers, finds the upper bounds and marks what stays.
+__attribute__((visibility("hidden"))) hipError_t lay_out(const Inputs &in, int max_S, hipStream_t stream);
+// Runs the passes of all multipliers, finds the upper bounds and marks what stays.
 // max_rows: layers times (strategies / 64, rounded up).  held: most layers have the matrix of the one before.
 __attribute__((visibility("hidden")))
-hipError_t launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_rows, int max_S, int max_K, bool held, const Inputs &in,
+hipError_t launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_rows, int max_S, int max_K, bool held,
                   hipStream_t stream);
 // The DP over what stays, after it: a workgroup per instance (gdp_frontier.hip), or per key of each (gdp_key_labels.hip; up to
 // GDP_KEY_LABELS_MAX_L layers).

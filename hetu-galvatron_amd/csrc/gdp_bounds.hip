@@ -532,14 +532,17 @@ void bounds::multipliers(const gdp_problem *q, int n_lam, double *lam)
     for (int i = 1; i < n_lam; ++i) lam[i] = base * exp2(-6.0 + 12.0 * (i - 1) / (n_lam - 2));
 }
 
-hipError_t bounds::launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_rows, int max_S, int max_K, bool held, const Inputs &in,
-                          hipStream_t stream)
+hipError_t bounds::lay_out(const Inputs &in, int max_S, hipStream_t stream)
 {
     const int bands = (max_S + 15) / 16, n_head = in.head ? (int)(in.head_bytes / 16) : 0;
+    if (n_head == 0 && in.n_matrices == 0) return hipSuccess;
     gdp_bound_transpose_kernel<<<(unsigned)((n_head + HEAD - 1) / HEAD + in.n_matrices * bands), 256, 0, stream>>>(
         in.matrices, bands, static_cast<const uint4v *>(in.head), static_cast<uint4v *>(in.head_to), n_head);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    return hipGetLastError();
+}
+
+hipError_t bounds::launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS, int max_rows, int max_S, int max_K, bool held, hipStream_t stream)
+{
     const dim3 grid(2u * (unsigned)n_lam, (unsigned)n);
     const unsigned threads = 64u * (unsigned)((max_S + TARGETS - 1) / TARGETS);
 #define GDP_PASS(E, AHEAD) \
@@ -554,7 +557,7 @@ hipError_t bounds::launch(const GdpBoundInst *inst, int n, int n_lam, int max_LS
     else GDP_PASS(22, 2);
     else GDP_PASS(32, 2);
 #undef GDP_PASS
-    e = hipGetLastError();
+    hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     gdp_bound_upper_kernel<<<dim3((unsigned)((max_LS + 255) / 256), (unsigned)max_K, (unsigned)n), 256, 0, stream>>>(inst, n_lam);
     e = hipGetLastError();

@@ -316,8 +316,8 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     hipError_t e = hipMemcpy(base, g_stage, up_bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) return gdp_fail_hip(e, "gdp_solve_static: upload");
     const GdpBoundInst *inst = reinterpret_cast<const GdpBoundInst *>(base + off_inst);
-    e = bounds::launch(inst, 1, (int)NL, (int)LS, L * ((S + 63) / 64), S, K, changes * 4 <= L,
-                       {reinterpret_cast<const GdpBoundMatrix *>(base + off_matrices), T, nullptr, nullptr, 0}, stream);
+    e = bounds::lay_out({reinterpret_cast<const GdpBoundMatrix *>(base + off_matrices), T, nullptr, nullptr, 0}, S, stream);
+    if (e == hipSuccess) e = bounds::launch(inst, 1, (int)NL, (int)LS, L * ((S + 63) / 64), S, K, changes * 4 <= L, stream);
     if (e == hipSuccess) e = alone ? bounds::launch_key_labels(inst, 1, K, stream) : bounds::launch_labels(inst, 1, K, stream);
     if (e != hipSuccess) {
         (void)hipDeviceSynchronize();
