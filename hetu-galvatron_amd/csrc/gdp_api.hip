@@ -2738,7 +2738,9 @@ static double undominated(int32_t n, const gdp_problem *const *p)
 }
 
 // Whether the keys of these instances have a workgroup each (gdp_key_labels.hip).  Not where next to no strategy is dominated by another:
-// labels are many either way then, and most such calls are given up as they were.
+// labels are many either way then, and most such calls are given up as they were.  120 random calls, ms by a workgroup for each instance / for
+// each key: up to 0.3 of the strategies undominated 9.6 / 7.6, to 0.7 9.3 / 8.6, none more than 1.10 times as slow; to 0.8 0.51 / 0.55, the worst
+// 1.26; above, 8 calls, 0.75 / 0.67, too few to move the line.
 static bool keys_alone(int32_t n, const gdp_problem *const *p)
 {
     for (int32_t i = 0; i < n; ++i)

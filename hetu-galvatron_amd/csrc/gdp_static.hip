@@ -230,7 +230,7 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     if (!bounds::has_form(&form) || !(magnitude < 1e100)) return GDP_OK;
     // The bounds take 35 us at least (L = 5: S = 8 58 us whole, 60 with them, S = 11 79 and 60).
     if (dense_ns(L, S) < 36e3 && !forced) return GDP_OK;
-    // (calls of more keys go the way they went, and end it where they did)
+    // (calls of more keys go the way they went, and end it where they did; 21 of 5 keys would take 0.84 of their time with a workgroup each)
     constexpr int MOST_ALONE = 4;
     int64_t budget[GDP_BOUND_MAX_KEY], least = 0;
     for (int l = 0; l < L; ++l) {
@@ -307,7 +307,10 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     b.out = reinterpret_cast<GdpFrontierOut *>(base + off_out);
     b.res = reinterpret_cast<int32_t *>(base + off_res);
     b.magnitude = magnitude;
-    b.limit = dense_ns(L, S);
+    // Half of it for keys with a workgroup each, whose account (gdp_key_labels.hip) says what is ahead but not the bounds behind them: 75 random
+    // calls 10.2 ms dense or by the shared workgroup, 8.5 with the whole, 2 of them more than 5 % slower than before, the worst 1.58; 8.3
+    // with half, none; 8.7 with 0.3, one 2.5.
+    b.limit = (alone ? 0.5 : 1.0) * dense_ns(L, S);
     b.L = L; b.V = p->V; b.S = S; b.K = K; b.T = T;
     b.n_hist = b.n_hist_turns = (int32_t)labels;
     b.n_lam = (int32_t)NL;
