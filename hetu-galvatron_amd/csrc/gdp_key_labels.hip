@@ -81,7 +81,7 @@ struct Shared {
 static_assert(sizeof(Shared) <= 160 * 1024, "LDS of a compute unit");
 
 constexpr unsigned long long GIVEN_UP = ~0ull - 1;   // (as a bound it would be a NaN)
-enum { GOES_ON = 0, TOO_MANY = 4, NONE_LEFT = 3, UNSORTED = -1 };
+enum { GOES_ON = 0, NO_PATH = 1, TOO_MANY_KEPT = 2, NONE_LEFT = 3, TOO_MANY = 4, UNSORTED = -1 };
 
 __device__ __forceinline__ int prefix_sum(int x)
 {
@@ -170,7 +170,8 @@ __global__ __launch_bounds__(THREADS) void gdp_key_labels_kernel(const GdpBoundI
         }
     };
     const int64_t B = GLOBAL(const __attribute__((address_space(1))) int64_t *, I.budget)[own_key];
-    const unsigned long long known = GLOBAL(const __attribute__((address_space(1))) unsigned long long *, I.ub)[own_key];
+    unsigned long long known = 0;   // the workgroup of another key may write here by now: one wave asks, and decides for all
+    if (t < 64) known = __hip_atomic_load(I.ub + own_key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     const int best = GLOBAL(gint, I.best)[own_key];
     const __attribute__((address_space(1))) int4v *marks = GLOBAL(const __attribute__((address_space(1))) int4v *, I.marks) + (size_t)own_key * L;
     int4v mark = marks[min(lane, L - 1)];
@@ -184,12 +185,7 @@ __global__ __launch_bounds__(THREADS) void gdp_key_labels_kernel(const GdpBoundI
         }
         return;
     }
-    if (known >= GIVEN_UP) {
-        give_up(known == GIVEN_UP ? TOO_MANY : 1);
-        return;
-    }
     const int32_t budget = uniform((int32_t)B);
-    double ub = uniform(gdp_unordered(known));
     const gdouble Q = GLOBAL(gdouble, I.Q), intra = GLOBAL(gdouble, I.intra), inter = GLOBAL(gdouble, I.inter_f);
     const gint Q_mem = GLOBAL(gint, I.Q_mem), mem = GLOBAL(gint, I.mem);
     const glabel hist = GLOBAL(glabel, I.hist) + (size_t)own_key * I.n_hist;
@@ -234,7 +230,8 @@ __global__ __launch_bounds__(THREADS) void gdp_key_labels_kernel(const GdpBoundI
         const bool any_bad = lanes_where(bad) != 0;   // (of all lanes)
         if (lane == 0) {
             sh.layer[L] = make_int4(0, sum, turns, 0);
-            sh.lost = any_bad || sum > ALL_KEPT;
+            sh.lost = known == ~0ull ? NO_PATH : known == GIVEN_UP ? TOO_MANY : any_bad || sum > ALL_KEPT ? TOO_MANY_KEPT : GOES_ON;
+            sh.ub = gdp_unordered(known);
         }
     }
     for (int e = t; e < 2 * (LABELS + KEY_PAD); e += THREADS) sh.f.key[0][e] = INFINITY;   // both
@@ -247,10 +244,11 @@ __global__ __launch_bounds__(THREADS) void gdp_key_labels_kernel(const GdpBoundI
         sh.single[0] = 0.0;
     }
     __syncthreads();
-    if (sh.lost) {
-        give_up(2);
+    if (const int why = uniform(sh.lost); why != GOES_ON) {
+        give_up(why);
         return;
     }
+    double ub = uniform(sh.ub);
     for (int l = wave; l < L; l += WAVES) {
         const int4 m = sh.mark[l];
         const unsigned long long lo = (unsigned long long)(uint32_t)uniform(m.y) << 32 | (uint32_t)uniform(m.x),
