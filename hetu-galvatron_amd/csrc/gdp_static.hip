@@ -217,6 +217,60 @@ double work(const gdp_problem *p) { return (double)p->L * p->V * (double)p->S * 
 // V = 18405, S = 26 13.3, V = 12602, S = 41 20).
 double dense_ns(int L, int S) { return L * (4000.0 + 350.0 * S); }
 
+// Where the arrays of the bounds lie from the start of `scratch`.  alone: with a workgroup for every key.
+struct BoundLayout {
+    int NL;
+    size_t off_inst, off_matrices, off_mem, off_intra, off_inter, off_index, off_lam, off_budget, off_other_time, up_bytes;   // what is uploaded
+    size_t off_out, off_res, back_bytes;   // what is copied back
+    size_t off_keep, off_marks, off_inter_f, off_inter_t, off_P, off_Q, off_P_mem, off_Q_mem, off_end, off_best, off_ub, off_hist, off_turns, off_hist_mem,
+        off_hist_intra, bytes, labels;
+};
+
+BoundLayout bound_layout(const gdp_problem *p, int matrices, int multipliers, bool alone)
+{
+    const size_t L = (size_t)p->L, K = (size_t)p->n_key, T = (size_t)matrices, NL = (size_t)multipliers, LS = L * p->S, SS = (size_t)p->S * p->S,
+                 keys = alone ? K : 1;
+    BoundLayout y;
+    y.NL = multipliers;
+    y.labels = L * (alone ? GDP_KEY_LABELS : GDP_FRONTIER_LABELS);
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        const size_t o = off;
+        off = align_up(off + bytes, 256);
+        return o;
+    };
+    y.off_inst = take(sizeof(GdpBoundInst));
+    y.off_matrices = take(sizeof(GdpBoundMatrix) * T);
+    y.off_mem = take(4 * LS);
+    y.off_intra = take(8 * LS);
+    y.off_inter = take(8 * SS * T);
+    y.off_index = take(4 * L);
+    y.off_lam = take(8 * NL);
+    y.off_budget = take(8 * K);
+    y.off_other_time = take(8 * K);
+    y.up_bytes = off;
+    y.off_out = take(sizeof(GdpFrontierOut));
+    y.off_res = take(4 * K * L);
+    y.back_bytes = off - y.up_bytes;
+    y.off_keep = take(LS);
+    y.off_marks = take(16 * K * L);
+    y.off_inter_f = take(8 * SS * T);
+    y.off_inter_t = take(8 * SS * T);
+    y.off_P = take(8 * LS * NL);
+    y.off_Q = take(8 * LS * NL);
+    y.off_P_mem = take(4 * LS * NL);
+    y.off_Q_mem = take(4 * LS * NL);
+    y.off_end = take(8 * NL);
+    y.off_best = take(4 * K);
+    y.off_ub = take(8 * K);
+    y.off_hist = take(sizeof(GdpFrontierLabel) * y.labels * keys);
+    y.off_turns = take(alone ? 0 : 8 * y.labels);
+    y.off_hist_mem = take(4 * GDP_FRONTIER_KEPT);
+    y.off_hist_intra = take(8 * GDP_FRONTIER_KEPT);
+    y.bytes = off;
+    return y;
+}
+
 // Solves p by bounds if that is possible: *done.  Initial costs are zeros.  *marked: that is left to the dense recurrence, and
 // g_keep says which strategies can matter to it.
 int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base, gdp_result *r, bool *done, bool *marked)
@@ -247,96 +301,84 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     }
     if (!any) return GDP_OK;
     const bool alone = K <= MOST_ALONE && L <= GDP_KEY_LABELS_MAX_L && bounds::undominated(p) <= GDP_KEY_LABELS_MOST;
-    const size_t NL = alone ? (size_t)bounds::key_multipliers(p) : 64, keys = alone ? (size_t)K : 1;
-    const size_t LS = (size_t)L * S, SS = (size_t)S * S, labels = (size_t)L * (alone ? GDP_KEY_LABELS : GDP_FRONTIER_LABELS);
-    size_t off = 0;
-    auto take = [&](size_t bytes) {
-        const size_t o = off;
-        off = align_up(off + bytes, 256);
-        return o;
-    };
-    const size_t off_inst = take(sizeof(GdpBoundInst)), off_matrices = take(sizeof(GdpBoundMatrix) * (size_t)T), off_mem = take(4 * LS),
-                 off_intra = take(8 * LS), off_inter = take(8 * SS * (size_t)T), off_index = take(4 * (size_t)L),
-                 off_lam = take(8 * NL), off_budget = take(8 * (size_t)K), off_other_time = take(8 * (size_t)K), up_bytes = off,
-                 off_out = take(sizeof(GdpFrontierOut)), off_res = take(4 * (size_t)K * L), back_bytes = off - up_bytes,
-                 off_keep = take(LS), off_marks = take(16 * (size_t)K * L), off_inter_f = take(8 * SS * (size_t)T), off_inter_t = take(8 * SS * (size_t)T),
-                 off_P = take(8 * LS * NL), off_Q = take(8 * LS * NL), off_P_mem = take(4 * LS * NL), off_Q_mem = take(4 * LS * NL),
-                 off_end = take(8 * NL), off_best = take(4 * (size_t)K), off_ub = take(8 * (size_t)K),
-                 off_hist = take(sizeof(GdpFrontierLabel) * labels * keys), off_turns = take(alone ? 0 : 8 * labels),
-                 off_hist_mem = take(4 * GDP_FRONTIER_KEPT), off_hist_intra = take(8 * GDP_FRONTIER_KEPT);
-    if (off > (size_t)GDP_STATIC_SCRATCH_BYTES || up_bytes > STAGE_BYTES || back_bytes > STAGE_BYTES) return GDP_OK;
-    memcpy(g_stage + off_mem, p->mem, 4 * LS);
-    memcpy(g_stage + off_intra, p->intra, 8 * LS);
-    memcpy(g_stage + off_inter, p->inter, 8 * SS * (size_t)T);
-    int32_t *index = reinterpret_cast<int32_t *>(g_stage + off_index);
+    BoundLayout y = bound_layout(p, T, alone ? bounds::key_multipliers(p) : 64, alone);
+    // Where 128 multipliers do not fit into the workspace 64 do (L = 128, S = 128, 4 keys, 40 matrices: 70.6 MB, 45.4;
+    // dense 4.9 ms, by these bounds 1.15).
+    if (y.bytes > (size_t)GDP_STATIC_SCRATCH_BYTES && y.NL > 64) y = bound_layout(p, T, 64, alone);
+    if (y.bytes > (size_t)GDP_STATIC_SCRATCH_BYTES || y.up_bytes > STAGE_BYTES || y.back_bytes > STAGE_BYTES) return GDP_OK;
+    const size_t NL = (size_t)y.NL, LS = (size_t)L * S, SS = (size_t)S * S;
+    memcpy(g_stage + y.off_mem, p->mem, 4 * LS);
+    memcpy(g_stage + y.off_intra, p->intra, 8 * LS);
+    memcpy(g_stage + y.off_inter, p->inter, 8 * SS * (size_t)T);
+    int32_t *index = reinterpret_cast<int32_t *>(g_stage + y.off_index);
     int changes = 0;
     for (int l = 0; l < L; ++l) {
         index[l] = p->inter_index ? p->inter_index[l] : l;
         changes += l > 0 && index[l] != index[l - 1];
     }
-    bounds::multipliers(p, (int)NL, reinterpret_cast<double *>(g_stage + off_lam));
-    memcpy(g_stage + off_budget, budget, 8 * (size_t)K);
-    memcpy(g_stage + off_other_time, p->other_time, 8 * (size_t)K);
-    GdpBoundMatrix *matrices = reinterpret_cast<GdpBoundMatrix *>(g_stage + off_matrices);
+    bounds::multipliers(p, (int)NL, reinterpret_cast<double *>(g_stage + y.off_lam));
+    memcpy(g_stage + y.off_budget, budget, 8 * (size_t)K);
+    memcpy(g_stage + y.off_other_time, p->other_time, 8 * (size_t)K);
+    GdpBoundMatrix *matrices = reinterpret_cast<GdpBoundMatrix *>(g_stage + y.off_matrices);
     for (int t = 0; t < T; ++t)
-        matrices[t] = {reinterpret_cast<const double *>(base + off_inter) + SS * (size_t)t, reinterpret_cast<double *>(base + off_inter_f) + SS * (size_t)t,
-                       reinterpret_cast<double *>(base + off_inter_t) + SS * (size_t)t, S, 0};
+        matrices[t] = {reinterpret_cast<const double *>(base + y.off_inter) + SS * (size_t)t, reinterpret_cast<double *>(base + y.off_inter_f) + SS * (size_t)t,
+                       reinterpret_cast<double *>(base + y.off_inter_t) + SS * (size_t)t, S, 0};
     GdpBoundInst b;
     memset(&b, 0, sizeof b);
-    b.mem = reinterpret_cast<const int32_t *>(base + off_mem);
-    b.intra = reinterpret_cast<const double *>(base + off_intra);
-    b.inter_f = reinterpret_cast<double *>(base + off_inter_f);
-    b.inter_t = reinterpret_cast<double *>(base + off_inter_t);
-    b.index = reinterpret_cast<const int32_t *>(base + off_index);
-    b.lam = reinterpret_cast<const double *>(base + off_lam);
-    b.budget = reinterpret_cast<const int64_t *>(base + off_budget);
-    b.P = reinterpret_cast<double *>(base + off_P);
-    b.Q = reinterpret_cast<double *>(base + off_Q);
-    b.P_mem = reinterpret_cast<uint32_t *>(base + off_P_mem);
-    b.Q_mem = reinterpret_cast<uint32_t *>(base + off_Q_mem);
-    b.end = reinterpret_cast<double *>(base + off_end);
-    b.ub = reinterpret_cast<unsigned long long *>(base + off_ub);
-    b.best = reinterpret_cast<int32_t *>(base + off_best);
-    b.keep = base + off_keep;
-    b.marks = reinterpret_cast<unsigned long long *>(base + off_marks);
-    b.other_time = reinterpret_cast<const double *>(base + off_other_time);
-    b.hist = reinterpret_cast<GdpFrontierLabel *>(base + off_hist);
-    b.hist_mem = reinterpret_cast<int32_t *>(base + off_hist_mem);
-    b.hist_turns = reinterpret_cast<double *>(base + off_turns);
-    b.hist_intra = reinterpret_cast<double *>(base + off_hist_intra);
-    b.out = reinterpret_cast<GdpFrontierOut *>(base + off_out);
-    b.res = reinterpret_cast<int32_t *>(base + off_res);
+    b.mem = reinterpret_cast<const int32_t *>(base + y.off_mem);
+    b.intra = reinterpret_cast<const double *>(base + y.off_intra);
+    b.inter_f = reinterpret_cast<double *>(base + y.off_inter_f);
+    b.inter_t = reinterpret_cast<double *>(base + y.off_inter_t);
+    b.index = reinterpret_cast<const int32_t *>(base + y.off_index);
+    b.lam = reinterpret_cast<const double *>(base + y.off_lam);
+    b.budget = reinterpret_cast<const int64_t *>(base + y.off_budget);
+    b.P = reinterpret_cast<double *>(base + y.off_P);
+    b.Q = reinterpret_cast<double *>(base + y.off_Q);
+    b.P_mem = reinterpret_cast<uint32_t *>(base + y.off_P_mem);
+    b.Q_mem = reinterpret_cast<uint32_t *>(base + y.off_Q_mem);
+    b.end = reinterpret_cast<double *>(base + y.off_end);
+    b.ub = reinterpret_cast<unsigned long long *>(base + y.off_ub);
+    b.best = reinterpret_cast<int32_t *>(base + y.off_best);
+    b.keep = base + y.off_keep;
+    b.marks = reinterpret_cast<unsigned long long *>(base + y.off_marks);
+    b.other_time = reinterpret_cast<const double *>(base + y.off_other_time);
+    b.hist = reinterpret_cast<GdpFrontierLabel *>(base + y.off_hist);
+    b.hist_mem = reinterpret_cast<int32_t *>(base + y.off_hist_mem);
+    b.hist_turns = reinterpret_cast<double *>(base + y.off_turns);
+    b.hist_intra = reinterpret_cast<double *>(base + y.off_hist_intra);
+    b.out = reinterpret_cast<GdpFrontierOut *>(base + y.off_out);
+    b.res = reinterpret_cast<int32_t *>(base + y.off_res);
     b.magnitude = magnitude;
     // Half of it for keys with a workgroup each, whose account (gdp_key_labels.hip) says what is ahead but not the bounds behind them: 75 random
     // calls 10.2 ms dense or by the shared workgroup, 8.5 with the whole, 2 of them more than 5 % slower than before, the worst 1.58; 8.3
     // with half, none; 8.7 with 0.3, one 2.5.
     b.limit = (alone ? 0.5 : 1.0) * dense_ns(L, S);
     b.L = L; b.V = p->V; b.S = S; b.K = K; b.T = T;
-    b.n_hist = b.n_hist_turns = (int32_t)labels;
+    b.n_hist = b.n_hist_turns = (int32_t)y.labels;
     b.n_lam = (int32_t)NL;
-    memcpy(g_stage + off_inst, &b, sizeof b);
+    memcpy(g_stage + y.off_inst, &b, sizeof b);
     hipStream_t stream = nullptr;
-    hipError_t e = hipMemcpy(base, g_stage, up_bytes, hipMemcpyHostToDevice);
+    hipError_t e = hipMemcpy(base, g_stage, y.up_bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) return gdp_fail_hip(e, "gdp_solve_static: upload");
-    const GdpBoundInst *inst = reinterpret_cast<const GdpBoundInst *>(base + off_inst);
-    e = bounds::lay_out({reinterpret_cast<const GdpBoundMatrix *>(base + off_matrices), T, nullptr, nullptr, 0}, S, stream);
+    const GdpBoundInst *inst = reinterpret_cast<const GdpBoundInst *>(base + y.off_inst);
+    e = bounds::lay_out({reinterpret_cast<const GdpBoundMatrix *>(base + y.off_matrices), T, nullptr, nullptr, 0}, S, stream);
     if (e == hipSuccess) e = bounds::launch(inst, 1, (int)NL, (int)LS, L * ((S + 63) / 64), S, K, changes * 4 <= L, stream);
     if (e == hipSuccess) e = alone ? bounds::launch_key_labels(inst, 1, K, stream) : bounds::launch_labels(inst, 1, K, stream);
     if (e != hipSuccess) {
         (void)hipDeviceSynchronize();
         return gdp_fail_hip(e, "gdp_solve_static: kernel launch");
     }
-    e = hipMemcpy(g_stage, base + off_out, back_bytes, hipMemcpyDeviceToHost);   // after the kernels, in stream order
+    e = hipMemcpy(g_stage, base + y.off_out, y.back_bytes, hipMemcpyDeviceToHost);   // after the kernels, in stream order
     if (e != hipSuccess) return gdp_fail_hip(e, "gdp_solve_static: download");
     const GdpFrontierOut *out = reinterpret_cast<const GdpFrontierOut *>(g_stage);
     const int status = bounds::status_of(*out, K);
     if (status > 1) {
-        e = hipMemcpy(g_keep, base + off_keep, LS, hipMemcpyDeviceToHost);
+        e = hipMemcpy(g_keep, base + y.off_keep, LS, hipMemcpyDeviceToHost);
         if (e != hipSuccess) return gdp_fail_hip(e, "gdp_solve_static: download");
         *marked = true;
     }
     if (status != 0) return GDP_OK;
-    const int32_t *res = reinterpret_cast<const int32_t *>(g_stage + (off_res - off_out));
+    const int32_t *res = reinterpret_cast<const int32_t *>(g_stage + (y.off_res - y.off_out));
     for (int k = 0; k < K; ++k) {
         r->total[k] = out->total[k];
         r->remaining[k] = out->remaining[k];

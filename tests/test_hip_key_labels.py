@@ -152,3 +152,19 @@ def test_a_key_that_is_given_up_takes_the_others_along(n, monkeypatch):
         _lib.solve_batch(probs)
     for x, prob in zip(xs, probs):
         _same(prob, x, V, f"{n}")
+
+
+# The bounds of 128 multipliers beside 4 keys need 70.6 of 67.1 MB
+@pytest.mark.gpu
+def test_static_calls_whose_bounds_need_most_of_the_workspace(monkeypatch):
+    monkeypatch.delenv("GALVATRON_DP_REDUCE", raising=False)
+    monkeypatch.delenv("GALVATRON_DP_SKIP", raising=False)
+    L, S, V, T = 128, 128, 2000, 40
+    mem, intra, inter, om, ot = _instance(L, S, V, "each", 4)
+    index = (np.arange(L) * T // L).astype(np.int32)
+    prob = _lib.Problem(mem, intra, inter[:T], V, om, ot, inter_index=index)
+    _lib.batch_stats_begin()
+    _lib.solve_static(prob)
+    s = _lib.batch_stats_end()
+    _same(prob, (mem, intra, np.ascontiguousarray(inter[:T][index]), om, ot), V, "static")
+    assert s.executed < 0.01 * s.relaxations
