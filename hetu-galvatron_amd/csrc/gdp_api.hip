@@ -2917,6 +2917,25 @@ static size_t bound_bytes(const gdp_problem *q, const HostInst &h, int n_lam, bo
            (alone ? 16 * K * L * GDP_KEY_LABELS : 24 * L * GDP_FRONTIER_LABELS + 12 * GDP_FRONTIER_KEPT) + 256 * ARRAYS;
 }
 
+// How the bounds of some instances may be laid out: with a workgroup for every key or one for all of them.
+struct BoundForm {
+    bool alone;
+    int n_lam;
+};
+
+// Those that come into question, each for where there is no room for the one before it.  only: the instance, if it is one.  L = 80, S = 64,
+// V = 4000, 1 key: 24 MB with 128 multipliers and 339 us, 16 with 64 and 337; whole 705.  L = 40, S = 64, V = 60000, 8 keys: 10 MB and
+// 215 us, 9 with one workgroup for all keys and 314; whole 1340.
+static std::vector<BoundForm> bound_forms(bool alone, size_t instances, const gdp_problem *only)
+{
+    const int n_lam = bound_multipliers(instances), most = alone && only ? bounds::key_multipliers(only) : n_lam;
+    std::vector<BoundForm> forms;
+    if (most > n_lam) forms.push_back({true, most});
+    if (alone) forms.push_back({true, n_lam});
+    forms.push_back({false, n_lam});
+    return forms;
+}
+
 // What the bounds of a slice work with; given back on every way out, the stream idle.
 struct BoundLease {
     int device = 0;
@@ -3117,12 +3136,13 @@ hipError_t BoundSlice::enqueue(char *dev, hipStream_t stream) const
 
 // Bounds of the instances of one slice in one set of launches, and behind them the DP over what stays.  out[i]: the
 // results of instance i; the smaller instance that is left of it where its labels are too many; empty where it is to be
-// solved whole.  The calling thread looks through initial costs while the device works.
-static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &magnitude, BoundEntry *es, int m, int n_lam,
-                        bool alone, bool forced, InitialScan &scan, std::vector<std::unique_ptr<Reduced>> &out)
+// solved whole.  *room: false where the device has not the memory, then all are empty.  The calling thread looks through initial costs
+// while the device works.
+static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &magnitude, BoundEntry *es, int m, const BoundForm &form,
+                        bool forced, InitialScan &scan, std::vector<std::unique_ptr<Reduced>> &out, bool *room)
 {
     BoundSlice slice;
-    slice.lay_out(p, es, m, n_lam, alone);
+    slice.lay_out(p, es, m, form.n_lam, form.alone);
     // What stays as smaller instances takes about half of what the whole ones take (labels_pay, 1.2 10^13 relaxations a second),
     // and a second layout and round trip.  ms in all, whole / with limit_ns as it is / with this one:
     //   245 calls above the rule's line, L = 3 to 128, S = 5 to 88  156 / 82.0 / 77.1 (more than 10 % slower than whole: 9, now 2)
@@ -3135,10 +3155,15 @@ static int reduce_slice(const gdp_problem *const *p, const std::vector<double> &
     // A device or a host that is out of memory solves the instances whole, in the parts that fit; what else may be
     // wrong with the device is found, and reported, there.
     BoundLease lease;
-    if (hipGetDevice(&lease.device) != hipSuccess || lane_take(lease.device, slice.back_bytes, slice.up_bytes, &lease.lane) != hipSuccess ||
-        arena_take(lease.device, slice.bytes, &lease.dev, &lease.dev_bytes) != hipSuccess) {
+    *room = true;
+    if (hipGetDevice(&lease.device) != hipSuccess || lane_take(lease.device, slice.back_bytes, slice.up_bytes, &lease.lane) != hipSuccess) {
+        (void)hipGetLastError();
+        return GDP_OK;
+    }
+    if (arena_take(lease.device, slice.bytes, &lease.dev, &lease.dev_bytes) != hipSuccess) {
         (void)hipGetLastError();
         lease.dev = nullptr;
+        *room = false;
         return GDP_OK;
     }
     const Lane &lane = lease.lane;
@@ -3234,18 +3259,24 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
         BoundEntry e;
         if (bound_entry(p[i], i, magnitude[(size_t)i], e)) es.push_back(std::move(e));
     }
-    const bool alone = keys_alone(n, p);
-    const int n_lam = alone && es.size() == 1 ? bounds::key_multipliers(p[es[0].orig]) : bound_multipliers(es.size());
+    const std::vector<BoundForm> forms = bound_forms(keys_alone(n, p), es.size(), es.size() == 1 ? p[es[0].orig] : nullptr);
     int rc = GDP_OK;
     for (size_t begin = 0; begin < es.size() && rc == GDP_OK;) {
-        size_t end = begin, bytes = 0;
-        while (end < es.size() && end - begin < 65535) {
-            const size_t b = bound_bytes(p[es[end].orig], es[end].h, n_lam, alone);
-            if (bytes + b > limit) break;
-            bytes += b;
-            ++end;
+        size_t end = begin, tried = SIZE_MAX;
+        bool room = false;
+        for (size_t f = 0; f < forms.size() && !room && rc == GDP_OK; ++f) {
+            size_t to = begin, bytes = 0;
+            while (to < es.size() && to - begin < 65535) {
+                const size_t b = bound_bytes(p[es[to].orig], es[to].h, forms[f].n_lam, forms[f].alone);
+                if (bytes + b > limit) break;
+                bytes += b;
+                ++to;
+            }
+            if (to == begin || bytes >= tried) continue;
+            end = to;
+            tried = bytes;
+            rc = reduce_slice(p, magnitude, es.data() + begin, (int)(end - begin), forms[f], forced, scan, out, &room);
         }
-        if (end > begin) rc = reduce_slice(p, magnitude, es.data() + begin, (int)(end - begin), n_lam, alone, forced, scan, out);
         begin = std::max(end, begin + 1);
     }
     return rc;
@@ -3266,34 +3297,31 @@ static void take_bounds(int32_t n, const gdp_problem *const *p, const std::vecto
     bool forced = false;
     if (plan->keep_marks || !bounds::allowed(&forced) || (!forced && !bounds_pay(n, p))) return;
     std::unique_ptr<PlanBounds> b(new PlanBounds());
-    size_t bytes = 0;
     const size_t limit = std::min(arena_budget(), REDUCE_MAX_BYTES);
     for (int i = 0; i < n; ++i) {
         BoundEntry e;
         if (!bound_entry(p[i], i, magnitude[(size_t)i], e)) return;
         b->es.push_back(std::move(e));
     }
-    bool alone = keys_alone(n, p);
-    int n_lam = 0;
-    auto fits = [&](bool key_alone) {
-        n_lam = key_alone && n == 1 ? bounds::key_multipliers(p[0]) : bound_multipliers((size_t)n);
-        bytes = 0;
-        for (int i = 0; i < n; ++i) bytes += bound_bytes(p[i], b->es[(size_t)i].h, n_lam, key_alone);
-        return bytes <= limit;
-    };
-    if (alone && !fits(true)) alone = false;
-    if (!fits(alone)) return;
-    b->slice.lay_out(p, b->es.data(), n, n_lam, alone);
+    b->lease.device = plan->device;
+    for (const BoundForm &form : bound_forms(keys_alone(n, p), (size_t)n, n == 1 ? p[0] : nullptr)) {
+        size_t bytes = 0;
+        for (int i = 0; i < n; ++i) bytes += bound_bytes(p[i], b->es[(size_t)i].h, form.n_lam, form.alone);
+        if (bytes > limit) continue;
+        b->slice = BoundSlice();
+        b->slice.lay_out(p, b->es.data(), n, form.n_lam, form.alone);
+        if (arena_take(plan->device, b->slice.bytes, &b->lease.dev, &b->lease.dev_bytes) == hipSuccess) break;
+        (void)hipGetLastError();
+        b->lease.dev = nullptr;
+    }
+    if (!b->lease.dev) return;
+    if (lane_take(plan->device, b->slice.back_bytes, 0, &b->lease.lane) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
     plan->bounds_out.resize((size_t)plan->n_key_total);
     plan->bounds_res.resize(plan->n_res_total);
     std::vector<char> up(b->slice.up_bytes);
-    b->lease.device = plan->device;
-    if (lane_take(plan->device, b->slice.back_bytes, 0, &b->lease.lane) != hipSuccess ||
-        arena_take(plan->device, b->slice.bytes, &b->lease.dev, &b->lease.dev_bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        b->lease.dev = nullptr;
-        return;
-    }
     b->slice.fill(p, magnitude, up.data(), b->lease.dev, b->lease.dev, b->lease.lane.back);
     if (hipMemcpyAsync(b->lease.dev, up.data(), b->slice.up_bytes, hipMemcpyHostToDevice, plan->stream) != hipSuccess ||
         b->slice.bring(nullptr, b->lease.dev, plan->stream) != hipSuccess ||

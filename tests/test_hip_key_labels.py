@@ -168,3 +168,39 @@ def test_static_calls_whose_bounds_need_most_of_the_workspace(monkeypatch):
     s = _lib.batch_stats_end()
     _same(prob, (mem, intra, np.ascontiguousarray(inter[:T][index]), om, ot), V, "static")
     assert s.executed < 0.01 * s.relaxations
+
+
+# Less memory than a workgroup for every key works in, of the device or allowed for, and not less than one for all of them (8 keys), or
+# than 64 multipliers (1 key, 24 MB with 128)
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,S,n_keys,limit_mb", [(40, 20, 8, 3), (80, 64, 1, 20)])
+@pytest.mark.parametrize("limit", ["GALVATRON_DP_ARENA_MB", "GALVATRON_DP_DEVICE_LIMIT_MB"])
+def test_calls_and_batches_whose_bounds_have_little_room(L, S, n_keys, limit_mb, limit, monkeypatch):
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    monkeypatch.setenv(limit, str(limit_mb))
+    _lib.cache_trim()
+    V = 4000
+    for many in (1, 2):
+        xs = [_instance(L, S, V + i, "each", n_keys) for i in range(many)]
+        probs = [_lib.Problem(x[0], x[1], x[2], V, x[3], x[4]) for x in xs]
+        if many > 1 and limit == "GALVATRON_DP_DEVICE_LIMIT_MB":
+            monkeypatch.setenv(limit, str(many * limit_mb))   # (a batch whose bounds are not to be had in one piece is solved whole)
+        _lib.batch_stats_begin()
+        _lib.solve_batch(probs)
+        s = _lib.batch_stats_end()
+        assert s.executed < 0.01 * s.relaxations
+        for x, prob in zip(xs, probs):
+            _same(prob, x, V, f"{many} {limit}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,S,n_keys,limit_mb", [(40, 20, 8, 3), (80, 64, 1, 20)])
+def test_plans_whose_bounds_have_little_room(L, S, n_keys, limit_mb, monkeypatch):
+    monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
+    monkeypatch.setenv("GALVATRON_DP_ARENA_MB", str(limit_mb))
+    V, x = 2000, _instance(L, S, 2000, "each", n_keys)
+    prob = _lib.Problem(x[0], x[1], x[2], V, x[3], x[4])
+    with _lib.Plan([prob]) as plan:
+        assert plan.run().relax_launches == 0
+        plan.fetch()
+    _same(prob, x, V, "plan")
