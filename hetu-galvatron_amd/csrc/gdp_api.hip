@@ -2724,28 +2724,43 @@ static int bound_multipliers(size_t instances) { return instances <= 32 ? 64 : 3
 
 // Share of the strategies that no other one dominates: most others go.  From one layer each of at most 8 instances (batches of 2 to
 // 1000, share of the relaxations left: random costs 0.15 on average and 0.06; costs where memory is traded for time 0.44 and 0.40).
-static double undominated(int32_t n, const gdp_problem *const *p)
-{
-    constexpr int32_t LOOKED_AT = 8;
-    if (n == 1) return bounds::undominated(p[0]);
-    double share = 0;
-    const int32_t m = std::min(n, LOOKED_AT);
-    for (int32_t k = 0; k < m; ++k) {
-        const gdp_problem *q = p[(int64_t)n * k / m];
-        share += bounds::undominated(q, q->L / 2);
+// Asked for by several rules of a call, looked at once (4 layers of S = 64 are sorted in 14 us when they are new; L = 16, S = 88 234 -> 227 us).
+class Undominated {
+public:
+    Undominated(int32_t n, const gdp_problem *const *p) : n_(n), p_(p) {}
+    double share()
+    {
+        if (share_ < 0) share_ = look();
+        return share_;
     }
-    return share / m;
-}
+
+private:
+    double look() const
+    {
+        constexpr int32_t LOOKED_AT = 8;
+        if (n_ == 1) return bounds::undominated(p_[0]);
+        double share = 0;
+        const int32_t m = std::min(n_, LOOKED_AT);
+        for (int32_t k = 0; k < m; ++k) {
+            const gdp_problem *q = p_[(int64_t)n_ * k / m];
+            share += bounds::undominated(q, q->L / 2);
+        }
+        return share / m;
+    }
+    int32_t n_;
+    const gdp_problem *const *p_;
+    double share_ = -1;
+};
 
 // Whether the keys of these instances have a workgroup each (gdp_key_labels.hip).  Not where next to no strategy is dominated by another:
 // labels are many either way then, and most such calls are given up as they were.  120 random calls, ms by a workgroup for each instance / for
 // each key: up to 0.3 of the strategies undominated 9.6 / 7.6, to 0.7 9.3 / 8.6, none more than 1.10 times as slow; to 0.8 0.51 / 0.55, the worst
 // 1.26; above, 8 calls, 0.75 / 0.67, too few to move the line.
-static bool keys_alone(int32_t n, const gdp_problem *const *p)
+static bool keys_alone(int32_t n, const gdp_problem *const *p, Undominated &undominated)
 {
     for (int32_t i = 0; i < n; ++i)
         if (p[i]->L > GDP_KEY_LABELS_MAX_L) return false;
-    return undominated(n, p) <= GDP_KEY_LABELS_MOST;
+    return undominated.share() <= GDP_KEY_LABELS_MOST;
 }
 
 // Whether the bounds of a batch or plan are worth their time (GALVATRON_DP_REDUCE=1 takes them for every instance that has the
@@ -2770,7 +2785,7 @@ static bool keys_alone(int32_t n, const gdp_problem *const *p)
 //   32 x L = 14, S = 40  V = 8000 * 1.33 / 0.71, not taken 1.08 / 1.13    V = 30000 * 2.79 / 0.71; 2.61 / 1.29
 //   64 x L = 28, S = 64, V = 8000 * 24.6 / 18.5; 9.3 / 10.6
 // (Single calls are taken earlier where labels_pay says so.)
-static bool bounds_pay(int32_t n, const gdp_problem *const *p)
+static bool bounds_pay(int32_t n, const gdp_problem *const *p, Undominated &undominated)
 {
     constexpr double RATE = 1e13, FLOOR = 0.2e-3, STEP = 5e-6, STEP_16 = 25e-6, BUSY = 1.5e-6, BUSY_16 = 13e-6, ENTRY = 3e-9, GROUP = 0.1e-3;
     double work = 0, layers = 0, entries = 0;
@@ -2793,7 +2808,7 @@ static bool bounds_pay(int32_t n, const gdp_problem *const *p)
     if (save < FLOOR) return false;
     const bool wide = max_S > 88;
     const double passes = layers * 2 * bound_multipliers((size_t)n) / 1024;
-    return save >= std::max(max_L * (wide ? STEP_16 : STEP), passes * (wide ? BUSY_16 : BUSY)) + (n > 1 ? entries * ENTRY * undominated(n, p) : 0.0);
+    return save >= std::max(max_L * (wide ? STEP_16 : STEP), passes * (wide ? BUSY_16 : BUSY)) + (n > 1 ? entries * ENTRY * undominated.share() : 0.0);
 }
 
 // The same for a call of one instance, below bounds_pay's floor.  The launch schemes take 60 us + L * (2.8 + 0.085 S) us and their
@@ -2809,14 +2824,14 @@ static bool bounds_pay(int32_t n, const gdp_problem *const *p)
 // The workgroup that all keys share is slower; for its sake layers of their own with 80 at most, however many keys there are, and
 // everything from 5e7 a layer, as in bounds_pay.  Initial costs are looked through while the device works, at 45 GB/s of
 // memory: where that takes longer than the launch schemes nothing is gained.
-static bool labels_pay(const gdp_problem *q, size_t scanned)
+static bool labels_pay(const gdp_problem *q, size_t scanned, Undominated &undominated)
 {
     constexpr double LEAST = 3e7, MANY = 3e8, MANY_LAYER = 5e7, FEW = 80, FEW_OF_KEYS = 500, EACH = 0.5e-6;
     if (!bounds::has_form(q) || q->S > 88) return false;
     const double work = (double)q->L * q->V * q->S * q->S, chain = q->L * (2.8e-6 + 0.085e-6 * q->S), whole = chain + work / 1.2e13;
     if (work < LEAST || (double)scanned / 45e9 > whole) return false;
     if (work >= std::max(MANY, MANY_LAYER * q->L)) return true;
-    const double share = bounds::undominated(q), expected = share * q->S * q->L;
+    const double share = undominated.share(), expected = share * q->S * q->L;
     if (q->L <= GDP_KEY_LABELS_MAX_L && share <= GDP_KEY_LABELS_MOST && expected * q->n_key <= std::max(FEW_OF_KEYS, whole / EACH)) return true;
     int alike = 0;
     for (int l = 1; l < q->L; ++l) {
@@ -2923,12 +2938,14 @@ struct BoundForm {
     int n_lam;
 };
 
-// Those that come into question, each for where there is no room for the one before it.  only: the instance, if it is one.  L = 80, S = 64,
-// V = 4000, 1 key: 24 MB with 128 multipliers and 339 us, 16 with 64 and 337; whole 705.  L = 40, S = 64, V = 60000, 8 keys: 10 MB and
-// 215 us, 9 with one workgroup for all keys and 314; whole 1340.
-static std::vector<BoundForm> bound_forms(bool alone, size_t instances, const gdp_problem *only)
+// Those that come into question for what of n instances has bounds, each for where there is no room for the one before it.  first: one of
+// those.  L = 80, S = 64, V = 4000, 1 key: 24 MB with 128 multipliers and 339 us, 16 with 64 and 337; whole 705.  L = 40, S = 64, V = 60000,
+// 8 keys: 10 MB and 215 us, 9 with one workgroup for all keys and 314; whole 1340.
+static std::vector<BoundForm> bound_forms(int32_t n, const gdp_problem *const *p, size_t instances, const gdp_problem *first, Undominated &undominated)
 {
-    const int n_lam = bound_multipliers(instances), most = alone && only ? bounds::key_multipliers(only) : n_lam;
+    const bool alone = keys_alone(n, p, undominated);
+    const int n_lam = bound_multipliers(instances),
+              most = alone && instances == 1 ? bounds::key_multipliers(first, n == 1 ? undominated.share() : bounds::undominated(first)) : n_lam;
     std::vector<BoundForm> forms;
     if (most > n_lam) forms.push_back({true, most});
     if (alone) forms.push_back({true, n_lam});
@@ -3251,7 +3268,9 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
 {
     bool forced = false;
     if (!bounds::allowed(&forced)) return GDP_OK;
-    if (!forced && !(bounds_pay(n, p) && InitialScan::device_bound(dense_work(n, p), scan.alone())) && !(n == 1 && labels_pay(p[0], scan.alone())))
+    Undominated undominated(n, p);
+    if (!forced && !(bounds_pay(n, p, undominated) && InitialScan::device_bound(dense_work(n, p), scan.alone())) &&
+        !(n == 1 && labels_pay(p[0], scan.alone(), undominated)))
         return GDP_OK;
 
     std::vector<BoundEntry> es;
@@ -3259,7 +3278,8 @@ static int reduce_batch(int32_t n, const gdp_problem *const *p, const std::vecto
         BoundEntry e;
         if (bound_entry(p[i], i, magnitude[(size_t)i], e)) es.push_back(std::move(e));
     }
-    const std::vector<BoundForm> forms = bound_forms(keys_alone(n, p), es.size(), es.size() == 1 ? p[es[0].orig] : nullptr);
+    if (es.empty()) return GDP_OK;
+    const std::vector<BoundForm> forms = bound_forms(n, p, es.size(), p[es[0].orig], undominated);
     int rc = GDP_OK;
     for (size_t begin = 0; begin < es.size() && rc == GDP_OK;) {
         size_t end = begin, tried = SIZE_MAX;
@@ -3295,7 +3315,8 @@ static void give_back(PlanBounds *b) { delete b; }
 static void take_bounds(int32_t n, const gdp_problem *const *p, const std::vector<double> &magnitude, gdp_plan *plan)
 {
     bool forced = false;
-    if (plan->keep_marks || !bounds::allowed(&forced) || (!forced && !bounds_pay(n, p))) return;
+    Undominated undominated(n, p);
+    if (plan->keep_marks || !bounds::allowed(&forced) || (!forced && !bounds_pay(n, p, undominated))) return;
     std::unique_ptr<PlanBounds> b(new PlanBounds());
     const size_t limit = std::min(arena_budget(), REDUCE_MAX_BYTES);
     for (int i = 0; i < n; ++i) {
@@ -3304,7 +3325,7 @@ static void take_bounds(int32_t n, const gdp_problem *const *p, const std::vecto
         b->es.push_back(std::move(e));
     }
     b->lease.device = plan->device;
-    for (const BoundForm &form : bound_forms(keys_alone(n, p), (size_t)n, n == 1 ? p[0] : nullptr)) {
+    for (const BoundForm &form : bound_forms(n, p, (size_t)n, p[0], undominated)) {
         size_t bytes = 0;
         for (int i = 0; i < n; ++i) bytes += bound_bytes(p[i], b->es[(size_t)i].h, form.n_lam, form.alone);
         if (bytes > limit) continue;

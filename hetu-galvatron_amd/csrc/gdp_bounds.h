@@ -82,8 +82,8 @@ __attribute__((visibility("hidden"))) bool allowed(bool *forced);
 // Share of the strategies of a layer, and on average of 4 layers, that are cheaper in time than every one that needs no more memory.
 __attribute__((visibility("hidden"))) double undominated(const gdp_problem *q, int layer);
 __attribute__((visibility("hidden"))) double undominated(const gdp_problem *q);
-// How many multipliers an instance takes whose keys have a workgroup each.
-__attribute__((visibility("hidden"))) int key_multipliers(const gdp_problem *q);
+// How many multipliers an instance takes whose keys have a workgroup each, given the share of its undominated strategies.
+__attribute__((visibility("hidden"))) int key_multipliers(const gdp_problem *q, double undominated);
 // The multipliers of an instance: 0 and a geometric series around (range of times) / (range of memory costs).
 __attribute__((visibility("hidden"))) void multipliers(const gdp_problem *q, int n_lam, double *lam);
 // What is laid out before a set of launches: head_bytes (a multiple of 16) are copied from `head`, if there is one, page-locked host memory,

@@ -511,10 +511,10 @@ double bounds::undominated(const gdp_problem *q)
 // Twice as many leave fewer labels where those are many, which the undominated strategies of all layers tell best, and take 3 us longer (a
 // wave of passes on every compute unit instead of every second).  110 calls of random inputs, us with 64 / 128: up to 250 of these strategies 64 is as fast or up to
 // 4 us faster; above 183 / 172, 190 / 153, 228 / 140, 235 / 219, 351 / 269, 1263 / 424.  256 are slower in nearly all.
-int bounds::key_multipliers(const gdp_problem *q)
+int bounds::key_multipliers(const gdp_problem *q, double undominated)
 {
     constexpr double MANY = 250;
-    return undominated(q) * q->S * q->L <= MANY ? 64 : GDP_BOUND_MAX_LAM;
+    return undominated * q->S * q->L <= MANY ? 64 : GDP_BOUND_MAX_LAM;
 }
 
 void bounds::multipliers(const gdp_problem *q, int n_lam, double *lam)

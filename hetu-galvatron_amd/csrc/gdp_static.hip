@@ -300,8 +300,10 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
         any = any || b >= least;
     }
     if (!any) return GDP_OK;
-    const bool alone = K <= MOST_ALONE && L <= GDP_KEY_LABELS_MAX_L && bounds::undominated(p) <= GDP_KEY_LABELS_MOST;
-    BoundLayout y = bound_layout(p, T, alone ? bounds::key_multipliers(p) : 64, alone);
+    const bool may = K <= MOST_ALONE && L <= GDP_KEY_LABELS_MAX_L;
+    const double undominated = may ? bounds::undominated(p) : 1.0;
+    const bool alone = may && undominated <= GDP_KEY_LABELS_MOST;
+    BoundLayout y = bound_layout(p, T, alone ? bounds::key_multipliers(p, undominated) : 64, alone);
     // Where 128 multipliers do not fit into the workspace 64 do (L = 128, S = 128, 4 keys, 40 matrices: 70.6 MB, 45.4;
     // dense 4.9 ms, by these bounds 1.15).
     if (y.bytes > (size_t)GDP_STATIC_SCRATCH_BYTES && y.NL > 64) y = bound_layout(p, T, 64, alone);
