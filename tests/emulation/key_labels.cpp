@@ -51,6 +51,15 @@ size_t instance_size() { return sizeof(GdpBoundInst); }
 size_t result_size() { return sizeof(GdpFrontierOut); }
 int labels_a_layer() { return GDP_KEY_LABELS; }
 
+// Of the workgroup that ran last: the most labels of a layer, strategies that stay, transitions between them.
+void seen(int layers, int *most_labels, int *kept, int *transitions)
+{
+    const Shared &sh = *reinterpret_cast<const Shared *>(emulated_lds);
+    *most_labels = *std::max_element(sh.labels_of, sh.labels_of + layers);
+    *kept = sh.layer[layers].y;
+    *transitions = sh.layer[layers].z;
+}
+
 // The workgroup of a key.  order: waves first to last, last to first, or (seed) at random.  From the moment on that `told_at` waves
 // have begun another key of the instance says in this one's upper bound that it has been given up (-1: none does).  0: all
 // threads have ended; 1: some never would; 2: a wave had left when others met at a barrier.

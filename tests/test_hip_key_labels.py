@@ -47,14 +47,24 @@ def _same(prob, x, V, tag):
             assert [int(v) for v in prob.res[k]] == [int(v) for v in res[k]], f"{tag} key {k}"
 
 
+def _executed(probs, solve=_lib.solve_batch):
+    """The share of the relaxations that are looked at: next to none where labels solve them."""
+    _lib.batch_stats_begin()
+    solve(probs)
+    s = _lib.batch_stats_end()
+    return s.executed / s.relaxations
+
+
 # Layers: 2, around 64 (a word of marks), 128, and one more, which has a workgroup per instance; strategies: 2, around 64 (the
-# words of a layer's marks), 128; labels: one (runs of layers with one strategy), up to 16, 32 and 64 beside each other, more (trade)
+# words of a layer's marks), 128; labels: one (runs of layers with one strategy), up to 16, 32 and 64 beside each other, more, in buckets
+# (trade: 485 with L = 16, 1200 with L = 24 are given up); layers whose strategies and transitions do not fit into LDS at a time (ties, L = 50:
+# 472 and 4406).  How many there are, and that the kernel solves them, is checked on the CPU as well (test_key_labels_on_cpu.py).
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind,L,S,V", [("each", 2, 2, 60), ("each", 9, 12, 3000), ("each", 20, 63, 4000), ("each", 20, 64, 4000), ("each", 20, 65, 4000),
                                         ("each", 6, 128, 2000), ("each", 63, 7, 6000), ("each", 64, 7, 6000), ("each", 65, 7, 6000), ("runs", 127, 6, 4000),
                                         ("runs", 128, 6, 4000), ("runs", 129, 6, 4000), ("runs", 40, 20, 5000), ("alike", 30, 24, 5000),
                                         ("trade", 8, 9, 2000), ("trade", 12, 24, 5000), ("trade", 16, 33, 9000), ("trade", 24, 48, 12000), ("ties", 12, 24, 300),
-                                        ("ties", 30, 40, 900), ("ties", 70, 9, 1000)])
+                                        ("ties", 30, 40, 900), ("ties", 70, 9, 1000), ("ties", 50, 40, 1500)])
 @pytest.mark.parametrize("n_keys", [1, 3, 4, 8])
 def test_calls_against_the_oracle(kind, L, S, V, n_keys, monkeypatch):
     monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
@@ -64,8 +74,9 @@ def test_calls_against_the_oracle(kind, L, S, V, n_keys, monkeypatch):
     _lib.solve_batch([prob])
     s = _lib.batch_stats_end()
     _same(prob, x, V, f"{kind} {L} {S} {V}")
-    if kind in ("each", "runs") and V > 1000:
-        assert s.executed < 0.01 * s.relaxations
+    if V > 60:                                              # (of a small instance labels are no small part)
+        given_up = (kind, L) == ("trade", 24) and n_keys != 3
+        assert (s.executed < 0.01 * s.relaxations) == (not given_up)
 
 
 @pytest.mark.gpu
@@ -75,7 +86,7 @@ def test_batches_of_different_shapes(many, monkeypatch):
     monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
     V, xs = 1500, [_instance(3 + i % 9, 5 + 11 * (i % 7), 1500 + i, ("each", "ties")[i % 2], 1 + i % 6) for i in range(many)]
     probs = [_lib.Problem(x[0], x[1], x[2], V, x[3], x[4]) for x in xs]
-    _lib.solve_batch(probs)
+    assert _executed(probs) < 0.01
     for i, (x, prob) in enumerate(zip(xs, probs)):
         _same(prob, x, V, f"instance {i}")
 
@@ -86,12 +97,12 @@ def test_static_calls_and_plans(kind, L, S, V, n_keys, monkeypatch):
     monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
     x = _instance(L, S, V, kind, n_keys)
     prob = _lib.Problem(x[0], x[1], x[2], V, x[3], x[4])
-    _lib.solve_static(prob)
+    assert _executed(prob, _lib.solve_static) < 0.01
     _same(prob, x, V, f"static {kind}")
     prob.total[:], prob.remaining[:], prob.res[:] = 0, 0, 0
     with _lib.Plan([prob]) as plan:
         for _ in range(2):
-            plan.run()
+            assert plan.run().relax_launches == 0
             plan.fetch()
             _same(prob, x, V, f"plan {kind}")
 
@@ -133,14 +144,15 @@ def test_calls_around_the_rule(kind, L, S, V, n_keys, zeros, labels, monkeypatch
     _same(prob, x, V, f"{kind} {L} {S} {V} {n_keys} {zeros}")
 
 
-# One key with many labels among keys with few: what it is given up for takes the others along, and the next run starts from bounds of its own
+# One key with many labels among keys with few, which by themselves are solved by labels: what it is given up for takes them along, and
+# the next run starts from bounds of its own.  In a batch the other instances go on by labels.
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 6])
 def test_a_key_that_is_given_up_takes_the_others_along(n, monkeypatch):
     monkeypatch.setenv("GALVATRON_DP_REDUCE", "1")
     L, S, V = 24, 64, 12000
     xs = []
-    for k in range(n):
+    for k in (3, 0, 1, 2, 4, 5)[:n]:
         rng = np.random.Generator(np.random.PCG64([L, S, k]))
         per = V // L
         mem = np.repeat(rng.integers(per // 4, 3 * per, size=(1, S)), L, 0).astype(np.int32)
@@ -148,6 +160,10 @@ def test_a_key_that_is_given_up_takes_the_others_along(n, monkeypatch):
         intra[:, ::3] += 1e3                       # a third is dominated
         xs.append((mem, intra, np.repeat(rng.uniform(0, 0.05, size=(1, S, S)), L, 0), [0, V // 2, 6 * V // 10], [0.0, 0.5, 1.0]))
     probs = [_lib.Problem(x[0], x[1], x[2], V, x[3], x[4]) for x in xs]
+    given_up = [_executed([prob]) for prob in probs]
+    assert given_up[0] > 0.01 and max(given_up[1:], default=0) < 1e-3
+    x = xs[0]
+    assert all(_executed([_lib.Problem(x[0], x[1], x[2], V, x[3][k:k + 1], x[4][k:k + 1])]) < 1e-3 for k in (1, 2))
     for _ in range(3):
         _lib.solve_batch(probs)
     for x, prob in zip(xs, probs):

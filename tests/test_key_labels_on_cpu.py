@@ -13,6 +13,7 @@ import pytest
 
 from galvatron_dp import _build
 from oracle import dp_oracle as O
+from test_hip_key_labels import _instance
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CLANG = "/opt/rocm/llvm/bin/clang++"
@@ -52,27 +53,6 @@ def lib(tmp_path_factory):
     lib.run_key.argtypes = [ctypes.c_void_p] + [ctypes.c_int] * 2 + [ctypes.c_uint, ctypes.c_int]
     assert lib.instance_size() == ctypes.sizeof(Instance) and lib.result_size() == ctypes.sizeof(Out)
     return lib
-
-
-def _instance(L, S, V, kind, n_keys):
-    """'each': random costs; 'trade': layers alike in which a third of the strategies trades memory for time, so that labels are many;
-    'ties': small whole numbers; 'runs': one strategy is the best by far in most layers."""
-    rng = np.random.Generator(np.random.PCG64([L, S, V, n_keys]))
-    per, n = max(2, V // L), 1 if kind == "trade" else L
-    mem = rng.integers(max(1, per // 4), 3 * per, size=(n, S)).astype(np.int32)
-    intra, inter = rng.lognormal(2.5, 0.5, size=(n, S)), rng.uniform(0, 5, size=(n, S, S))
-    if kind == "trade":
-        intra, inter = 40.0 * per / mem * rng.uniform(0.98, 1.02, size=mem.shape), inter * 0.05
-        intra[:, rng.permutation(S)[:2 * S // 3]] += 1e3
-    if kind == "ties":
-        mem, intra, inter = (mem // max(1, per // 4) + 1).astype(np.int32), rng.integers(1, 5, size=(n, S)).astype(float), rng.integers(0, 3, size=(n, S, S)).astype(float)
-    if kind == "runs":
-        for l in range(L):
-            if l % 7 != 3:
-                intra[l, rng.integers(S)] = 1e-3
-                mem[l, np.argmin(intra[l])] = 1
-    mem, intra, inter = (np.ascontiguousarray(np.repeat(a, L // n, 0)) for a in (mem, intra, inter))
-    return mem, intra, inter, [int(V * f) for f in (0.1, 0.3, 0.0, 0.999)[:n_keys]], [k / 3 for k in range(n_keys)]
 
 
 class Emulated:
@@ -129,6 +109,11 @@ class Emulated:
         assert self.lib.run_key(ctypes.byref(self.inst), key, order, seed, told_at) == 0
         return self.out.status[key]
 
+    def seen(self):
+        found = [ctypes.c_int() for _ in range(3)]
+        self.lib.seen(self.L, *map(ctypes.byref, found))
+        return [v.value for v in found]
+
     def check(self, key, want):
         total, res, left = want
         assert np.float64(self.out.total[key]).tobytes() == np.float64(total[key]).tobytes()
@@ -141,17 +126,22 @@ def _want(x, V):
     return O.solve(x[0], x[1], x[2], V, dict(zip(keys, x[3])), dict(zip(keys, x[4])))[:3]
 
 
-# One wave's labels and all waves' (trade: up to some hundred, in buckets), runs of layers with one strategy, ties; strategies on both sides
-# of 64, more layers than a word of marks; what does not fit into LDS at a time (4096 strategies, 3072 transitions)
-@pytest.mark.parametrize("kind,L,S,V,n_lam", [("each", 2, 2, 60, 64), ("each", 9, 12, 3000, 64), ("each", 20, 65, 4000, 64), ("runs", 70, 6, 4000, 64),
-                                              ("trade", 12, 24, 5000, 64), ("trade", 16, 33, 9000, 128), ("ties", 30, 40, 900, 64)])
+# One wave's labels and all waves' (trade: hundreds, in buckets), runs of layers with one strategy, ties; strategies on both sides of 64, more
+# layers than a word of marks; more strategies or transitions than LDS holds at a time (448, 3072).  least: labels of a layer, strategies that
+# stay and transitions that some key has.
+@pytest.mark.parametrize("kind,L,S,V,n_lam,least", [("each", 2, 2, 60, 64, (1, 2, 2)), ("each", 9, 12, 3000, 64, (2, 9, 9)), ("each", 20, 65, 4000, 64, (2, 20, 20)),
+                                                    ("runs", 128, 6, 4000, 64, (1, 128, 128)), ("alike", 30, 24, 5000, 64, (33, 200, 1000)),
+                                                    ("trade", 16, 33, 9000, 64, (193, 128, 900)), ("trade", 16, 48, 9000, 128, (65, 64, 300)),
+                                                    ("ties", 30, 40, 900, 64, (9, 300, 3073)), ("ties", 50, 40, 1500, 64, (9, 449, 3073))])
 @pytest.mark.parametrize("order", [0, 1, 2])
-def test_in_any_order_of_waves(lib, kind, L, S, V, n_lam, order):
+def test_in_any_order_of_waves(lib, kind, L, S, V, n_lam, least, order):
     x = _instance(L, S, V, kind, 4)
-    e, want = Emulated(lib, x, V, n_lam), _want(x, V)
+    e, want, seen = Emulated(lib, x, V, n_lam), _want(x, V), []
     for key in range(4):
         assert e.run(key, order) == 0
         e.check(key, want)
+        seen.append(e.seen())
+    assert all(max(most) >= bound for most, bound in zip(zip(*seen), least)), seen
 
 
 # Another key's workgroup writes into the upper bound of this one between its waves: all of them go by the one or by the other
