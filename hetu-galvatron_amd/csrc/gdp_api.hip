@@ -198,7 +198,7 @@ struct Lane {
     int device = 0;
     hipStream_t stream = nullptr;
     hipEvent_t ev_begin = nullptr, ev_end = nullptr;
-    hipEvent_t ev_back = nullptr;  // after the copy of the results (a flow run queues more work behind it)
+    hipEvent_t ev_back = nullptr;  // after the kernel that writes the results (a flow run queues more work behind it)
     hipStream_t side = nullptr;    // second stream: the upload of a small plan's inputs runs beside the kernel that
     hipEvent_t ev_side = nullptr;  // prepares its cost buffers; the event joins it to the main stream
     char *back = nullptr;  // page-locked host memory the results are written into
@@ -688,7 +688,7 @@ static int scan_f0(const gdp_problem *p, bool *live, double *maxabs)
 namespace {
 
 // Looks through the initial costs of a batch for anything but zeros, on threads beside the one that prepares and
-// waits for the device: one thread reads 35 GB/s from memory, so the 184 MB of a call with S = 88, V = 262144 took 4.5 ms
+// waits for the device: the 184 MB of a call with S = 88, V = 262144 took 4.5 ms
 // of its own once the device needed less.  The arrays are cut into pieces that the threads draw from a counter; the
 // caller helps with what is left when it needs the answer, so a thread that could not be had only costs time.  7 threads
 // (GALVATRON_DP_SCAN_THREADS: so many, 0 for none) where the machine has them, from 64 MB on.  Lines that other cores
@@ -700,6 +700,7 @@ namespace {
 //   185 MB 9.6 -> 1.5;  4.6 -> 9.0;  8.6 -> 11.4
 class InitialScan {
 public:
+    static constexpr double READ = 45e9;   // bytes a second that one core reads of an array that fits no cache (1 to 184 MB: 45 to 47; again 350)
     void start(int32_t n, const gdp_problem *const *p, double relaxations)
     {
         for (int i = 0; i < n; ++i) {
@@ -719,10 +720,10 @@ public:
         } catch (const std::system_error &) {   // no thread to be had: the caller does what is left
         }
     }
-    // A caller that looks through `bytes` (35 GB/s) for longer than the whole instances' relaxations keep the device
-    // (10^13 a second) waits for itself: bounds would come on top, and what helpers save is lost when the array is
+    // Whether the whole instances' relaxations (10^13 a second) keep the device for about twice as long as the caller looks through
+    // `bytes`.  One that looks for longer waits for itself: bounds would come on top, and what helpers save is lost when the array is
     // filled again (75 MB: the call 1.60 -> 1.00 ms, filling the next array 3.7 -> 5.3 ms).
-    static bool device_bound(double relaxations, size_t bytes) { return relaxations / 1e13 >= 1.5 * (double)bytes / 35e9; }
+    static bool device_bound(double relaxations, size_t bytes) { return relaxations / 1e13 >= 1.93 * (double)bytes / READ; }
     // true: anything but zeros has been seen already
     bool found() const { return found_.load(std::memory_order_relaxed); }
     // bytes that the calling thread has to look through by itself
@@ -2753,9 +2754,10 @@ private:
 };
 
 // Whether the keys of these instances have a workgroup each (gdp_key_labels.hip).  Not where next to no strategy is dominated by another:
-// labels are many either way then, and most such calls are given up as they were.  120 random calls, ms by a workgroup for each instance / for
-// each key: up to 0.3 of the strategies undominated 9.6 / 7.6, to 0.7 9.3 / 8.6, none more than 1.10 times as slow; to 0.8 0.51 / 0.55, the worst
-// 1.26; above, 8 calls, 0.75 / 0.67, too few to move the line.
+// labels are many either way then, and most such calls are given up as they were.  ms by a workgroup for each instance / for each key, random
+// calls: up to 0.3 of the strategies undominated 9.6 / 7.6, none more than 1.10 times as slow; 40 of 0.5 to 0.6 6.15 / 5.21, 39 to 0.7
+// 5.64 / 5.30 (one 1.32), 55 to 0.8 8.69 / 8.04, none slower; 45 static calls of 0.7 to 0.8 5.59 / 4.62, three 1.07 to 1.09.  Above, 124 calls
+// 16.68 / 16.12, four of them 1.13 to 1.51.
 static bool keys_alone(int32_t n, const gdp_problem *const *p, Undominated &undominated)
 {
     for (int32_t i = 0; i < n; ++i)
@@ -2815,21 +2817,26 @@ static bool bounds_pay(int32_t n, const gdp_problem *const *p, Undominated &undo
 // relaxations; by labels it is a round trip of 50 us and, where each key has its workgroup, what its labels take: which is not known
 // before, what tells it best is how many strategies no other one dominates, over the layers (4 of them are looked at) and keys -- a
 // key whose labels are too many takes the call back to the launch schemes.  500 of them are taken from 3e7 relaxations on, more where
-// that is 0.5 us each at most.  Of 520 random calls (L = 3 to 80, S = 5 to 88, 1 to 5 keys; layers alike, two sorts, their own) 286
-// go by labels then, in 53.5 of 97 ms; 4 of them are more than 1.05 times as slow as whole.  us, whole / by labels (*: taken):
+// that is 0.5 us each at most.
+//   3000 random calls (L = 3 to 80, S = 5 to 88, 1 to 5 keys; layers alike, two sorts, their own): 919 are taken for that, 96 ms of 153 whole.
+// 32 of these are more than 1.1 times as slow as whole (112 / 266 the worst): 24 with layers alike or of two sorts that trade memory for
+// time (of 238), 7 with layers alike and random costs (of 289).  Nor does anything that is known before tell them apart: a line on the
+// strategies, layers, keys, budget or their products that leaves out half of them costs three times what it saves; where 0.59 us each
+// and 18 layers would, ten gain 700 us and eleven lose 570 (73 -> 206 the worst).  Of 209 with L = 30 to 80, S = 5 to 9 19 are slower, 27 ms of 44.
+// us, whole / by labels (*: taken):
 //   layers alike, random costs  * L = 24, S = 22, 1.9e8, 4 keys 157 / 70    L = 8, S = 16, 2.9e7 80 / 62
-//   layers of their own  * L = 32, S = 44, 4e9 668 / 150   * L = 27, S = 16, 5.3e7 155 / 113   * L = 53, S = 5, 4.4e7 219 / 294
+//   layers of their own  * L = 32, S = 44, 4e9 668 / 150   * L = 27, S = 16, 5.3e7 155 / 113   ... that follow a layout * L = 33, S = 8, 5.8e7, 2 keys 165 / 277
 //   layers alike that follow a layout (7 to 20 undominated)  * L = 13, S = 18, 3e7 104 / 96    L = 28, S = 40, 1.3e9 282 / 258 to 440
 //     L = 58, S = 12, 4.8e7 251 / 604    L = 28, S = 80, 6.8e8 354 / 389
 // The workgroup that all keys share is slower; for its sake layers of their own with 80 at most, however many keys there are, and
-// everything from 5e7 a layer, as in bounds_pay.  Initial costs are looked through while the device works, at 45 GB/s of
-// memory: where that takes longer than the launch schemes nothing is gained.
+// everything from 5e7 a layer, as in bounds_pay.  Initial costs are looked through while the device works: where that takes longer than
+// the launch schemes nothing is gained.
 static bool labels_pay(const gdp_problem *q, size_t scanned, Undominated &undominated)
 {
     constexpr double LEAST = 3e7, MANY = 3e8, MANY_LAYER = 5e7, FEW = 80, FEW_OF_KEYS = 500, EACH = 0.5e-6;
     if (!bounds::has_form(q) || q->S > 88) return false;
     const double work = (double)q->L * q->V * q->S * q->S, chain = q->L * (2.8e-6 + 0.085e-6 * q->S), whole = chain + work / 1.2e13;
-    if (work < LEAST || (double)scanned / 45e9 > whole) return false;
+    if (work < LEAST || (double)scanned / InitialScan::READ > whole) return false;
     if (work >= std::max(MANY, MANY_LAYER * q->L)) return true;
     const double share = undominated.share(), expected = share * q->S * q->L;
     if (q->L <= GDP_KEY_LABELS_MAX_L && share <= GDP_KEY_LABELS_MOST && expected * q->n_key <= std::max(FEW_OF_KEYS, whole / EACH)) return true;

@@ -27,7 +27,7 @@ namespace {
 
 static_assert(GDP_BOUND_MAX_S == 128, "two blocks of 64 targets; a strategy in the low 7 bits of a candidate");
 
-// The inputs as the passes read them.  First workgroups of 16 KB of `head` each, which go where they are read from then on; then a
+// The inputs as the passes read them, which takes more than its name says.  First workgroups of 16 KB of `head` each, which go where they are read from then on; then a
 // 16-row band of a matrix each, as it is and transposed, +inf replaced by GDP_BOUND_FAR; LDS turns the band around so that both
 // sides are read and written along rows.
 // Both may lie in page-locked host memory: what the copy engine would bring in a copy of its own, and the first kernel would wait for

@@ -99,7 +99,8 @@ __global__ __launch_bounds__(THREADS) void gdp_frontier_kernel(const GdpBoundIns
     // Keys whose lines, and whose multipliers, are held in registers; the others' are read from LDS.  All where there is room for
     // them: no kernel here may need scratch memory, which the runtime would have to obtain for the launch, and gdp_solve_static
     // promises that nothing is obtained.  (8 keys with all of them held took 252 bytes a lane and longer: L = 80, S = 64 408 -> 377 us;
-    // 5 keys with two lines held 12 to 16 bytes, 522 -> 517 us; since each key has a status of its own one held is too many.)
+    // 5 keys with two lines held 12 to 16 bytes, 522 -> 517 us; since each key has a status of its own one held is too many by 12: 80
+    // static calls of 5 keys 12.06 ms, 12.00 with it.)
     constexpr int LINES_HELD = KEYS <= 4 ? KEYS : KEYS == 5 ? 0 : 2, KEYS_HELD = KEYS <= 5 ? KEYS : 0;
     extern __shared__ __align__(16) char lds[];
     Shared &sh = *reinterpret_cast<Shared *>(lds);

@@ -2,7 +2,7 @@
 //
 // Between the layers of a call lies latency, not work: a wave issues one instruction in 4 clocks at best, one that waits for
 // the one before in 9, one that waits for LDS in 120, a round trip to memory is 2000.  What this kernel does about it:
-// * The labels of a key by itself are a third of those of 4 keys together, and are held against one upper bound, by 8
+// * The labels of a key by itself are fewer than those of 4 keys together, and are held against one upper bound, by 8
 //   multipliers instead of 4, wider apart (L = 80, S = 64, labels per layer: 42 of all keys, 10 of one).
 // * The upper bound becomes better on the way: every label, completed by the cheapest ways on from its strategy under two
 //   multipliers, is a path (30 layers of two kinds that trade memory for time: a third of the labels of the first bound).

@@ -284,7 +284,8 @@ int solve_by_bounds(const gdp_problem *p, double magnitude, unsigned char *base,
     if (!bounds::has_form(&form) || !(magnitude < 1e100)) return GDP_OK;
     // The bounds take 35 us at least (L = 5: S = 8 58 us whole, 60 with them, S = 11 79 and 60).
     if (dense_ns(L, S) < 36e3 && !forced) return GDP_OK;
-    // (calls of more keys go the way they went, and end it where they did; 21 of 5 keys would take 0.84 of their time with a workgroup each)
+    // (Calls of more keys have one workgroup for all of them.  21 of 5 keys would take 0.84 of their time with a workgroup each; that some
+    // of 5, 6 and 8 are given up, or not, where the shared workgroup does is held by tests, no limit of the other kernel.)
     constexpr int MOST_ALONE = 4;
     int64_t budget[GDP_BOUND_MAX_KEY], least = 0;
     for (int l = 0; l < L; ++l) {
